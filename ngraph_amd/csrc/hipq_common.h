@@ -39,6 +39,7 @@ namespace hipq
     // share a block, so callers that run on streams of their own may overlap.  Growing a block waits
     // for its stream and frees the old one.
     int workspace(size_t bytes, hipStream_t stream, void** ptr);
+    bool workspace_holds(size_t bytes); // whether workspace() can hand out that much on this thread at all (see noalloc_begin)
     // a second block per (device, stream) for reductions split over workgroups: zeroed tile counters
     // (kSplitCounterBytes of them) followed by `partial_bytes` for partial sums
     constexpr size_t kSplitCounterBytes = 64 * 1024;
@@ -271,6 +272,9 @@ namespace hipq
                             void* out, hipStream_t s);
 
     int launch_transpose(const void* in, void* out, int64_t N, int64_t R, int64_t Cc, int elem_bytes, hipStream_t s);
+    // the same for bytes, rows of the result padded to `pitch` bytes (a multiple of 16) with *zp
+    int launch_transpose_pad(const void* in, void* out, int64_t N, int64_t R, int64_t Cc, int64_t pitch, const void* zp, int zp_t, hipStream_t s);
+    int launch_pad_rows(const void* in, void* out, int64_t rows, int64_t cols, int64_t pitch, const void* zp, int zp_t, hipStream_t s);
     int launch_pad_channels(const void* in, void* out, int64_t N, int64_t X, int64_t Cc, bool in_ncx, const void* zp, int zp_t, hipStream_t s);
     bool conv_pad_eligible(const ConvGeom& g, ConvGeom* padded);
     int launch_im2col_nxc(const ConvGeom& g, const void* x_nxc, void* a, const void* zp, int zp_t, hipStream_t s);

@@ -102,6 +102,134 @@ namespace hipq
         }
     }
 
+    // 16 bytes from any address whose last byte lies inside the tensor (global loads need no alignment
+    // on this chip); a piece that runs past the tensor's end takes the bytes that exist one by one
+    __device__ __forceinline__ v4t load16_inside(const uint8_t* p, int64_t left)
+    {
+        v4t v = v4t{0, 0, 0, 0};
+        if (left >= 16)
+            __builtin_memcpy(&v, p, 16);
+        else
+        {
+            uint32_t w[4] = {0u, 0u, 0u, 0u};
+            for (int i = 0; i < 16; ++i)
+                if (i < left)
+                    w[i >> 2] |= static_cast<uint32_t>(p[i]) << (8 * (i & 3));
+            v = v4t{static_cast<int>(w[0]), static_cast<int>(w[1]), static_cast<int>(w[2]), static_cast<int>(w[3])};
+        }
+        return v;
+    }
+
+    // in [B][R][Cc] bytes -> out [B][Cc][Rp], Rp >= R a multiple of 16, rows R .. Rp - 1 holding the byte
+    // *zp (0 without one): transpose_bytes_kernel for extents that are multiples of nothing.  What a
+    // convolution over such a channel count or picture size reads in place of its NCX tensor, and the
+    // packed form of a QuantizedDot operand.  The rows of the input start at any address, so its loads
+    // are unaligned 16-byte ones; the output's rows are whole 16-byte pieces.  Bound by HBM where
+    // the tensor is large; u8 [8][90][35 * 29] takes 4.9 us in a kernel trace, most of it launch and latency.
+    __global__ __launch_bounds__(256) void transpose_pad_bytes_kernel(const uint8_t* __restrict__ in, uint8_t* __restrict__ out, int32_t R, int32_t Cc, int32_t Rp, int32_t tiles_c,
+                                                                      int64_t bytes, const void* zp, int32_t zp_t)
+    {
+        __shared__ uint32_t tile[4][64][17];
+        const int wave = threadIdx.x >> 6;
+        const int t = threadIdx.x & 63;
+        const int tc = wave % tiles_c, tr = wave / tiles_c;
+        const int r0 = (static_cast<int>(blockIdx.y) * (4 / tiles_c) + tr) * 64;
+        const int c0 = (static_cast<int>(blockIdx.x) * tiles_c + tc) * 64;
+        const int fill = static_cast<int>((static_cast<uint32_t>(load_zp(zp, zp_t)) & 0xffu) * 0x01010101u);
+        const int64_t plane = static_cast<int64_t>(blockIdx.z) * R * Cc;
+        uint8_t* const dst = out + static_cast<int64_t>(blockIdx.z) * Cc * Rp;
+        {
+            const int rg = t >> 2, cb = t & 3; // rows 4rg..4rg+3, columns 16cb..16cb+15 of the tile
+            v4t l[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+            {
+                const int r = r0 + 4 * rg + i, c = c0 + 16 * cb;
+                const int64_t at = plane + static_cast<int64_t>(r) * Cc + c;
+                l[i] = (r < R && c < Cc) ? load16_inside(in + at, bytes - at) : v4t{fill, fill, fill, fill};
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+            {
+                const uint32_t d[4] = {static_cast<uint32_t>(l[0][q]), static_cast<uint32_t>(l[1][q]), static_cast<uint32_t>(l[2][q]), static_cast<uint32_t>(l[3][q])};
+                uint32_t o[4];
+                transpose4x4(d, o);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    tile[wave][16 * cb + 4 * q + j][rg] = o[j];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int it = 0; it < 4; ++it)
+        {
+            const int col = it * 16 + (t >> 2), q = t & 3;
+            const v4t v = v4t{static_cast<int>(tile[wave][col][4 * q]), static_cast<int>(tile[wave][col][4 * q + 1]), static_cast<int>(tile[wave][col][4 * q + 2]),
+                              static_cast<int>(tile[wave][col][4 * q + 3])};
+            const int c = c0 + col, r = r0 + 16 * q;
+            if (c < Cc && r < Rp)
+                *reinterpret_cast<v4t*>(dst + static_cast<int64_t>(c) * Rp + r) = v;
+        }
+    }
+
+    int launch_transpose_pad(const void* in, void* out, int64_t B, int64_t R, int64_t Cc, int64_t Rp, const void* zp, int zp_t, hipStream_t s)
+    {
+        if (B == 0 || R == 0 || Cc == 0)
+            return HIPQ_OK;
+        HIPQ_REQUIRE(B <= 65535 && Rp % 16 == 0 && Rp >= R && Rp < (1ll << 31) && Cc < (1ll << 31), "extent too large for the padded transpose");
+        const int tiles_c = Cc > 128 ? 4 : (Cc > 64 ? 2 : 1);
+        const int64_t gx = (Cc + 64 * tiles_c - 1) / (64 * tiles_c), gy = (Rp + 64 * (4 / tiles_c) - 1) / (64 * (4 / tiles_c));
+        HIPQ_REQUIRE(gy <= 65535, "extent too large for the transpose grid");
+        dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(gy), static_cast<unsigned>(B));
+        transpose_pad_bytes_kernel<<<grid, 256, 0, s>>>(static_cast<const uint8_t*>(in), static_cast<uint8_t*>(out), static_cast<int32_t>(R), static_cast<int32_t>(Cc), static_cast<int32_t>(Rp),
+                                                       tiles_c, B * R * Cc, zp, zp_t);
+        return check_launch("transpose_pad_bytes");
+    }
+
+    // rows of `cols` bytes -> rows of `pitch` bytes (a multiple of 16), the bytes behind a row's end holding
+    // *zp (0 without one); 16 bytes of the result a lane.  The MFMA kernels read matrices and
+    // channels-last tensors in aligned 16-byte pieces of a row; this is the copy they read when a row is
+    // not a whole number of them.  Bound by HBM where it is large (reads 1, writes pitch / cols).
+    __global__ __launch_bounds__(256) void pad_rows_kernel(const uint8_t* __restrict__ in, v4t* __restrict__ out, int64_t pieces, uint32_t pieces_per_row, int32_t cols, int64_t bytes, const void* zp,
+                                                           int32_t zp_t)
+    {
+        const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+        if (i >= pieces)
+            return;
+        const uint32_t fill = (static_cast<uint32_t>(load_zp(zp, zp_t)) & 0xffu) * 0x01010101u;
+        const uint32_t row = static_cast<uint32_t>(i) / pieces_per_row;
+        const int32_t c = static_cast<int32_t>(static_cast<uint32_t>(i) - row * pieces_per_row) * 16;
+        const int32_t n = cols - c; // bytes of the piece that the row has
+        v4t v = v4t{0, 0, 0, 0};
+        if (n > 0)
+        {
+            const int64_t at = static_cast<int64_t>(row) * cols + c;
+            v = load16_inside(in + at, bytes - at);
+        }
+        if (n < 16)
+        {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+            {
+                const int k = n - 4 * q; // bytes of this dword that the row has
+                const uint32_t keep = k >= 4 ? 0xffffffffu : (k <= 0 ? 0u : (1u << (8 * k)) - 1u);
+                v[q] = static_cast<int>((static_cast<uint32_t>(v[q]) & keep) | (fill & ~keep));
+            }
+        }
+        out[i] = v;
+    }
+
+    int launch_pad_rows(const void* in, void* out, int64_t rows, int64_t cols, int64_t pitch, const void* zp, int zp_t, hipStream_t s)
+    {
+        const int64_t pieces = rows * (pitch / 16);
+        if (pieces == 0)
+            return HIPQ_OK;
+        HIPQ_REQUIRE(pitch % 16 == 0 && pitch >= cols && pieces < (1ll << 31), "matrix too large for the row padding");
+        pad_rows_kernel<<<static_cast<unsigned>((pieces + 255) / 256), 256, 0, s>>>(static_cast<const uint8_t*>(in), static_cast<v4t*>(out), pieces, static_cast<uint32_t>(pitch / 16),
+                                                                                   static_cast<int32_t>(cols), rows * cols, zp, zp_t);
+        return check_launch("pad_rows");
+    }
+
     int launch_transpose(const void* in, void* out, int64_t B, int64_t R, int64_t Cc, int elem_bytes, hipStream_t s)
     {
         if (B == 0 || R == 0 || Cc == 0)
@@ -301,14 +429,18 @@ namespace hipq
         return check_launch("im2col_nxc");
     }
 
-    // Fewer than 16 input channels (a network's first layer): the MFMA kernels take the layer with the
-    // channels padded to 16 -- zero weights in the packed filter, a padded copy of the data
+    // Channel counts that are no multiple of 16 (a network's first layer, widths that were not chosen for
+    // a matrix core): the MFMA kernels take the layer with the channels padded to the next one -- zero
+    // weights in the packed filter, a padded copy of the data.  From 16 channels on only layers of at
+    // least 2^20 multiply-adds, which the direct kernel takes about as long for as the copy's launch.
     bool conv_pad_eligible(const ConvGeom& g, ConvGeom* padded)
     {
-        if (g.C >= 16 || g.C < 1)
+        if (g.C < 1 || g.C % 16 == 0)
             return false;
         ConvGeom p = g;
-        p.C = 16;
+        p.C = static_cast<int64_t>(align_up(static_cast<size_t>(g.C), 16));
+        if (g.C > 16 && g.out_count() < (1ll << 31) && g.out_count() * (g.C * g.taps()) < (1ll << 20))
+            return false;
         p.data_layout = HIPQ_LAYOUT_NXC;
         if (!conv_mfma_eligible(p))
             return false;

@@ -24,7 +24,7 @@ namespace hipq
     }
 
     // Runs the convolution with whatever layouts the descriptor names.
-    static int run_conv(const ConvGeom& g,
+    static int run_conv(const ConvGeom& whole,
                         const void* data,
                         const void* filter,
                         const void* packed,
@@ -36,75 +36,89 @@ namespace hipq
         // the MFMA kernels have no fused-policy instantiation with int32 output (no nGraph op asks for one)
         RowPack rp;
         // a first layer the band kernel takes whole: it reads the [N][C][H][W] bytes itself
-        if (packed && (reinterpret_cast<uintptr_t>(data) & 3) == 0 && conv_rowpack_eligible(g, &rp) && conv_stem_eligible(g, epi, zp, nullptr))
-            return launch_conv_stem(g, data, packed, zp, epi, nullptr, out, s);
-        if (packed && conv_rowpack_eligible(g, &rp))
+        if (packed && (reinterpret_cast<uintptr_t>(data) & 3) == 0 && conv_rowpack_eligible(whole, &rp) && conv_stem_eligible(whole, epi, zp, nullptr))
+            return launch_conv_stem(whole, data, packed, zp, epi, nullptr, out, s);
+        if (packed && conv_rowpack_eligible(whole, &rp))
         {
             // a first layer's three or four channels: a copy with the padding materialised, whose
             // filter rows are single 32-byte runs, then the tile kernel that loads straight into LDS
             void* ws = nullptr;
-            int rc = workspace(align_up(static_cast<size_t>(g.N * rp.Hp * rp.Wp * 4), 256), s, &ws);
+            int rc = workspace(align_up(static_cast<size_t>(whole.N * rp.Hp * rp.Wp * 4), 256), s, &ws);
             if (rc)
                 return rc;
-            rc = launch_stage_rows(g, rp, data, ws, zp.data_zp, zp.data_t, s);
+            rc = launch_stage_rows(whole, rp, data, ws, zp.data_zp, zp.data_t, s);
             if (rc)
                 return rc;
-            return launch_conv_rowpack(g, rp, ws, packed, zp, epi, out, s);
+            return launch_conv_rowpack(whole, rp, ws, packed, zp, epi, out, s);
         }
         ConvGeom padded;
-        if (packed && !conv_mfma_eligible(g) && conv_pad_eligible(g, &padded) && !(epi.mode == EPI_FUSED && g.out_t == HIPQ_I32))
-        {
-            // a first layer's few channels: a 16-channel channels-last copy, then the MFMA kernel
-            void* ws = nullptr;
-            const int64_t in_sp = g.in[1] * g.in[2];
-            int rc = workspace(align_up(static_cast<size_t>(g.N * in_sp * 16), 256), s, &ws);
-            if (rc)
-                return rc;
-            rc = launch_pad_channels(data, ws, g.N, in_sp, g.C, g.data_layout == HIPQ_LAYOUT_NCX, zp.data_zp, zp.data_t, s);
-            if (rc)
-                return rc;
-            return launch_conv_mfma(padded, ws, packed, zp, epi, out, g.out_layout == HIPQ_LAYOUT_NCX && g.K > 1, s);
-        }
-        if (!packed || !conv_mfma_eligible(g) || (epi.mode == EPI_FUSED && g.out_t == HIPQ_I32))
-            return launch_conv_direct(g, data, filter, zp, epi, out, s);
+        // (the entry point that allocates nothing keeps the direct kernel where the copy would not fit its array)
+        const bool pad = packed && !conv_mfma_eligible(whole) && conv_pad_eligible(whole, &padded) && (whole.C < 16 || workspace_holds(static_cast<size_t>(padded.in_count()) + 256));
+        if (!packed || (!pad && !conv_mfma_eligible(whole)) || (epi.mode == EPI_FUSED && whole.out_t == HIPQ_I32))
+            return launch_conv_direct(whole, data, filter, zp, epi, out, s);
+        // the geometry the MFMA kernels see: channels in whole 16-byte pieces
+        const ConvGeom& g = pad ? padded : whole;
 
-        // layers bound by HBM traffic that widen 64 channels: weights in registers, loads a tile ahead
-        if (conv_pw64_eligible(g, epi, zp))
-            return launch_conv_pw64(g, data, packed, epi, out, s);
-
-        // 3x3 layers over 64 channels with an NCHW output keep their filter in registers and read the
-        // input in whichever layout it has: no transposition, no scratch
-        if (conv_regw_eligible(g, g.out_layout == HIPQ_LAYOUT_NCX && g.K > 1))
-            return launch_conv_regw(g, data, packed, zp, epi, out, true, s);
-
-        // The other kernels read channels-last data; an NCHW input is transposed through the workspace.
-        // The output is written directly in either layout (sum_in is indexed like the output).
         // A layer with few output pixels in all (M <= 64: the deepest layers of a network at batch 1)
         // is a skinny GEMM over its receptive-field matrix [M][taps * C] -- the data itself for a 1x1
         // stride-1 filter, an im2col copy in the workspace otherwise -- and takes the weight-streaming
         // GEMM kernels, which spread the filter over every CU where tiles of M would fill a few.
         const int64_t in_sp = g.in[1] * g.in[2];
-        const bool tr_in = g.data_layout == HIPQ_LAYOUT_NCX && g.C > 1;
+        const bool out_ncx = g.out_layout == HIPQ_LAYOUT_NCX && g.K > 1;
+        const bool tr_in = !pad && g.data_layout == HIPQ_LAYOUT_NCX && g.C > 1;
         const int64_t M = g.N * g.out[1] * g.out[2];
         const int64_t kred = g.C * g.taps();
         const bool pointwise = g.taps() == 1 && g.st[1] == 1 && g.st[2] == 1 && g.pb[1] == 0 && g.pb[2] == 0 && g.out[1] == g.in[1] && g.out[2] == g.in[2];
-        const bool as_gemm = !(g.out_layout == HIPQ_LAYOUT_NCX && g.K > 1) && M <= 64 && kred % 64 == 0 && kred >= 256 && M * kred < (1ll << 31) &&
-                             g.filter_t == HIPQ_I8 && getenv("HIPQ_NO_SKINNY") == nullptr;
-        const size_t tr_bytes = tr_in ? align_up(static_cast<size_t>(g.in_count()), 256) : 0;
+        const bool as_gemm = !out_ncx && M <= 64 && kred % 64 == 0 && kred >= 256 && M * kred < (1ll << 31) && g.filter_t == HIPQ_I8 && getenv("HIPQ_NO_SKINNY") == nullptr;
+        const size_t tr_bytes = pad || tr_in ? align_up(static_cast<size_t>(g.in_count()), 256) : 0;
         const size_t col_bytes = (as_gemm && !pointwise) ? align_up(static_cast<size_t>(M * kred), 256) : 0;
         const void* x = data;
         uint8_t* ws = nullptr;
-        if (tr_bytes + col_bytes)
-        {
+        auto scratch = [&]() {
             void* p = nullptr;
-            int rc = workspace(tr_bytes + col_bytes, s, &p);
+            const int rc = tr_bytes + col_bytes ? workspace(tr_bytes + col_bytes, s, &p) : HIPQ_OK;
+            ws = static_cast<uint8_t*>(p);
+            return rc;
+        };
+        if (pad)
+        {
+            // the channels-last copy with the missing channels of every pixel at the data zero point (they
+            // meet zero weights; as the zero point they also vanish on the exact path for a non-zero
+            // filter zero point)
+            int rc = scratch();
             if (rc)
                 return rc;
-            ws = static_cast<uint8_t*>(p);
+            if (whole.C < 16)
+                rc = launch_pad_channels(data, ws, g.N, in_sp, whole.C, whole.data_layout == HIPQ_LAYOUT_NCX, zp.data_zp, zp.data_t, s);
+            else if (whole.data_layout == HIPQ_LAYOUT_NCX)
+                rc = launch_transpose_pad(data, ws, g.N, whole.C, in_sp, g.C, zp.data_zp, zp.data_t, s);
+            else
+                rc = launch_pad_rows(data, ws, g.N * in_sp, whole.C, g.C, zp.data_zp, zp.data_t, s);
+            if (rc)
+                return rc;
+            x = ws;
+        }
+
+        // layers bound by HBM traffic that widen 64 channels: weights in registers, loads a tile ahead
+        if (conv_pw64_eligible(g, epi, zp))
+            return launch_conv_pw64(g, x, packed, epi, out, s);
+
+        // 3x3 layers over 64 channels with an NCHW output keep their filter in registers and read the
+        // input in whichever layout it has: no transposition, no scratch
+        if (conv_regw_eligible(g, out_ncx))
+            return launch_conv_regw(g, x, packed, zp, epi, out, true, s);
+
+        // The other kernels read channels-last data; an NCHW input is transposed through the workspace.
+        // The output is written directly in either layout (sum_in is indexed like the output).
+        if (!pad)
+        {
+            const int rc = scratch();
+            if (rc)
+                return rc;
         }
         if (tr_in)
         {
-            int rc = launch_transpose(data, ws, g.N, g.C, in_sp, 1, s);
+            const int rc = in_sp % 16 == 0 ? launch_transpose(data, ws, g.N, g.C, in_sp, 1, s) : launch_transpose_pad(data, ws, g.N, g.C, in_sp, g.C, nullptr, HIPQ_U8, s);
             if (rc)
                 return rc;
             x = ws;
@@ -132,7 +146,6 @@ namespace hipq
                 return launch_dot_mfma(dd, x, packed, wsum, zp, epi, out, s);
             }
         }
-        const bool out_ncx = g.out_layout == HIPQ_LAYOUT_NCX && g.K > 1;
         // layers whose filter fits in LDS take the band kernel (HIPQ_NO_BAND=1 forces the generic one)
         const bool no_band = getenv("HIPQ_NO_BAND") != nullptr;
         // (a 1 x 1 filter over every pixel, 8-bit channels-last output in whole 16-byte rows: the data
@@ -179,34 +192,76 @@ namespace hipq
 
     static int dot_pack(const hipq_dot_desc_t& d, const void* b, void* packed, bool with_fragments, hipStream_t s);
 
-    // Layout of a packed dot operand: [N][K] weights (only when the caller's are [K][N]), the column
-    // sums, and -- for products the weight-streaming kernels take -- the weights once more in MFMA
-    // fragment order.  Each part starts on a 256-byte boundary.
-    static size_t dot_blob_weights(const hipq_dot_desc_t& d) { return d.b_layout == HIPQ_B_KN ? align_up(static_cast<size_t>(d.N * d.K), 256) : 0; }
+    // The product the MFMA kernels see: reductions in whole 16-byte pieces of a row.  A reduction that is
+    // not is padded to whole 64-byte steps -- zero weights in the packed operand, a padded copy of the
+    // rows of `a` in the workspace.  Below 64 there is less to multiply than to pad: the direct kernel.
+    static bool dot_is_padded(const hipq_dot_desc_t& d) { return d.K >= 64 && d.K % 16 != 0; }
+    static hipq_dot_desc_t dot_seen(const hipq_dot_desc_t& d)
+    {
+        hipq_dot_desc_t p = d;
+        if (dot_is_padded(d))
+            p.K = static_cast<int64_t>(align_up(static_cast<size_t>(d.K), 64));
+        return p;
+    }
+
+    // Layout of a packed dot operand: [N][K] weights (only when the caller's are [K][N] or need padding),
+    // the column sums, and -- for products the weight-streaming kernels take -- the weights once more in
+    // MFMA fragment order.  Each part starts on a 256-byte boundary.
+    static bool dot_blob_has_weights(const hipq_dot_desc_t& d) { return d.b_layout == HIPQ_B_KN || dot_is_padded(d); }
+    static size_t dot_blob_weights(const hipq_dot_desc_t& d) { return dot_blob_has_weights(d) ? align_up(static_cast<size_t>(d.N * dot_seen(d).K), 256) : 0; }
     static size_t dot_blob_sums(const hipq_dot_desc_t& d) { return align_up(static_cast<size_t>(d.N) * sizeof(int32_t), 256); }
 
-    // weights [N,K] + column sums for the MFMA dot, either prepacked or built in the workspace
+    // Operands of the MFMA dot: the rows of `a` (padded through the workspace where the reduction is) and
+    // the weights [N,K] with their column sums, either prepacked or built in the workspace
     // (built on the fly there is no fragment-ordered copy: making one costs more than it saves a call)
-    static int dot_operands(const hipq_dot_desc_t& d, const void* b, const void* packed, const void** w, const int32_t** wsum, const void** wfrag, hipStream_t s)
+    struct DotOperands
     {
+        hipq_dot_desc_t d; // as the kernels see it
+        const void* a;
+        const void* w;
+        const void* wfrag;
+        const int32_t* wsum;
+    };
+    static size_t dot_padded_rows_bytes(const hipq_dot_desc_t& d) { return dot_is_padded(d) ? align_up(static_cast<size_t>(d.M * dot_seen(d).K), 256) : 0; }
+
+    // scratch (may be null: the workspace): where the copies go, for a caller that holds a part of the
+    // workspace itself
+    static int dot_operands(const hipq_dot_desc_t& d, const void* a, const void* b, const void* packed, const ZeroPoints& zp, DotOperands* o, hipStream_t s, uint8_t* scratch = nullptr)
+    {
+        o->d = dot_seen(d);
+        o->a = a;
+        o->wfrag = nullptr;
         const size_t wbytes = dot_blob_weights(d);
+        const size_t blob_bytes = packed ? 0 : wbytes + dot_blob_sums(d);
+        const size_t a_bytes = dot_padded_rows_bytes(d);
         const uint8_t* blob = static_cast<const uint8_t*>(packed);
-        *wfrag = nullptr;
-        if (!blob)
+        if (blob_bytes + a_bytes)
         {
-            uint8_t* ws = nullptr;
-            int rc = workspace(wbytes + dot_blob_sums(d), s, reinterpret_cast<void**>(&ws));
+            uint8_t* ws = scratch;
+            int rc = ws ? HIPQ_OK : workspace(blob_bytes + a_bytes, s, reinterpret_cast<void**>(&ws));
             if (rc)
                 return rc;
-            rc = dot_pack(d, b, ws, false, s);
-            if (rc)
-                return rc;
-            blob = ws;
+            if (a_bytes)
+            {
+                // (the bytes behind a row's end meet zero weights; as the zero point they also vanish on the
+                // exact path for a non-zero weight zero point)
+                rc = launch_pad_rows(a, ws + blob_bytes, d.M, d.K, o->d.K, zp.data_zp, zp.data_t, s);
+                if (rc)
+                    return rc;
+                o->a = ws + blob_bytes;
+            }
+            if (blob_bytes)
+            {
+                rc = dot_pack(d, b, ws, false, s);
+                if (rc)
+                    return rc;
+                blob = ws;
+            }
         }
-        else if (dot_fragments_eligible(d))
-            *wfrag = blob + wbytes + dot_blob_sums(d);
-        *w = d.b_layout == HIPQ_B_KN ? static_cast<const void*>(blob) : b;
-        *wsum = reinterpret_cast<const int32_t*>(blob + wbytes);
+        if (packed && dot_fragments_eligible(o->d))
+            o->wfrag = blob + wbytes + dot_blob_sums(d);
+        o->w = dot_blob_has_weights(d) ? static_cast<const void*>(blob) : b;
+        o->wsum = reinterpret_cast<const int32_t*>(blob + wbytes);
         return HIPQ_OK;
     }
 
@@ -217,21 +272,24 @@ namespace hipq
                        const ZeroPoints& zp,
                        const Epilogue& epi,
                        void* out,
-                       hipStream_t s)
+                       hipStream_t s,
+                       uint8_t* scratch = nullptr)
     {
         if (d.M == 0 || d.N == 0)
             return HIPQ_OK;
         HIPQ_REQUIRE(out && (d.K == 0 || (a && b)), "null tensor pointer");
-        if (!dot_mfma_eligible(d) || (reinterpret_cast<uintptr_t>(a) & 15) || (reinterpret_cast<uintptr_t>(b) & 15) ||
-            (reinterpret_cast<uintptr_t>(out) & 15))
+        // (operands that the padded copies replace may start anywhere)
+        const bool copied = dot_is_padded(d);
+        const uintptr_t misaligned = reinterpret_cast<uintptr_t>(out) | (copied ? 0 : reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b));
+        // Padding and packing a reduction on the fly is three launches ahead of the product: from 2^24
+        // multiply-adds on, where the direct kernel takes ten times as long as those
+        if (!dot_mfma_eligible(dot_seen(d)) || (misaligned & 15) || (copied && !packed && d.M * d.N < (1ll << 31) && d.M * d.N * d.K < (1ll << 24)))
             return launch_dot_direct(d, a, b, zp, epi, out, s);
-        const void* w = nullptr;
-        const void* wfrag = nullptr;
-        const int32_t* wsum = nullptr;
-        int rc = dot_operands(d, b, packed, &w, &wsum, &wfrag, s);
+        DotOperands o;
+        const int rc = dot_operands(d, a, b, packed, zp, &o, s, scratch);
         if (rc)
             return rc;
-        return launch_dot_mfma(d, a, w, wsum, zp, epi, out, s, wfrag);
+        return launch_dot_mfma(o.d, o.a, o.w, o.wsum, zp, epi, out, s, o.wfrag);
     }
 
     static int dot_pack(const hipq_dot_desc_t& d, const void* b, void* packed, bool with_fragments, hipStream_t s)
@@ -239,17 +297,21 @@ namespace hipq
         uint8_t* blob = static_cast<uint8_t*>(packed);
         const void* w = b;
         const size_t wbytes = dot_blob_weights(d);
-        if (d.b_layout == HIPQ_B_KN)
+        const hipq_dot_desc_t seen = dot_seen(d);
+        if (dot_blob_has_weights(d))
         {
-            int rc = launch_transpose(b, blob, 1, d.K, d.N, 1, s); // [K][N] -> [N][K]
+            // [K][N] -> [N][K], or [N][K] rows padded
+            const int rc = d.b_layout != HIPQ_B_KN ? launch_pad_rows(b, blob, d.N, d.K, seen.K, nullptr, HIPQ_I8, s)
+                           : d.N % 16 == 0 && seen.K == d.K ? launch_transpose(b, blob, 1, d.K, d.N, 1, s)
+                                                            : launch_transpose_pad(b, blob, 1, d.K, d.N, seen.K, nullptr, HIPQ_I8, s);
             if (rc)
                 return rc;
             w = blob;
         }
-        int rc = launch_row_sums_i8(w, d.N, d.K, reinterpret_cast<int32_t*>(blob + wbytes), s);
-        if (rc || !with_fragments || !dot_fragments_eligible(d))
+        const int rc = launch_row_sums_i8(w, d.N, seen.K, reinterpret_cast<int32_t*>(blob + wbytes), s);
+        if (rc || !with_fragments || !dot_fragments_eligible(seen))
             return rc;
-        return launch_pack_dot_fragments(w, d.N, d.K, blob + wbytes + dot_blob_sums(d), s);
+        return launch_pack_dot_fragments(w, d.N, seen.K, blob + wbytes + dot_blob_sums(d), s);
     }
 }
 
@@ -429,15 +491,16 @@ int hipq_quantized_convolution_fused_max_pool(const hipq_conv_desc_t* desc,
 
 size_t hipq_dot_packed_bytes(const hipq_dot_desc_t* d)
 {
-    if (!d || !dot_mfma_eligible(*d))
+    if (!d || !dot_mfma_eligible(dot_seen(*d)))
         return 0;
-    return dot_blob_weights(*d) + dot_blob_sums(*d) + (dot_fragments_eligible(*d) ? dot_fragment_bytes(*d) : 0);
+    const hipq_dot_desc_t seen = dot_seen(*d);
+    return dot_blob_weights(*d) + dot_blob_sums(*d) + (dot_fragments_eligible(seen) ? dot_fragment_bytes(seen) : 0);
 }
 
 int hipq_dot_pack(const hipq_dot_desc_t* d, const void* b, void* packed, void* stream)
 {
     HIPQ_REQUIRE(d && b && packed, "null pointer");
-    if (!dot_mfma_eligible(*d))
+    if (!dot_mfma_eligible(dot_seen(*d)))
         return fail(HIPQ_ERR_UNSUPPORTED, "shape is not eligible for the MFMA path (hipq_dot_packed_bytes is 0)");
     return dot_pack(*d, b, packed, true, as_stream(stream));
 }
@@ -531,12 +594,10 @@ int hipq_quantized_dot_bias_gelu_quantize(const hipq_dot_desc_t* d,
         return rc;
     hipStream_t s = as_stream(stream);
     // in the epilogue of the product, where the kernels that take it apply
-    if (dot_mfma_eligible(*d) && d->M > 256 && (reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && (reinterpret_cast<uintptr_t>(quant->out) & 15) == 0)
+    if (dot_mfma_eligible(*d) && d->K % 16 == 0 && d->M > 256 && (reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && (reinterpret_cast<uintptr_t>(quant->out) & 15) == 0)
     {
-        const void* wn = nullptr;
-        const void* wfrag = nullptr;
-        const int32_t* wsum = nullptr;
-        rc = dot_operands(*d, w, packed_w, &wn, &wsum, &wfrag, s);
+        DotOperands o;
+        rc = dot_operands(*d, a, w, packed_w, ZeroPoints{nullptr, nullptr, d->a_t, d->b_t}, &o, s);
         if (rc)
             return rc;
         Epilogue post = e;
@@ -545,7 +606,7 @@ int hipq_quantized_dot_bias_gelu_quantize(const hipq_dot_desc_t* d,
         post.post_t = quant->quant_t;
         post.post_mode = quant->round_mode;
         ZeroPoints zp{nullptr, nullptr, d->a_t, d->b_t};
-        rc = launch_rows_gelu_q8(a, d->a_t == HIPQ_U8, static_cast<const int8_t*>(wn), wsum, d->M, static_cast<int32_t>(d->N), static_cast<int32_t>(d->K), zp, post, quant->out, s);
+        rc = launch_rows_gelu_q8(a, d->a_t == HIPQ_U8, static_cast<const int8_t*>(o.w), o.wsum, d->M, static_cast<int32_t>(d->N), static_cast<int32_t>(d->K), zp, post, quant->out, s);
         if (rc != HIPQ_ERR_UNSUPPORTED)
             return rc;
     }
@@ -554,11 +615,12 @@ int hipq_quantized_dot_bias_gelu_quantize(const hipq_dot_desc_t* d,
     if (!packed_w)
         return fail(HIPQ_ERR_UNSUPPORTED, "QuantizedDotBias + Gelu + Quantize outside the fused kernels needs prepacked weights (hipq_dot_pack)");
     float* product = nullptr;
-    rc = workspace(static_cast<size_t>(d->M) * static_cast<size_t>(d->N) * sizeof(float), s, reinterpret_cast<void**>(&product));
+    const size_t product_bytes = align_up(static_cast<size_t>(d->M) * static_cast<size_t>(d->N) * sizeof(float), 256);
+    rc = workspace(product_bytes + dot_padded_rows_bytes(*d), s, reinterpret_cast<void**>(&product));
     if (rc)
         return rc;
     ZeroPoints zp{nullptr, nullptr, d->a_t, d->b_t};
-    rc = run_dot(*d, a, w, packed_w, zp, e, product, s);
+    rc = run_dot(*d, a, w, packed_w, zp, e, product, s, reinterpret_cast<uint8_t*>(product) + product_bytes);
     if (rc)
         return rc;
     return hipq_gelu_quantize_f32(product, nullptr, quant, d->M * d->N, stream);

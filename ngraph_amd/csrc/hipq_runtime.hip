@@ -137,6 +137,8 @@ namespace hipq
         return HIPQ_OK;
     }
 
+    bool workspace_holds(size_t bytes) { return !t_noalloc || bytes <= kScratchWorkspaceBytes; }
+
     int workspace(size_t bytes, hipStream_t stream, void** ptr)
     {
         int dev = 0;

@@ -523,8 +523,9 @@ namespace
             if (!is_type<op::v0::QuantizedDotBias>(dot) || !single_user(dot) || dot->get_output_element_type(0) != element::f32 || !dot->get_argument(1)->is_constant())
                 continue;
             {
-                // the fused entry point needs the weights lower_dot prepacks: shapes the library does not
-                // pack (a reduction that is not a multiple of 16, ...) keep Gelu and Quantize as they are
+                // the fused entry point needs the weights lower_dot prepacks, and a reduction that the
+                // kernels with both in their epilogue take as it is (one that is not a multiple of 16 goes
+                // through padded copies): other shapes keep Gelu and Quantize as they are
                 hipq_dot_desc_t d;
                 memset(&d, 0, sizeof(d));
                 d.a_t = dtype_of(dot->get_input_element_type(0));
@@ -534,7 +535,7 @@ namespace
                 d.M = static_cast<int64_t>(dot->get_input_shape(0).at(0));
                 d.K = static_cast<int64_t>(dot->get_input_shape(0).at(1));
                 d.N = static_cast<int64_t>(dot->get_input_shape(1).at(0));
-                if (hipq_dot_packed_bytes(&d) == 0)
+                if (d.K % 16 != 0 || hipq_dot_packed_bytes(&d) == 0)
                     continue;
             }
             QuantizedCopy copy = qc->second;
