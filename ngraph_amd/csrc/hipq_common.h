@@ -254,6 +254,8 @@ namespace hipq
                          void* out,
                          bool out_ncx, // false: out is channels-last; true: out is NCHW (written directly)
                          hipStream_t s);
+    // whether the kernels for layers too small to fill the chip take it (hipq_igemm_wk.hip)
+    bool conv_wk_preferred(const ConvGeom& g, int out_t, bool out_ncx);
     bool dot_mfma_eligible(const hipq_dot_desc_t& d);
     int launch_dot_mfma(const hipq_dot_desc_t& d,
                         const void* a,
@@ -277,7 +279,6 @@ namespace hipq
     int launch_pad_rows(const void* in, void* out, int64_t rows, int64_t cols, int64_t pitch, const void* zp, int zp_t, hipStream_t s);
     int launch_pad_channels(const void* in, void* out, int64_t N, int64_t X, int64_t Cc, bool in_ncx, const void* zp, int zp_t, hipStream_t s);
     bool conv_pad_eligible(const ConvGeom& g, ConvGeom* padded);
-    int launch_im2col_nxc(const ConvGeom& g, const void* x_nxc, void* a, const void* zp, int zp_t, hipStream_t s);
     // first layers (at most four channels): staged copy with materialised padding + row-packed filter
     struct RowPack
     {

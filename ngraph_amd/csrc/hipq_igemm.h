@@ -126,6 +126,7 @@ namespace hipq
         static constexpr bool kUniform = false;
         static constexpr bool kFloatOut = false;
         static constexpr bool kPads = false; // (only read by the kernels that load straight into LDS)
+        static constexpr bool kPadded = false; // no taps in a padding
 
         struct Row
         {
@@ -161,6 +162,7 @@ namespace hipq
         static constexpr bool kUniform = false;
         static constexpr bool kFloatOut = false;
         static constexpr bool kPads = false; // (only read by the kernels that load straight into LDS)
+        static constexpr bool kPadded = true; // taps in the padding are the data zero point
         const uint8_t* x; // [N][H][W][C]
         int32_t H, W, C, Q, R, S, sh, sw, dh, dw, pbh, pbw;
         int64_t PQ;
@@ -2112,4 +2114,13 @@ namespace hipq
         }
         return fail(HIPQ_ERR_UNSUPPORTED, "no MFMA kernel for this epilogue / output type");
     }
+
+    // small products and convolutions: the reduction split over a workgroup's wavefronts, fragments straight
+    // from memory (hipq_igemm_wk.hip); HIPQ_ERR_UNSUPPORTED (nothing launched, no error text) when the call
+    // is not of their kind
+    bool wk_preferred(int64_t M, int64_t N, bool dma);
+    int launch_rows_wk(const void* a, bool a_unsigned, const int8_t* w_nk, const void* w_frag, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi,
+                       void* out, hipStream_t s, const char* name);
+    int launch_conv_wk(const ConvX& xl, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, int x_unsigned, const ZeroPoints& zp, const Epilogue& epi, const OutMap& om, void* out,
+                       hipStream_t s, const char* name);
 }

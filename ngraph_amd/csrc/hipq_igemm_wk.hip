@@ -1,0 +1,436 @@
+// int8 products and implicit-GEMM convolutions too small to fill the chip with the tile kernels of
+// hipq_igemm.h: few output pixels or rows, where a launch lasts as long as its slowest chain of
+// dependent steps and not as long as its arithmetic.
+//
+// What bounds them: the tile kernels walk a tile's reduction slice by slice -- global memory to LDS,
+// barrier, LDS to registers, MFMA -- and a workgroup that is alone on its compute unit takes about
+// 400 ns a slice, nearly all of it latency (a 256 -> 256 3 x 3 layer on 14 x 14 pixels is 36 slices).
+// Here a workgroup owns a small output tile (MT x NT blocks of 16 x 16) and the whole reduction, its
+// wavefronts take a part of the reduction each, and a wavefront asks for the
+// v_mfma_i32_16x16x64_i8 fragments of all its steps at once, straight into registers: one memory
+// latency instead of one a slice, no LDS and no barrier in front of the MFMAs.  The partial tiles meet
+// in LDS once.  Fragment loads from a row-major matrix take half of every cache line they touch, so
+// a compute unit takes operands in at about half of its best rate: the launcher gives these kernels
+// only what that costs less for than the slices would.
+//
+// Measured, one launch of a replayed graph: 256 -> 256 3 x 3 on one 14 x 14 picture 17.4 -> 6.1 us,
+// 512 -> 512 3 x 3 on 7 x 7 (an unrolled copy and a skinny product before) 16.3 -> 8.3, 1024 -> 256
+// 1 x 1 on 14 x 14 10.7 -> 4.9, 128 x 768 x 768 with float outputs 8.5 -> 3.8; a launch that does
+// nothing takes 1.7.
+#include <cstdlib>
+
+#include "hipq_igemm.h"
+
+namespace hipq
+{
+    typedef int v4acc __attribute__((ext_vector_type(4)));
+
+    struct WkParams
+    {
+        const int8_t* w;      // weights: [N][Kred] rows, or 1 KB blocks in fragment order
+        const int8_t* w_rows; // the [N][Kred] rows in either case
+        const int32_t* wsum;
+        uint32_t w_bytes;
+        int32_t w_row;        // bytes from one 16-row block's lane to its next row (rows) / 0 (fragments)
+        int32_t w_block;      // bytes between column blocks of 16
+        int32_t w_step;       // bytes between 64-byte reduction steps
+        int32_t w_lane_chunk; // bytes between a lane's 16-byte chunks of a step (rows: 16, fragments: 256)
+        int32_t fragments;
+        int64_t M;
+        int32_t Kred;
+        int32_t x_unsigned;
+        int32_t inner;        // tiles along the inner dimension of the tile order
+        int32_t m_inner;      // 1: consecutive tiles share a column block, 0: a row block
+    };
+
+    // KW wavefronts split the reduction of a tile of MT x NT blocks, TW such tiles (one below the other)
+    // make a workgroup; U: reduction steps of 64 bytes a wavefront has in flight.
+    // X_ON_A: the activations are MFMA source A, so that a lane's four accumulators are four consecutive
+    // pixels of one channel (NCHW outputs); otherwise four consecutive channels of one pixel
+    template <class XL, int MT, int NT, int KW, int TW, int U, bool X_ON_A>
+    __global__ __launch_bounds__(KW * TW * 64) void igemm_wk_kernel(XL xl, WkParams p, ZeroPoints zp, Epilogue epi, OutMap om, void* __restrict__ out)
+    {
+        constexpr int BM = MT * 16, BN = NT * 16;
+        constexpr int BLOCKS = MT * NT;
+        static_assert(BLOCKS % KW == 0 || KW % BLOCKS == 0, "the wavefronts of a tile share its blocks evenly");
+        constexpr int ITER = BLOCKS >= KW ? BLOCKS / KW : 1; // blocks a wavefront finishes
+        __shared__ v4acc red[KW > 1 ? KW * TW * BLOCKS * 64 : 1];
+        __shared__ __attribute__((aligned(16))) int32_t col_corr[BN];
+        __shared__ __attribute__((aligned(16))) float col_bias[BN], col_scale[BN];
+
+        const int tid = threadIdx.x;
+        const int lane = tid & 63;
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int kw = wave % KW, tw = wave / KW;
+        const int r16 = lane & 15, kc = lane >> 4;
+        const int N = om.N;
+        const bool fused = epi.mode == EPI_FUSED;
+        // workgroups are dealt round robin to the eight compute dies: a die gets consecutive tiles, which
+        // share the operand that is the larger one
+        const int grid = static_cast<int>(gridDim.x);
+        const int id = (grid & 7) == 0 ? (static_cast<int>(blockIdx.x) & 7) * (grid >> 3) + (static_cast<int>(blockIdx.x) >> 3) : static_cast<int>(blockIdx.x);
+        const int outer_i = id / p.inner, inner_i = id - outer_i * p.inner;
+        const int64_t m0 = (static_cast<int64_t>(p.m_inner ? inner_i : outer_i) * TW + tw) * BM;
+        const int n0 = (p.m_inner ? outer_i : inner_i) * BN;
+
+        // ---- operands: fragments of this wavefront's steps
+        const int steps = (p.Kred + 63) >> 6;
+        const int per = (steps + KW - 1) / KW;
+        const int s_begin = ((kw + id) % KW) * per;
+        const int s_end = min(steps, s_begin + per);
+        const __amdgpu_buffer_rsrc_t xrs = make_rsrc(xl.x, xl.bytes);
+        const __amdgpu_buffer_rsrc_t wrs = make_rsrc(p.w, p.w_bytes);
+        typename XL::Row xr[MT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+            xl.init_row(xr[i], m0 + i * 16 + r16, p.M);
+        int32_t woff[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+        {
+            const int n = n0 + j * 16 + r16;
+            // (a block of the fragment-ordered copy holds zeros beyond N)
+            const bool ok = p.fragments ? n0 + j * 16 < N : n < N;
+            woff[j] = ok ? ((n0 >> 4) + j) * p.w_block + r16 * p.w_row + kc * p.w_lane_chunk : kOob;
+        }
+        v4i xf[U][MT], wf[U][NT];
+        uint32_t pads = 0; // bit u * MT + i: the data fragment lies in the padding
+        auto load = [&](int u, int s) {
+            const int kbyte = s * 64 + kc * 16;
+            const bool in_k = (s < s_end) & (kbyte < p.Kred);
+            typename XL::Cursor cur;
+            xl.init_cursor(cur, kbyte);
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+            {
+                const int32_t off = in_k ? xl.offset(xr[i], cur) : kOob;
+                if (XL::kPadded)
+                    pads = (pads & ~(1u << (u * MT + i))) | ((off == kOob ? 1u : 0u) << (u * MT + i));
+                xf[u][i] = buffer_load16(xrs, off);
+            }
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                wf[u][j] = buffer_load16(wrs, (in_k && woff[j] != kOob) ? woff[j] + s * p.w_step : kOob);
+        };
+        // what the epilogue needs from memory is asked for in front of the operands, none of it looked at
+        // before the reduction is done: per-channel constants, the scalars, the residual
+        int32_t raw_wsum = 0, raw_bias = 0;
+        float raw_scale = 0.0f;
+        const bool with_bias = fused && epi.bias != nullptr, per_channel = fused && epi.per_channel != 0;
+        if (tid < BN)
+        {
+            const int n = n0 + tid < N ? n0 + tid : 0;
+            raw_wsum = p.wsum[n];
+            raw_bias = (with_bias ? epi.bias : p.wsum)[n];
+            raw_scale = (per_channel ? epi.scale : reinterpret_cast<const float*>(p.wsum))[n];
+        }
+        HeadWords hw = head_scalars_load(zp, epi, p.wsum);
+        // this wavefront finishes blocks it * KW + kw of its tile, a group of four outputs a lane
+        const bool has_sum = fused && epi.sum_in != nullptr;
+        const bool vec_ok = X_ON_A ? (!om.ncx || (om.PQ & 3) == 0) : (N & 3) == 0;
+        int64_t o_at[ITER];
+        int o_left[ITER]; // outputs of the group that exist
+        uint32_t res[ITER];
+#pragma unroll
+        for (int it = 0; it < ITER; ++it)
+        {
+            const int blk = it * KW + kw;
+            const int mi = blk / NT, ni = blk % NT;
+            const int64_t m = m0 + mi * 16 + (X_ON_A ? 4 * kc : r16);
+            const int n = n0 + ni * 16 + (X_ON_A ? r16 : 4 * kc);
+            const bool live = blk < BLOCKS && m < p.M && n < N;
+            o_left[it] = !live ? 0 : X_ON_A ? static_cast<int>(p.M - m < 4 ? p.M - m : 4) : (N - n < 4 ? N - n : 4);
+            o_at[it] = live ? om.index(m, n) : 0;
+            res[it] = 0;
+            if (has_sum && o_left[it] > 0)
+            {
+                if (vec_ok)
+                    res[it] = *reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(epi.sum_in) + o_at[it]);
+                else
+                {
+                    for (int e = 0; e < o_left[it]; ++e)
+                        res[it] |= static_cast<uint32_t>(static_cast<const uint8_t*>(epi.sum_in)[X_ON_A ? om.index(m + e, n) : o_at[it] + e]) << (8 * e);
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            load(u, s_begin + u);
+
+        const int xor_mask = p.x_unsigned ? static_cast<int>(0x80808080u) : 0;
+        const int32_t xzp_early = XL::kPadded ? load_zp(zp.data_zp, zp.data_t) : 0;
+        const int fill = (xzp_early & 0xFF) * 0x01010101;
+        v4acc acc[MT][NT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                acc[i][j] = v4acc{0, 0, 0, 0};
+        auto multiply = [&](int u) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+            {
+                v4i x = xf[u][i];
+                if (XL::kPadded && fill != 0) // uniform: padding taps hold the data zero point
+                {
+                    const bool pad = (pads >> (u * MT + i)) & 1u;
+                    x = v4i{pad ? fill : x[0], pad ? fill : x[1], pad ? fill : x[2], pad ? fill : x[3]};
+                }
+                // (steps past the reduction read zero weights, which cancel whatever is here)
+                x = v4i{x[0] ^ xor_mask, x[1] ^ xor_mask, x[2] ^ xor_mask, x[3] ^ xor_mask};
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    acc[i][j] = X_ON_A ? __builtin_amdgcn_mfma_i32_16x16x64_i8(x, wf[u][j], acc[i][j], 0, 0, 0) : __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[u][j], x, acc[i][j], 0, 0, 0);
+            }
+        };
+        for (int s = s_begin; s + U < s_end; s += U) // (uniform; most launches ask for everything above)
+        {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+            {
+                multiply(u);
+                load(u, s + U + u);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            multiply(u);
+
+        head_scalars_settle(hw);
+        const HeadScalars hs = head_scalars_finish(hw, zp, epi);
+        if (hs.wzp != 0) // uniform; w - wzp does not fit a signed byte: exact, slow
+        {
+            slow_tile(xl, p.w_rows, p.M, p.Kred, p.x_unsigned, hs.xzp, hs.wzp, epi, om, out, m0 - tw * BM, n0, TW * BM, BN);
+            return;
+        }
+        // ---- the partial tiles meet in LDS
+        if constexpr (KW > 1)
+        {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    red[(wave * BLOCKS + i * NT + j) * 64 + lane] = acc[i][j];
+        }
+        if (tid < BN)
+        {
+            col_corr[tid] = ((p.x_unsigned ? 128 : 0) - hs.xzp) * raw_wsum;
+            col_bias[tid] = with_bias ? static_cast<float>(raw_bias) : 0.0f;
+            col_scale[tid] = per_channel ? raw_scale : hs.ec.scale;
+        }
+        const EpiConst ec = hs.ec;
+        const bool relu = epi.relu != 0;
+        const bool gelu = epi.post_scale != nullptr;
+        const float post_scale = gelu ? *epi.post_scale : 1.0f;
+        const int32_t post_zp = gelu ? load_zp(epi.post_zp, epi.post_t) : 0;
+        __syncthreads();
+        // (one instantiation of the arithmetic a policy and output kind, chosen by uniform branches: the kernel
+        // runs it once)
+        auto finish = [&](auto mode_c, auto kind_c) {
+            constexpr int MODE = decltype(mode_c)::value;
+            constexpr int KIND = decltype(kind_c)::value;
+#pragma unroll
+            for (int it = 0; it < ITER; ++it)
+            {
+                if (o_left[it] == 0)
+                    continue;
+                const int blk = it * KW + kw;
+                v4acc a;
+                if constexpr (KW > 1)
+                {
+                    a = red[(tw * KW * BLOCKS + blk) * 64 + lane];
+#pragma unroll
+                    for (int v = 1; v < KW; ++v)
+                        a += red[((tw * KW + v) * BLOCKS + blk) * 64 + lane];
+                }
+                else
+                    a = acc[it / NT][it % NT];
+                const int nl = (blk % NT) * 16 + (X_ON_A ? r16 : 4 * kc); // column within the tile
+                int32_t v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                {
+                    const int c = X_ON_A ? nl : nl + e;
+                    const int32_t sum = a[e] + col_corr[c];
+                    const uint32_t rb = (res[it] >> (8 * e)) & 0xFFu;
+                    const float sv = epi.sum_t == HIPQ_I8 ? static_cast<float>(static_cast<int8_t>(rb)) : static_cast<float>(rb);
+                    v[e] = MODE == EPI_INTERP ? epi_interp<KIND>(ec, sum) : epi_fused<KIND == OUT_GELU_Q8 ? OUT_F32 : KIND>(ec, sum, col_bias[c], col_scale[c], has_sum, sv, relu);
+                }
+                if constexpr (KIND == OUT_GELU_Q8)
+                {
+                    // Gelu and Quantize with the arithmetic of their own kernels: the bytes equal the three launches'
+                    const f32x4 r4 = f32x4{gelu1(__int_as_float(v[0])), gelu1(__int_as_float(v[1])), gelu1(__int_as_float(v[2])), gelu1(__int_as_float(v[3]))};
+                    uint32_t packed = 0;
+                    if (epi.post_mode == HIPQ_ROUND_NEAREST_TOWARD_EVEN) // uniform
+                        packed = epi.post_t == HIPQ_U8 ? quantize4<uint8_t, true>(r4, post_scale, static_cast<float>(post_zp), epi.post_mode)
+                                                       : quantize4<int8_t, true>(r4, post_scale, static_cast<float>(post_zp), epi.post_mode);
+                    else
+                    {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            packed |= (epi.post_t == HIPQ_U8 ? static_cast<uint32_t>(quantize_one<float, uint8_t>(r4[e], post_scale, static_cast<uint8_t>(post_zp), epi.post_mode))
+                                                             : static_cast<uint32_t>(static_cast<uint8_t>(quantize_one<float, int8_t>(r4[e], post_scale, static_cast<int8_t>(post_zp), epi.post_mode))))
+                                      << (8 * e);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        v[e] = static_cast<int32_t>((packed >> (8 * e)) & 0xFFu);
+                }
+                if (vec_ok && o_left[it] == 4)
+                {
+                    if (KIND == OUT_Q8 || KIND == OUT_GELU_Q8)
+                        *reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(out) + o_at[it]) = pack4(v);
+                    else
+                        *reinterpret_cast<v4i*>(static_cast<int32_t*>(out) + o_at[it]) = v4i{v[0], v[1], v[2], v[3]};
+                }
+                else
+                {
+                    const int64_t m = m0 + (blk / NT) * 16 + 4 * kc;
+                    for (int e = 0; e < o_left[it]; ++e)
+                        store_out(out, KIND == OUT_Q8 || KIND == OUT_GELU_Q8 ? HIPQ_U8 : HIPQ_I32, X_ON_A ? om.index(m + e, n0 + nl) : o_at[it] + e, e == 0 ? v[0] : e == 1 ? v[1] : e == 2 ? v[2] : v[3]);
+                }
+            }
+        };
+        using std::integral_constant;
+        const bool q8 = epi.out_t == HIPQ_U8 || epi.out_t == HIPQ_I8;
+        if (!fused)
+        {
+            if (q8)
+                finish(integral_constant<int, EPI_INTERP>{}, integral_constant<int, OUT_Q8>{});
+            else
+                finish(integral_constant<int, EPI_INTERP>{}, integral_constant<int, OUT_I32>{});
+        }
+        else if (q8)
+            finish(integral_constant<int, EPI_FUSED>{}, integral_constant<int, OUT_Q8>{});
+        else if constexpr (!X_ON_A && !XL::kPadded)
+        {
+            if (gelu)
+                finish(integral_constant<int, EPI_FUSED>{}, integral_constant<int, OUT_GELU_Q8>{});
+            else
+                finish(integral_constant<int, EPI_FUSED>{}, integral_constant<int, OUT_F32>{});
+        }
+    }
+
+    enum class WkShape
+    {
+        kTile1181, // 16 x 16, eight wavefronts on the reduction
+        kTile1241, // 16 x 32, four
+        kTile2241, // 32 x 32, four
+        kTile2222, // two tiles of 32 x 32, two wavefronts each
+        kTile2214  // four tiles of 32 x 32, a wavefront each
+    };
+    static int64_t wk_tiles(int64_t M, int64_t N, int bm, int bn) { return (M + bm - 1) / bm * ((N + bn - 1) / bn); }
+
+    // Which tile: the largest that still gives every compute unit work.  From three 32 x 32 tiles for two
+    // compute units on those; their reduction is worth splitting over all four wavefronts unless it is
+    // short and there are many of them.  Fewer tiles: 16 x 32, and where even those leave half of the chip
+    // idle on a reduction of eight steps or more, 16 x 16 with eight wavefronts on it.  (The lines are those
+    // that cost least over 200 products and convolutions of 1 to 90 000 rows, 64 to 9 600 bytes of reduction
+    // and 16 to 4 000 outputs, each timed in all five shapes: 1.7 % above the best shape of each on average.)
+    static WkShape wk_shape(int64_t M, int64_t N, int64_t Kred)
+    {
+        const int64_t t22 = wk_tiles(M, N, 32, 32), steps = (Kred + 63) / 64, units = device_compute_units();
+        if (t22 * 2 >= units * 3)
+        {
+            if (t22 < units * 3 || steps > 6)
+                return WkShape::kTile2241;
+            return steps <= 2 ? WkShape::kTile2214 : WkShape::kTile2222;
+        }
+        return wk_tiles(M, N, 16, 32) * 2 >= units || steps < 8 ? WkShape::kTile1241 : WkShape::kTile1181;
+    }
+
+    // Whether these kernels are the better ones.  Against the kernels that load straight into LDS (`dma`: 8-bit
+    // or fused float rows in whole 16-byte pieces, channels in whole 64-byte slices) up to three 32 x 32
+    // tiles a compute unit: above that those kernels' whole-line loads and larger tiles win (985 x 512 x
+    // 1536: 8.6 us there, 9.9 us here; 985 x 512 x 512: 7.9, 5.5).  Against the register-staged ones up to
+    // sixteen.
+    bool wk_preferred(int64_t M, int64_t N, bool dma)
+    {
+        // (the switches that name a kernel of the other family mean that family)
+        for (const char* name : {"HIPQ_NO_WK", "HIPQ_SPLIT_K", "HIPQ_NO_DMA", "HIPQ_NO_PIPE", "HIPQ_NO_CONV_DMA", "HIPQ_NO_HALF_TILES", "HIPQ_NO_REGW"})
+            if (getenv(name) != nullptr)
+                return false;
+        return wk_tiles(M, N, 32, 32) <= static_cast<int64_t>(device_compute_units()) * (dma ? 3 : 16);
+    }
+
+    template <class XL, int MT, int NT, int KW, int TW, int U, bool X_ON_A>
+    static int launch_wk_tile(const XL& xl, WkParams p, const ZeroPoints& zp, const Epilogue& epi, const OutMap& om, void* out, hipStream_t s, const char* name)
+    {
+        const int64_t m_tiles = (p.M + TW * MT * 16 - 1) / (TW * MT * 16), n_tiles = (om.N + NT * 16 - 1) / (NT * 16);
+        HIPQ_REQUIRE(fits_i32(m_tiles * n_tiles), "too many tiles");
+        p.m_inner = p.M <= om.N ? 1 : 0; // the larger operand is the one that consecutive tiles share
+        p.inner = static_cast<int32_t>(p.m_inner ? m_tiles : n_tiles);
+        igemm_wk_kernel<XL, MT, NT, KW, TW, U, X_ON_A><<<static_cast<unsigned>(m_tiles * n_tiles), KW * TW * 64, 0, s>>>(xl, p, zp, epi, om, out);
+        return check_launch(name);
+    }
+
+    template <class XL, bool X_ON_A>
+    static int launch_wk(const XL& xl, const WkParams& p, const ZeroPoints& zp, const Epilogue& epi, const OutMap& om, void* out, hipStream_t s, const char* name)
+    {
+        const bool q8 = epi.out_t == HIPQ_U8 || epi.out_t == HIPQ_I8;
+        if (epi.mode == EPI_FUSED && !q8 && (X_ON_A || XL::kPadded || epi.out_t != HIPQ_F32))
+            return HIPQ_ERR_UNSUPPORTED;
+        const int steps = (p.Kred + 63) / 64;
+        // as many steps in flight as a wavefront has, up to what its registers hold: a load that has no step
+        // would still take its turn in the texture path, which is what bounds these kernels
+#define WK(MT, NT, KW, TW, BIG)                                                                           \
+    case WkShape::kTile##MT##NT##KW##TW:                                                              \
+        switch ((steps + KW - 1) / KW)                                                                     \
+        {                                                                                                  \
+        case 1: return launch_wk_tile<XL, MT, NT, KW, TW, 1, X_ON_A>(xl, p, zp, epi, om, out, s, name);     \
+        case 2: return launch_wk_tile<XL, MT, NT, KW, TW, 2, X_ON_A>(xl, p, zp, epi, om, out, s, name);     \
+        case 3: return launch_wk_tile<XL, MT, NT, KW, TW, 3, X_ON_A>(xl, p, zp, epi, om, out, s, name);     \
+        case 4: return launch_wk_tile<XL, MT, NT, KW, TW, 4, X_ON_A>(xl, p, zp, epi, om, out, s, name);     \
+        default: return launch_wk_tile<XL, MT, NT, KW, TW, BIG, X_ON_A>(xl, p, zp, epi, om, out, s, name);  \
+        }
+        switch (wk_shape(p.M, om.N, p.Kred))
+        {
+            WK(1, 1, 8, 1, 6);
+            WK(1, 2, 4, 1, 6);
+            WK(2, 2, 1, 4, 5);
+            WK(2, 2, 2, 2, 5);
+            WK(2, 2, 4, 1, 5);
+        }
+#undef WK
+        return HIPQ_ERR_UNSUPPORTED; // (not reached)
+    }
+
+    static WkParams wk_params(const int8_t* w_nk, const void* w_frag, const int32_t* wsum, int64_t M, int32_t N, int32_t K, int x_unsigned)
+    {
+        WkParams p;
+        p.fragments = w_frag != nullptr;
+        p.w = w_frag ? static_cast<const int8_t*>(w_frag) : w_nk;
+        p.w_rows = w_nk;
+        p.wsum = wsum;
+        p.w_bytes = w_frag ? static_cast<uint32_t>((N + 15) / 16) * static_cast<uint32_t>(K / 64) * 1024u : static_cast<uint32_t>(N) * static_cast<uint32_t>(K);
+        p.w_row = w_frag ? 16 : K;
+        p.w_block = w_frag ? (K / 64) * 1024 : 16 * K;
+        p.w_step = w_frag ? 1024 : 64;
+        p.w_lane_chunk = w_frag ? 256 : 16;
+        p.M = M;
+        p.Kred = K;
+        p.x_unsigned = x_unsigned;
+        p.inner = p.m_inner = 1;
+        return p;
+    }
+
+    int launch_rows_wk(const void* a, bool a_unsigned, const int8_t* w_nk, const void* w_frag, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi,
+                       void* out, hipStream_t s, const char* name)
+    {
+        GemmX xl;
+        xl.x = static_cast<const uint8_t*>(a);
+        xl.K = K;
+        xl.bytes = static_cast<uint32_t>(M * K);
+        const OutMap om{0, N, 1};
+        return launch_wk<GemmX, false>(xl, wk_params(w_nk, w_frag, wsum, M, N, K, a_unsigned ? 1 : 0), zp, epi, om, out, s, name);
+    }
+
+    int launch_conv_wk(const ConvX& xl, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, int x_unsigned, const ZeroPoints& zp, const Epilogue& epi, const OutMap& om, void* out,
+                       hipStream_t s, const char* name)
+    {
+        const WkParams p = wk_params(w, nullptr, wsum, M, N, K, x_unsigned);
+        if (om.ncx)
+            return launch_wk<ConvX, true>(xl, p, zp, epi, om, out, s, name);
+        return launch_wk<ConvX, false>(xl, p, zp, epi, om, out, s, name);
+    }
+}

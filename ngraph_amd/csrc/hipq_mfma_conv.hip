@@ -26,6 +26,13 @@ namespace hipq
         return true;
     }
 
+    bool conv_wk_preferred(const ConvGeom& g, int out_t, bool out_ncx)
+    {
+        const bool pointwise = g.taps() == 1 && g.st[1] == 1 && g.st[2] == 1;
+        const bool dma = !out_ncx && g.K % 16 == 0 && (out_t == HIPQ_U8 || out_t == HIPQ_I8) && (g.C % 64 == 0 || pointwise);
+        return wk_preferred(g.N * g.out[1] * g.out[2], g.K, dma);
+    }
+
     int launch_conv_mfma(const ConvGeom& g,
                          const void* data_nxc,
                          const void* packed,
@@ -69,6 +76,14 @@ namespace hipq
             reinterpret_cast<const int32_t*>(static_cast<const uint8_t*>(packed) + align_up(static_cast<size_t>(g.K) * Kred, 256));
         OutMap om{out_ncx ? 1 : 0, N, xl.PQ};
         const int xu = g.data_t == HIPQ_U8 ? 1 : 0;
+        if (conv_wk_preferred(g, epi.out_t, out_ncx))
+        {
+            // (a layer of at most 64 output pixels is a product of as many rows)
+            const bool rows = !out_ncx && M <= 64 && Kred % 64 == 0 && Kred >= 256;
+            const int rc = launch_conv_wk(xl, w, wsum, M, N, Kred, xu, zp, epi, om, out, s, rows ? "dot_skinny_wk_i8_16x16x64" : "conv_mfma_wk_i8_16x16x64");
+            if (rc != HIPQ_ERR_UNSUPPORTED)
+                return rc;
+        }
         // a 1 x 1 filter over every pixel: the channels-last data is the [pixels][C] matrix itself
         if (!out_ncx && g.taps() == 1 && g.st[1] == 1 && g.st[2] == 1 && g.pb[1] == 0 && g.pb[2] == 0 && g.out[1] == g.in[1] && g.out[2] == g.in[2] &&
             g.C % 16 == 0)

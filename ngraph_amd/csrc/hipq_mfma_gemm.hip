@@ -1055,6 +1055,36 @@ namespace hipq
         HIPQ_REQUIRE((reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w_nk) & 15) == 0 &&
                          (reinterpret_cast<uintptr_t>(out) & 15) == 0,
                      "MFMA dot needs 16-byte aligned tensors");
+        // Products too small to fill the chip: fragments straight from memory, the reduction split over a
+        // workgroup's wavefronts.  Up to 32 rows with packed weights only short reductions: the kernel
+        // below asks for whole lines of both operands, which counts from twelve steps on (1 x 1024 x 1003:
+        // 3.3 us there, 3.5 here; 16 x 256 x 512: 3.6 there, 3.1 here).  From 65 rows on, where the kernel
+        // that keeps the whole reduction in one workgroup would take the product, only up to about
+        // 8192 step-tiles (77 x 1024 x 1003: 4.3 us here, 5.8 there; 77 x 4096 x 4096: 13.3, 10.8).
+        {
+            const bool skinny = dot_skinny_eligible(d) && getenv("HIPQ_NO_SKINNY") == nullptr;
+            const bool q8 = epi.out_t == HIPQ_U8 || epi.out_t == HIPQ_I8;
+            const bool dma = d.N % 16 == 0 && (q8 || (epi.out_t == HIPQ_F32 && epi.mode == EPI_FUSED));
+            const int64_t steps = (d.K + 63) / 64;
+            const bool rows64 = skinny && d.M > 64 && dot_rows64_eligible(d);
+            bool wk = wk_preferred(d.M, d.N, dma);
+            const char* name = "dot_mfma_wk_i8_16x16x64";
+            if (skinny && d.M <= 32 && w_frag && steps >= (d.M <= 16 ? 12 : 24))
+                wk = false;
+            else if (rows64)
+            {
+                wk = wk && ((d.M + 31) / 32) * ((d.N + 31) / 32) * steps <= 8192;
+                name = w_frag && d.K <= 4096 ? "dot_rows64w_wk_i8_16x16x64" : "dot_rows64_wk_i8_16x16x64";
+            }
+            else if (skinny && (d.M <= 64 || !dma))
+                name = w_frag && (d.M <= 16 ? d.K <= 8192 : d.M <= 32 && d.K <= 4096) ? "dot_skinnyf_wk_i8_16x16x64" : "dot_skinny_wk_i8_16x16x64";
+            if (wk)
+            {
+                const int rc = launch_rows_wk(a, d.a_t == HIPQ_U8, static_cast<const int8_t*>(w_nk), w_frag, wsum, d.M, static_cast<int32_t>(d.N), static_cast<int32_t>(d.K), zp, epi, out, s, name);
+                if (rc != HIPQ_ERR_UNSUPPORTED)
+                    return rc;
+            }
+        }
         if (dot_skinny_eligible(d) && getenv("HIPQ_NO_SKINNY") == nullptr)
         {
             // prepacked weights: whole-line loads (fragment-ordered weights, activations through LDS)

@@ -59,24 +59,16 @@ namespace hipq
         // the geometry the MFMA kernels see: channels in whole 16-byte pieces
         const ConvGeom& g = pad ? padded : whole;
 
-        // A layer with few output pixels in all (M <= 64: the deepest layers of a network at batch 1)
-        // is a skinny GEMM over its receptive-field matrix [M][taps * C] -- the data itself for a 1x1
-        // stride-1 filter, an im2col copy in the workspace otherwise -- and takes the weight-streaming
-        // GEMM kernels, which spread the filter over every CU where tiles of M would fill a few.
         const int64_t in_sp = g.in[1] * g.in[2];
         const bool out_ncx = g.out_layout == HIPQ_LAYOUT_NCX && g.K > 1;
         const bool tr_in = !pad && g.data_layout == HIPQ_LAYOUT_NCX && g.C > 1;
-        const int64_t M = g.N * g.out[1] * g.out[2];
-        const int64_t kred = g.C * g.taps();
-        const bool pointwise = g.taps() == 1 && g.st[1] == 1 && g.st[2] == 1 && g.pb[1] == 0 && g.pb[2] == 0 && g.out[1] == g.in[1] && g.out[2] == g.in[2];
-        const bool as_gemm = !out_ncx && M <= 64 && kred % 64 == 0 && kred >= 256 && M * kred < (1ll << 31) && g.filter_t == HIPQ_I8 && getenv("HIPQ_NO_SKINNY") == nullptr;
+        const bool small = conv_wk_preferred(g, epi.out_t, out_ncx); // too small to fill the chip
         const size_t tr_bytes = pad || tr_in ? align_up(static_cast<size_t>(g.in_count()), 256) : 0;
-        const size_t col_bytes = (as_gemm && !pointwise) ? align_up(static_cast<size_t>(M * kred), 256) : 0;
         const void* x = data;
         uint8_t* ws = nullptr;
         auto scratch = [&]() {
             void* p = nullptr;
-            const int rc = tr_bytes + col_bytes ? workspace(tr_bytes + col_bytes, s, &p) : HIPQ_OK;
+            const int rc = tr_bytes ? workspace(tr_bytes, s, &p) : HIPQ_OK;
             ws = static_cast<uint8_t*>(p);
             return rc;
         };
@@ -123,29 +115,6 @@ namespace hipq
                 return rc;
             x = ws;
         }
-        if (as_gemm)
-        {
-            if (!pointwise)
-            {
-                int rc = launch_im2col_nxc(g, x, ws + tr_bytes, zp.data_zp, zp.data_t, s);
-                if (rc)
-                    return rc;
-                x = ws + tr_bytes;
-            }
-            hipq_dot_desc_t dd;
-            memset(&dd, 0, sizeof(dd));
-            dd.a_t = g.data_t;
-            dd.b_t = g.filter_t;
-            dd.out_t = g.out_t;
-            dd.M = M;
-            dd.K = kred;
-            dd.N = g.K;
-            if (dot_mfma_eligible(dd))
-            {
-                const int32_t* wsum = reinterpret_cast<const int32_t*>(static_cast<const uint8_t*>(packed) + align_up(static_cast<size_t>(g.K * kred), 256));
-                return launch_dot_mfma(dd, x, packed, wsum, zp, epi, out, s);
-            }
-        }
         // layers whose filter fits in LDS take the band kernel (HIPQ_NO_BAND=1 forces the generic one)
         const bool no_band = getenv("HIPQ_NO_BAND") != nullptr;
         // (a 1 x 1 filter over every pixel, 8-bit channels-last output in whole 16-byte rows: the data
@@ -153,7 +122,7 @@ namespace hipq
         // channels at 56 x 56, batch 128: 15.8 us against 23 us)
         const bool row_matrix = !out_ncx && g.taps() == 1 && g.st[1] == 1 && g.st[2] == 1 && g.pb[1] == 0 && g.pb[2] == 0 && g.out[1] == g.in[1] && g.out[2] == g.in[2] &&
                                 (g.out_t == HIPQ_U8 || g.out_t == HIPQ_I8) && g.K % 16 == 0 && getenv("HIPQ_NO_DMA") == nullptr && getenv("HIPQ_NO_PIPE") == nullptr;
-        if (!no_band && !row_matrix && conv_band_eligible(g, out_ncx))
+        if (!small && !no_band && !row_matrix && conv_band_eligible(g, out_ncx))
             return launch_conv_band(g, x, packed, zp, epi, out, out_ncx, s);
         return launch_conv_mfma(g, x, packed, zp, epi, out, out_ncx, s);
     }
