@@ -1019,9 +1019,20 @@ namespace hipq
     // Quantize(Gelu(rows x weights -> f32)) with Gelu and Quantize in the epilogue of the kernels that
     // load straight into LDS; HIPQ_ERR_UNSUPPORTED (nothing launched, no error text) when the call is
     // not of their kind.  epi carries the Quantize in its post_* fields; out is the 8-bit tensor.
-    int launch_rows_gelu_q8(const void* a, bool a_unsigned, const int8_t* w_nk, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi,
+    bool dot_gelu_wk_preferred(const hipq_dot_desc_t& d) { return wk_preferred(d.M, d.N, d.N % 16 == 0); }
+
+    int launch_rows_gelu_q8(const void* a, bool a_unsigned, const int8_t* w_nk, const void* w_frag, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi,
                             void* out, hipStream_t s)
     {
+        if (wk_preferred(M, N, N % 16 == 0))
+        {
+            // (128 x 768 x 3072: product, then Gelu and Quantize from the workspace 14.4 us, in one kernel 5.4)
+            const int rc = launch_rows_wk(a, a_unsigned, w_nk, w_frag, wsum, M, N, K, zp, epi, out, s, M > 256 && N > 64 && N % 16 == 0 ? "dot_gelu_q8_wk_i8_16x16x64" : "dot_wk_gelu_vec");
+            if (rc != HIPQ_ERR_UNSUPPORTED)
+                return rc;
+        }
+        if (M <= 256)
+            return HIPQ_ERR_UNSUPPORTED;
         OutMap om{0, N, 1};
         RowsU xu;
         xu.x = static_cast<const uint8_t*>(a);

@@ -562,11 +562,15 @@ int hipq_quantized_dot_bias_gelu_quantize(const hipq_dot_desc_t* d,
     if (rc)
         return rc;
     hipStream_t s = as_stream(stream);
-    // in the epilogue of the product, where the kernels that take it apply
-    if (dot_mfma_eligible(*d) && d->K % 16 == 0 && d->M > 256 && (reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && (reinterpret_cast<uintptr_t>(quant->out) & 15) == 0)
+    // in the epilogue of the product, where the kernels that take it apply: the ones for products too
+    // small to fill the chip, and from 257 rows on the tile kernels
+    const bool q16 = (reinterpret_cast<uintptr_t>(quant->out) & 15) == 0;
+    const bool small = packed_w && dot_gelu_wk_preferred(*d);
+    if (dot_mfma_eligible(*d) && d->K % 16 == 0 && (small || d->M > 256) && (reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && q16)
     {
         DotOperands o;
-        rc = dot_operands(*d, a, w, packed_w, ZeroPoints{nullptr, nullptr, d->a_t, d->b_t}, &o, s);
+        ZeroPoints zp{nullptr, nullptr, d->a_t, d->b_t};
+        rc = dot_operands(*d, a, w, packed_w, zp, &o, s);
         if (rc)
             return rc;
         Epilogue post = e;
@@ -574,8 +578,7 @@ int hipq_quantized_dot_bias_gelu_quantize(const hipq_dot_desc_t* d,
         post.post_zp = quant->zero_point;
         post.post_t = quant->quant_t;
         post.post_mode = quant->round_mode;
-        ZeroPoints zp{nullptr, nullptr, d->a_t, d->b_t};
-        rc = launch_rows_gelu_q8(a, d->a_t == HIPQ_U8, static_cast<const int8_t*>(o.w), o.wsum, d->M, static_cast<int32_t>(d->N), static_cast<int32_t>(d->K), zp, post, quant->out, s);
+        rc = launch_rows_gelu_q8(a, d->a_t == HIPQ_U8, static_cast<const int8_t*>(o.w), o.wfrag, o.wsum, d->M, static_cast<int32_t>(d->N), static_cast<int32_t>(d->K), zp, post, quant->out, s);
         if (rc != HIPQ_ERR_UNSUPPORTED)
             return rc;
     }
