@@ -661,8 +661,9 @@ HIPQ_API int hipq_batch_matmul_view_f32(const float* a,
  * hipq_softmax_scaled_f32 and hipq_batch_matmul_view_f32 in sequence; the [queries, keys] scores stay
  * on the compute unit.  Q is [queries, depth], K and V are [keys, depth] per batch element, addressed
  * like the views above (strides in elements); factor may be null (no Multiply); out may be null when
- * quant is given.  Returns HIPQ_ERR_UNSUPPORTED (nothing launched) unless keys == 128, depth == 64 and
- * queries is a multiple of 32: callers then run the three ops.  No counterpart as a single reference op. */
+ * quant is given.  Returns HIPQ_ERR_UNSUPPORTED (nothing launched) unless depth == 64 and either queries ==
+ * keys, up to 512 of them but not 64, or keys == 128 and queries is a multiple of 32: callers then run the three
+ * ops.  No counterpart as a single reference op. */
 typedef struct hipq_attention_view
 {
     int64_t batch_inner;

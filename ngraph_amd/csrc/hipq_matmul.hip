@@ -321,21 +321,24 @@ namespace hipq
         // ---- attention of one head in one kernel -------------------------------------------------------
         // out = BatchMatMul(Softmax(Multiply(BatchMatMulTranspose(Q, K), factor)), V), every op rounding
         // as the separate kernels round (the products through the same matrix instruction chain, the
-        // Softmax through softmax_piece with the same lanes on the same pieces), so the result equals
-        // the three launches bit for bit while the scores never leave the compute unit.
-        // A work item is 32 query rows of one head against its 128 keys of depth 64.  LDS: Q [32][64],
-        // K [128][64], V [128][64] as f32; the scores and probabilities [32][132] take K's place once K
-        // has been multiplied.  Rows of Q and K are swizzled by k ^ 4 (row % 16), rows of V by
-        // n ^ 16 (key % 4): fragment reads (16 rows x 4 consecutive k a wavefront) and the 16-byte
-        // writes touch every bank once, without padding, which is what lets two workgroups share a
-        // compute unit's 160 KB.
-        // A workgroup walks items: V is asked for when the item starts and laid into LDS after the
-        // scores, the next item's Q and K are asked for before the second product, and an item's
-        // results wait in registers until the next item's operands have arrived (loads and stores
-        // share one counter).
-        constexpr int AQ = 32, AKEYS = 128, AD = 64, ASP = AKEYS + 4;
-        constexpr size_t kAttnLdsBytes = static_cast<size_t>(AQ * AD + 2 * AKEYS * AD) * sizeof(float);
-        static_assert(AQ * ASP <= AKEYS * AD, "the scores must fit K's region");
+        // Softmax with the same lanes on the same elements as the Softmax kernel of that row length), so
+        // the result equals the three launches bit for bit while the scores never leave the compute unit.
+        // A workgroup takes RB blocks of 16 query rows of one head against all of its keys, depth 64.  Keys
+        // and values pass through one LDS region in chunks of 128 (those beyond the last key are neither
+        // multiplied nor summed), the next chunk on its way into registers while one is multiplied; every
+        // wavefront keeps the fragments of Q, which pass through the region that then holds the scores.
+        // Rows of Q, K and the scores are four floats longer than their data, so that fragment reads (16 rows
+        // x 4 consecutive k a wavefront) and the 16-byte writes touch every bank once at offsets known at
+        // compile time; rows of V are swizzled by n ^ 16 (key % 4).  32 rows x 384 keys are swizzled by
+        // column ^ 4 (row % 16) instead: without the four floats two workgroups fit a compute unit's LDS,
+        // and one multiplies while the other waits at a barrier or exponentiates (1440 items of 32 x 384:
+        // 112 us, with one workgroup a compute unit 133; the three launches 120).
+        // Bound by the f64 matrix instruction (64 cycles each) plus, not beside, the vector work of a SIMD:
+        // at 384 heads of 128 x 128 the instruction alone takes 20 us, the kernel 39 (with the swizzle
+        // computed for every fragment 42, as a resident grid that walks the items 42); 12 heads: 6.5 us
+        // (8 wavefronts on 32 rows 9.3; the three launches 18.5).
+        constexpr int AKEYS = 128, AD = 64; // keys of a chunk, depth
+        constexpr int AMAX = 512;          // keys
         struct AttnView
         {
             int64_t batch_inner;
@@ -344,209 +347,267 @@ namespace hipq
             int64_t v_outer, v_inner, ldv;
             int64_t o_outer, o_inner, ldo;
         };
-        struct AttnItem
+        // floats a row of Q, K and the scores is longer than its data; none: swizzled instead
+        constexpr int attn_pad(int rb, int chunks) { return rb == 2 && chunks == 3 ? 0 : 4; }
+        constexpr size_t attn_lds(int rb, int chunks)
         {
-            const float* Q;
-            const float* K;
-            const float* V;
-            int64_t o_base;
-        };
+            return (static_cast<size_t>(rb) * 16 * (AKEYS * chunks + attn_pad(rb, chunks)) + AKEYS * (AD + attn_pad(rb, chunks))) * sizeof(float);
+        }
 
-        __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                                                                                 const float* __restrict__ v, const float* __restrict__ factor,
-                                                                                                                 float* __restrict__ out, AttnView view, MatQuant mq, int32_t row_blocks,
-                                                                                                                 int32_t items)
+        // CH: chunks of keys; WHOLE: the keys fill them (a number known at compile time, and nothing to check)
+        template <int RB, int WAVES, int CH, bool WHOLE>
+        __global__ __launch_bounds__(WAVES * 64, 4) void attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+                                                                              const float* __restrict__ factor, float* __restrict__ out, AttnView view, MatQuant mq, int32_t queries,
+                                                                              int32_t keys_, int32_t row_blocks)
         {
-            extern __shared__ __attribute__((aligned(16))) float attn_lds[];
-            float* const Qs = attn_lds;
-            float* const Ks = Qs + AQ * AD;
-            float* const Vs = Ks + AKEYS * AD;
-            float* const Ss = Ks;
+            const int keys = WHOLE ? CH * AKEYS : keys_;
+            constexpr int QB = RB * 16;
+            constexpr int ROWS = WAVES * 4;      // rows that one piece a thread covers
+            constexpr int PIECES = AKEYS / ROWS; // 16-byte pieces a thread and chunk
+            constexpr int KB = 8 / WAVES;                            // 16-key blocks of a chunk a wavefront multiplies
+            constexpr int CB = RB * 4 >= WAVES ? RB * 4 / WAVES : 1; // 16 x 16 blocks of the context a wavefront owns
+            constexpr int PAD = attn_pad(RB, CH);
+            constexpr int pitch = CH * AKEYS + PAD, kpitch = AD + PAD; // of a row of scores, of a row of Q and K
+            static_assert(QB <= ROWS, "a piece of Q a thread");
+            extern __shared__ __attribute__((aligned(16))) float attn_lds_base[];
+            float* const Ss = attn_lds_base;
+            float* const KV = Ss + QB * pitch;
             const int tid = threadIdx.x;
-            const int lane = tid & 63, wave = tid >> 6;
+            const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
             const int r16 = lane & 15, kq = lane >> 4;
             const int64_t ldq = view.ldq, ldk = view.ldk, ldv = view.ldv, ldo = view.ldo;
             const bool scaled = factor != nullptr;
             const float c = scaled ? *factor : 1.0f;
             const int grid = static_cast<int>(gridDim.x);
             // (workgroups are dealt round-robin to the 8 XCDs: renumbered so that the row blocks of a head meet in one L2)
-            const int first = (grid & 7) == 0 ? (static_cast<int>(blockIdx.x) & 7) * (grid >> 3) + (static_cast<int>(blockIdx.x) >> 3) : static_cast<int>(blockIdx.x);
-            if (first >= items) // uniform
-                return;
+            const int t = (grid & 7) == 0 ? (static_cast<int>(blockIdx.x) & 7) * (grid >> 3) + (static_cast<int>(blockIdx.x) >> 3) : static_cast<int>(blockIdx.x);
+            const int rb = t % row_blocks;
+            const uint32_t batch = static_cast<uint32_t>(t / row_blocks);
             const uint32_t batch_inner = static_cast<uint32_t>(view.batch_inner < (1ll << 31) ? view.batch_inner : (1ll << 31));
-            auto item_at = [&](int t) -> AttnItem {
-                const int rb = t % row_blocks;
-                const uint32_t batch = static_cast<uint32_t>(t / row_blocks);
-                const int64_t bo = batch / batch_inner, bi = batch - bo * batch_inner;
-                return AttnItem{q + bo * view.q_outer + bi * view.q_inner + static_cast<int64_t>(rb) * AQ * ldq, k + bo * view.k_outer + bi * view.k_inner,
-                                v + bo * view.v_outer + bi * view.v_inner, bo * view.o_outer + bi * view.o_inner + static_cast<int64_t>(rb) * AQ * ldo};
-            };
-            // a thread's 16-byte pieces: row tid / 16 (+ 16 a piece), columns 4 (tid % 16) ..
+            const int64_t bo = batch / batch_inner, bi = batch - bo * batch_inner;
+            const float* const Q = q + bo * view.q_outer + bi * view.q_inner + static_cast<int64_t>(rb) * QB * ldq;
+            const float* const K = k + bo * view.k_outer + bi * view.k_inner;
+            const float* const V = v + bo * view.v_outer + bi * view.v_inner;
+            const int64_t o_base = bo * view.o_outer + bi * view.o_inner + static_cast<int64_t>(rb) * QB * ldo;
+            const int rows = min(QB, queries - rb * QB); // query rows that exist
+            // a thread's 16-byte pieces: row tid / 16 (+ ROWS a piece), columns 4 (tid % 16) ..
             const int prow = tid >> 4, pcol = (tid & 15) * 4;
-            f4 rq[2], rk[8], rv[8];
-            auto fetch_qk = [&](const AttnItem& w) {
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-                    rq[i] = *reinterpret_cast<const f4*>(w.Q + static_cast<int64_t>(prow + 16 * i) * ldq + pcol);
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    rk[i] = *reinterpret_cast<const f4*>(w.K + static_cast<int64_t>(prow + 16 * i) * ldk + pcol);
+            // (the compiler would compute every address of the loops below once and keep it: hundreds of registers.
+            // A value that it cannot see through makes it form them where they are used)
+            auto fresh = [](int x) {
+                asm volatile("" : "+v"(x));
+                return x;
             };
-            auto fetch_v = [&](const AttnItem& w) {
+            f4 rkv[PIECES];
+            auto fetch = [&](const float* from, int64_t ld, int chunk) {
+                const int row0 = chunk * AKEYS + fresh(tid >> 4);
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    rv[i] = *reinterpret_cast<const f4*>(w.V + static_cast<int64_t>(prow + 16 * i) * ldv + pcol);
+                for (int i = 0; i < PIECES; ++i)
+                {
+                    const int row = WHOLE ? row0 + ROWS * i : min(row0 + ROWS * i, keys - 1); // (keys past the last are not scored)
+                    rkv[i] = *reinterpret_cast<const f4*>(from + static_cast<int64_t>(row) * ld + pcol);
+                }
             };
-            auto put_qk = [&]() {
-                const int at = prow * AD + (pcol ^ (4 * prow)); // (row % 16 = tid / 16 for every piece of the thread)
+            auto swizzled = [](int col, int row) { return PAD ? col : col ^ (4 * (row & 15)); };
+            auto put_k = [&]() {
+                const int at = prow * kpitch + swizzled(pcol, prow); // (row % 16 = (tid / 16) % 16 for every piece of the thread)
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
-                    *reinterpret_cast<f4*>(Qs + at + i * 16 * AD) = rq[i];
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    *reinterpret_cast<f4*>(Ks + at + i * 16 * AD) = rk[i];
+                for (int i = 0; i < PIECES; ++i)
+                    *reinterpret_cast<f4*>(KV + at + i * ROWS * kpitch) = rkv[i];
             };
-            auto put_v = [&]() {
+            auto put_v = [&](int chunk) {
                 const int at = prow * AD + (pcol ^ (16 * (prow & 3))); // (key % 4 = (tid / 16) % 4 for every piece)
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    *reinterpret_cast<f4*>(Vs + at + i * 16 * AD) = rv[i];
-            };
-            const float qs = mq.out ? *mq.scale : 1.0f;
-            const int32_t qz = mq.out ? load_zp(mq.zero_point, mq.quant_t) : 0;
-            auto q1 = [&](float x) -> uint32_t {
-                return mq.quant_t == HIPQ_U8 ? static_cast<uint32_t>(quantize_one<float, uint8_t>(x, qs, static_cast<uint8_t>(qz), mq.mode))
-                                             : static_cast<uint32_t>(static_cast<uint8_t>(quantize_one<float, int8_t>(x, qs, static_cast<int8_t>(qz), mq.mode)));
-            };
-            // second product: block i, register e of lane (r16, kq) = row 16 i + 4 e + kq, column 16 wave + r16
-            float res[2][4];
-            auto store_item = [&](const AttnItem& w) {
-                if (out) // uniform
+                for (int i = 0; i < PIECES; ++i)
                 {
-#pragma unroll
-                    for (int i = 0; i < 2; ++i)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            out[w.o_base + static_cast<int64_t>(16 * i + 4 * e + kq) * ldo + 16 * wave + r16] = res[i][e];
-                }
-                if (mq.out) // uniform
-                {
-                    const bool rne = mq.mode == HIPQ_ROUND_NEAREST_TOWARD_EVEN; // uniform: the Quantize kernels' four-at-a-time arithmetic
-#pragma unroll
-                    for (int i = 0; i < 2; ++i)
-                    {
-                        uint32_t four = 0;
-                        if (rne)
-                        {
-                            const f4 x = f4{res[i][0], res[i][1], res[i][2], res[i][3]};
-                            four = mq.quant_t == HIPQ_U8 ? quantize4<uint8_t, true>(x, qs, static_cast<float>(qz), mq.mode) : quantize4<int8_t, true>(x, qs, static_cast<float>(qz), mq.mode);
-                        }
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            static_cast<uint8_t*>(mq.out)[w.o_base + static_cast<int64_t>(16 * i + 4 * e + kq) * ldo + 16 * wave + r16] =
-                                static_cast<uint8_t>(rne ? (four >> (8 * e)) & 0xFFu : q1(res[i][e]));
-                    }
+                    // (values past the last key meet zero probabilities: zeros themselves, whatever the last row holds)
+                    const f4 zero = f4{0.0f, 0.0f, 0.0f, 0.0f};
+                    *reinterpret_cast<f4*>(KV + at + i * ROWS * AD) = (WHOLE || chunk * AKEYS + prow + ROWS * i < keys) ? rkv[i] : zero;
                 }
             };
-
-            int t = first;
-            AttnItem cur = item_at(t);
-            AttnItem done = cur;
-            bool unsaved = false; // uniform
-            fetch_qk(cur);
-            for (;;)
             {
-                put_qk();
-                __syncthreads();
-                fetch_v(cur);
-                if (unsaved)
+                const f4 piece = *reinterpret_cast<const f4*>(Q + static_cast<int64_t>(min(prow, rows - 1)) * ldq + pcol); // (rows past the last are not stored)
+                fetch(K, ldk, 0);
+                if (QB == ROWS || prow < QB)
+                    *reinterpret_cast<f4*>(Ss + prow * kpitch + swizzled(pcol, prow)) = piece;
+                put_k();
+            }
+            // ---- scores, a chunk of keys at a time; this wavefront KB blocks of 16 keys of every chunk
+            float qf[RB][AD / 4];
+#pragma unroll
+            for (int ch = 0; ch < CH; ++ch)
+            {
+                __syncthreads(); // the chunk (and Q) is in LDS
+                if (ch + 1 < CH)
+                    fetch(K, ldk, ch + 1);
+                else
+                    fetch(V, ldv, 0);
+                const int swz = PAD ? 0 : fresh(4 * r16);
+                if (ch == 0)
                 {
-                    store_item(done);
-                    unsaved = false;
+#pragma unroll
+                    for (int s = 0; s < AD / 4; ++s)
+#pragma unroll
+                        for (int i = 0; i < RB; ++i)
+                            qf[i][s] = Ss[(16 * i + r16) * kpitch + ((4 * s) ^ swz) + kq];
                 }
-                // ---- scores: 32 x 128 over depth 64; this wavefront the 32 keys 32 wave .. as 2 x 2 blocks
-                d4 acc[2][2];
+                const int key0 = ch * AKEYS + wave * KB * 16;
+                d4 acc[RB][KB];
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
+                for (int i = 0; i < RB; ++i)
 #pragma unroll
-                    for (int j = 0; j < 2; ++j)
+                    for (int j = 0; j < KB; ++j)
                         acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+                const bool some = WHOLE || ch + 1 < CH || key0 < keys; // uniform
+                if (some)
                 {
-                    const float* const qa = Qs + r16 * AD + kq;
-                    const float* const kb = Ks + (32 * wave + r16) * AD + kq;
+                    const float* const kb = KV + (wave * KB * 16 + r16) * kpitch + kq;
 #pragma unroll
                     for (int s = 0; s < AD / 4; ++s)
                     {
-                        const int off = (4 * s) ^ (4 * r16);
-                        double ad[2], bd[2];
+                        double bd[KB];
 #pragma unroll
-                        for (int i = 0; i < 2; ++i)
+                        for (int j = 0; j < KB; ++j)
+                            bd[j] = static_cast<double>(kb[((4 * s) ^ swz) + j * 16 * kpitch]);
+#pragma unroll
+                        for (int i = 0; i < RB; ++i)
+#pragma unroll
+                            for (int j = 0; j < KB; ++j)
+                                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(qf[i][s]), bd[j], acc[i][j], 0, 0, 0);
+                    }
+                }
+                __syncthreads(); // every wavefront has read the chunk (and Q): the next one takes its place
+                if (some)
+                {
+#pragma unroll
+                    for (int i = 0; i < RB; ++i)
+#pragma unroll
+                        for (int j = 0; j < KB; ++j)
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                            {
+                                const int row = 4 * e + kq;
+                                Ss[(16 * i + row) * pitch + swizzled(key0 + 16 * j + r16, row)] = static_cast<float>(acc[i][j][e]);
+                            }
+                }
+                if (ch + 1 < CH)
+                    put_k();
+                else
+                    put_v(0);
+            }
+            __syncthreads();
+            // ---- Softmax: 32 lanes a row as in the Softmax kernel, two rows a wavefront at a time
+#pragma unroll
+            for (int it = 0; it < QB / WAVES / 2; ++it)
+            {
+                const int row = QB / WAVES * wave + 2 * it + (lane >> 5);
+                f4* const at = reinterpret_cast<f4*>(Ss + row * pitch + swizzled(4 * (lane & 31), row));
+                f4 p[CH];
+#pragma unroll
+                for (int i = 0; i < CH; ++i)
+                    p[i] = at[32 * i];
+                softmax_row<32, CH>(p, lane & 31, keys, scaled, c);
+#pragma unroll
+                for (int i = 0; i < CH; ++i)
+                    at[32 * i] = p[i]; // (zeros past the last key)
+            }
+            // ---- context over the keys, a chunk at a time: this wavefront's blocks are row blocks cr .. cr + CB - 1
+            // of column block cc; register e of lane (r16, kq) is row 4 e + kq, column r16 of a block
+            const int cc = wave & 3;
+            const int cr = WAVES == 4 ? 0 : (wave >> 2) * CB;
+            const bool has_context = RB * 4 >= WAVES || wave < RB * 4; // uniform
+            d4 ctx[CB];
+#pragma unroll
+            for (int i = 0; i < CB; ++i)
+                ctx[i] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int ch = 0; ch < CH; ++ch)
+            {
+                __syncthreads(); // the chunk of V (and the probabilities) are in LDS
+                if (ch + 1 < CH)
+                    fetch(V, ldv, ch + 1);
+                if (has_context)
+                {
+                    const int swz = PAD ? 0 : fresh(4 * r16);
+                    const float* const pa = Ss + (cr * 16 + r16) * pitch + kq + ch * AKEYS;
+                    const float* const vb = KV + kq * AD + ((16 * cc + r16) ^ (16 * kq));
+#pragma unroll
+                    for (int g = 0; g < AKEYS / 16; ++g)
+                        if (WHOLE || ch + 1 < CH || ch * AKEYS + g * 16 < keys) // uniform
                         {
-                            ad[i] = static_cast<double>(qa[off + i * 16 * AD]);
-                            bd[i] = static_cast<double>(kb[off + i * 16 * AD]);
+#pragma unroll
+                            for (int s = 4 * g; s < 4 * g + 4; ++s)
+                            {
+                                const double bd = static_cast<double>(vb[4 * s * AD]);
+#pragma unroll
+                                for (int i = 0; i < CB; ++i)
+                                    ctx[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(pa[((4 * s) ^ swz) + i * 16 * pitch]), bd, ctx[i], 0, 0, 0);
+                            }
                         }
-#pragma unroll
-                        for (int i = 0; i < 2; ++i)
-#pragma unroll
-                            for (int j = 0; j < 2; ++j)
-                                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ad[i], bd[j], acc[i][j], 0, 0, 0);
-                    }
                 }
-                __syncthreads(); // every wavefront has read K: the scores take its place
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            Ss[(16 * i + 4 * e + kq) * ASP + 32 * wave + 16 * j + r16] = static_cast<float>(acc[i][j][e]);
-                put_v();
-                __syncthreads();
-                // ---- Softmax of the rows: this wavefront rows 8 wave .., two at a time, 32 lanes a row
-#pragma unroll
-                for (int it = 0; it < 4; ++it)
+                if (ch + 1 < CH)
                 {
-                    f4* const piece = reinterpret_cast<f4*>(Ss + (8 * wave + 2 * it + (lane >> 5)) * ASP) + (lane & 31);
-                    *piece = softmax_piece<32>(*piece, true, scaled, c);
+                    __syncthreads(); // every wavefront has read the chunk
+                    put_v(ch + 1);
                 }
-                __syncthreads();
-                // the next item's Q and K
-                const int t_next = t + grid;
-                const bool more = t_next < items; // uniform
-                AttnItem next = cur;
-                if (more)
-                {
-                    next = item_at(t_next);
-                    fetch_qk(next);
-                }
-                // ---- context: 32 x 64 over the 128 keys; this wavefront columns 16 wave .. as 2 x 1 blocks
-                d4 ctx[2] = {d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}};
-                {
-                    const float* const pa = Ss + r16 * ASP + kq;
-                    const float* const vb = Vs + kq * AD + ((16 * wave + r16) ^ (16 * kq));
+            }
+            if (!has_context)
+                return;
+            const float qs = mq.out ? *mq.scale : 1.0f;
+            const int32_t qz = mq.out ? load_zp(mq.zero_point, mq.quant_t) : 0;
+            const bool rne = mq.mode == HIPQ_ROUND_NEAREST_TOWARD_EVEN; // uniform: the Quantize kernels' four-at-a-time arithmetic
 #pragma unroll
-                    for (int s = 0; s < AKEYS / 4; ++s)
-                    {
-                        const double bd = static_cast<double>(vb[4 * s * AD]);
-#pragma unroll
-                        for (int i = 0; i < 2; ++i)
-                            ctx[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(pa[4 * s + i * 16 * ASP]), bd, ctx[i], 0, 0, 0);
-                    }
-                }
-                __syncthreads(); // every wavefront has read Q's, the probabilities' and V's regions
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < CB; ++i)
+            {
+                const f4 x = f4{static_cast<float>(ctx[i][0]), static_cast<float>(ctx[i][1]), static_cast<float>(ctx[i][2]), static_cast<float>(ctx[i][3])};
+                uint32_t four = 0;
+                if (mq.out && rne)
+                    four = mq.quant_t == HIPQ_U8 ? quantize4<uint8_t, true>(x, qs, static_cast<float>(qz), mq.mode) : quantize4<int8_t, true>(x, qs, static_cast<float>(qz), mq.mode);
+                else if (mq.out)
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        res[i][e] = static_cast<float>(ctx[i][e]);
-                done = cur;
-                if (!more)
-                    break;
-                unsaved = true;
-                cur = next;
-                t = t_next;
+                        four |= (mq.quant_t == HIPQ_U8 ? static_cast<uint32_t>(quantize_one<float, uint8_t>(x[e], qs, static_cast<uint8_t>(qz), mq.mode))
+                                                       : static_cast<uint32_t>(static_cast<uint8_t>(quantize_one<float, int8_t>(x[e], qs, static_cast<int8_t>(qz), mq.mode))))
+                                << (8 * e);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                {
+                    const int row = 16 * (cr + i) + 4 * e + kq;
+                    if (row >= rows)
+                        continue;
+                    const int64_t at = o_base + static_cast<int64_t>(row) * ldo + 16 * cc + r16;
+                    if (out) // uniform
+                        out[at] = x[e];
+                    if (mq.out) // uniform
+                        static_cast<uint8_t*>(mq.out)[at] = static_cast<uint8_t>(four >> (8 * e));
+                }
             }
-            store_item(done);
+        }
+
+        template <int RB, int WAVES>
+        int launch_attention(const float* q, const float* k, const float* v, const float* factor, float* out, const AttnView& av, const MatQuant& mq, int64_t batch, int64_t queries, int64_t keys,
+                             hipStream_t s)
+        {
+            const int ch = static_cast<int>((keys + AKEYS - 1) / AKEYS);
+            const auto kernel = keys == AKEYS ? attention_f32_kernel<RB, WAVES, 1, true>
+                                : ch == 1     ? attention_f32_kernel<RB, WAVES, 1, false>
+                                : ch == 2     ? attention_f32_kernel<RB, WAVES, 2, false>
+                                : ch == 3     ? attention_f32_kernel<RB, WAVES, 3, false>
+                                              : attention_f32_kernel<RB, WAVES, 4, false>;
+            static bool configured[16][5] = {};
+            const int which = keys == AKEYS ? 0 : ch;
+            int dev = 0;
+            HIPQ_HIP(hipGetDevice(&dev));
+            if (dev >= 0 && dev < 16 && !configured[dev][which])
+            {
+                HIPQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+                configured[dev][which] = true;
+            }
+            const int64_t row_blocks = (queries + RB * 16 - 1) / (RB * 16);
+            HIPQ_REQUIRE(batch * row_blocks < (1ll << 31) - (1 << 20), "too many work items for one launch");
+            kernel<<<static_cast<unsigned>(batch * row_blocks), WAVES * 64, attn_lds(RB, ch), s>>>(q, k, v, factor, out, av, mq, static_cast<int32_t>(queries), static_cast<int32_t>(keys),
+                                                                                                    static_cast<int32_t>(row_blocks));
+            return check_launch("attention_f32");
         }
     }
 }
@@ -619,8 +680,10 @@ int hipq_attention_f32(const float* q, const float* k, const float* v, const flo
 {
     HIPQ_REQUIRE(view, "null view");
     HIPQ_REQUIRE(batch >= 0 && queries >= 0 && keys >= 0 && depth >= 0, "negative extent");
-    if (keys != AKEYS || depth != AD || queries % AQ != 0)
-        return fail(HIPQ_ERR_UNSUPPORTED, "the one-kernel attention takes 128 keys of depth 64 and query rows in multiples of 32 (run the three ops otherwise)");
+    // (64 keys are one tile of the products' own kernel: the three ops)
+    const bool self = queries == keys && keys > 0 && keys <= AMAX && keys != 64;
+    if (depth != AD || !(self || (keys == AKEYS && queries % 32 == 0)))
+        return fail(HIPQ_ERR_UNSUPPORTED, "the one-kernel attention takes depth 64 and as many queries as keys, up to 512 but not 64, or 128 keys and query rows in multiples of 32 (run the three ops otherwise)");
     if (batch == 0 || queries == 0)
         return HIPQ_OK;
     MatQuant mq{nullptr, nullptr, nullptr, HIPQ_I8, HIPQ_ROUND_NEAREST_TOWARD_EVEN};
@@ -639,21 +702,14 @@ int hipq_attention_f32(const float* q, const float* k, const float* v, const flo
     auto rows16 = [](const float* p, int64_t ld, int64_t outer, int64_t inner) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0 && ld % 4 == 0 && outer % 4 == 0 && inner % 4 == 0; };
     HIPQ_REQUIRE(rows16(q, view->ldq, view->q_outer, view->q_inner) && rows16(k, view->ldk, view->k_outer, view->k_inner) && rows16(v, view->ldv, view->v_outer, view->v_inner),
                  "rows of Q, K and V must start 16-byte aligned");
-    const int64_t row_blocks = queries / AQ;
-    HIPQ_REQUIRE(batch * row_blocks < (1ll << 31) - (1 << 20), "too many work items for one launch");
-    static bool configured[16] = {};
-    int dev = 0;
-    HIPQ_HIP(hipGetDevice(&dev));
-    if (dev >= 0 && dev < 16 && !configured[dev])
-    {
-        HIPQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(attention_f32_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kAttnLdsBytes)));
-        configured[dev] = true;
-    }
     const AttnView av{view->batch_inner, view->q_outer, view->q_inner, view->ldq, view->k_outer, view->k_inner, view->ldk,
                       view->v_outer, view->v_inner, view->ldv, view->o_outer, view->o_inner, view->ldo};
-    const int64_t items = batch * row_blocks;
-    // two workgroups a compute unit (their LDS fits twice), each walking its share of the items
-    const int64_t grid = std::min<int64_t>(items, 2ll * device_compute_units());
-    attention_f32_kernel<<<static_cast<unsigned>(grid), 256, kAttnLdsBytes, as_stream(stream)>>>(q, k, v, factor, out, av, mq, static_cast<int32_t>(row_blocks), static_cast<int32_t>(items));
-    return check_launch("attention_f32");
+    // 16 query rows a workgroup, or 32: two blocks of rows share the fragments of K, the chunks staged and the
+    // barriers, so that an item of 32 rows costs about 1.75 items of 16, measured from 12 x 128 x 128 to 120 x
+    // 384 x 384; whichever leaves the fullest compute unit with less
+    const int64_t cus = device_compute_units();
+    auto items_a_cu = [&](int64_t rows) { return (batch * ((queries + rows - 1) / rows) + cus - 1) / cus; };
+    if (4 * items_a_cu(16) <= 7 * items_a_cu(32))
+        return launch_attention<1, 8>(q, k, v, factor, out, av, mq, batch, queries, keys, as_stream(stream));
+    return launch_attention<2, 8>(q, k, v, factor, out, av, mq, batch, queries, keys, as_stream(stream));
 }

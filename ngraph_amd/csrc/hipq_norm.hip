@@ -48,12 +48,66 @@ namespace hipq
         constexpr int kRowVecs = 8; // float4 pieces of a row a lane keeps: rows up to 64 * 4 * 8 = 2048 elements
 
         // out = exp(x - max(x)) / sum(exp(x - max(x))) along contiguous rows
-        // (src/ngraph/runtime/reference/softmax.hpp:31-57); one wavefront a row.
-        template <bool CACHED>
-        __global__ __launch_bounds__(256) void softmax_rows_kernel(const float* __restrict__ in, const float* __restrict__ factor, float* __restrict__ out, int64_t rows, int32_t cols)
+        // (src/ngraph/runtime/reference/softmax.hpp:31-57).  W lanes own a row, P pieces of four elements
+        // each: 64 / W rows a wavefront, W and P the smallest that hold the row, so that the lanes have work
+        // (an attention row of 128 is 32 pieces, one of 384 three times 32).  `vec`: rows start 16-byte
+        // aligned; otherwise (any length) the elements of a piece are loaded one by one, still once.
+        template <int W, int P>
+        __global__ __launch_bounds__(256) void softmax_rows_kernel(const float* __restrict__ in, const float* __restrict__ factor, float* __restrict__ out, int64_t rows, int32_t cols,
+                                                                   int vec)
         {
             // factor (may be null): the input is Multiply(x, factor) -- the product is rounded to f32 as the
             // Multiply op would round it
+            const bool scaled = factor != nullptr;
+            const float c = scaled ? *factor : 1.0f;
+            const int lane = threadIdx.x & 63;
+            const int sub = lane & (W - 1);
+            const int64_t row = (static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * (64 / W) + lane / W;
+            const int live = row < rows ? cols : 0;
+            const float* const x = in + row * cols;
+            float* const y = out + row * cols;
+            f4 v[P];
+#pragma unroll
+            for (int i = 0; i < P; ++i)
+            {
+                const int at = 4 * (W * i + sub);
+                v[i] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+                if (vec) // uniform
+                {
+                    if (at < live)
+                        v[i] = *reinterpret_cast<const f4*>(x + at);
+                }
+                else
+                {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (at + e < live)
+                            v[i][e] = x[at + e];
+                }
+            }
+            softmax_row<W, P>(v, sub, live, scaled, c);
+#pragma unroll
+            for (int i = 0; i < P; ++i)
+            {
+                const int at = 4 * (W * i + sub);
+                if (vec) // uniform
+                {
+                    if (at < live)
+                        *reinterpret_cast<f4*>(y + at) = v[i];
+                }
+                else
+                {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (at + e < live)
+                            y[at + e] = v[i][e];
+                }
+            }
+        }
+
+        // rows longer than that: one wavefront a row, read three times
+        __global__ __launch_bounds__(256) void softmax_long_rows_kernel(const float* __restrict__ in, const float* __restrict__ factor, float* __restrict__ out, int64_t rows, int32_t cols)
+        {
             const bool scaled = factor != nullptr;
             const float c = scaled ? *factor : 1.0f;
             const int lane = threadIdx.x & 63;
@@ -62,80 +116,17 @@ namespace hipq
                 return;
             const float* x = in + row * cols;
             float* y = out + row * cols;
-            if (CACHED) // cols % 4 == 0, 16-byte aligned rows, cols <= 2048
-            {
-                const int vecs = cols >> 2;
-                f4 v[kRowVecs];
-                float m = -INFINITY;
-#pragma unroll
-                for (int i = 0; i < kRowVecs; ++i)
-                {
-                    const int j = i * 64 + lane;
-                    if (j < vecs)
-                    {
-                        v[i] = reinterpret_cast<const f4*>(x)[j];
-                        if (scaled)
-                            v[i] = f4{__fmul_rn(v[i][0], c), __fmul_rn(v[i][1], c), __fmul_rn(v[i][2], c), __fmul_rn(v[i][3], c)};
-                        m = fmaxf(fmaxf(fmaxf(m, v[i][0]), fmaxf(v[i][1], v[i][2])), v[i][3]);
-                    }
-                }
-                m = wave_max(m);
-                float s = 0.0f;
-#pragma unroll
-                for (int i = 0; i < kRowVecs; ++i)
-                    if (i * 64 + lane < vecs)
-                    {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                        {
-                            v[i][e] = expf(v[i][e] - m);
-                            s += v[i][e];
-                        }
-                    }
-                s = wave_sum(s);
-#pragma unroll
-                for (int i = 0; i < kRowVecs; ++i)
-                {
-                    const int j = i * 64 + lane;
-                    if (j < vecs)
-                        reinterpret_cast<f4*>(y)[j] = f4{v[i][0] / s, v[i][1] / s, v[i][2] / s, v[i][3] / s};
-                }
-            }
-            else
-            {
-                auto at = [&](int j) { return scaled ? __fmul_rn(x[j], c) : x[j]; };
-                float m = -INFINITY;
-                for (int j = lane; j < cols; j += 64)
-                    m = fmaxf(m, at(j));
-                m = wave_max(m);
-                float s = 0.0f;
-                for (int j = lane; j < cols; j += 64)
-                    s += expf(at(j) - m);
-                s = wave_sum(s);
-                for (int j = lane; j < cols; j += 64)
-                    y[j] = expf(at(j) - m) / s;
-            }
-        }
-
-        // short rows (at most W float4 pieces, W = 32, 16 or 8 lanes): 64 / W rows a wavefront, one
-        // piece a lane, so that every lane has work (an attention row of 128 is 32 pieces)
-        template <int W>
-        __global__ __launch_bounds__(256) void softmax_short_rows_kernel(const float* __restrict__ in, const float* __restrict__ factor, float* __restrict__ out, int64_t rows, int32_t cols)
-        {
-            const bool scaled = factor != nullptr;
-            const float c = scaled ? *factor : 1.0f;
-            constexpr int RPW = 64 / W;
-            const int lane = threadIdx.x & 63;
-            const int sub = lane & (W - 1);
-            const int64_t row = (static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * RPW + lane / W;
-            const int vecs = cols >> 2;
-            const bool live = row < rows && sub < vecs;
-            f4 v = f4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-            if (live)
-                v = reinterpret_cast<const f4*>(in + row * cols)[sub];
-            v = softmax_piece<W>(v, live, scaled, c);
-            if (live)
-                reinterpret_cast<f4*>(out + row * cols)[sub] = v;
+            auto at = [&](int j) { return scaled ? __fmul_rn(x[j], c) : x[j]; };
+            float m = -INFINITY;
+            for (int j = lane; j < cols; j += 64)
+                m = fmaxf(m, at(j));
+            m = wave_max(m);
+            float s = 0.0f;
+            for (int j = lane; j < cols; j += 64)
+                s += expf(at(j) - m);
+            s = wave_sum(s);
+            for (int j = lane; j < cols; j += 64)
+                y[j] = expf(at(j) - m) / s;
         }
 
         // the same over a strided axis: the tensor is [outer][axis][inner], one lane a column (o, i)
@@ -326,25 +317,30 @@ static int launch_softmax(const float* in, const float* factor, float* out, int6
     hipStream_t s = as_stream(stream);
     if (inner == 1)
     {
-        const bool cached = axis % 4 == 0 && axis <= 64 * 4 * kRowVecs && aligned16(in) && aligned16(out);
-        if (cached && axis <= 128)
-        {
-            const int w = axis > 64 ? 32 : (axis > 32 ? 16 : 8);
-            const int64_t rows_per_block = 4 * (64 / w);
-            const unsigned blocks = static_cast<unsigned>((outer + rows_per_block - 1) / rows_per_block);
-            if (w == 32)
-                softmax_short_rows_kernel<32><<<blocks, 256, 0, s>>>(in, factor, out, outer, static_cast<int32_t>(axis));
-            else if (w == 16)
-                softmax_short_rows_kernel<16><<<blocks, 256, 0, s>>>(in, factor, out, outer, static_cast<int32_t>(axis));
-            else
-                softmax_short_rows_kernel<8><<<blocks, 256, 0, s>>>(in, factor, out, outer, static_cast<int32_t>(axis));
-            return check_launch("softmax_rows");
-        }
-        const unsigned grid = static_cast<unsigned>((outer + 3) / 4);
-        if (cached)
-            softmax_rows_kernel<true><<<grid, 256, 0, s>>>(in, factor, out, outer, static_cast<int32_t>(axis));
+        const int32_t cols = static_cast<int32_t>(axis);
+        const int vec = axis % 4 == 0 && aligned16(in) && aligned16(out);
+        auto rows_with = [&](auto kernel, int lanes) {
+            const int64_t a_block = 4 * (64 / lanes);
+            kernel<<<static_cast<unsigned>((outer + a_block - 1) / a_block), 256, 0, s>>>(in, factor, out, outer, cols, vec);
+        };
+        if (axis <= 32)
+            rows_with(softmax_rows_kernel<8, 1>, 8);
+        else if (axis <= 64)
+            rows_with(softmax_rows_kernel<16, 1>, 16);
+        else if (axis <= 128)
+            rows_with(softmax_rows_kernel<32, 1>, 32);
+        else if (axis <= 256)
+            rows_with(softmax_rows_kernel<32, 2>, 32);
+        else if (axis <= 384)
+            rows_with(softmax_rows_kernel<32, 3>, 32);
+        else if (axis <= 512)
+            rows_with(softmax_rows_kernel<32, 4>, 32);
+        else if (axis <= 1024)
+            rows_with(softmax_rows_kernel<64, 4>, 64);
+        else if (axis <= 64 * 4 * kRowVecs)
+            rows_with(softmax_rows_kernel<64, kRowVecs>, 64);
         else
-            softmax_rows_kernel<false><<<grid, 256, 0, s>>>(in, factor, out, outer, static_cast<int32_t>(axis));
+            softmax_long_rows_kernel<<<static_cast<unsigned>((outer + 3) / 4), 256, 0, s>>>(in, factor, out, outer, cols);
         return check_launch("softmax_rows");
     }
     softmax_strided_kernel<<<static_cast<unsigned>((outer * inner + 255) / 256), 256, 0, s>>>(in, factor, out, outer, static_cast<int32_t>(axis), inner);

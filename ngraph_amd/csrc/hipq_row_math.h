@@ -10,47 +10,92 @@ namespace hipq
 {
     typedef float row_f4 __attribute__((ext_vector_type(4)));
 
-    // reductions over aligned groups of W lanes of a wavefront
+    // Reductions over aligned groups of W lanes of a wavefront: a butterfly whose distance halves from W / 2
+    // down, every lane ending with the result.  Data-parallel-primitive moves and the half-wavefront swaps
+    // instead of shuffles: a shuffle goes through LDS, and the six of a row in sequence are what a short row
+    // waits for (LayerNorm of 128 rows of 768: 4.37 us with shuffles, 4.11 so; Softmax of 7880 rows of 197,
+    // with its single pass over unaligned rows: 7.30, 6.10).
+    template <int CTRL>
+    __device__ __forceinline__ float dpp_move(float v)
+    {
+        const int x = __builtin_bit_cast(int, v);
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(x, x, CTRL, 0xf, 0xf, false));
+    }
+    template <int W, typename F>
+    __device__ __forceinline__ float butterfly(float v, F combine)
+    {
+        // distances 32 and 16: v_permlane*_swap of two copies leaves the lower halves in one register and the
+        // upper ones in the other (the two wait states are the ones a freshly written operand needs)
+        if (W >= 64)
+        {
+            float a = v, b = v;
+            asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+            v = combine(a, b);
+        }
+        if (W >= 32)
+        {
+            float a = v, b = v;
+            asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+            v = combine(a, b);
+        }
+        // distance 8: a rotation within 16 lanes; 4: the same, since what the lanes hold has period 8 by then. In
+        // groups of 8 a mirror of eight lanes and one of four
+        if (W >= 16)
+        {
+            v = combine(v, dpp_move<0x128>(v)); // row_ror:8
+            v = combine(v, dpp_move<0x124>(v)); // row_ror:4
+        }
+        else if (W == 8)
+            v = combine(v, dpp_move<0x1b>(dpp_move<0x141>(v))); // row_half_mirror (l ^ 7), then quad_perm:[3,2,1,0] (l ^ 3)
+        if (W >= 4)
+            v = combine(v, dpp_move<0x4e>(v)); // quad_perm:[2,3,0,1]
+        return combine(v, dpp_move<0xb1>(v));  // quad_perm:[1,0,3,2]
+    }
     template <int W = 64>
     __device__ __forceinline__ float wave_max(float v)
     {
-#pragma unroll
-        for (int o = W / 2; o > 0; o >>= 1)
-            v = fmaxf(v, __shfl_xor(v, o));
-        return v;
+        return butterfly<W>(v, [](float a, float b) { return fmaxf(a, b); });
     }
     template <int W = 64>
     __device__ __forceinline__ float wave_sum(float v)
     {
-#pragma unroll
-        for (int o = W / 2; o > 0; o >>= 1)
-            v += __shfl_xor(v, o);
-        return v;
+        return butterfly<W>(v, [](float a, float b) { return a + b; });
     }
 
-    // Softmax of a row of at most 4 W elements held one 16-byte piece a lane by W neighbouring lanes
+    // Softmax of a row held in 16-byte pieces by W neighbouring lanes, lane l pieces l, l + W, ..
     // (src/ngraph/runtime/reference/softmax.hpp:31-57): exp(x - max) / sum(exp(x - max)); with `scaled`
-    // the input is Multiply(x, c), the product rounded to f32 as the Multiply op rounds it.  Lanes
-    // past the row's end pass live = false.  The sum: a lane's four terms in order, then the lanes'
-    // sums through the butterfly of wave_sum.
-    template <int W>
-    __device__ __forceinline__ row_f4 softmax_piece(row_f4 v, bool live, bool scaled, float c)
+    // the input is Multiply(x, c), the product rounded to f32 as the Multiply op rounds it.  `live` of the
+    // row's elements exist (the others come out as zero, or NaN in a row that is NaN throughout).  The sum:
+    // a lane's terms in order, then the lanes' sums through the butterfly of wave_sum.
+    template <int W, int P>
+    __device__ __forceinline__ void softmax_row(row_f4 (&v)[P], int lane, int live, bool scaled, float c)
     {
-        if (!live)
-            v = row_f4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-        else if (scaled)
-            v = row_f4{__fmul_rn(v[0], c), __fmul_rn(v[1], c), __fmul_rn(v[2], c), __fmul_rn(v[3], c)};
-        const float m = wave_max<W>(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])));
+        float m = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < P; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+            {
+                const float x = scaled ? __fmul_rn(v[i][e], c) : v[i][e];
+                v[i][e] = 4 * (W * i + lane) + e < live ? x : -INFINITY;
+                m = fmaxf(m, v[i][e]);
+            }
+        m = wave_max<W>(m);
         float s = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-        {
-            v[e] = live ? expf(v[e] - m) : 0.0f;
-            s += v[e];
-        }
+        for (int i = 0; i < P; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+            {
+                v[i][e] = expf(v[i][e] - m);
+                s += v[i][e];
+            }
         s = wave_sum<W>(s);
-        return row_f4{v[0] / s, v[1] / s, v[2] / s, v[3] / s};
+#pragma unroll
+        for (int i = 0; i < P; ++i)
+            v[i] = row_f4{v[i][0] / s, v[i][1] / s, v[i][2] / s, v[i][3] / s};
     }
+
     // a / b rounded as the division rounds it, from r = fl(1 / b): q0 = a r, e = a - b q0 (exact in a fused
     // multiply-add), q = q0 + e r -- three instructions where the division sequence takes eleven.
     // (Markstein's correction: with a correctly rounded reciprocal the result is the correctly rounded
