@@ -186,15 +186,21 @@ namespace hipq
         // (src/ngraph/op/layer_norm.cpp:96-139 with builder::mean / builder::variance,
         // src/ngraph/builder/reduce_ops.cpp:68-124): mean = sum(x) / n, var = sum((x - mean)^2) / n,
         // out = (x - mean) / sqrt(var + eps) * scale + bias.  One wavefront a row.
-        template <bool CACHED>
-        __global__ __launch_bounds__(256) void layer_norm_kernel(const float* __restrict__ in, const float* __restrict__ addend, const float* __restrict__ scale,
-                                                                 const float* __restrict__ bias, float* __restrict__ out, QuantOut qo, float* __restrict__ mean_out,
-                                                                 float* __restrict__ var_out, int64_t rows, int32_t cols, float eps)
+        // P: 16-byte pieces a lane keeps of its row (0: a row of any length and alignment, re-read), ROWS: rows
+        // a workgroup.  A short tensor is bound by the chain load, sum, sum of squares, store: everything that
+        // does not hang on the row (scale, bias, the quantizer's parameters) is fetched beside it, and up to
+        // four rows a compute unit each take a workgroup of their own, spread over the chip (128 rows of 768:
+        // 3.55 us, with four rows a workgroup and the parameters fetched where they are used 4.11); a tall one
+        // is a stream (4096 rows of 768: 41 MB in 8.4 us).
+        template <int P, int ROWS>
+        __global__ __launch_bounds__(64 * ROWS) void layer_norm_kernel(const float* __restrict__ in, const float* __restrict__ addend, const float* __restrict__ scale,
+                                                                       const float* __restrict__ bias, float* __restrict__ out, QuantOut qo, float* __restrict__ mean_out,
+                                                                       float* __restrict__ var_out, int64_t rows, int32_t cols, float eps)
         {
             // addend (may be null): the input is Add(in, addend), the sum rounded to f32 as the Add op rounds it;
             // qo.out (may be null): Quantize of the result beside it
             const int lane = threadIdx.x & 63;
-            const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+            const int64_t row = static_cast<int64_t>(blockIdx.x) * ROWS + (threadIdx.x >> 6);
             if (row >= rows)
                 return;
             const float* x = in + row * cols;
@@ -203,27 +209,39 @@ namespace hipq
             const float n = static_cast<float>(cols);
             const float qs = qo.out ? *qo.scale : 1.0f;
             const int32_t qz = qo.out ? load_zp(qo.zero_point, qo.quant_t) : 0;
-            if (CACHED)
+            if (P > 0)
             {
                 const int vecs = cols >> 2;
-                f4 v[kRowVecs];
+                f4 v[P > 0 ? P : 1], w[P > 0 ? P : 1], sc[P > 0 ? P : 1], bi[P > 0 ? P : 1];
+#pragma unroll
+                for (int i = 0; i < P; ++i)
+                {
+                    // (lanes past the row's end fetch its first piece and count for nothing)
+                    const int j = i * 64 + lane < vecs ? i * 64 + lane : 0;
+                    v[i] = reinterpret_cast<const f4*>(x)[j];
+                    if (x2) // uniform
+                        w[i] = reinterpret_cast<const f4*>(x2)[j];
+                    sc[i] = f4{1.0f, 1.0f, 1.0f, 1.0f};
+                    bi[i] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+                    if (scale) // uniform
+                    {
+                        sc[i] = reinterpret_cast<const f4*>(scale)[j];
+                        bi[i] = reinterpret_cast<const f4*>(bias)[j];
+                    }
+                }
                 float s = 0.0f;
 #pragma unroll
-                for (int i = 0; i < kRowVecs; ++i)
+                for (int i = 0; i < P; ++i)
+                {
+                    if (x2)
+                        v[i] = f4{__fadd_rn(v[i][0], w[i][0]), __fadd_rn(v[i][1], w[i][1]), __fadd_rn(v[i][2], w[i][2]), __fadd_rn(v[i][3], w[i][3])};
                     if (i * 64 + lane < vecs)
-                    {
-                        v[i] = reinterpret_cast<const f4*>(x)[i * 64 + lane];
-                        if (x2)
-                        {
-                            const f4 w = reinterpret_cast<const f4*>(x2)[i * 64 + lane];
-                            v[i] = f4{__fadd_rn(v[i][0], w[0]), __fadd_rn(v[i][1], w[1]), __fadd_rn(v[i][2], w[2]), __fadd_rn(v[i][3], w[3])};
-                        }
                         s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
-                    }
+                }
                 const float mean = __fdiv_rn(wave_sum(s), n);
                 float q = 0.0f;
 #pragma unroll
-                for (int i = 0; i < kRowVecs; ++i)
+                for (int i = 0; i < P; ++i)
                     if (i * 64 + lane < vecs)
                     {
 #pragma unroll
@@ -241,19 +259,17 @@ namespace hipq
                 const float rsd = __fdiv_rn(1.0f, sd);
                 const bool by_reciprocal = sd > 1e-30f && sd < 1e30f; // uniform
 #pragma unroll
-                for (int i = 0; i < kRowVecs; ++i)
+                for (int i = 0; i < P; ++i)
                 {
                     const int j = i * 64 + lane;
                     if (j < vecs)
                     {
                         f4 r;
-                        const f4 sc = scale ? reinterpret_cast<const f4*>(scale)[j] : f4{1.0f, 1.0f, 1.0f, 1.0f};
-                        const f4 bi = scale ? reinterpret_cast<const f4*>(bias)[j] : f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
                         {
                             const float nv = by_reciprocal ? div_by_reciprocal(v[i][e], sd, rsd) : __fdiv_rn(v[i][e], sd);
-                            r[e] = scale ? __fadd_rn(__fmul_rn(nv, sc[e]), bi[e]) : nv;
+                            r[e] = scale ? __fadd_rn(__fmul_rn(nv, sc[i][e]), bi[i][e]) : nv;
                         }
                         reinterpret_cast<f4*>(y)[j] = r;
                         if (qo.out)
@@ -421,12 +437,22 @@ static int launch_layer_norm(const float* in, const float* addend, const float* 
         return rc;
     const bool cached = cols % 4 == 0 && cols <= 64 * 4 * kRowVecs && aligned16(in) && aligned16(out) && (!scale || (aligned16(scale) && aligned16(bias))) &&
                         (!addend || aligned16(addend)) && (!qo.out || (reinterpret_cast<uintptr_t>(qo.out) & 3) == 0);
-    const unsigned grid = static_cast<unsigned>((rows + 3) / 4);
     hipStream_t s = as_stream(stream);
-    if (cached)
-        layer_norm_kernel<true><<<grid, 256, 0, s>>>(in, addend, scale, bias, out, qo, mean, var, rows, static_cast<int32_t>(cols), static_cast<float>(epsilon));
+    auto rows_with = [&](auto kernel, int a_block) {
+        kernel<<<static_cast<unsigned>((rows + a_block - 1) / a_block), 64 * a_block, 0, s>>>(in, addend, scale, bias, out, qo, mean, var, rows, static_cast<int32_t>(cols),
+                                                                                              static_cast<float>(epsilon));
+    };
+    const bool few = rows <= 4 * static_cast<int64_t>(device_compute_units());
+    if (!cached)
+        rows_with(layer_norm_kernel<0, 4>, 4);
+    else if (cols <= 512)
+        few ? rows_with(layer_norm_kernel<2, 1>, 1) : rows_with(layer_norm_kernel<2, 4>, 4);
+    else if (cols <= 768)
+        few ? rows_with(layer_norm_kernel<3, 1>, 1) : rows_with(layer_norm_kernel<3, 4>, 4);
+    else if (cols <= 1024)
+        few ? rows_with(layer_norm_kernel<4, 1>, 1) : rows_with(layer_norm_kernel<4, 4>, 4);
     else
-        layer_norm_kernel<false><<<grid, 256, 0, s>>>(in, addend, scale, bias, out, qo, mean, var, rows, static_cast<int32_t>(cols), static_cast<float>(epsilon));
+        few ? rows_with(layer_norm_kernel<kRowVecs, 1>, 1) : rows_with(layer_norm_kernel<kRowVecs, 4>, 4);
     return check_launch("layer_norm_rows");
 }
 
