@@ -4,13 +4,15 @@
 // the nGraph tree: true IEEE division by the scale, the reference's floor/ceil rounding formulas,
 // zero point added in REAL, clamp in REAL, then the cast.
 //
-// Two kernel families:
+// Three kernel families:
 //   *_vec4    f32 <-> {i8,u8}, scale laid along one run of adjacent axes (or scalar) and the
 //             innermost non-axis extent a multiple of 4.  Each lane moves groups of 4 elements:
 //             one 16-byte load/store on the f32 side, one 4-byte store/load on the quantized side,
 //             lane-contiguous, so a wavefront touches 1 KiB + 256 B of consecutive memory per step.
-//   *_generic every other case (f64, i32, ragged inner extent, scattered axes): one element per
-//             lane, coordinates recovered with 64-bit div/mod.
+//   *_ragged  the same types and the same accesses where a group of 4 may reach into the next row of
+//             the scale table (an inner extent that is no multiple of 4) or past the end.
+//   *_generic every other case (f64, i32, scattered axes): one element per lane, coordinates
+//             recovered with 64-bit div/mod.
 #include "hipq_common.h"
 #include "hipq_index_div.h"
 #include "hipq_quant_math.h"
@@ -97,7 +99,10 @@ namespace hipq
     }
 
     // Groups a lane handles per launch, one wavefront-contiguous step of 256 groups apart (measured
-    // on f32[64,1024,1024]: 3 is best for Quantize, 2 for Dequantize).
+    // on f32[64,1024,1024]: 3 is best for Quantize, 2 for Dequantize).  A short tensor, whose steps do
+    // not fill the compute units eight times, takes one: it waits for one load and not for bandwidth,
+    // and shorter workgroups spread over more compute units (both directions of f32[13, 1, 16868]: 5.34
+    // us with the long ones, 4.12 so).
     constexpr int kQuantUnroll = 3;
     constexpr int kDequantUnroll = 2;
 
@@ -110,7 +115,7 @@ namespace hipq
     {
         return run_index(v, ROW_UNIFORM ? first_group_of_step : g);
     }
-    template <typename QUANT, bool RNE, bool ROW_UNIFORM>
+    template <typename QUANT, bool RNE, bool ROW_UNIFORM, int UNROLL>
     __global__ __launch_bounds__(256) void quantize_vec4_kernel(const f32x4* __restrict__ in,
                                                                 const float* __restrict__ scale,
                                                                 const QUANT* __restrict__ zp,
@@ -119,14 +124,13 @@ namespace hipq
                                                                 RunView view,
                                                                 int mode)
     {
-        constexpr int kUnroll = kQuantUnroll;
-        uint32_t first = blockIdx.x * (256u * kUnroll);
+        uint32_t first = blockIdx.x * (256u * UNROLL);
         uint32_t base = first + threadIdx.x;
-        f32x4 x[kUnroll];
-        float s[kUnroll];
-        float z[kUnroll];
+        f32x4 x[UNROLL];
+        float s[UNROLL];
+        float z[UNROLL];
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u)
+        for (int u = 0; u < UNROLL; ++u)
         {
             uint32_t g = base + u * 256u;
             if (g < groups)
@@ -138,7 +142,7 @@ namespace hipq
             }
         }
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u)
+        for (int u = 0; u < UNROLL; ++u)
         {
             uint32_t g = base + u * 256u;
             if (g < groups)
@@ -148,7 +152,7 @@ namespace hipq
 
     // The quantized side is read with ordinary loads (4 bytes a lane: streaming hints on so narrow a
     // load cost a sixth of the rate), the f32 side written with streaming stores.
-    template <typename QUANT, bool ROW_UNIFORM>
+    template <typename QUANT, bool ROW_UNIFORM, int UNROLL>
     __global__ __launch_bounds__(256) void dequantize_vec4_kernel(const uint32_t* __restrict__ in,
                                                                   const float* __restrict__ scale,
                                                                   const QUANT* __restrict__ zp,
@@ -156,14 +160,13 @@ namespace hipq
                                                                   uint32_t groups,
                                                                   RunView view)
     {
-        constexpr int kUnroll = kDequantUnroll;
-        uint32_t first = blockIdx.x * (256u * kUnroll);
+        uint32_t first = blockIdx.x * (256u * UNROLL);
         uint32_t base = first + threadIdx.x;
-        uint32_t q[kUnroll];
-        float s[kUnroll];
-        int32_t z[kUnroll];
+        uint32_t q[UNROLL];
+        float s[UNROLL];
+        int32_t z[UNROLL];
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u)
+        for (int u = 0; u < UNROLL; ++u)
         {
             uint32_t g = base + u * 256u;
             if (g < groups)
@@ -175,7 +178,7 @@ namespace hipq
             }
         }
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u)
+        for (int u = 0; u < UNROLL; ++u)
         {
             uint32_t g = base + u * 256u;
             if (g < groups)
@@ -189,6 +192,160 @@ namespace hipq
                 }
                 f32x4 o = {r[0], r[1], r[2], r[3]};
                 __builtin_nontemporal_store(o, &out[g]);
+            }
+        }
+    }
+
+    // ---- rows of any length ----------------------------------------------------------------------
+    // Groups of 4 consecutive elements whatever the rows' length: in a row of `inner` >= 4 a group lies in
+    // one row or in two, and an element takes the parameters of the first as long as it is one of the
+    // `left` that remain of it.  Bound by memory like the kernels above, and with their accesses (one
+    // element a lane, its index by 64-bit division: f32[1, 894, 43045] 279 us for Quantize and Dequantize,
+    // f32[1, 128, 51474] 57, f32[19, 834, 238] 35; so 75, 17 and 11.5).
+    enum RaggedForm
+    {
+        RAGGED_STEP, // inner >= 1024: the 1024 elements of a workgroup's step lie in two rows at most, known from its index alone
+        RAGGED_LANE, // inner >= 4: every lane looks its row up
+        RAGGED_EACH  // shorter rows: every element does
+    };
+    struct RaggedView
+    {
+        IndexDiv div_inner, div_a;
+        uint32_t inner, a, groups, tail; // full groups, elements behind the last
+    };
+    constexpr uint32_t kRaggedStep = 1024; // elements of a workgroup's step
+
+    struct RaggedRow
+    {
+        uint32_t j0, j1; // scale index of the row that an element lies in, of the row behind it
+        int32_t left;    // elements from this one to the row's end
+    };
+    __device__ __forceinline__ RaggedRow ragged_row(const RaggedView& v, uint32_t element)
+    {
+        const uint32_t row = fastdiv(element, v.div_inner);
+        const uint32_t j = row - fastdiv(row, v.div_a) * v.a;
+        return RaggedRow{j, j + 1 == v.a ? 0 : j + 1, static_cast<int32_t>((row + 1) * v.inner - element)};
+    }
+
+    template <typename QUANT, bool RNE, int FORM, int UNROLL>
+    __global__ __launch_bounds__(256) void quantize_ragged_kernel(const float* __restrict__ in, const float* __restrict__ scale, const QUANT* __restrict__ zp, QUANT* __restrict__ out,
+                                                                  RaggedView view, int mode)
+    {
+        const uint32_t first = blockIdx.x * (256u * UNROLL);
+        f32x4 x[UNROLL];
+        float s0[UNROLL], s1[UNROLL], z0[UNROLL], z1[UNROLL];
+        int32_t left[UNROLL];
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u)
+        {
+            const uint32_t step = first + u * 256u, g = step + threadIdx.x;
+            if (FORM != RAGGED_EACH && g < view.groups)
+            {
+                x[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(in) + g);
+                const RaggedRow r = ragged_row(view, 4 * (FORM == RAGGED_STEP ? step : g));
+                s0[u] = scale[r.j0];
+                s1[u] = scale[r.j1];
+                z0[u] = static_cast<float>(zp[r.j0]);
+                z1[u] = static_cast<float>(zp[r.j1]);
+                left[u] = FORM == RAGGED_STEP ? r.left - 4 * static_cast<int32_t>(threadIdx.x) : r.left;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u)
+        {
+            const uint32_t g = first + u * 256u + threadIdx.x;
+            if (FORM != RAGGED_EACH && g < view.groups)
+            {
+                const bool in_first = left[u] > 0;
+                uint32_t q = quantize4<QUANT, RNE>(x[u], in_first ? s0[u] : s1[u], in_first ? z0[u] : z1[u], mode);
+                if (in_first && left[u] < 4)
+                {
+                    const uint32_t mask = (1u << (8 * left[u])) - 1;
+                    q = (q & mask) | (quantize4<QUANT, RNE>(x[u], s1[u], z1[u], mode) & ~mask);
+                }
+                __builtin_nontemporal_store(q, reinterpret_cast<uint32_t*>(out) + g);
+            }
+            else if (FORM == RAGGED_EACH && g < view.groups)
+            {
+                const f32x4 v = reinterpret_cast<const f32x4*>(in)[g];
+                uint32_t q = 0;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                {
+                    const uint32_t j = ragged_row(view, 4 * g + e).j0;
+                    q |= static_cast<uint32_t>(static_cast<uint8_t>(quantize_one<float, QUANT>(v[e], scale[j], zp[j], RNE ? HIPQ_ROUND_NEAREST_TOWARD_EVEN : mode))) << (8 * e);
+                }
+                reinterpret_cast<uint32_t*>(out)[g] = q;
+            }
+            else if (g == view.groups)
+            {
+                for (uint32_t e = 0; e < view.tail; ++e)
+                {
+                    const uint32_t j = ragged_row(view, 4 * g + e).j0;
+                    out[4 * g + e] = quantize_one<float, QUANT>(in[4 * g + e], scale[j], zp[j], mode);
+                }
+            }
+        }
+    }
+
+    template <typename QUANT, int FORM, int UNROLL>
+    __global__ __launch_bounds__(256) void dequantize_ragged_kernel(const QUANT* __restrict__ in, const float* __restrict__ scale, const QUANT* __restrict__ zp, float* __restrict__ out,
+                                                                    RaggedView view)
+    {
+        const uint32_t first = blockIdx.x * (256u * UNROLL);
+        uint32_t q[UNROLL];
+        float s0[UNROLL], s1[UNROLL];
+        int32_t z0[UNROLL], z1[UNROLL], left[UNROLL];
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u)
+        {
+            const uint32_t step = first + u * 256u, g = step + threadIdx.x;
+            if (FORM != RAGGED_EACH && g < view.groups)
+            {
+                q[u] = reinterpret_cast<const uint32_t*>(in)[g];
+                const RaggedRow r = ragged_row(view, 4 * (FORM == RAGGED_STEP ? step : g));
+                s0[u] = scale[r.j0];
+                s1[u] = scale[r.j1];
+                z0[u] = static_cast<int32_t>(zp[r.j0]);
+                z1[u] = static_cast<int32_t>(zp[r.j1]);
+                left[u] = FORM == RAGGED_STEP ? r.left - 4 * static_cast<int32_t>(threadIdx.x) : r.left;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u)
+        {
+            const uint32_t g = first + u * 256u + threadIdx.x;
+            if (FORM != RAGGED_EACH && g < view.groups)
+            {
+                f32x4 r;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                {
+                    const int32_t v = static_cast<int32_t>(static_cast<QUANT>((q[u] >> (8 * e)) & 0xFFu));
+                    r[e] = __fmul_rn(static_cast<float>(v - (e < left[u] ? z0[u] : z1[u])), e < left[u] ? s0[u] : s1[u]);
+                }
+                __builtin_nontemporal_store(r, reinterpret_cast<f32x4*>(out) + g);
+            }
+            else if (FORM == RAGGED_EACH && g < view.groups)
+            {
+                const uint32_t b = reinterpret_cast<const uint32_t*>(in)[g];
+                f32x4 r;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                {
+                    const uint32_t j = ragged_row(view, 4 * g + e).j0;
+                    const int32_t v = static_cast<int32_t>(static_cast<QUANT>((b >> (8 * e)) & 0xFFu));
+                    r[e] = __fmul_rn(static_cast<float>(v - static_cast<int32_t>(zp[j])), scale[j]);
+                }
+                reinterpret_cast<f32x4*>(out)[g] = r;
+            }
+            else if (g == view.groups)
+            {
+                for (uint32_t e = 0; e < view.tail; ++e)
+                {
+                    const uint32_t j = ragged_row(view, 4 * g + e).j0;
+                    out[4 * g + e] = __fmul_rn(static_cast<float>(static_cast<int32_t>(in[4 * g + e]) - static_cast<int32_t>(zp[j])), scale[j]);
+                }
             }
         }
     }
@@ -264,11 +421,15 @@ namespace hipq
         return static_cast<unsigned>(b > 65536 ? 65536 : (b < 1 ? 1 : b));
     }
 
+    static bool ragged_ok(const hipq_quant_desc_t& d, const Canon& c, const void* f32_ptr, const void* q_ptr)
+    {
+        return d.real_t == HIPQ_F32 && (d.quant_t == HIPQ_U8 || d.quant_t == HIPQ_I8) && c.single_run && c.count < (1ll << 31) &&
+               (reinterpret_cast<uintptr_t>(f32_ptr) & 15) == 0 && (reinterpret_cast<uintptr_t>(q_ptr) & 3) == 0;
+    }
+    // groups of 4 lie in one row of the scale table each
     static bool vec4_ok(const hipq_quant_desc_t& d, const Canon& c, const void* f32_ptr, const void* q_ptr)
     {
-        return d.real_t == HIPQ_F32 && (d.quant_t == HIPQ_U8 || d.quant_t == HIPQ_I8) && c.single_run &&
-               c.count < (1ll << 31) && c.count % 4 == 0 && (c.a == 1 || c.inner % 4 == 0) &&
-               (reinterpret_cast<uintptr_t>(f32_ptr) & 15) == 0 && (reinterpret_cast<uintptr_t>(q_ptr) & 3) == 0;
+        return ragged_ok(d, c, f32_ptr, q_ptr) && c.count % 4 == 0 && (c.a == 1 || c.inner % 4 == 0);
     }
 
     // every 256-group step of a workgroup lies inside one row of the scale table
@@ -282,6 +443,21 @@ namespace hipq
         v.div_a = make_fastdiv(v.a);
         return v;
     }
+    static RaggedView make_ragged_view(const Canon& c)
+    {
+        RaggedView v;
+        v.a = static_cast<uint32_t>(c.a);
+        v.inner = static_cast<uint32_t>(c.a == 1 ? c.count : c.inner);
+        v.div_inner = make_fastdiv(v.inner);
+        v.div_a = make_fastdiv(v.a);
+        v.groups = static_cast<uint32_t>(c.count / 4);
+        v.tail = static_cast<uint32_t>(c.count % 4);
+        return v;
+    }
+    static RaggedForm ragged_form(const RaggedView& v) { return v.inner >= kRaggedStep ? RAGGED_STEP : (v.inner >= 4 ? RAGGED_LANE : RAGGED_EACH); }
+    // (the group behind the last full one holds the tail)
+    static unsigned ragged_blocks(const RaggedView& v, int unroll) { return (v.groups + 1 + 256 * unroll - 1) / (256 * unroll); }
+    static bool is_short(uint32_t groups) { return (groups + 255) / 256 <= 8u * static_cast<unsigned>(device_compute_units()); }
 }
 
 using namespace hipq;
@@ -302,18 +478,16 @@ int hipq_quantize(const hipq_quant_desc_t* d, const void* in, const void* scale,
     if (vec4_ok(*d, c, in, out))
     {
         uint32_t groups = static_cast<uint32_t>(c.count / 4);
-        unsigned blocks = (groups + 256 * kQuantUnroll - 1) / (256 * kQuantUnroll);
+        const bool few = is_short(groups);
+        const unsigned step = 256 * (few ? 1 : kQuantUnroll);
+        unsigned blocks = (groups + step - 1) / step;
         RunView v = make_view(c);
         bool rne = d->round_mode == HIPQ_ROUND_NEAREST_TOWARD_EVEN;
         bool uniform = row_uniform(c);
-#define LAUNCH_Q4(QT, RNE, UNI)                                                                    \
-    quantize_vec4_kernel<QT, RNE, UNI><<<blocks, 256, 0, s>>>(static_cast<const f32x4*>(in),      \
-                                                              static_cast<const float*>(scale),    \
-                                                              static_cast<const QT*>(zp),          \
-                                                              static_cast<uint32_t*>(out),         \
-                                                              groups,                              \
-                                                              v,                                   \
-                                                              d->round_mode)
+#define LAUNCH_Q4_U(QT, RNE, UNI, U)                                                                                                                                                     \
+    quantize_vec4_kernel<QT, RNE, UNI, U><<<blocks, 256, 0, s>>>(static_cast<const f32x4*>(in), static_cast<const float*>(scale), static_cast<const QT*>(zp), static_cast<uint32_t*>(out), \
+                                                                 groups, v, d->round_mode)
+#define LAUNCH_Q4(QT, RNE, UNI) (few ? LAUNCH_Q4_U(QT, RNE, UNI, 1) : LAUNCH_Q4_U(QT, RNE, UNI, kQuantUnroll))
 #define LAUNCH_Q4_T(QT)                                                                            \
     do                                                                                             \
     {                                                                                              \
@@ -332,7 +506,30 @@ int hipq_quantize(const hipq_quant_desc_t* d, const void* in, const void* scale,
             LAUNCH_Q4_T(uint8_t);
 #undef LAUNCH_Q4_T
 #undef LAUNCH_Q4
+#undef LAUNCH_Q4_U
         return check_launch("quantize_vec4");
+    }
+    if (ragged_ok(*d, c, in, out))
+    {
+        const RaggedView v = make_ragged_view(c);
+        const bool rne = d->round_mode == HIPQ_ROUND_NEAREST_TOWARD_EVEN;
+#define LAUNCH_QR(QT, RNE, FORM, U)                                                                                                                                           \
+    quantize_ragged_kernel<QT, RNE, FORM, U><<<ragged_blocks(v, U), 256, 0, s>>>(static_cast<const float*>(in), static_cast<const float*>(scale), static_cast<const QT*>(zp), \
+                                                                                 static_cast<QT*>(out), v, d->round_mode)
+#define LAUNCH_QR_U(QT, RNE, FORM) (is_short(v.groups) ? LAUNCH_QR(QT, RNE, FORM, 1) : LAUNCH_QR(QT, RNE, FORM, kQuantUnroll))
+#define LAUNCH_QR_F(QT, FORM) (rne ? LAUNCH_QR_U(QT, true, FORM) : LAUNCH_QR_U(QT, false, FORM))
+#define LAUNCH_QR_T(FORM) (d->quant_t == HIPQ_I8 ? LAUNCH_QR_F(int8_t, FORM) : LAUNCH_QR_F(uint8_t, FORM))
+        switch (ragged_form(v))
+        {
+        case RAGGED_STEP: LAUNCH_QR_T(RAGGED_STEP); break;
+        case RAGGED_LANE: LAUNCH_QR_T(RAGGED_LANE); break;
+        case RAGGED_EACH: LAUNCH_QR_T(RAGGED_EACH); break;
+        }
+#undef LAUNCH_QR_T
+#undef LAUNCH_QR_F
+#undef LAUNCH_QR_U
+#undef LAUNCH_QR
+        return check_launch("quantize_ragged");
     }
     DimInfo di = dim_info(*d);
     unsigned blocks = generic_blocks(c.count);
@@ -379,16 +576,14 @@ int hipq_dequantize(const hipq_quant_desc_t* d, const void* in, const void* scal
     if (vec4_ok(*d, c, out, in))
     {
         uint32_t groups = static_cast<uint32_t>(c.count / 4);
-        unsigned blocks = (groups + 256 * kDequantUnroll - 1) / (256 * kDequantUnroll);
+        const bool few = is_short(groups);
+        const unsigned step = 256 * (few ? 1 : kDequantUnroll);
+        unsigned blocks = (groups + step - 1) / step;
         RunView v = make_view(c);
         bool uniform = row_uniform(c);
-#define LAUNCH_D4(QT, UNI)                                                                         \
-    dequantize_vec4_kernel<QT, UNI><<<blocks, 256, 0, s>>>(static_cast<const uint32_t*>(in),       \
-                                                           static_cast<const float*>(scale),       \
-                                                           static_cast<const QT*>(zp),             \
-                                                           static_cast<f32x4*>(out),               \
-                                                           groups,                                 \
-                                                           v)
+#define LAUNCH_D4_U(QT, UNI, U)                                                                                                                                                            \
+    dequantize_vec4_kernel<QT, UNI, U><<<blocks, 256, 0, s>>>(static_cast<const uint32_t*>(in), static_cast<const float*>(scale), static_cast<const QT*>(zp), static_cast<f32x4*>(out), groups, v)
+#define LAUNCH_D4(QT, UNI) (few ? LAUNCH_D4_U(QT, UNI, 1) : LAUNCH_D4_U(QT, UNI, kDequantUnroll))
         if (d->quant_t == HIPQ_I8)
         {
             if (uniform)
@@ -404,7 +599,27 @@ int hipq_dequantize(const hipq_quant_desc_t* d, const void* in, const void* scal
                 LAUNCH_D4(uint8_t, false);
         }
 #undef LAUNCH_D4
+#undef LAUNCH_D4_U
         return check_launch("dequantize_vec4");
+    }
+    if (ragged_ok(*d, c, out, in))
+    {
+        const RaggedView v = make_ragged_view(c);
+#define LAUNCH_DR(QT, FORM, U)                                                                                                                                              \
+    dequantize_ragged_kernel<QT, FORM, U><<<ragged_blocks(v, U), 256, 0, s>>>(static_cast<const QT*>(in), static_cast<const float*>(scale), static_cast<const QT*>(zp), \
+                                                                              static_cast<float*>(out), v)
+#define LAUNCH_DR_U(QT, FORM) (is_short(v.groups) ? LAUNCH_DR(QT, FORM, 1) : LAUNCH_DR(QT, FORM, kDequantUnroll))
+#define LAUNCH_DR_T(FORM) (d->quant_t == HIPQ_I8 ? LAUNCH_DR_U(int8_t, FORM) : LAUNCH_DR_U(uint8_t, FORM))
+        switch (ragged_form(v))
+        {
+        case RAGGED_STEP: LAUNCH_DR_T(RAGGED_STEP); break;
+        case RAGGED_LANE: LAUNCH_DR_T(RAGGED_LANE); break;
+        case RAGGED_EACH: LAUNCH_DR_T(RAGGED_EACH); break;
+        }
+#undef LAUNCH_DR_T
+#undef LAUNCH_DR_U
+#undef LAUNCH_DR
+        return check_launch("dequantize_ragged");
     }
     DimInfo di = dim_info(*d);
     unsigned blocks = generic_blocks(c.count);
