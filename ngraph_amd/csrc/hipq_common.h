@@ -256,6 +256,11 @@ namespace hipq
                          hipStream_t s);
     // whether the kernels for layers too small to fill the chip take it (hipq_igemm_wk.hip)
     bool conv_wk_preferred(const ConvGeom& g, int out_t, bool out_ncx);
+    // whether they read channels-last data of `whole`, whose channels are no multiple of 16, in place
+    bool conv_ragged_preferred(const ConvGeom& whole, const ConvGeom& padded, const Epilogue& epi, bool out_ncx);
+    // those kernels on channels-last data whose channels are no multiple of 16, without a padded copy:
+    // `whole` is the layer, `padded` its form with the packed filter's channel count
+    int launch_conv_ragged(const ConvGeom& whole, const ConvGeom& padded, const void* data_nxc, const void* packed, const ZeroPoints& zp, const Epilogue& epi, void* out, bool out_ncx, hipStream_t s);
     bool dot_mfma_eligible(const hipq_dot_desc_t& d);
     int launch_dot_mfma(const hipq_dot_desc_t& d,
                         const void* a,
@@ -265,7 +270,10 @@ namespace hipq
                         const Epilogue& epi,
                         void* out,
                         hipStream_t s,
-                        const void* w_frag = nullptr); // fragment-ordered copy of the weights (prepacked blobs), or null
+                        const void* w_frag = nullptr, // fragment-ordered copy of the weights (prepacked blobs), or null
+                        int64_t a_row = 0); // bytes of a row of `a` where it is read in place (dot_ragged_preferred), 0: d.K
+    // whether a product whose reduction was padded to d.K reads the rows of `a` where they lie
+    bool dot_ragged_preferred(const hipq_dot_desc_t& d, int64_t row_bytes, const Epilogue& epi);
 
     int launch_rows_mfma(const void* a, bool a_unsigned, const int8_t* w_nk, const int32_t* wsum, int64_t M, int32_t N, int32_t K,
                          const ZeroPoints& zp, const Epilogue& epi, void* out, hipStream_t s, const char* name);

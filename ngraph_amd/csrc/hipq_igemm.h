@@ -127,6 +127,7 @@ namespace hipq
         static constexpr bool kFloatOut = false;
         static constexpr bool kPads = false; // (only read by the kernels that load straight into LDS)
         static constexpr bool kPadded = false; // no taps in a padding
+        static constexpr bool kRagged = false; // 16-byte chunks of the data are aligned
 
         struct Row
         {
@@ -163,6 +164,7 @@ namespace hipq
         static constexpr bool kFloatOut = false;
         static constexpr bool kPads = false; // (only read by the kernels that load straight into LDS)
         static constexpr bool kPadded = true; // taps in the padding are the data zero point
+        static constexpr bool kRagged = false; // 16-byte chunks of the data are aligned
         const uint8_t* x; // [N][H][W][C]
         int32_t H, W, C, Q, R, S, sh, sw, dh, dw, pbh, pbw;
         int64_t PQ;
@@ -227,7 +229,8 @@ namespace hipq
                             (static_cast<uint32_t>(xx) < static_cast<uint32_t>(W));
             return ok ? rw.base + (y * W + xx) * C + c.c : kOob;
         }
-        __device__ __forceinline__ int32_t direct(int64_t m, const int8_t* wrow, int32_t xzp, int32_t wzp, bool x_unsigned) const
+        __device__ __forceinline__ int32_t direct(int64_t m, const int8_t* wrow, int32_t xzp, int32_t wzp, bool x_unsigned) const { return direct_taps(m, wrow, C, xzp, wzp, x_unsigned); }
+        __device__ __forceinline__ int32_t direct_taps(int64_t m, const int8_t* wrow, int32_t tap_bytes, int32_t xzp, int32_t wzp, bool x_unsigned) const
         {
             Row rw;
             init_row(rw, m, m + 1);
@@ -240,7 +243,7 @@ namespace hipq
                     if (static_cast<uint32_t>(y) >= static_cast<uint32_t>(H) || static_cast<uint32_t>(xx) >= static_cast<uint32_t>(W))
                         continue;
                     const uint8_t* p = x + rw.base + (y * W + xx) * C;
-                    const int8_t* wp = wrow + (r * S + s) * C;
+                    const int8_t* wp = wrow + (r * S + s) * tap_bytes;
                     for (int32_t c = 0; c < C; ++c)
                     {
                         int32_t a = x_unsigned ? static_cast<int32_t>(p[c]) : static_cast<int32_t>(static_cast<int8_t>(p[c]));
@@ -249,6 +252,28 @@ namespace hipq
                 }
             return acc;
         }
+    };
+
+    // ---- loaders of data whose channels or reduction are no multiple of 16 bytes, read where it lies -----
+    // The reduction they walk is the packed weights': every tap's channels (or every row) padded with zero
+    // weights to whole 16-byte chunks.  A chunk that runs over the end of its pixel (row) holds the next
+    // one's first bytes, which meet those zeros.
+    struct GemmRaggedX : GemmX // K: bytes of a row
+    {
+        static constexpr bool kRagged = true;
+    };
+    struct ConvRaggedX : ConvX // C: bytes of a pixel; by_c divides by Cp
+    {
+        static constexpr bool kRagged = true;
+        int32_t Cp; // channels of a tap in the packed weights
+        __device__ __forceinline__ void init_cursor(Cursor& c, int kbyte) const
+        {
+            const int tap = static_cast<int>(by_c.div(static_cast<uint32_t>(kbyte)));
+            c.c = kbyte - tap * Cp;
+            c.r = static_cast<int>(by_s.div(static_cast<uint32_t>(tap)));
+            c.s = tap - c.r * S;
+        }
+        __device__ __forceinline__ int32_t direct(int64_t m, const int8_t* wrow, int32_t xzp, int32_t wzp, bool x_unsigned) const { return direct_taps(m, wrow, Cp, xzp, wzp, x_unsigned); }
     };
 
     // ---- loaders of the kernels that load straight into LDS -------------------------------------
@@ -2119,8 +2144,13 @@ namespace hipq
     // from memory (hipq_igemm_wk.hip); HIPQ_ERR_UNSUPPORTED (nothing launched, no error text) when the call
     // is not of their kind
     bool wk_preferred(int64_t M, int64_t N, bool dma);
+    bool ragged_preferred(int64_t M, int64_t N, int64_t row_bytes, int64_t steps, bool dma, bool pointwise);
     int launch_rows_wk(const void* a, bool a_unsigned, const int8_t* w_nk, const void* w_frag, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi,
                        void* out, hipStream_t s, const char* name);
+    int launch_rows_wk_ragged(const void* a, int32_t a_row, bool a_unsigned, const int8_t* w_nk, const void* w_frag, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp,
+                              const Epilogue& epi, void* out, hipStream_t s, const char* name); // rows of a_row bytes, any a_row >= 16
+    int launch_conv_wk_ragged(const ConvRaggedX& xl, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, int x_unsigned, const ZeroPoints& zp, const Epilogue& epi,
+                              const OutMap& om, void* out, hipStream_t s, const char* name);
     int launch_conv_wk(const ConvX& xl, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, int x_unsigned, const ZeroPoints& zp, const Epilogue& epi, const OutMap& om, void* out,
                        hipStream_t s, const char* name);
 }

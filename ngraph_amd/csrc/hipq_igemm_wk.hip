@@ -17,6 +17,9 @@
 // 512 -> 512 3 x 3 on 7 x 7 (an unrolled copy and a skinny product before) 16.3 -> 8.3, 1024 -> 256
 // 1 x 1 on 14 x 14 10.7 -> 4.9, 128 x 768 x 768 with float outputs 8.5 -> 3.8; a launch that does
 // nothing takes 1.7.
+//
+// Rows and pixels that are no multiple of 16 bytes are read where they lie (ragged_preferred): u8
+// [8,90,35,29] x i8 [150,90,3,3] 14.4 -> 13.1 us, 77 x 1000 x 1003 8.2 -> 4.1 with the copy's launch gone.
 #include <cstdlib>
 
 #include "hipq_igemm.h"
@@ -24,6 +27,10 @@
 namespace hipq
 {
     typedef int v4acc __attribute__((ext_vector_type(4)));
+    // (global loads and stores need no alignment on this chip)
+    typedef v4i v4i_any __attribute__((aligned(1)));
+    typedef uint32_t u32_any __attribute__((aligned(1)));
+    typedef v4i v4i_word __attribute__((aligned(4)));
 
     struct WkParams
     {
@@ -95,6 +102,13 @@ namespace hipq
         }
         v4i xf[U][MT], wf[U][NT];
         uint32_t pads = 0; // bit u * MT + i: the data fragment lies in the padding
+        // Ragged data: a chunk that would run past the tensor's last byte is read as far to the front as it
+        // takes to end there; the bytes it starts late by, four bits a step in flight
+        const int32_t x_last = static_cast<int32_t>(xl.bytes) - 16;
+        uint32_t late[MT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+            late[i] = 0;
         auto load = [&](int u, int s) {
             const int kbyte = s * 64 + kc * 16;
             const bool in_k = (s < s_end) & (kbyte < p.Kred);
@@ -106,7 +120,16 @@ namespace hipq
                 const int32_t off = in_k ? xl.offset(xr[i], cur) : kOob;
                 if (XL::kPadded)
                     pads = (pads & ~(1u << (u * MT + i))) | ((off == kOob ? 1u : 0u) << (u * MT + i));
-                xf[u][i] = buffer_load16(xrs, off);
+                if constexpr (XL::kRagged)
+                {
+                    // (a fragment that does not exist is whatever the tensor starts with: its weights are zeros,
+                    // its row is not stored, or the padding replaces it)
+                    const int32_t at = min(max(off, 0), x_last);
+                    late[i] = (late[i] & ~(15u << (4 * u))) | static_cast<uint32_t>(max(off, at) - at) << (4 * u);
+                    xf[u][i] = *reinterpret_cast<const v4i_any*>(xl.x + static_cast<uint32_t>(at));
+                }
+                else
+                    xf[u][i] = buffer_load16(xrs, off);
             }
 #pragma unroll
             for (int j = 0; j < NT; ++j)
@@ -127,7 +150,7 @@ namespace hipq
         HeadWords hw = head_scalars_load(zp, epi, p.wsum);
         // this wavefront finishes blocks it * KW + kw of its tile, a group of four outputs a lane
         const bool has_sum = fused && epi.sum_in != nullptr;
-        const bool vec_ok = X_ON_A ? (!om.ncx || (om.PQ & 3) == 0) : (N & 3) == 0;
+        const bool vec_ok = !X_ON_A || !om.ncx || (om.PQ & 3) == 0; // the group is contiguous (rows of N may start anywhere)
         int64_t o_at[ITER];
         int o_left[ITER]; // outputs of the group that exist
         uint32_t res[ITER];
@@ -144,8 +167,8 @@ namespace hipq
             res[it] = 0;
             if (has_sum && o_left[it] > 0)
             {
-                if (vec_ok)
-                    res[it] = *reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(epi.sum_in) + o_at[it]);
+                if (vec_ok && o_left[it] == 4)
+                    res[it] = *reinterpret_cast<const u32_any*>(static_cast<const uint8_t*>(epi.sum_in) + o_at[it]);
                 else
                 {
                     for (int e = 0; e < o_left[it]; ++e)
@@ -171,7 +194,23 @@ namespace hipq
             for (int i = 0; i < MT; ++i)
             {
                 v4i x = xf[u][i];
-                if (XL::kPadded && fill != 0) // uniform: padding taps hold the data zero point
+                if constexpr (XL::kRagged)
+                {
+                    const uint32_t n = (late[i] >> (4 * u)) & 15u;
+                    if (__builtin_amdgcn_ballot_w64(n != 0) != 0) // uniform, and rare
+                    {
+                        const int q = static_cast<int>(n >> 2);
+                        const int d[8] = {x[0], x[1], x[2], x[3], 0, 0, 0, 0};
+                        int y[5];
+#pragma unroll
+                        for (int e = 0; e < 5; ++e)
+                            y[e] = q == 0 ? d[e] : q == 1 ? d[e + 1] : q == 2 ? d[e + 2] : d[e + 3];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            x[e] = static_cast<int>(__builtin_amdgcn_alignbyte(static_cast<uint32_t>(y[e + 1]), static_cast<uint32_t>(y[e]), n & 3u));
+                    }
+                }
+                if (XL::kPadded && (XL::kRagged || fill != 0)) // uniform: padding taps hold the data zero point
                 {
                     const bool pad = (pads >> (u * MT + i)) & 1u;
                     x = v4i{pad ? fill : x[0], pad ? fill : x[1], pad ? fill : x[2], pad ? fill : x[3]};
@@ -279,9 +318,9 @@ namespace hipq
                 if (vec_ok && o_left[it] == 4)
                 {
                     if (KIND == OUT_Q8 || KIND == OUT_GELU_Q8)
-                        *reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(out) + o_at[it]) = pack4(v);
+                        *reinterpret_cast<u32_any*>(static_cast<uint8_t*>(out) + o_at[it]) = pack4(v);
                     else
-                        *reinterpret_cast<v4i*>(static_cast<int32_t*>(out) + o_at[it]) = v4i{v[0], v[1], v[2], v[3]};
+                        *reinterpret_cast<v4i_word*>(static_cast<int32_t*>(out) + o_at[it]) = v4i{v[0], v[1], v[2], v[3]};
                 }
                 else
                 {
@@ -344,13 +383,38 @@ namespace hipq
     // tiles a compute unit: above that those kernels' whole-line loads and larger tiles win (985 x 512 x
     // 1536: 8.6 us there, 9.9 us here; 985 x 512 x 512: 7.9, 5.5).  Against the register-staged ones up to
     // sixteen.
-    bool wk_preferred(int64_t M, int64_t N, bool dma)
+    static bool wk_enabled()
     {
         // (the switches that name a kernel of the other family mean that family)
         for (const char* name : {"HIPQ_NO_WK", "HIPQ_SPLIT_K", "HIPQ_NO_DMA", "HIPQ_NO_PIPE", "HIPQ_NO_CONV_DMA", "HIPQ_NO_HALF_TILES", "HIPQ_NO_REGW"})
             if (getenv(name) != nullptr)
                 return false;
-        return wk_tiles(M, N, 32, 32) <= static_cast<int64_t>(device_compute_units()) * (dma ? 3 : 16);
+        return true;
+    }
+    bool wk_preferred(int64_t M, int64_t N, bool dma) { return wk_enabled() && wk_tiles(M, N, 32, 32) <= static_cast<int64_t>(device_compute_units()) * (dma ? 3 : 16); }
+
+    // Whether rows (pixels) of `row_bytes` that are no multiple of 16 are read where they lie, instead of
+    // through a copy padded to whole chunks (a launch, 2.5 us and more, and rows a power of two apart).
+    // Chunks then start at any byte.  On rows of whole dwords that costs nothing seen (4096 x 1500 x 1003:
+    // copy and product 58.5 us, in place 39.5; 16 x 1000 x 1003: 6.6, 3.7); on others a chunk takes about
+    // twice its time in the memory path, so only while there are few of them: 32 steps of 64 bytes (40 with a
+    // window's taps, which hit the same lines) and 8192 step-tiles (24576 with taps or up to six steps):
+    // 77 x 2001 x 1003 7.1 there, 6.2 in place; 600 x 1301 x 1003 12.0, 14.4; 16 x 4001 x 150 6.7, 8.7;
+    // 90 -> 150 channels 3 x 3 on 8 x 35 x 35 pixels 15.4, 14.8, on 64 x 35 x 35 68, 82.
+    // Where no kernel that loads straight into LDS would take the call, short reductions stay here beyond
+    // the sizes of wk_preferred: 90 -> 150 channels 1 x 1 on 128 x 56 x 56 179 there, 79 in place.
+    bool ragged_preferred(int64_t M, int64_t N, int64_t row_bytes, int64_t steps, bool dma, bool pointwise)
+    {
+        if (!wk_enabled())
+            return false;
+        const int64_t tiles = wk_tiles(M, N, 32, 32), units = device_compute_units();
+        if (!dma && pointwise && (steps <= 3 || (steps <= 6 && tiles <= units * 40)))
+            return true;
+        if (!wk_preferred(M, N, dma))
+            return false;
+        if (row_bytes % 4 == 0)
+            return pointwise || steps <= 40;
+        return steps <= (pointwise ? 32 : 40) && tiles * steps <= (steps <= 6 || !pointwise ? 24576 : 8192);
     }
 
     template <class XL, int MT, int NT, int KW, int TW, int U, bool X_ON_A>
@@ -414,15 +478,37 @@ namespace hipq
         return p;
     }
 
+    template <class XL>
+    static XL rows_of(const void* a, int64_t M, int32_t row_bytes)
+    {
+        XL xl;
+        xl.x = static_cast<const uint8_t*>(a);
+        xl.K = row_bytes;
+        xl.bytes = static_cast<uint32_t>(M * row_bytes);
+        return xl;
+    }
+
     int launch_rows_wk(const void* a, bool a_unsigned, const int8_t* w_nk, const void* w_frag, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi,
                        void* out, hipStream_t s, const char* name)
     {
-        GemmX xl;
-        xl.x = static_cast<const uint8_t*>(a);
-        xl.K = K;
-        xl.bytes = static_cast<uint32_t>(M * K);
         const OutMap om{0, N, 1};
-        return launch_wk<GemmX, false>(xl, wk_params(w_nk, w_frag, wsum, M, N, K, a_unsigned ? 1 : 0), zp, epi, om, out, s, name);
+        return launch_wk<GemmX, false>(rows_of<GemmX>(a, M, K), wk_params(w_nk, w_frag, wsum, M, N, K, a_unsigned ? 1 : 0), zp, epi, om, out, s, name);
+    }
+
+    int launch_rows_wk_ragged(const void* a, int32_t a_row, bool a_unsigned, const int8_t* w_nk, const void* w_frag, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp,
+                              const Epilogue& epi, void* out, hipStream_t s, const char* name)
+    {
+        const OutMap om{0, N, 1};
+        return launch_wk<GemmRaggedX, false>(rows_of<GemmRaggedX>(a, M, a_row), wk_params(w_nk, w_frag, wsum, M, N, K, a_unsigned ? 1 : 0), zp, epi, om, out, s, name);
+    }
+
+    int launch_conv_wk_ragged(const ConvRaggedX& xl, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, int x_unsigned, const ZeroPoints& zp, const Epilogue& epi,
+                              const OutMap& om, void* out, hipStream_t s, const char* name)
+    {
+        const WkParams p = wk_params(w, nullptr, wsum, M, N, K, x_unsigned);
+        if (om.ncx)
+            return launch_wk<ConvRaggedX, true>(xl, p, zp, epi, om, out, s, name);
+        return launch_wk<ConvRaggedX, false>(xl, p, zp, epi, om, out, s, name);
     }
 
     int launch_conv_wk(const ConvX& xl, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, int x_unsigned, const ZeroPoints& zp, const Epilogue& epi, const OutMap& om, void* out,

@@ -33,19 +33,17 @@ namespace hipq
         return wk_preferred(g.N * g.out[1] * g.out[2], g.K, dma);
     }
 
-    int launch_conv_mfma(const ConvGeom& g,
-                         const void* data_nxc,
-                         const void* packed,
-                         const ZeroPoints& zp,
-                         const Epilogue& epi,
-                         void* out,
-                         bool out_ncx,
-                         hipStream_t s)
+    bool conv_ragged_preferred(const ConvGeom& whole, const ConvGeom& padded, const Epilogue& epi, bool out_ncx)
     {
-        HIPQ_REQUIRE(conv_mfma_eligible(g), "shape not eligible for the MFMA convolution");
-        HIPQ_REQUIRE((reinterpret_cast<uintptr_t>(data_nxc) & 15) == 0 && (reinterpret_cast<uintptr_t>(packed) & 15) == 0 &&
-                         (reinterpret_cast<uintptr_t>(out) & 15) == 0,
-                     "MFMA convolution needs 16-byte aligned tensors");
+        if (whole.C < 16 || whole.data_layout != HIPQ_LAYOUT_NXC)
+            return false;
+        const bool pointwise = whole.taps() == 1;
+        const bool dma = !out_ncx && padded.K % 16 == 0 && (epi.out_t == HIPQ_U8 || epi.out_t == HIPQ_I8) && (padded.C % 64 == 0 || (pointwise && whole.st[1] == 1 && whole.st[2] == 1));
+        return ragged_preferred(whole.N * whole.out[1] * whole.out[2], whole.K, whole.C, (padded.C * whole.taps() + 63) / 64, dma, pointwise);
+    }
+
+    static ConvX conv_loader(const ConvGeom& g, const void* data_nxc)
+    {
         ConvX xl;
         xl.x = static_cast<const uint8_t*>(data_nxc);
         xl.H = static_cast<int32_t>(g.in[1]);
@@ -62,13 +60,45 @@ namespace hipq
         xl.pbw = static_cast<int32_t>(g.pb[2]);
         xl.PQ = g.out[1] * g.out[2];
         xl.bytes = static_cast<uint32_t>(g.in_count());
-        const int64_t M = g.N * xl.PQ;
         xl.by_pq = fast_div(xl.PQ);
-        if (M >= (1ll << 31))
+        if (g.N * xl.PQ >= (1ll << 31))
             xl.by_pq.sh = 0xffffffffu;
         xl.by_q = fast_div(xl.Q);
         xl.by_c = fast_div(xl.C);
         xl.by_s = fast_div(xl.S);
+        return xl;
+    }
+
+    int launch_conv_ragged(const ConvGeom& whole, const ConvGeom& padded, const void* data_nxc, const void* packed, const ZeroPoints& zp, const Epilogue& epi, void* out, bool out_ncx, hipStream_t s)
+    {
+        HIPQ_REQUIRE(conv_mfma_eligible(padded), "shape not eligible for the MFMA convolution");
+        HIPQ_REQUIRE((reinterpret_cast<uintptr_t>(packed) & 15) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0, "MFMA convolution needs 16-byte aligned tensors");
+        ConvRaggedX xl;
+        static_cast<ConvX&>(xl) = conv_loader(whole, data_nxc);
+        xl.Cp = static_cast<int32_t>(padded.C);
+        xl.by_c = fast_div(xl.Cp);
+        const int32_t N = static_cast<int32_t>(whole.K);
+        const int32_t Kred = static_cast<int32_t>(padded.C * whole.taps());
+        const int32_t* wsum = reinterpret_cast<const int32_t*>(static_cast<const uint8_t*>(packed) + align_up(static_cast<size_t>(whole.K) * Kred, 256));
+        const OutMap om{out_ncx ? 1 : 0, N, xl.PQ};
+        return launch_conv_wk_ragged(xl, static_cast<const int8_t*>(packed), wsum, whole.N * xl.PQ, N, Kred, whole.data_t == HIPQ_U8 ? 1 : 0, zp, epi, om, out, s, "conv_mfma_wk_ragged_i8_16x16x64");
+    }
+
+    int launch_conv_mfma(const ConvGeom& g,
+                         const void* data_nxc,
+                         const void* packed,
+                         const ZeroPoints& zp,
+                         const Epilogue& epi,
+                         void* out,
+                         bool out_ncx,
+                         hipStream_t s)
+    {
+        HIPQ_REQUIRE(conv_mfma_eligible(g), "shape not eligible for the MFMA convolution");
+        HIPQ_REQUIRE((reinterpret_cast<uintptr_t>(data_nxc) & 15) == 0 && (reinterpret_cast<uintptr_t>(packed) & 15) == 0 &&
+                         (reinterpret_cast<uintptr_t>(out) & 15) == 0,
+                     "MFMA convolution needs 16-byte aligned tensors");
+        const ConvX xl = conv_loader(g, data_nxc);
+        const int64_t M = g.N * xl.PQ;
         const int32_t N = static_cast<int32_t>(g.K);
         const int32_t Kred = static_cast<int32_t>(g.C * g.taps());
         const int8_t* w = static_cast<const int8_t*>(packed);

@@ -1052,6 +1052,18 @@ namespace hipq
         return true;
     }
 
+    bool dot_ragged_preferred(const hipq_dot_desc_t& d, int64_t row_bytes, const Epilogue& epi)
+    {
+        const bool q8 = epi.out_t == HIPQ_U8 || epi.out_t == HIPQ_I8;
+        if (epi.mode == EPI_FUSED && !q8 && epi.out_t != HIPQ_F32)
+            return false;
+        // (the kernel that keeps a whole reduction in one workgroup wins later than on aligned rows, the copy being
+        // part of its price: 256 x 1000 x 4001 8.8 us with it, 7.1 in place; 250 x 2004 x 4000 11.3, 11.8)
+        if (dot_rows64_eligible(d) && ((d.M + 31) / 32) * ((d.N + 31) / 32) * (d.K / 64) > 16384)
+            return false;
+        return ragged_preferred(d.M, d.N, row_bytes, d.K / 64, d.N % 16 == 0 && (q8 || epi.mode == EPI_FUSED), true);
+    }
+
     int launch_dot_mfma(const hipq_dot_desc_t& d,
                         const void* a,
                         const void* w_nk,
@@ -1060,12 +1072,16 @@ namespace hipq
                         const Epilogue& epi,
                         void* out,
                         hipStream_t s,
-                        const void* w_frag)
+                        const void* w_frag,
+                        int64_t a_row)
     {
         HIPQ_REQUIRE(dot_mfma_eligible(d), "shape not eligible for the MFMA dot");
-        HIPQ_REQUIRE((reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w_nk) & 15) == 0 &&
+        HIPQ_REQUIRE((a_row != 0 || (reinterpret_cast<uintptr_t>(a) & 15) == 0) && (reinterpret_cast<uintptr_t>(w_nk) & 15) == 0 &&
                          (reinterpret_cast<uintptr_t>(out) & 15) == 0,
                      "MFMA dot needs 16-byte aligned tensors");
+        if (a_row != 0)
+            return launch_rows_wk_ragged(a, static_cast<int32_t>(a_row), d.a_t == HIPQ_U8, static_cast<const int8_t*>(w_nk), w_frag, wsum, d.M, static_cast<int32_t>(d.N), static_cast<int32_t>(d.K), zp,
+                                         epi, out, s, "dot_mfma_wk_ragged_i8_16x16x64");
         // Products too small to fill the chip: fragments straight from memory, the reduction split over a
         // workgroup's wavefronts.  Up to 32 rows with packed weights only short reductions: the kernel
         // below asks for whole lines of both operands, which counts from twelve steps on (1 x 1024 x 1003:

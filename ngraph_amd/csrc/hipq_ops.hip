@@ -64,6 +64,9 @@ namespace hipq
         const bool tr_in = !pad && g.data_layout == HIPQ_LAYOUT_NCX && g.C > 1;
         const bool small = conv_wk_preferred(g, epi.out_t, out_ncx); // too small to fill the chip
         const size_t tr_bytes = pad || tr_in ? align_up(static_cast<size_t>(g.in_count()), 256) : 0;
+        // channels-last pixels of any width, where reading them as they lie costs less than the copy
+        if (pad && conv_ragged_preferred(whole, g, epi, out_ncx) && !conv_pw64_eligible(g, epi, zp) && !conv_regw_eligible(g, out_ncx))
+            return launch_conv_ragged(whole, g, data, packed, zp, epi, out, out_ncx, s);
         const void* x = data;
         uint8_t* ws = nullptr;
         auto scratch = [&]() {
@@ -190,19 +193,23 @@ namespace hipq
         const void* w;
         const void* wfrag;
         const int32_t* wsum;
+        int64_t a_row; // bytes of a row of `a` where it stays unpadded, 0: the padded reduction
     };
     static size_t dot_padded_rows_bytes(const hipq_dot_desc_t& d) { return dot_is_padded(d) ? align_up(static_cast<size_t>(d.M * dot_seen(d).K), 256) : 0; }
 
     // scratch (may be null: the workspace): where the copies go, for a caller that holds a part of the
     // workspace itself
-    static int dot_operands(const hipq_dot_desc_t& d, const void* a, const void* b, const void* packed, const ZeroPoints& zp, DotOperands* o, hipStream_t s, uint8_t* scratch = nullptr)
+    static int dot_operands(const hipq_dot_desc_t& d, const void* a, const void* b, const void* packed, const ZeroPoints& zp, const Epilogue& epi, DotOperands* o, hipStream_t s,
+                            uint8_t* scratch = nullptr)
     {
         o->d = dot_seen(d);
         o->a = a;
         o->wfrag = nullptr;
         const size_t wbytes = dot_blob_weights(d);
         const size_t blob_bytes = packed ? 0 : wbytes + dot_blob_sums(d);
-        const size_t a_bytes = dot_padded_rows_bytes(d);
+        const bool in_place = dot_is_padded(d) && dot_ragged_preferred(o->d, d.K, epi);
+        o->a_row = in_place ? d.K : 0;
+        const size_t a_bytes = in_place ? 0 : dot_padded_rows_bytes(d);
         const uint8_t* blob = static_cast<const uint8_t*>(packed);
         if (blob_bytes + a_bytes)
         {
@@ -255,10 +262,10 @@ namespace hipq
         if (!dot_mfma_eligible(dot_seen(d)) || (misaligned & 15) || (copied && !packed && d.M * d.N < (1ll << 31) && d.M * d.N * d.K < (1ll << 24)))
             return launch_dot_direct(d, a, b, zp, epi, out, s);
         DotOperands o;
-        const int rc = dot_operands(d, a, b, packed, zp, &o, s, scratch);
+        const int rc = dot_operands(d, a, b, packed, zp, epi, &o, s, scratch);
         if (rc)
             return rc;
-        return launch_dot_mfma(o.d, o.a, o.w, o.wsum, zp, epi, out, s, o.wfrag);
+        return launch_dot_mfma(o.d, o.a, o.w, o.wsum, zp, epi, out, s, o.wfrag, o.a_row);
     }
 
     static int dot_pack(const hipq_dot_desc_t& d, const void* b, void* packed, bool with_fragments, hipStream_t s)
@@ -570,7 +577,7 @@ int hipq_quantized_dot_bias_gelu_quantize(const hipq_dot_desc_t* d,
     {
         DotOperands o;
         ZeroPoints zp{nullptr, nullptr, d->a_t, d->b_t};
-        rc = dot_operands(*d, a, w, packed_w, zp, &o, s);
+        rc = dot_operands(*d, a, w, packed_w, zp, e, &o, s);
         if (rc)
             return rc;
         Epilogue post = e;
