@@ -381,8 +381,11 @@ namespace hipq
     // Whether these kernels are the better ones.  Against the kernels that load straight into LDS (`dma`: 8-bit
     // or fused float rows in whole 16-byte pieces, channels in whole 64-byte slices) up to three 32 x 32
     // tiles a compute unit: above that those kernels' whole-line loads and larger tiles win (985 x 512 x
-    // 1536: 8.6 us there, 9.9 us here; 985 x 512 x 512: 7.9, 5.5).  Against the register-staged ones up to
-    // sixteen.
+    // 1536: 8.6 us there, 9.9 us here; 985 x 512 x 512: 7.9, 5.5); up to four on reductions of at most 256
+    // bytes and seven on those of one step, where their larger tiles wait for one slice as long as these do
+    // and leave compute units idle (784 x 256 x 1024 6.4, 5.6; 3136 x 64 x 256 6.4, 5.2; 6272 x 64 x 256 6.8, 5.9;
+    // but 1568 x 256 x 1024, six tiles a unit: 6.8, 7.9).  Not for at most 64 outputs (12544 x 256 x 64: 6.4,
+    // 6.7).  Against the register-staged ones up to sixteen.
     static bool wk_enabled()
     {
         // (the switches that name a kernel of the other family mean that family)
@@ -391,7 +394,11 @@ namespace hipq
                 return false;
         return true;
     }
-    bool wk_preferred(int64_t M, int64_t N, bool dma) { return wk_enabled() && wk_tiles(M, N, 32, 32) <= static_cast<int64_t>(device_compute_units()) * (dma ? 3 : 16); }
+    bool wk_preferred(int64_t M, int64_t N, int64_t steps, bool dma)
+    {
+        const int64_t limit = !dma ? 16 : N <= 64 || steps > 4 ? 3 : steps > 1 ? 4 : 7;
+        return wk_enabled() && wk_tiles(M, N, 32, 32) <= static_cast<int64_t>(device_compute_units()) * limit;
+    }
 
     // Whether rows (pixels) of `row_bytes` that are no multiple of 16 are read where they lie, instead of
     // through a copy padded to whole chunks (a launch, 2.5 us and more, and rows a power of two apart).
@@ -410,7 +417,7 @@ namespace hipq
         const int64_t tiles = wk_tiles(M, N, 32, 32), units = device_compute_units();
         if (!dma && pointwise && (steps <= 3 || (steps <= 6 && tiles <= units * 40)))
             return true;
-        if (!wk_preferred(M, N, dma))
+        if (!wk_preferred(M, N, steps, dma))
             return false;
         if (row_bytes % 4 == 0)
             return pointwise || steps <= 40;

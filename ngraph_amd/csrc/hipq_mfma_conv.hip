@@ -30,7 +30,7 @@ namespace hipq
     {
         const bool pointwise = g.taps() == 1 && g.st[1] == 1 && g.st[2] == 1;
         const bool dma = !out_ncx && g.K % 16 == 0 && (out_t == HIPQ_U8 || out_t == HIPQ_I8) && (g.C % 64 == 0 || pointwise);
-        return wk_preferred(g.N * g.out[1] * g.out[2], g.K, dma);
+        return wk_preferred(g.N * g.out[1] * g.out[2], g.K, (g.C * g.taps() + 63) / 64, dma);
     }
 
     bool conv_ragged_preferred(const ConvGeom& whole, const ConvGeom& padded, const Epilogue& epi, bool out_ncx)
