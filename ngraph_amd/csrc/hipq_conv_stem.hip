@@ -441,8 +441,12 @@ namespace hipq
             }
             else
                 out_rows = p.P;
-            // the largest band that fits LDS and the loader's registers
+            // of the bands that fit LDS and the loader's registers the one whose workgroups end first: rounds of
+            // items over the compute units times the convolution rows of an item (and about two rows' worth of
+            // latency).  224 x 224 images, 7 x 7 / 2 and a 3 x 3 / 2 pool: bands of four pooled rows from 16
+            // images on, single rows up to four (one image 12.2 -> 9.4 us)
             bool found = false;
+            int64_t least = 0;
             for (int rows = pool ? 4 : 8; rows >= 1; rows >>= 1)
             {
                 const int64_t CR = pool ? static_cast<int64_t>(rows - 1) * p.psh + p.wh : rows;
@@ -451,13 +455,17 @@ namespace hipq
                 const size_t need = static_cast<size_t>(IR * p.pitch) + raw_bytes + (pool ? static_cast<size_t>(CR * p.Q * kConvPixel) : 0) + 512;
                 if (need > kStemLdsLimit)
                     continue;
+                const int64_t units = device_compute_units();
+                const int64_t cost = (g.N * ((out_rows + rows - 1) / rows) + units - 1) / units * (CR + 2);
+                if (found && cost >= least)
+                    continue;
+                least = cost;
                 p.raw_bytes = static_cast<int32_t>(raw_bytes);
                 p.band_rows = rows;
                 p.CR = static_cast<int32_t>(CR);
                 p.IR = static_cast<int32_t>(IR);
                 *lds_bytes = need;
                 found = true;
-                break;
             }
             if (!found)
                 return false;
