@@ -353,6 +353,7 @@ namespace hipq
     enum class WkShape
     {
         kTile1181, // 16 x 16, eight wavefronts on the reduction
+        kTile11161, // the same, sixteen
         kTile1241, // 16 x 32, four
         kTile2241, // 32 x 32, four
         kTile2222, // two tiles of 32 x 32, two wavefronts each
@@ -365,7 +366,10 @@ namespace hipq
     // short and there are many of them.  Fewer tiles: 16 x 32, and where even those leave half of the chip
     // idle on a reduction of eight steps or more, 16 x 16 with eight wavefronts on it.  (The lines are those
     // that cost least over 200 products and convolutions of 1 to 90 000 rows, 64 to 9 600 bytes of reduction
-    // and 16 to 4 000 outputs, each timed in all five shapes: 1.7 % above the best shape of each on average.)
+    // and 16 to 4 000 outputs, each timed in five shapes: 1.7 % above the best shape of each on average.)
+    // Reductions that eight wavefronts cannot ask for at once (more than 48 steps) and sixteen ask for in four
+    // loads each take sixteen: 40 x 4096 x 512 5.6 -> 5.3 us, 100 x 4004 x 200 5.6 -> 5.1, 400 -> 400 3 x 3 on 9 x 9
+    // 6.8 -> 6.2; from five loads on the larger exchange costs more (512 -> 512 3 x 3 on 7 x 7 8.0 -> 8.2).
     static WkShape wk_shape(int64_t M, int64_t N, int64_t Kred)
     {
         const int64_t t22 = wk_tiles(M, N, 32, 32), steps = (Kred + 63) / 64, units = device_compute_units();
@@ -375,7 +379,9 @@ namespace hipq
                 return WkShape::kTile2241;
             return steps <= 2 ? WkShape::kTile2214 : WkShape::kTile2222;
         }
-        return wk_tiles(M, N, 16, 32) * 2 >= units || steps < 8 ? WkShape::kTile1241 : WkShape::kTile1181;
+        if (wk_tiles(M, N, 16, 32) * 2 >= units || steps < 8)
+            return WkShape::kTile1241;
+        return steps > 48 && steps <= 64 ? WkShape::kTile11161 : WkShape::kTile1181;
     }
 
     // Whether these kernels are the better ones.  Against the kernels that load straight into LDS (`dma`: 8-bit
@@ -457,6 +463,7 @@ namespace hipq
         switch (wk_shape(p.M, om.N, p.Kred))
         {
             WK(1, 1, 8, 1, 6);
+            WK(1, 1, 16, 1, 6);
             WK(1, 2, 4, 1, 6);
             WK(2, 2, 1, 4, 5);
             WK(2, 2, 2, 2, 5);

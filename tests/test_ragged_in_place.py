@@ -11,9 +11,10 @@ from ngraph_amd import synth
 pytestmark = pytest.mark.gpu
 
 
-# reductions of every remainder (a step more or less than whole), one row, a row more than a block, several
+# reductions of every remainder (a step more or less than whole), one row, a row more than a block, several;
+# of 49 and 63 steps, which sixteen wavefronts share unevenly
 @pytest.mark.parametrize("M", [1, 17, 67])
-@pytest.mark.parametrize("K", [65, 66, 71, 77, 79, 127, 129, 334, 1000, 1535, 2044])
+@pytest.mark.parametrize("K", [65, 66, 71, 77, 79, 127, 129, 334, 1000, 1535, 2044, 3076, 4004])
 def test_dot_rows(gpu_lib, M, K):
     N = 101
     a = synth.uniform_int(21, (M, K), 0, 255, np.uint8)
