@@ -52,8 +52,12 @@ namespace hipq
             return launch_conv_rowpack(whole, rp, ws, packed, zp, epi, out, s);
         }
         ConvGeom padded;
-        // (the entry point that allocates nothing keeps the direct kernel where the copy would not fit its array)
-        const bool pad = packed && !conv_mfma_eligible(whole) && conv_pad_eligible(whole, &padded) && (whole.C < 16 || workspace_holds(static_cast<size_t>(padded.in_count()) + 256));
+        // (widths above 16 that are no multiple of it: tensors that start on no 16-byte boundary keep the direct
+        // kernel, as products do, and so does the entry point that allocates nothing where the copy would not
+        // fit its array)
+        const bool aligned = ((reinterpret_cast<uintptr_t>(packed) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(epi.sum_in)) & 15) == 0;
+        const bool pad =
+            packed && !conv_mfma_eligible(whole) && conv_pad_eligible(whole, &padded) && (whole.C < 16 || (aligned && workspace_holds(static_cast<size_t>(padded.in_count()) + 256)));
         if (!packed || (!pad && !conv_mfma_eligible(whole)) || (epi.mode == EPI_FUSED && whole.out_t == HIPQ_I32))
             return launch_conv_direct(whole, data, filter, zp, epi, out, s);
         // the geometry the MFMA kernels see: channels in whole 16-byte pieces
@@ -254,9 +258,9 @@ namespace hipq
         if (d.M == 0 || d.N == 0)
             return HIPQ_OK;
         HIPQ_REQUIRE(out && (d.K == 0 || (a && b)), "null tensor pointer");
-        // (operands that the padded copies replace may start anywhere)
+        // (operands that the padded copies replace may start anywhere, the packed weights they are read from may not)
         const bool copied = dot_is_padded(d);
-        const uintptr_t misaligned = reinterpret_cast<uintptr_t>(out) | (copied ? 0 : reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b));
+        const uintptr_t misaligned = reinterpret_cast<uintptr_t>(out) | (copied ? reinterpret_cast<uintptr_t>(packed) : reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b));
         // Padding and packing a reduction on the fly is three launches ahead of the product: from 2^24
         // multiply-adds on, where the direct kernel takes ten times as long as those
         if (!dot_mfma_eligible(dot_seen(d)) || (misaligned & 15) || (copied && !packed && d.M * d.N < (1ll << 31) && d.M * d.N * d.K < (1ll << 24)))

@@ -86,3 +86,40 @@ def test_dot_odd_reductions(gpu_lib, shape):
             got = H.quantized_dot_bias(d, f, a, w, bias, scales)
             assert np.array_equal(got.view(np.uint8), exp.view(np.uint8)), (a_t, out_t, H.last_kernel())
     O.port().orc_set_threads(1)
+
+
+# (through the kernel that reads pixels where they lie, the padded copies, the pointwise kernel and the one
+# that keeps the filter in registers)
+@pytest.mark.parametrize("case", [(1, 50, 33, (17, 13), 3, H.NXC, H.NXC), (2, 50, 33, (17, 13), 3, H.NCX, H.NCX), (2, 63, 256, (16, 12), 1, H.NXC, H.NXC), (1, 63, 64, (16, 16), 3, H.NCX, H.NCX)])
+def test_conv_odd_channels_at_any_address(gpu_lib, case, monkeypatch):
+    """tensors that start on no 16-byte boundary are taken, each of them alone: what lies around the output stays"""
+    N, Cc, K, sp, f, dl, ol = case
+    monkeypatch.setenv("HIPQ_PW64_MIN_ROWS", "1")
+    pad = (f // 2, f // 2)
+    kw = dict(pad_below=pad, pad_above=pad, out_t="u8")
+    d0 = H.make_conv_desc(N, Cc, K, sp, (f, f), **kw)
+    d = H.make_conv_desc(N, Cc, K, sp, (f, f), data_layout=dl, out_layout=ol, **kw)
+    fd = H.make_fused_desc(has_bias=True, has_sum=True, sum_t="u8", with_relu=True, scale_count=K)
+    data = synth.uniform_int(41, d0.data_shape(), 0, 255, np.uint8)
+    filt = synth.uniform_int(42, d0.filter_shape(), -128, 127, np.int8)
+    bias = synth.uniform_int(43, (K,), -3000, 3000, np.int32)
+    scale = synth.uniform_f32(44, (K,), 0.8, 1.2) * np.float32(0.01 / np.sqrt(Cc * f * f))
+    res = synth.uniform_int(45, d0.out_shape(), 0, 255, np.uint8)
+    exp = O.quantized_convolution_fused(d0, fd, data, filt, bias, res, scale, 0.5)
+    x, r = (to_nxc(data) if dl == H.NXC else data), (to_nxc(res) if ol == H.NXC else res)
+    bf = H.DeviceBuffer.from_numpy(filt)
+    packed = H.pack_filter(d, bf)
+    whole, bb, bs, bss = packed.to_numpy(np.uint8, (packed.nbytes,)), H._dev(bias), H._dev(scale), H._dev(np.float32(0.5))
+
+    def at(a, offset):
+        return H.DeviceBuffer.from_numpy(np.concatenate([np.full(offset, 77, np.uint8), np.ascontiguousarray(a).view(np.uint8).ravel(), np.full(32, 77, np.uint8)]))
+
+    for o_data, o_packed, o_sum, o_out in ((0, 0, 0, 0), (1, 0, 0, 0), (0, 4, 0, 0), (0, 0, 1, 0), (0, 0, 0, 1), (0, 0, 0, 8)):
+        print("odd conv at", case, o_data, o_packed, o_sum, o_out, flush=True)
+        bx, bp, br, out = at(x, o_data), at(whole, o_packed), at(r, o_sum), at(np.zeros(exp.size, np.uint8), o_out)
+        H.check(gpu_lib.hipq_quantized_convolution_fused(H.C.byref(d), H.C.byref(fd), bx.ptr + o_data, bf.ptr, bp.ptr + o_packed, bb.ptr, br.ptr + o_sum, bs.ptr, bss.ptr, out.ptr + o_out, None))
+        H.check(gpu_lib.hipq_stream_sync(None))
+        got = out.to_numpy(np.uint8, (out.nbytes,))
+        inner = got[o_out : o_out + exp.size].reshape(d.out_shape())
+        assert np.array_equal(to_ncx(inner) if ol == H.NXC else inner, exp), H.last_kernel()
+        assert (got[:o_out] == 77).all() and (got[o_out + exp.size :] == 77).all()
