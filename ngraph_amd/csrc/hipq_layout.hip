@@ -126,63 +126,70 @@ namespace hipq
     // packed form of a QuantizedDot operand.  The rows of the input start at any address, so its loads
     // are unaligned 16-byte ones; the output's rows are whole 16-byte pieces.  Bound by HBM where
     // the tensor is large; u8 [8][90][35 * 29] takes 4.9 us in a kernel trace, most of it launch and latency.
-    __global__ __launch_bounds__(256) void transpose_pad_bytes_kernel(const uint8_t* __restrict__ in, uint8_t* __restrict__ out, int32_t R, int32_t Cc, int32_t Rp, int32_t tiles_c,
+    __global__ __launch_bounds__(256) void transpose_pad_bytes_kernel(const uint8_t* __restrict__ in, uint8_t* __restrict__ out, int32_t B, int32_t R, int32_t Cc, int32_t Rp, int32_t tiles_c,
                                                                       int64_t bytes, const void* zp, int32_t zp_t)
     {
         __shared__ uint32_t tile[4][64][17];
         const int wave = threadIdx.x >> 6;
         const int t = threadIdx.x & 63;
         const int tc = wave % tiles_c, tr = wave / tiles_c;
-        const int r0 = (static_cast<int>(blockIdx.y) * (4 / tiles_c) + tr) * 64;
+        const int rows = (4 / tiles_c) * 64; // of a workgroup
         const int c0 = (static_cast<int>(blockIdx.x) * tiles_c + tc) * 64;
         const int fill = static_cast<int>((static_cast<uint32_t>(load_zp(zp, zp_t)) & 0xffu) * 0x01010101u);
-        const int64_t plane = static_cast<int64_t>(blockIdx.z) * R * Cc;
-        uint8_t* const dst = out + static_cast<int64_t>(blockIdx.z) * Cc * Rp;
-        {
-            const int rg = t >> 2, cb = t & 3; // rows 4rg..4rg+3, columns 16cb..16cb+15 of the tile
-            v4t l[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
+        // (a launch has at most 65535 workgroups along these two axes; one trip each below that)
+        for (int32_t b = static_cast<int32_t>(blockIdx.z); b < B; b += static_cast<int32_t>(gridDim.z))
+            for (int32_t row0 = static_cast<int32_t>(blockIdx.y) * rows; row0 < Rp; row0 += static_cast<int32_t>(gridDim.y) * rows)
             {
-                const int r = r0 + 4 * rg + i, c = c0 + 16 * cb;
-                const int64_t at = plane + static_cast<int64_t>(r) * Cc + c;
-                l[i] = (r < R && c < Cc) ? load16_inside(in + at, bytes - at) : v4t{fill, fill, fill, fill};
+                const int r0 = row0 + tr * 64;
+                const int64_t plane = static_cast<int64_t>(b) * R * Cc;
+                uint8_t* const dst = out + static_cast<int64_t>(b) * Cc * Rp;
+                {
+                    const int rg = t >> 2, cb = t & 3; // rows 4rg..4rg+3, columns 16cb..16cb+15 of the tile
+                    v4t l[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                    {
+                        const int r = r0 + 4 * rg + i, c = c0 + 16 * cb;
+                        const int64_t at = plane + static_cast<int64_t>(r) * Cc + c;
+                        l[i] = (r < R && c < Cc) ? load16_inside(in + at, bytes - at) : v4t{fill, fill, fill, fill};
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                    {
+                        const uint32_t d[4] = {static_cast<uint32_t>(l[0][q]), static_cast<uint32_t>(l[1][q]), static_cast<uint32_t>(l[2][q]), static_cast<uint32_t>(l[3][q])};
+                        uint32_t o[4];
+                        transpose4x4(d, o);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            tile[wave][16 * cb + 4 * q + j][rg] = o[j];
+                    }
+                }
+                __syncthreads();
+#pragma unroll
+                for (int it = 0; it < 4; ++it)
+                {
+                    const int col = it * 16 + (t >> 2), q = t & 3;
+                    const v4t v = v4t{static_cast<int>(tile[wave][col][4 * q]), static_cast<int>(tile[wave][col][4 * q + 1]), static_cast<int>(tile[wave][col][4 * q + 2]),
+                                      static_cast<int>(tile[wave][col][4 * q + 3])};
+                    const int c = c0 + col, r = r0 + 16 * q;
+                    if (c < Cc && r < Rp)
+                        *reinterpret_cast<v4t*>(dst + static_cast<int64_t>(c) * Rp + r) = v;
+                }
+                __syncthreads(); // the tile is read: the next trip may write it
             }
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-            {
-                const uint32_t d[4] = {static_cast<uint32_t>(l[0][q]), static_cast<uint32_t>(l[1][q]), static_cast<uint32_t>(l[2][q]), static_cast<uint32_t>(l[3][q])};
-                uint32_t o[4];
-                transpose4x4(d, o);
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    tile[wave][16 * cb + 4 * q + j][rg] = o[j];
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int it = 0; it < 4; ++it)
-        {
-            const int col = it * 16 + (t >> 2), q = t & 3;
-            const v4t v = v4t{static_cast<int>(tile[wave][col][4 * q]), static_cast<int>(tile[wave][col][4 * q + 1]), static_cast<int>(tile[wave][col][4 * q + 2]),
-                              static_cast<int>(tile[wave][col][4 * q + 3])};
-            const int c = c0 + col, r = r0 + 16 * q;
-            if (c < Cc && r < Rp)
-                *reinterpret_cast<v4t*>(dst + static_cast<int64_t>(c) * Rp + r) = v;
-        }
     }
 
     int launch_transpose_pad(const void* in, void* out, int64_t B, int64_t R, int64_t Cc, int64_t Rp, const void* zp, int zp_t, hipStream_t s)
     {
         if (B == 0 || R == 0 || Cc == 0)
             return HIPQ_OK;
-        HIPQ_REQUIRE(B <= 65535 && Rp % 16 == 0 && Rp >= R && Rp < (1ll << 31) && Cc < (1ll << 31), "extent too large for the padded transpose");
+        // (B and R with room for the last trip's step beyond them)
+        HIPQ_REQUIRE(B < (1ll << 31) - 65535 && Rp % 16 == 0 && Rp >= R && Rp < (1ll << 31) - 65535 * 256 && Cc < (1ll << 31), "extent too large for the padded transpose");
         const int tiles_c = Cc > 128 ? 4 : (Cc > 64 ? 2 : 1);
         const int64_t gx = (Cc + 64 * tiles_c - 1) / (64 * tiles_c), gy = (Rp + 64 * (4 / tiles_c) - 1) / (64 * (4 / tiles_c));
-        HIPQ_REQUIRE(gy <= 65535, "extent too large for the transpose grid");
-        dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(gy), static_cast<unsigned>(B));
-        transpose_pad_bytes_kernel<<<grid, 256, 0, s>>>(static_cast<const uint8_t*>(in), static_cast<uint8_t*>(out), static_cast<int32_t>(R), static_cast<int32_t>(Cc), static_cast<int32_t>(Rp),
-                                                       tiles_c, B * R * Cc, zp, zp_t);
+        dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(std::min<int64_t>(gy, 65535)), static_cast<unsigned>(std::min<int64_t>(B, 65535)));
+        transpose_pad_bytes_kernel<<<grid, 256, 0, s>>>(static_cast<const uint8_t*>(in), static_cast<uint8_t*>(out), static_cast<int32_t>(B), static_cast<int32_t>(R), static_cast<int32_t>(Cc),
+                                                       static_cast<int32_t>(Rp), tiles_c, B * R * Cc, zp, zp_t);
         return check_launch("transpose_pad_bytes");
     }
 

@@ -117,6 +117,7 @@ namespace hipq
         }
         if (tr_in)
         {
+            HIPQ_REQUIRE(g.N <= 65535, "batch %lld beyond 65535", (long long)g.N);
             const int rc = in_sp % 16 == 0 ? launch_transpose(data, ws, g.N, g.C, in_sp, 1, s) : launch_transpose_pad(data, ws, g.N, g.C, in_sp, g.C, nullptr, HIPQ_U8, s);
             if (rc)
                 return rc;

@@ -123,3 +123,30 @@ def test_conv_odd_channels_at_any_address(gpu_lib, case, monkeypatch):
         inner = got[o_out : o_out + exp.size].reshape(d.out_shape())
         assert np.array_equal(to_ncx(inner) if ol == H.NXC else inner, exp), H.last_kernel()
         assert (got[:o_out] == 77).all() and (got[o_out + exp.size :] == 77).all()
+
+
+@pytest.mark.parametrize("N", [65535, 65536, 140001])
+def test_conv_odd_channels_of_large_batches(gpu_lib, N):
+    """more pictures than a launch has workgroups along one axis, [N][C][X] and odd widths: all are transposed"""
+    print("odd conv, batch", N, flush=True)
+    O.port().orc_set_threads(8)
+    d = H.make_conv_desc(N, 17, 5, (2, 1), (1, 1), out_t="i8")
+    data = synth.uniform_int(46, d.data_shape(), 0, 255, np.uint8)
+    filt = synth.uniform_int(47, d.filter_shape(), -128, 127, np.int8)
+    exp = O.quantized_convolution(d, data, filt, 0.02, 7, 0.005, 0, 0.5, 3)
+    got = H.quantized_convolution(d, data, filt, 0.02, 7, 0.005, 0, 0.5, 3)
+    assert H.last_kernel() != "conv_direct" and np.array_equal(got, exp)
+    O.port().orc_set_threads(1)
+
+
+def test_dot_odd_reduction_longer_than_a_grid(gpu_lib):
+    """weights [K, N] whose padded transposition has more row tiles than a launch has workgroups along one axis"""
+    K, N = 65535 * 256 + 17, 3
+    print("odd dot, long reduction", K, flush=True)
+    a = synth.uniform_int(48, (1, K), 0, 1, np.uint8)
+    b = synth.uniform_int(49, (K, N), -1, 1, np.int8)
+    a[0, -5:], b[-5:] = 1, 127
+    d = H.make_dot_desc(1, K, N, a_t="u8", out_t="i32")
+    got = H.quantized_dot(d, a, b, 1.0, 0, 1.0, 0, 1.0, 0)
+    assert H.last_kernel() != "dot_direct"
+    assert np.array_equal(got, (a.astype(np.int64) @ b.astype(np.int64)).astype(np.int32))
