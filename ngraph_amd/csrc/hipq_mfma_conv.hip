@@ -108,9 +108,7 @@ namespace hipq
         const int xu = g.data_t == HIPQ_U8 ? 1 : 0;
         if (conv_wk_preferred(g, epi.out_t, out_ncx))
         {
-            // (a layer of at most 64 output pixels is a product of as many rows)
-            const bool rows = !out_ncx && M <= 64 && Kred % 64 == 0 && Kred >= 256;
-            const int rc = launch_conv_wk(xl, w, wsum, M, N, Kred, xu, zp, epi, om, out, s, rows ? "dot_skinny_wk_i8_16x16x64" : "conv_mfma_wk_i8_16x16x64");
+            const int rc = launch_conv_wk(xl, w, wsum, M, N, Kred, xu, zp, epi, om, out, s, "conv_mfma_wk_i8_16x16x64");
             if (rc != HIPQ_ERR_UNSUPPORTED)
                 return rc;
         }

@@ -1027,7 +1027,7 @@ namespace hipq
         if (wk_preferred(M, N, (K + 63) / 64, N % 16 == 0))
         {
             // (128 x 768 x 3072: product, then Gelu and Quantize from the workspace 14.4 us, in one kernel 5.4)
-            const int rc = launch_rows_wk(a, a_unsigned, w_nk, w_frag, wsum, M, N, K, zp, epi, out, s, M > 256 && N > 64 && N % 16 == 0 ? "dot_gelu_q8_wk_i8_16x16x64" : "dot_wk_gelu_vec");
+            const int rc = launch_rows_wk(a, a_unsigned, w_nk, w_frag, wsum, M, N, K, zp, epi, out, s, "dot_gelu_q8_wk_i8_16x16x64");
             if (rc != HIPQ_ERR_UNSUPPORTED)
                 return rc;
         }
@@ -1095,19 +1095,14 @@ namespace hipq
             const int64_t steps = (d.K + 63) / 64;
             const bool rows64 = skinny && d.M > 64 && dot_rows64_eligible(d);
             bool wk = wk_preferred(d.M, d.N, steps, dma);
-            const char* name = "dot_mfma_wk_i8_16x16x64";
             if (skinny && d.M <= 32 && w_frag && steps >= (d.M <= 16 ? 12 : 24))
                 wk = false;
             else if (rows64)
-            {
                 wk = wk && ((d.M + 31) / 32) * ((d.N + 31) / 32) * steps <= 8192;
-                name = w_frag && d.K <= 4096 ? "dot_rows64w_wk_i8_16x16x64" : "dot_rows64_wk_i8_16x16x64";
-            }
-            else if (skinny && (d.M <= 64 || !dma))
-                name = w_frag && (d.M <= 16 ? d.K <= 8192 : d.M <= 32 && d.K <= 4096) ? "dot_skinnyf_wk_i8_16x16x64" : "dot_skinny_wk_i8_16x16x64";
             if (wk)
             {
-                const int rc = launch_rows_wk(a, d.a_t == HIPQ_U8, static_cast<const int8_t*>(w_nk), w_frag, wsum, d.M, static_cast<int32_t>(d.N), static_cast<int32_t>(d.K), zp, epi, out, s, name);
+                const int rc = launch_rows_wk(a, d.a_t == HIPQ_U8, static_cast<const int8_t*>(w_nk), w_frag, wsum, d.M, static_cast<int32_t>(d.N), static_cast<int32_t>(d.K), zp, epi, out, s,
+                                              "dot_mfma_wk_i8_16x16x64");
                 if (rc != HIPQ_ERR_UNSUPPORTED)
                     return rc;
             }

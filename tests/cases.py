@@ -123,3 +123,9 @@ def dot_bias_closed_form(a, w, bias, scales, out_t, relu):
         return v
     lo, hi = (0, 255) if out_t == "u8" else (-128, 127)
     return np.clip(np.rint(v), lo, hi).astype(np.uint8 if out_t == "u8" else np.int8)
+
+
+def ran(family, *prefixes):
+    """the last call's kernel is one of `prefixes`; as the library chooses it may be one for small products instead"""
+    kernel = H.last_kernel()
+    assert family == "chosen" if "_wk_" in kernel else kernel.startswith(prefixes), kernel

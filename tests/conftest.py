@@ -48,3 +48,12 @@ def gpu_lib():
     assert n.value >= 1, "no HIP device visible"
     H.check(lib.hipq_set_device(0))
     return lib
+
+
+@pytest.fixture(params=["chosen", "large"])
+def family(request, monkeypatch):
+    """Products and convolutions of few tiles run on the kernels for small ones ("chosen": as the library
+    has it), and with those switched off on the kernels that larger ones run on ("large")."""
+    if request.param == "large":
+        monkeypatch.setenv("HIPQ_NO_WK", "1")
+    return request.param

@@ -57,8 +57,9 @@ def test_pw64_against_oracle_and_tile_kernel(gpu_lib, i, monkeypatch):
     assert np.array_equal(cases.to_ncx(got), exp), CASES[i]
     assert len(np.unique(got)) > 30
     monkeypatch.setenv("HIPQ_NO_PW64", "1")
+    monkeypatch.setenv("HIPQ_NO_WK", "1")
     other = H.quantized_convolution_fused(d, f, x, filt, bias, sm, scales, ss)
-    assert H.last_kernel().startswith("conv_mfma"), H.last_kernel()
+    assert H.last_kernel() == "conv_mfma_i8_32x32x32", H.last_kernel()
     assert np.array_equal(other, got)
     O.port().orc_set_threads(1)
 

@@ -222,7 +222,7 @@ def test_conv_kats(gpu_lib, kats):
             assert got.reshape(-1).astype(np.int64).tolist() == exp.astype(np.int64).tolist(), (k["name"], name)
 
 
-def test_conv_reference_vectors(gpu_lib, ref_vectors):
+def test_conv_reference_vectors(gpu_lib, family, ref_vectors):
     """compiled-reference outputs, including BASELINE config 1 with its wrapped outputs"""
     manifest, arrays = ref_vectors
     used = set()
@@ -238,7 +238,7 @@ def test_conv_reference_vectors(gpu_lib, ref_vectors):
         dl = cases.conv_from_manifest(m, H.NXC, H.NXC)[0]
         for name, got, kern in _conv_both(dl, cases.to_nxc(data), filt, s, z):
             assert np.array_equal(cases.to_ncx(got), arrays[m["name"]]), (m["name"], name, "nxc")
-    assert "conv_direct" in used and any(k.startswith(("conv_mfma", "dot_skinny")) for k in used), used
+    assert "conv_direct" in used and any(k.startswith("conv_mfma") for k in used), used
 
 
 MFMA_SHAPES = [
@@ -259,7 +259,7 @@ MFMA_SHAPES = [
 
 
 @pytest.mark.parametrize("i", range(len(MFMA_SHAPES)))
-def test_conv_mfma_shapes(gpu_lib, i):
+def test_conv_mfma_shapes(gpu_lib, family, i):
     N, Cc, K, in_sp, f_sp, kw = MFMA_SHAPES[i]
     say("mfma conv", MFMA_SHAPES[i])
     for out_t, s, z in (("i32", (1.0, 1.0, 1.0), (0, 0, 0)), ("i8", (0.02, 0.005, 0.9), (0, 0, -3)), ("i8", (0.02, 0.005, 0.7), (131, 0, 0))):
@@ -270,7 +270,7 @@ def test_conv_mfma_shapes(gpu_lib, i):
         exp = O.quantized_convolution(d, data, filt, s[0], z[0], s[1], z[1], s[2], z[2])
         O.port().orc_set_threads(1)
         got = H.quantized_convolution(d, data, filt, s[0], z[0], s[1], z[1], s[2], z[2])
-        assert H.last_kernel().startswith(("conv_mfma", "conv_band", "conv_regw", "dot_skinny")), H.last_kernel()
+        cases.ran(family, "conv_mfma", "conv_band", "conv_regw")
         assert np.array_equal(got, exp), (out_t, z)
     # reference layouts in and out (transposed through the workspace)
     d = H.make_conv_desc(N, Cc, K, in_sp, f_sp, out_t="i8", **kw)
@@ -279,11 +279,11 @@ def test_conv_mfma_shapes(gpu_lib, i):
     exp = O.quantized_convolution(d, data, filt, 0.02, 0, 0.005, 0, 0.9, 0)
     O.port().orc_set_threads(1)
     got = H.quantized_convolution(d, data, filt, 0.02, 0, 0.005, 0, 0.9, 0)
-    assert H.last_kernel().startswith(("conv_mfma", "conv_band", "conv_regw", "dot_skinny")), H.last_kernel()
+    cases.ran(family, "conv_mfma", "conv_band", "conv_regw")
     assert np.array_equal(got, exp)
 
 
-def test_conv_mfma_nonzero_filter_zero_point(gpu_lib):
+def test_conv_mfma_nonzero_filter_zero_point(gpu_lib, family):
     """packed filter handed over although the filter zero point is not zero: the kernel's slow
     in-kernel path must still give the reference's numbers"""
     say("mfma conv, filter zp != 0")
@@ -295,7 +295,7 @@ def test_conv_mfma_nonzero_filter_zero_point(gpu_lib):
     assert np.array_equal(got, exp)
 
 
-def test_conv_i8_data(gpu_lib):
+def test_conv_i8_data(gpu_lib, family):
     say("i8 data")
     d = H.make_conv_desc(1, 32, 48, (9, 9), (3, 3), pad_below=(1, 1), pad_above=(1, 1), data_t="i8", out_t="i32", data_layout=H.NXC, out_layout=H.NXC)
     data = synth.uniform_int(41, d.data_shape(), -128, 127, np.int8)
@@ -320,7 +320,7 @@ def test_conv_linearity_at_config1_batch(gpu_lib):
     a = H.quantized_convolution(d, data, f1, 1.0, 0, 1.0, 0, 1.0, 0).astype(np.int64)
     b = H.quantized_convolution(d, data, f2, 1.0, 0, 1.0, 0, 1.0, 0).astype(np.int64)
     c = H.quantized_convolution(d, data, (f1 + f2).astype(np.int8), 1.0, 0, 1.0, 0, 1.0, 0).astype(np.int64)
-    assert H.last_kernel().startswith(("conv_mfma", "conv_band", "conv_regw", "dot_skinny"))
+    assert H.last_kernel().startswith(("conv_mfma", "conv_band", "conv_regw"))
     assert np.array_equal(a + b, c)
     d1 = H.make_conv_desc(1, 64, 64, (56, 56), (3, 3), **kw)
     O.port().orc_set_threads(8)
@@ -371,7 +371,7 @@ def test_quant_conv_linear_rne_kat(gpu_lib, kats):
 @pytest.mark.parametrize("relu", [False, True])
 @pytest.mark.parametrize("has_sum", [False, True])
 @pytest.mark.parametrize("layout", [H.NCX, H.NXC])
-def test_fused_conv_random(gpu_lib, relu, has_sum, layout):
+def test_fused_conv_random(gpu_lib, family, relu, has_sum, layout):
     """ResNet-style bottleneck piece: per-channel scales, bias, residual sum, relu; both kernels"""
     say("fused conv", relu, has_sum, layout)
     out_t = "u8" if relu else "i8"
@@ -469,23 +469,22 @@ def test_conv_band(gpu_lib, i, monkeypatch):
     assert any(k.startswith("conv_band") for k in kernels), kernels
 
 
-SKINNY_CONV_SHAPES = [
+FEW_PIXEL_SHAPES = [
     # N, C, K, in_sp, f_sp, kw : at most 64 output pixels in all and a reduction of whole 64-byte steps
-    (1, 256, 64, (8, 7), (1, 1), dict()),                                                    # the data is the matrix
-    (1, 512, 512, (7, 7), (3, 3), dict(pad_below=(1, 1), pad_above=(1, 1))),                 # im2col, padding taps
+    (1, 256, 64, (8, 7), (1, 1), dict()),                                                    # one tap
+    (1, 512, 512, (7, 7), (3, 3), dict(pad_below=(1, 1), pad_above=(1, 1))),                 # padding taps
     (1, 64, 96, (12, 12), (3, 3), dict(stride=(2, 2), pad_below=(1, 1), pad_above=(0, 1))),  # stride, ragged K
     (1, 128, 40, (7, 8), (2, 2), dict(dilation=(2, 1), pad_below=(1, 0), pad_above=(1, 0))),
     (3, 256, 1000, (1, 1), (1, 1), dict()),                                                  # a classifier as a convolution
 ]
 
 
-@pytest.mark.parametrize("i", range(len(SKINNY_CONV_SHAPES)))
-def test_conv_as_skinny_gemm(gpu_lib, i):
-    """layers with few output pixels run as a GEMM over their receptive-field matrix on the
-    weight-streaming kernels: both policies, zero points (padding holds the data zero point; a filter
-    zero point takes the exact path), reference-layout input (transposed, then gathered), residual sum"""
-    N, Cc, K, in_sp, f_sp, kw = SKINNY_CONV_SHAPES[i]
-    say("skinny conv", SKINNY_CONV_SHAPES[i])
+@pytest.mark.parametrize("i", range(len(FEW_PIXEL_SHAPES)))
+def test_conv_few_pixels(gpu_lib, family, i):
+    """layers with few output pixels: both policies, zero points (padding holds the data zero point; a filter
+    zero point takes the exact path), reference-layout input (transposed first), residual sum"""
+    N, Cc, K, in_sp, f_sp, kw = FEW_PIXEL_SHAPES[i]
+    say("few pixels", FEW_PIXEL_SHAPES[i])
     O.port().orc_set_threads(8)
     for dl in (H.NXC, H.NCX):
         for out_t, z in (("i8", (0, 0, -3)), ("u8", (131, 0, 7)), ("i32", (3, 0, 0)), ("i8", (9, -7, 1))):
@@ -496,7 +495,7 @@ def test_conv_as_skinny_gemm(gpu_lib, i):
             s = (1.0, 1.0, 1.0) if out_t == "i32" else (0.02, 0.005, 0.9)
             exp = O.quantized_convolution(dn, data, filt, s[0], z[0], s[1], z[1], s[2], z[2])
             got = H.quantized_convolution(d, cases.to_nxc(data) if dl == H.NXC else data, filt, s[0], z[0], s[1], z[1], s[2], z[2])
-            assert H.last_kernel().startswith("dot_skinny"), H.last_kernel()
+            cases.ran(family, "conv_mfma")
             assert np.array_equal(cases.to_ncx(got), exp), (dl, out_t, z)
         for relu, has_sum in ((True, True), (False, False)):
             out_t = "u8" if relu else "i8"
@@ -510,7 +509,7 @@ def test_conv_as_skinny_gemm(gpu_lib, i):
             f = H.make_fused_desc(has_bias=True, has_sum=has_sum, sum_t="u8", with_relu=relu, scale_count=K)
             exp = O.quantized_convolution_fused(dn, f, data, filt, bias, summ, scales, 0.37 if has_sum else None)
             got = H.quantized_convolution_fused(d, f, cases.to_nxc(data) if dl == H.NXC else data, filt, bias, cases.to_nxc(summ) if has_sum else None, scales, 0.37 if has_sum else None)
-            assert H.last_kernel().startswith("dot_skinny"), H.last_kernel()
+            cases.ran(family, "conv_mfma")
             assert np.array_equal(cases.to_ncx(got), exp), (dl, relu, has_sum)
     O.port().orc_set_threads(1)
 
@@ -524,7 +523,7 @@ SPLIT_CONV_SHAPES = [
 ]
 
 
-def test_conv_bias_in_accumulator(gpu_lib):
+def test_conv_bias_in_accumulator(gpu_lib, family):
     """short reductions add small biases to the accumulators as integers (exact: no float rounding
     happens below 2^24); a column block holding a bias beyond 2^24 keeps the float add -- both kinds
     in one call, with and without a residual, against the oracle"""
@@ -546,7 +545,7 @@ def test_conv_bias_in_accumulator(gpu_lib):
         f = H.make_fused_desc(has_bias=True, has_sum=has_sum, sum_t="u8", with_relu=True, scale_count=K)
         exp = O.quantized_convolution_fused(dn, f, data, filt, bias, summ, scales, 0.21 if has_sum else None)
         got = H.quantized_convolution_fused(d, f, cases.to_nxc(data), filt, bias, cases.to_nxc(summ) if has_sum else None, scales, 0.21 if has_sum else None)
-        assert H.last_kernel().startswith("conv_mfma"), H.last_kernel()
+        cases.ran(family, "conv_mfma")
         assert np.array_equal(cases.to_ncx(got), exp), has_sum
         assert len(np.unique(exp)) > 50  # the outputs are spread, not saturated
     O.port().orc_set_threads(1)
@@ -574,7 +573,7 @@ def _conv_sweep():
 
 
 @pytest.mark.parametrize("case", _conv_sweep())
-def test_conv_fused_nxc_sweep(gpu_lib, case):
+def test_conv_fused_nxc_sweep(gpu_lib, family, case):
     """QuantizedConvolutionBias(+Add)+ReLU, channels-last in and out, over seeded ResNet-like layers, against the oracle"""
     N, Cc, K, hw, r, st, res = case
     say("conv fused nxc sweep", case)
@@ -602,7 +601,7 @@ def test_conv_register_staged(gpu_lib, i, monkeypatch):
     take the kernels whose loads go straight into LDS unless this switch is set; there, padding
     with a non-zero data zero point is patched in after the load)"""
     monkeypatch.setenv("HIPQ_NO_CONV_DMA", "1")
-    test_conv_split_reduction(gpu_lib, i)
+    test_conv_split_reduction(gpu_lib, "large", i)  # (the switch means the larger kernels)
 
 
 @pytest.mark.parametrize("stride", [1, 2])
@@ -645,11 +644,11 @@ def test_conv_deep_slices_padding(gpu_lib, stride, monkeypatch):
 def test_conv_split_forced(gpu_lib, i, monkeypatch):
     """the same shapes with every reduction cut in two whatever the launch heuristic would choose"""
     monkeypatch.setenv("HIPQ_SPLIT_K", "2")
-    test_conv_split_reduction(gpu_lib, i)
+    test_conv_split_reduction(gpu_lib, "large", i)  # (the switch means the larger kernels)
 
 
 @pytest.mark.parametrize("i", range(len(SPLIT_CONV_SHAPES)))
-def test_conv_split_reduction(gpu_lib, i):
+def test_conv_split_reduction(gpu_lib, family, i):
     """few tiles with long reductions: the pipelined kernel cuts each reduction over several
     workgroups, which meet through partial sums and a counter that the last one resets; called
     several times in a row (the counters must be back at zero), both policies, zero points, residual"""
@@ -664,7 +663,7 @@ def test_conv_split_reduction(gpu_lib, i):
         s = (0.02, 0.005, 0.9)
         exp = O.quantized_convolution(dn, data, filt, s[0], z[0], s[1], z[1], s[2], z[2])
         got = H.quantized_convolution(d, cases.to_nxc(data), filt, s[0], z[0], s[1], z[1], s[2], z[2])
-        assert H.last_kernel().startswith("conv_mfma"), H.last_kernel()
+        cases.ran(family, "conv_mfma")
         assert np.array_equal(cases.to_ncx(got), exp), z
     for rep, (relu, has_sum) in enumerate(((True, True), (False, False), (True, True))):
         out_t = "u8" if relu else "i8"
@@ -678,7 +677,7 @@ def test_conv_split_reduction(gpu_lib, i):
         f = H.make_fused_desc(has_bias=True, has_sum=has_sum, sum_t="u8", with_relu=relu, scale_count=K)
         exp = O.quantized_convolution_fused(dn, f, data, filt, bias, summ, scales, 0.37 if has_sum else None)
         got = H.quantized_convolution_fused(d, f, cases.to_nxc(data), filt, bias, cases.to_nxc(summ) if has_sum else None, scales, 0.37 if has_sum else None)
-        assert H.last_kernel().startswith("conv_mfma"), H.last_kernel()
+        cases.ran(family, "conv_mfma")
         assert np.array_equal(cases.to_ncx(got), exp), (relu, has_sum)
     O.port().orc_set_threads(1)
 
@@ -686,7 +685,7 @@ def test_conv_split_reduction(gpu_lib, i):
 @pytest.mark.parametrize("image,pads", [((30, 26), ((3, 3), (3, 3))), ((30, 28), ((3, 3), (3, 3))), ((19, 32), ((2, 5), (4, 0)))], ids=["rows26", "rows28", "rows32_uneven_pads"])
 @pytest.mark.parametrize("K", [24, 32])
 @pytest.mark.parametrize("Cc", [1, 3, 4, 15])
-def test_conv_few_input_channels(gpu_lib, Cc, K, image, pads):
+def test_conv_few_input_channels(gpu_lib, family, Cc, K, image, pads):
     """a network's first layer (3 input channels, 7x7 stride 2): the data is padded to 16 channels on
     the way into the MFMA kernel, or -- at most four channels, channels-last 8-bit output in whole
     16-byte pixels (K = 32 here) -- staged with its padding so that a filter row is one 32-byte run;
@@ -704,7 +703,7 @@ def test_conv_few_input_channels(gpu_lib, Cc, K, image, pads):
             filt = synth.uniform_int(800 + Cc, dn.filter_shape(), -128, 127, np.int8)
             exp = O.quantized_convolution(dn, data, filt, 0.02, z[0], 0.01, z[1], 0.8, z[2])
             got = H.quantized_convolution(d, cases.to_nxc(data) if dl == H.NXC else data, filt, 0.02, z[0], 0.01, z[1], 0.8, z[2])
-            assert H.last_kernel().startswith("conv_mfma"), H.last_kernel()
+            cases.ran(family, "conv_mfma")
             assert np.array_equal(cases.to_ncx(got) if ol == H.NXC else got, exp), (dl, ol, out_t, z)
         d = H.make_conv_desc(2, Cc, K, image, (7, 7), out_t="u8", data_layout=dl, out_layout=ol, **kw)
         dn = H.make_conv_desc(2, Cc, K, image, (7, 7), out_t="u8", **kw)
@@ -715,7 +714,7 @@ def test_conv_few_input_channels(gpu_lib, Cc, K, image, pads):
         f = H.make_fused_desc(has_bias=True, with_relu=True, scale_count=K)
         exp = O.quantized_convolution_fused(dn, f, data, filt, bias, None, scales, None)
         got = H.quantized_convolution_fused(d, f, cases.to_nxc(data) if dl == H.NXC else data, filt, bias, None, scales, None)
-        assert H.last_kernel().startswith("conv_mfma"), H.last_kernel()
+        cases.ran(family, "conv_mfma")
         assert np.array_equal(cases.to_ncx(got) if ol == H.NXC else got, exp), (dl, ol, "fused")
     O.port().orc_set_threads(1)
 
@@ -774,7 +773,7 @@ def test_dot_kats(gpu_lib, kats):
         assert got.reshape(-1).tolist() == k["expected"], k["name"]
 
 
-def test_dot_reference_vectors(gpu_lib, ref_vectors):
+def test_dot_reference_vectors(gpu_lib, family, ref_vectors):
     manifest, arrays = ref_vectors
     used = set()
     for m in manifest:
@@ -790,7 +789,7 @@ def test_dot_reference_vectors(gpu_lib, ref_vectors):
 
 
 @pytest.mark.parametrize("M", [1, 32, 256, 130])
-def test_dot_mfma_vs_oracle(gpu_lib, M):
+def test_dot_mfma_vs_oracle(gpu_lib, family, M):
     say("dot mfma M", M)
     K, N = 512, 384
     a = synth.uniform_int(81, (M, K), 0, 255, np.uint8)
@@ -800,7 +799,7 @@ def test_dot_mfma_vs_oracle(gpu_lib, M):
         d = H.make_dot_desc(M, K, N, out_t=out_t)
         exp = O.quantized_dot(d, a, b, s[0], z[0], s[1], z[1], s[2], z[2])
         got = H.quantized_dot(d, a, b, s[0], z[0], s[1], z[1], s[2], z[2])
-        assert H.last_kernel().startswith(("dot_mfma", "dot_skinny", "dot_rows64")), H.last_kernel()
+        cases.ran(family, "dot_mfma", "dot_skinny", "dot_rows64")
         assert np.array_equal(got, exp), (out_t, z)
     O.port().orc_set_threads(1)
 
@@ -823,7 +822,7 @@ def test_dot_bias_kat(gpu_lib, kats):
 
 
 @pytest.mark.parametrize("M", [1, 32, 256])
-def test_dot_bias_config2_shape(gpu_lib, M):
+def test_dot_bias_config2_shape(gpu_lib, family, M):
     """BASELINE config 2 at K = N = 1024 (the oracle needs minutes at 4096): per-output-channel
     scales, int32 bias, requantize to i8; and the f32 / relu variants"""
     say("config2 M", M)
@@ -838,15 +837,15 @@ def test_dot_bias_config2_shape(gpu_lib, M):
         f = H.make_fused_desc(has_bias=True, with_relu=relu, scale_count=N)
         exp = O.quantized_dot_bias(d, f, a, w, bias, scales)
         got = H.quantized_dot_bias(d, f, a, w, bias, scales)
-        assert H.last_kernel().startswith(("dot_mfma", "dot_skinny", "dot_rows64")), H.last_kernel()
+        cases.ran(family, "dot_mfma", "dot_skinny", "dot_rows64")
         assert np.array_equal(got, exp), (out_t, relu)
         assert len(np.unique(exp)) > 20  # the case is not degenerate (all saturated)
     O.port().orc_set_threads(1)
 
 
 @pytest.mark.parametrize("shape", [(200, 192, 144), (130, 4096, 64), (333, 768, 272), (4096, 64, 128)])
-def test_dot_bias_f32_tiles(gpu_lib, shape, monkeypatch):
-    """float outputs of QuantizedDotBias through the tile kernels: ragged row and column tiles, a
+def test_dot_bias_f32_tiles(gpu_lib, family, shape, monkeypatch):
+    """float outputs of QuantizedDotBias (the tile kernels, where the kernels for small products are off): ragged row and column tiles, a
     long reduction that is split over workgroups, a single-slice reduction; small biases (added to
     the accumulators as integers) and one beyond 2^24 (kept as a float add); with and without relu"""
     M, K, N = shape
@@ -867,19 +866,19 @@ def test_dot_bias_f32_tiles(gpu_lib, shape, monkeypatch):
                 got = H.quantized_dot_bias(d, f, a, w, bias, scales)
                 # (up to 256 rows with a long reduction and few tiles: one workgroup per 64 x 64 tile, whole reduction)
                 rows64 = 64 < M <= 256 and K >= 1024
-                assert H.last_kernel().startswith("dot_rows64" if rows64 else "dot_mfma"), H.last_kernel()
+                cases.ran(family, "dot_rows64" if rows64 else "dot_mfma")
                 assert np.array_equal(got.view(np.uint32), exp.view(np.uint32)), (a_t, big_bias, relu)
                 if rows64:
                     monkeypatch.setenv("HIPQ_NO_ROWS64", "1")
                     got = H.quantized_dot_bias(d, f, a, w, bias, scales)
                     monkeypatch.delenv("HIPQ_NO_ROWS64")
-                    assert H.last_kernel().startswith("dot_mfma"), H.last_kernel()
+                    cases.ran(family, "dot_mfma")
                     assert np.array_equal(got.view(np.uint32), exp.view(np.uint32)), (a_t, big_bias, relu, "tiles")
     O.port().orc_set_threads(1)
 
 
 @pytest.mark.parametrize("shape", [(512, 256, 384), (1024, 128, 640), (12288, 64, 1024), (16384, 64, 1152), (5000, 192, 400), (2048, 512, 1152)])
-def test_dot_tile_order(gpu_lib, shape):
+def test_dot_tile_order(gpu_lib, family, shape):
     """the persistent tile kernels number their tiles in groups of column blocks (squares per
     compute die): full groups of 2, 4 and 8, a narrower last group, more tiles than resident
     workgroups, ragged edges -- every output element must still be written exactly once"""
@@ -895,14 +894,14 @@ def test_dot_tile_order(gpu_lib, shape):
         f = H.make_fused_desc(has_bias=True, with_relu=relu, scale_count=N)
         exp = O.quantized_dot_bias(d, f, a, w, bias, scales)
         got = H.quantized_dot_bias(d, f, a, w, bias, scales)
-        assert H.last_kernel().startswith("dot_mfma"), H.last_kernel()
+        cases.ran(family, "dot_mfma")
         assert np.array_equal(got.view(np.uint8), exp.view(np.uint8)), (out_t, relu)
         assert len(np.unique(exp)) > 20
     O.port().orc_set_threads(1)
 
 
 @pytest.mark.parametrize("shape", [(1000, 768, 400), (2000, 512, 1104), (4096, 768, 768)])
-def test_dot_half_height_tiles(gpu_lib, shape, monkeypatch):
+def test_dot_half_height_tiles(gpu_lib, family, shape, monkeypatch):
     """row matrices whose 128 x 128 tiles would leave compute units idle run on 64 x 128 tiles with
     whole reductions: ragged last tiles in both directions, 8-bit and float outputs, against the
     oracle and against the 128 x 128 tiles (reductions split over workgroups) behind the switch"""
@@ -918,7 +917,7 @@ def test_dot_half_height_tiles(gpu_lib, shape, monkeypatch):
         f = H.make_fused_desc(has_bias=True, with_relu=relu, scale_count=N)
         exp = O.quantized_dot_bias(d, f, a, w, bias, scales)
         got = H.quantized_dot_bias(d, f, a, w, bias, scales)
-        assert H.last_kernel().startswith("dot_mfma"), H.last_kernel()
+        cases.ran(family, "dot_mfma")
         monkeypatch.setenv("HIPQ_NO_HALF_TILES", "1")
         full = H.quantized_dot_bias(d, f, a, w, bias, scales)
         monkeypatch.delenv("HIPQ_NO_HALF_TILES")
@@ -944,7 +943,7 @@ def _sweep_shapes():
 
 
 @pytest.mark.parametrize("shape", _sweep_shapes())
-def test_dot_dispatch_sweep(gpu_lib, shape):
+def test_dot_dispatch_sweep(gpu_lib, family, shape):
     """QuantizedDotBias over shapes drawn around the dispatch edges, 8-bit and float outputs, against the oracle"""
     M, K, N = shape
     say("dot dispatch sweep", shape)
@@ -1038,7 +1037,7 @@ def test_dot_bias_config2_benchmarked_form(gpu_lib, M):
 
 
 @pytest.mark.parametrize("M", [1, 7, 16, 17, 33, 64, 100, 129, 256])
-def test_dot_skinny(gpu_lib, M):
+def test_dot_skinny(gpu_lib, family, M):
     """the weight-streaming kernel for a handful of rows: ragged row and column tiles, a reduction
     that does not split evenly over the four wavefronts, signed and unsigned data, zero points,
     both requantization policies, f32 output, and the exact path for a non-zero weight zero point"""
@@ -1074,7 +1073,7 @@ def test_dot_skinny(gpu_lib, M):
                     got = H.quantized_dot(d, a, w, s[0], z[0], s[1], z[1], s[2], z[2], prepare=prepacked)
                     # (more than 64 rows with an 8-bit output in whole 16-byte rows go to the tile kernels)
                     want = kernel_of(M > 64 and out_t != "i32" and N % 16 == 0, K, prepacked)
-                    assert H.last_kernel().startswith(want), (H.last_kernel(), want)
+                    cases.ran(family, want)
                     assert np.array_equal(got, exp), (K, N, a_t, out_t, z, prepacked)
                 bias = synth.uniform_int(803, (N,), -(2**15), 2**15, np.int32)
                 scales = synth.uniform_f32(804, (N,), 0.001, 0.01) * np.float32(0.05)
@@ -1084,7 +1083,7 @@ def test_dot_skinny(gpu_lib, M):
                     exp = O.quantized_dot_bias(d, f, a, w, bias, scales)
                     got = H.quantized_dot_bias(d, f, a, w, bias, scales, prepare=prepacked)
                     want = kernel_of(M > 64 and N % 16 == 0, K, prepacked)
-                    assert H.last_kernel().startswith(want), (H.last_kernel(), want)
+                    cases.ran(family, want)
                     assert np.array_equal(got, exp), (K, N, a_t, out_t, relu, prepacked)
     O.port().orc_set_threads(1)
 
@@ -1108,7 +1107,7 @@ def test_transposes(gpu_lib, eb):
         assert np.array_equal(back.to_numpy(dt, (N, Cc, X)), a)
 
 
-def test_mfma_requant_ties(gpu_lib):
+def test_mfma_requant_ties(gpu_lib, family):
     """exact .5 ties of both signs and both parities on the MFMA path: half away from zero for the
     INTERPRETER policy, half to even for the fused policy"""
     say("requant ties")
@@ -1120,7 +1119,7 @@ def test_mfma_requant_ties(gpu_lib):
     exp_acc = np.tile(w[:, 0].astype(np.int32), (M, 1))
     d = H.make_dot_desc(M, K, N, out_t="i8", b_layout=H.B_NK)
     got = H.quantized_dot(d, a, w, 0.5, 0, 1.0, 0, 1.0, 0)
-    assert H.last_kernel().startswith(("dot_mfma", "dot_skinny")), H.last_kernel()
+    cases.ran(family, "dot_mfma", "dot_skinny")
     half_away = np.sign(exp_acc) * np.floor(np.abs(exp_acc) / 2 + 0.5)
     assert np.array_equal(got.astype(np.int64), half_away.astype(np.int64))
     assert np.array_equal(got, O.quantized_dot(d, a, w, 0.5, 0, 1.0, 0, 1.0, 0))
@@ -1136,7 +1135,7 @@ def test_mfma_requant_ties(gpu_lib):
 
 
 @pytest.mark.parametrize("shape", [(65, 1088, 64), (200, 1152, 130), (256, 2048, 48), (129, 1024, 1000), (192, 3008, 200), (72, 4096, 40), (130, 4160, 72)])
-def test_dot_rows64(gpu_lib, shape):
+def test_dot_rows64(gpu_lib, family, shape):
     """the whole-reduction kernels for 65-256 rows (prepacked weights: the one that reads their
     fragment-ordered copy; weights packed on the fly: the one that reads the row-major matrix): ragged row and column tiles, reductions that end in
     half a 128-byte piece (K % 128 == 64) or leave wavefronts without a piece, signed and unsigned
@@ -1153,7 +1152,7 @@ def test_dot_rows64(gpu_lib, shape):
             exp = O.quantized_dot(d, a, w, s[0], z[0], s[1], z[1], s[2], z[2])
             for prepacked, name in ((True, "dot_rows64w_" if K <= 4096 else "dot_rows64_"), (False, "dot_rows64_")):  # (the fragment-ordered kernel holds a reduction of 4096 bytes in registers)
                 got = H.quantized_dot(d, a, w, s[0], z[0], s[1], z[1], s[2], z[2], prepare=prepacked)
-                assert H.last_kernel().startswith(name), H.last_kernel()
+                cases.ran(family, name)
                 assert np.array_equal(got, exp), (a_t, out_t, z, prepacked)
         bias = synth.uniform_int(1503, (N,), -(2**15), 2**15, np.int32)
         scales = synth.uniform_f32(1504, (N,), 0.001, 0.01) * np.float32(0.05)
@@ -1163,7 +1162,7 @@ def test_dot_rows64(gpu_lib, shape):
             exp = O.quantized_dot_bias(d, f, a, w, bias, scales)
             for prepacked, name in ((True, "dot_rows64w_" if K <= 4096 else "dot_rows64_"), (False, "dot_rows64_")):  # (the fragment-ordered kernel holds a reduction of 4096 bytes in registers)
                 got = H.quantized_dot_bias(d, f, a, w, bias, scales, prepare=prepacked)
-                assert H.last_kernel().startswith(name), H.last_kernel()
+                cases.ran(family, name)
                 assert np.array_equal(got.view(np.uint8), exp.view(np.uint8)), (a_t, out_t, relu, prepacked)
     O.port().orc_set_threads(1)
 
@@ -1197,7 +1196,7 @@ def _random_conv_case(rng):
 
 
 @pytest.mark.parametrize("block", range(6))
-def test_conv_random_geometries(gpu_lib, block):
+def test_conv_random_geometries(gpu_lib, family, block):
     """seeded sweep: every case against the oracle, bit for bit, in the reference's layouts and (2-D and
     below) channels-last; INTERPRETER arithmetic with zero points on all three tensors"""
     rng = np.random.default_rng(9000 + block)
@@ -1229,7 +1228,7 @@ def test_conv_random_geometries(gpu_lib, block):
 
 
 @pytest.mark.parametrize("block", range(3))
-def test_dot_random_shapes(gpu_lib, block):
+def test_dot_random_shapes(gpu_lib, family, block):
     """seeded sweep of QuantizedDot (INTERPRETER arithmetic, [K, N] weights, zero points) and
     QuantizedDotBias (fused arithmetic, [N, K] weights, per-channel scales) against the oracle"""
     rng = np.random.default_rng(9100 + block)

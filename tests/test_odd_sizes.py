@@ -29,7 +29,7 @@ CONVS = [
 
 
 @pytest.mark.parametrize("case", CONVS)
-def test_conv_odd_channels(gpu_lib, case):
+def test_conv_odd_channels(gpu_lib, family, case):
     N, Cc, K, sp, f, stride, dil = case
     pad = (f - 1) * dil // 2
     kw = dict(stride=(stride,) * 2, dilation=(dil,) * 2, pad_below=(pad, pad), pad_above=(pad, pad))
@@ -61,7 +61,7 @@ def test_conv_odd_channels(gpu_lib, case):
 
 
 @pytest.mark.parametrize("shape", [(1, 65, 64), (77, 1000, 1003), (16, 71, 100), (33, 257, 65), (300, 333, 97), (130, 1090, 128), (1, 4001, 130)])
-def test_dot_odd_reductions(gpu_lib, shape):
+def test_dot_odd_reductions(gpu_lib, family, shape):
     M, K, N = shape
     say("odd dot", shape)
     O.port().orc_set_threads(8)
