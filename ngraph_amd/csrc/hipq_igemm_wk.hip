@@ -441,35 +441,37 @@ namespace hipq
         return check_launch(name);
     }
 
+    // as many steps in flight as a wavefront has, up to what its registers hold (the last of UPS): a load that
+    // has no step would still take its turn in the texture path, which is what bounds these kernels
+    template <class XL, bool X_ON_A, int MT, int NT, int KW, int TW, int U, int... UPS>
+    static int launch_wk_steps(const XL& xl, const WkParams& p, const ZeroPoints& zp, const Epilogue& epi, const OutMap& om, void* out, hipStream_t s, const char* name)
+    {
+        if constexpr (sizeof...(UPS) > 0)
+            if (((p.Kred + 63) / 64 + KW - 1) / KW > U)
+                return launch_wk_steps<XL, X_ON_A, MT, NT, KW, TW, UPS...>(xl, p, zp, epi, om, out, s, name);
+        return launch_wk_tile<XL, MT, NT, KW, TW, U, X_ON_A>(xl, p, zp, epi, om, out, s, name);
+    }
+
     template <class XL, bool X_ON_A>
     static int launch_wk(const XL& xl, const WkParams& p, const ZeroPoints& zp, const Epilogue& epi, const OutMap& om, void* out, hipStream_t s, const char* name)
     {
         const bool q8 = epi.out_t == HIPQ_U8 || epi.out_t == HIPQ_I8;
         if (epi.mode == EPI_FUSED && !q8 && (X_ON_A || XL::kPadded || epi.out_t != HIPQ_F32))
             return HIPQ_ERR_UNSUPPORTED;
-        const int steps = (p.Kred + 63) / 64;
-        // as many steps in flight as a wavefront has, up to what its registers hold: a load that has no step
-        // would still take its turn in the texture path, which is what bounds these kernels
-#define WK(MT, NT, KW, TW, BIG)                                                                           \
-    case WkShape::kTile##MT##NT##KW##TW:                                                              \
-        switch ((steps + KW - 1) / KW)                                                                     \
-        {                                                                                                  \
-        case 1: return launch_wk_tile<XL, MT, NT, KW, TW, 1, X_ON_A>(xl, p, zp, epi, om, out, s, name);     \
-        case 2: return launch_wk_tile<XL, MT, NT, KW, TW, 2, X_ON_A>(xl, p, zp, epi, om, out, s, name);     \
-        case 3: return launch_wk_tile<XL, MT, NT, KW, TW, 3, X_ON_A>(xl, p, zp, epi, om, out, s, name);     \
-        case 4: return launch_wk_tile<XL, MT, NT, KW, TW, 4, X_ON_A>(xl, p, zp, epi, om, out, s, name);     \
-        default: return launch_wk_tile<XL, MT, NT, KW, TW, BIG, X_ON_A>(xl, p, zp, epi, om, out, s, name);  \
-        }
+        // (of each shape the step counts that wk_shape gives it)
         switch (wk_shape(p.M, om.N, p.Kred))
         {
-            WK(1, 1, 8, 1, 6);
-            WK(1, 1, 16, 1, 6);
-            WK(1, 2, 4, 1, 6);
-            WK(2, 2, 1, 4, 5);
-            WK(2, 2, 2, 2, 5);
-            WK(2, 2, 4, 1, 5);
+        case WkShape::kTile1181: return launch_wk_steps<XL, X_ON_A, 1, 1, 8, 1, 1, 2, 3, 4, 6>(xl, p, zp, epi, om, out, s, name);
+        case WkShape::kTile11161: return launch_wk_steps<XL, X_ON_A, 1, 1, 16, 1, 4>(xl, p, zp, epi, om, out, s, name);
+        case WkShape::kTile1241: return launch_wk_steps<XL, X_ON_A, 1, 2, 4, 1, 1, 2, 3, 4, 6>(xl, p, zp, epi, om, out, s, name);
+        case WkShape::kTile2214:
+            if constexpr (std::is_same<XL, GemmRaggedX>::value) // (65 bytes and more, padded to whole steps)
+                return launch_wk_steps<XL, X_ON_A, 2, 2, 1, 4, 2>(xl, p, zp, epi, om, out, s, name);
+            else
+                return launch_wk_steps<XL, X_ON_A, 2, 2, 1, 4, 1, 2>(xl, p, zp, epi, om, out, s, name);
+        case WkShape::kTile2222: return launch_wk_steps<XL, X_ON_A, 2, 2, 2, 2, 2, 3>(xl, p, zp, epi, om, out, s, name);
+        case WkShape::kTile2241: return launch_wk_steps<XL, X_ON_A, 2, 2, 4, 1, 1, 2, 3, 4, 5>(xl, p, zp, epi, om, out, s, name);
         }
-#undef WK
         return HIPQ_ERR_UNSUPPORTED; // (not reached)
     }
 

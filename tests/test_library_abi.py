@@ -119,3 +119,26 @@ def test_fastdiv_exact():
         for n in ns:
             if 0 <= n < 2**31:
                 assert lib.hipq_debug_fastdiv(n, d) == n // d, (n, d)
+
+
+def test_kernels_for_small_products_are_those_the_rule_reaches():
+    """the instances of igemm_wk_kernel: of each tile shape the step counts a wavefront can get, and no other"""
+    import subprocess
+
+    reached = set()
+    for steps in range(1, 400):
+        # (the tile shapes that some number of rows and columns gives this reduction: MT, NT, KW, TW)
+        shapes = [(2, 2, 4, 1), (2, 2, 2, 2) if 2 < steps <= 6 else (2, 2, 1, 4) if steps <= 2 else (2, 2, 4, 1), (1, 2, 4, 1)]
+        if steps >= 8:
+            shapes.append((1, 1, 16, 1) if 48 < steps <= 64 else (1, 1, 8, 1))
+        for s in shapes:
+            per = -(-steps // s[2])
+            reached.add(s + (per if per <= 4 else 6 if s[0] == 1 else 5,))
+    out = subprocess.run(["nm", "-C", H.LIB_PATH], capture_output=True, text=True, check=True).stdout
+    built = {}
+    for loader, numbers, order in re.findall(r"__device_stub__igemm_wk_kernel<hipq::(\w+), ([\d, ]+), (true|false)>", out):
+        built.setdefault((loader, order), set()).add(tuple(int(n) for n in numbers.split(",")))
+    assert sorted(built) == [("ConvRaggedX", "false"), ("ConvRaggedX", "true"), ("ConvX", "false"), ("ConvX", "true"), ("GemmRaggedX", "false"), ("GemmX", "false")]
+    for which, tiles in built.items():
+        want = reached - {(2, 2, 1, 4, 1)} if which[0] == "GemmRaggedX" else reached  # (such rows have two steps at least)
+        assert tiles == want, (which, tiles ^ want)
