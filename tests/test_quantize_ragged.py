@@ -23,3 +23,20 @@ def test_quantize_rows_of_any_length(gpu_lib, shape):
         dq = H.dequantize(got, scale, zp, "f32", (1,))
         assert H.last_kernel() == "dequantize_ragged"
         assert np.array_equal(dq, O.dequantize(exp, scale, zp, "f32", (1,)))
+
+
+# (more than eight steps a compute unit, where a lane takes several groups: rows of whole steps, of whole groups, of
+# one step and more, of some groups, of less than one; the last step and the last group partly filled)
+@pytest.mark.parametrize("shape,kernel", [((2, 261, 4096), "vec4"), ((3, 85, 8228), "vec4"), ((2, 1043, 1027), "ragged"), ((200, 1543, 7), "ragged"), ((401, 1807, 3), "ragged")])
+def test_quantize_large(gpu_lib, shape, kernel):
+    print("quantize large", shape, flush=True)
+    x = synth.normal_f32(74, shape) * np.float32(20)
+    scale = synth.uniform_f32(75, (shape[1],), 0.05, 1.5)
+    for qt, mode in (("i8", H.RNE), ("u8", H.RNE), ("i8", 0), ("u8", 0)):
+        zp = synth.uniform_int(76, (shape[1],), 0, 40, H.NP_OF[H.dtype_code(qt)])
+        got, exp = H.quantize(x, scale, zp, qt, (1,), mode), O.quantize(x, scale, zp, qt, (1,), mode)
+        assert H.last_kernel() == "quantize_" + kernel
+        assert np.array_equal(got, exp)
+        dq = H.dequantize(got, scale, zp, "f32", (1,))
+        assert H.last_kernel() == "dequantize_" + kernel
+        assert np.array_equal(dq, O.dequantize(exp, scale, zp, "f32", (1,)))

@@ -2,6 +2,7 @@
 import numpy as np
 import pytest
 
+from cases import dot_bias_closed_form, to_nxc
 from ngraph_amd import hipq as H
 from ngraph_amd import synth
 
@@ -37,3 +38,40 @@ def test_conv_and_gelu_report_the_kernel_that_ran(gpu_lib, monkeypatch):
         assert H.last_kernel() == gelu
         monkeypatch.setenv("HIPQ_NO_WK", "1")
     assert np.array_equal(got[0], got[2]) and np.array_equal(got[1], got[3])
+
+
+# pictures, outputs, 64-byte steps of the reduction: every tile shape, and of each the steps its wavefronts have
+# in flight (the last of a line: more than that).  On 256 compute units.
+SHAPES = (
+    [((2, 4, 5), 200, s) for s in (8, 9, 24, 32, 48, 70, 49, 64)]  # 16 x 16, eight wavefronts (the last two: sixteen)
+    + [((2, 10, 10), 700, s) for s in (3, 7, 12, 16, 23, 40)]      # 16 x 32, four
+    + [((10, 8, 8), 640, s) for s in (4, 8, 11, 16, 20, 27)]       # 32 x 32, four
+    + [((4, 15, 15), 900, s) for s in (1, 2, 3, 6)]                # 32 x 32, one (1 and 2 steps) and two
+)
+
+
+@pytest.mark.parametrize("pictures,N,steps", SHAPES)
+@pytest.mark.parametrize("ragged", [False, True])
+def test_every_tile_shape(gpu_lib, pictures, N, steps, ragged):
+    """products and 1 x 1 convolutions of these sizes, rows in whole steps and rows that are not, against the closed form"""
+    K, M = 64 * steps - (4 if ragged else 0), int(np.prod(pictures))
+    print("small product", M, K, N, flush=True)
+    a = synth.uniform_int(71, (M, K), 0, 255, np.uint8)
+    w = synth.uniform_int(72, (N, K), -128, 127, np.int8)
+    bias = synth.uniform_int(73, (N,), -(2**15), 2**15, np.int32)
+    scale = synth.uniform_f32(74, (N,), 0.5, 1.5) * np.float32(0.003 / np.sqrt(K))
+    f = H.make_fused_desc(has_bias=True, with_relu=False, scale_count=N)
+    exp = dot_bias_closed_form(a, w, bias, scale, "i8", False)
+    assert len(np.unique(exp)) > 100
+    if K >= 64:
+        for out_t, want in (("i8", exp), ("f32", dot_bias_closed_form(a, w, bias, scale, "f32", False))):
+            d = H.make_dot_desc(M, K, N, out_t=out_t, b_layout=H.B_NK)
+            got = H.quantized_dot_bias(d, f, a, w, bias, scale)
+            assert H.last_kernel() == ("dot_mfma_wk_ragged_i8_16x16x64" if ragged else "dot_mfma_wk_i8_16x16x64")
+            assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), out_t
+    x = a.reshape(pictures + (K,))
+    for ol in (H.NXC, H.NCX):
+        d = H.make_conv_desc(pictures[0], K, N, pictures[1:], (1, 1), out_t="i8", data_layout=H.NXC, out_layout=ol)
+        got = H.quantized_convolution_fused(d, f, x, w.reshape(N, K, 1, 1), bias, None, scale, None)
+        assert H.last_kernel() == ("conv_mfma_wk_ragged_i8_16x16x64" if ragged else "conv_mfma_wk_i8_16x16x64")
+        assert np.array_equal(got if ol == H.NXC else to_nxc(got), exp.reshape(pictures + (N,))), ol
