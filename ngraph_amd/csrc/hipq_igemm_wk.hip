@@ -21,6 +21,9 @@
 // Rows and pixels that are no multiple of 16 bytes are read where they lie (ragged_preferred): u8
 // [8,90,35,29] x i8 [150,90,3,3] 14.4 -> 13.1 us, 77 x 1000 x 1003 8.2 -> 4.1 with the copy's launch gone.
 #include <cstdlib>
+#include <cstring>
+
+#include <unistd.h>
 
 #include "hipq_igemm.h"
 
@@ -394,17 +397,25 @@ namespace hipq
     // 6.7).  Against the register-staged ones up to sixteen.
     static bool wk_enabled()
     {
+        // one walk over the environment where nothing of the library's is set, as in any program that runs in
+        // earnest: a look-up by name costs as much, and there are seven
+        bool any = false;
+        for (char** e = environ; e && *e && !any; ++e)
+            any = strncmp(*e, "HIPQ_", 5) == 0;
+        if (!any)
+            return true;
         // (the switches that name a kernel of the other family mean that family)
         for (const char* name : {"HIPQ_NO_WK", "HIPQ_SPLIT_K", "HIPQ_NO_DMA", "HIPQ_NO_PIPE", "HIPQ_NO_CONV_DMA", "HIPQ_NO_HALF_TILES", "HIPQ_NO_REGW"})
             if (getenv(name) != nullptr)
                 return false;
         return true;
     }
-    bool wk_preferred(int64_t M, int64_t N, int64_t steps, bool dma)
+    static bool wk_fits(int64_t M, int64_t N, int64_t steps, bool dma)
     {
         const int64_t limit = !dma ? 16 : N <= 64 || steps > 4 ? 3 : steps > 1 ? 4 : 7;
-        return wk_enabled() && wk_tiles(M, N, 32, 32) <= static_cast<int64_t>(device_compute_units()) * limit;
+        return wk_tiles(M, N, 32, 32) <= static_cast<int64_t>(device_compute_units()) * limit;
     }
+    bool wk_preferred(int64_t M, int64_t N, int64_t steps, bool dma) { return wk_fits(M, N, steps, dma) && wk_enabled(); }
 
     // Whether rows (pixels) of `row_bytes` that are no multiple of 16 are read where they lie, instead of
     // through a copy padded to whole chunks (a launch, 2.5 us and more, and rows a power of two apart).
@@ -418,16 +429,10 @@ namespace hipq
     // the sizes of wk_preferred: 90 -> 150 channels 1 x 1 on 128 x 56 x 56 179 there, 79 in place.
     bool ragged_preferred(int64_t M, int64_t N, int64_t row_bytes, int64_t steps, bool dma, bool pointwise)
     {
-        if (!wk_enabled())
-            return false;
         const int64_t tiles = wk_tiles(M, N, 32, 32), units = device_compute_units();
-        if (!dma && pointwise && (steps <= 3 || (steps <= 6 && tiles <= units * 40)))
-            return true;
-        if (!wk_preferred(M, N, steps, dma))
-            return false;
-        if (row_bytes % 4 == 0)
-            return pointwise || steps <= 40;
-        return steps <= (pointwise ? 32 : 40) && tiles * steps <= (steps <= 6 || !pointwise ? 24576 : 8192);
+        const bool few_steps = !dma && pointwise && (steps <= 3 || (steps <= 6 && tiles <= units * 40));
+        const bool few_bytes = row_bytes % 4 == 0 ? pointwise || steps <= 40 : steps <= (pointwise ? 32 : 40) && tiles * steps <= (steps <= 6 || !pointwise ? 24576 : 8192);
+        return (few_steps || (few_bytes && wk_fits(M, N, steps, dma))) && wk_enabled();
     }
 
     template <class XL, int MT, int NT, int KW, int TW, int U, bool X_ON_A>

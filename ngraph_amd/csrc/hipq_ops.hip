@@ -66,7 +66,6 @@ namespace hipq
         const int64_t in_sp = g.in[1] * g.in[2];
         const bool out_ncx = g.out_layout == HIPQ_LAYOUT_NCX && g.K > 1;
         const bool tr_in = !pad && g.data_layout == HIPQ_LAYOUT_NCX && g.C > 1;
-        const bool small = conv_wk_preferred(g, epi.out_t, out_ncx); // too small to fill the chip
         const size_t tr_bytes = pad || tr_in ? align_up(static_cast<size_t>(g.in_count()), 256) : 0;
         // channels-last pixels of any width, where reading them as they lie costs less than the copy
         if (pad && conv_ragged_preferred(whole, g, epi, out_ncx) && !conv_pw64_eligible(g, epi, zp) && !conv_regw_eligible(g, out_ncx))
@@ -130,7 +129,8 @@ namespace hipq
         // channels at 56 x 56, batch 128: 15.8 us against 23 us)
         const bool row_matrix = !out_ncx && g.taps() == 1 && g.st[1] == 1 && g.st[2] == 1 && g.pb[1] == 0 && g.pb[2] == 0 && g.out[1] == g.in[1] && g.out[2] == g.in[2] &&
                                 (g.out_t == HIPQ_U8 || g.out_t == HIPQ_I8) && g.K % 16 == 0 && getenv("HIPQ_NO_DMA") == nullptr && getenv("HIPQ_NO_PIPE") == nullptr;
-        if (!small && !no_band && !row_matrix && conv_band_eligible(g, out_ncx))
+        // (nor layers too small to fill the chip)
+        if (!no_band && !row_matrix && conv_band_eligible(g, out_ncx) && !conv_wk_preferred(g, epi.out_t, out_ncx))
             return launch_conv_band(g, x, packed, zp, epi, out, out_ncx, s);
         return launch_conv_mfma(g, x, packed, zp, epi, out, out_ncx, s);
     }
@@ -577,8 +577,7 @@ int hipq_quantized_dot_bias_gelu_quantize(const hipq_dot_desc_t* d,
     // in the epilogue of the product, where the kernels that take it apply: the ones for products too
     // small to fill the chip, and from 257 rows on the tile kernels
     const bool q16 = (reinterpret_cast<uintptr_t>(quant->out) & 15) == 0;
-    const bool small = packed_w && dot_gelu_wk_preferred(*d);
-    if (dot_mfma_eligible(*d) && d->K % 16 == 0 && (small || d->M > 256) && (reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && q16)
+    if (dot_mfma_eligible(*d) && d->K % 16 == 0 && (d->M > 256 || (packed_w && dot_gelu_wk_preferred(*d))) && (reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && q16)
     {
         DotOperands o;
         ZeroPoints zp{nullptr, nullptr, d->a_t, d->b_t};

@@ -142,3 +142,54 @@ def test_kernels_for_small_products_are_those_the_rule_reaches():
     for which, tiles in built.items():
         want = reached - {(2, 2, 1, 4, 1)} if which[0] == "GemmRaggedX" else reached  # (such rows have two steps at least)
         assert tiles == want, (which, tiles ^ want)
+
+
+def test_a_call_looks_few_switches_up(tmp_path):
+    """environment look-ups of a one-row product and of a small convolution, counted by a program whose own getenv
+    stands in for the C library's (without a device the calls end where they would launch: the tensors are
+    addresses that nothing reads)"""
+    import subprocess
+
+    src = tmp_path / "count.c"
+    src.write_text(r"""
+#include <dlfcn.h>
+#include <stdio.h>
+#include <string.h>
+#include "hipq.h"
+static int n;
+extern char** environ;
+char* getenv(const char* name)
+{
+    size_t len = strlen(name);
+    n += strncmp(name, "HIPQ_", 5) == 0;
+    for (char** e = environ; *e; ++e)
+        if (strncmp(*e, name, len) == 0 && (*e)[len] == '=')
+            return *e + len + 1;
+    return 0;
+}
+int main(int argc, char** argv)
+{
+    static _Alignas(256) unsigned char at[512];
+    void* lib = dlopen(argv[1], RTLD_NOW);
+    hipq_fused_desc_t f = {.scale_count = 1};
+    hipq_dot_desc_t d = {.a_t = HIPQ_U8, .b_t = HIPQ_I8, .out_t = HIPQ_I8, .b_layout = HIPQ_B_NK, .M = 1, .K = 4096, .N = 4096};
+    hipq_conv_desc_t c = {.n_spatial = 2, .data_t = HIPQ_U8, .filter_t = HIPQ_I8, .out_t = HIPQ_U8, .data_layout = HIPQ_LAYOUT_NXC, .out_layout = HIPQ_LAYOUT_NXC,
+                          .N = 1, .C = 90, .K = 150, .in_sp = {35, 29}, .f_sp = {3, 3}, .out_sp = {35, 29}, .stride = {1, 1}, .dilation = {1, 1}, .data_dilation = {1, 1},
+                          .pad_below = {1, 1}, .pad_above = {1, 1}};
+    __typeof__(&hipq_quantized_dot_bias) dot = dlsym(lib, "hipq_quantized_dot_bias");
+    __typeof__(&hipq_quantized_convolution_fused) conv = dlsym(lib, "hipq_quantized_convolution_fused");
+    n = 0;
+    dot(&d, &f, at, at, at, 0, (float*)at, at + 256, 0);
+    printf("%d\n", n);
+    n = 0;
+    conv(&c, &f, at, at, at, 0, 0, (float*)at, 0, at + 256, 0);
+    printf("%d\n", n);
+    return 0;
+}
+""")
+    exe = tmp_path / "count"
+    subprocess.run(["gcc", "-std=gnu11", "-rdynamic", "-I", os.path.join(ROOT, "include"), str(src), "-o", str(exe), "-ldl"], check=True)
+    env = {k: v for k, v in os.environ.items() if not k.startswith("HIPQ_")}
+    env["HIP_VISIBLE_DEVICES"] = ""  # (no launch, on any machine)
+    dot, conv = (int(x) for x in subprocess.run([str(exe), H.LIB_PATH], env=env, capture_output=True, text=True, check=True).stdout.split())
+    assert dot <= 4 and conv <= 2, (dot, conv)
