@@ -394,7 +394,11 @@ namespace hipq
     // bytes and seven on those of one step, where their larger tiles wait for one slice as long as these do
     // and leave compute units idle (784 x 256 x 1024 6.4, 5.6; 3136 x 64 x 256 6.4, 5.2; 6272 x 64 x 256 6.8, 5.9;
     // but 1568 x 256 x 1024, six tiles a unit: 6.8, 7.9).  Not for at most 64 outputs (12544 x 256 x 64: 6.4,
-    // 6.7).  Against the register-staged ones up to sixteen.
+    // 6.7).  Against the register-staged ones up to sixteen, with more than 64 outputs up to 7 + 80 / steps: those
+    // take about 14 us and 0.64 a step while their 128 x 128 tiles are one round, these 4 us and 0.106 a step and
+    // tile of a unit (28 x 12 x 12 pixels of 512 -> 788 3 x 3, twelve tiles: 61 us there, 108 here; 985 x 5888 x
+    // 2971, eleven: 72, 127; 1824 x 4160 x 1001, seven: 59, 48); at most 64 outputs leave most units idle there
+    // (42 x 32 x 32 of 288 -> 46 3 x 3, ten: 79, 45).
     static bool wk_enabled()
     {
         // one walk over the environment where nothing of the library's is set, as in any program that runs in
@@ -410,12 +414,15 @@ namespace hipq
                 return false;
         return true;
     }
-    static bool wk_fits(int64_t M, int64_t N, int64_t steps, bool dma)
+    // spare: step-tiles a compute unit that these may take longer (80: the start of the register-staged ones)
+    static bool wk_fits(int64_t M, int64_t N, int64_t steps, bool dma, int64_t spare)
     {
-        const int64_t limit = !dma ? 16 : N <= 64 || steps > 4 ? 3 : steps > 1 ? 4 : 7;
-        return wk_tiles(M, N, 32, 32) <= static_cast<int64_t>(device_compute_units()) * limit;
+        const int64_t tiles = wk_tiles(M, N, 32, 32), units = device_compute_units();
+        if (!dma)
+            return tiles <= units * 16 && (N <= 64 || tiles * steps <= units * (7 * steps + spare));
+        return tiles <= units * (N <= 64 || steps > 4 ? 3 : steps > 1 ? 4 : 7);
     }
-    bool wk_preferred(int64_t M, int64_t N, int64_t steps, bool dma) { return wk_fits(M, N, steps, dma) && wk_enabled(); }
+    bool wk_preferred(int64_t M, int64_t N, int64_t steps, bool dma) { return wk_fits(M, N, steps, dma, 80) && wk_enabled(); }
 
     // Whether rows (pixels) of `row_bytes` that are no multiple of 16 are read where they lie, instead of
     // through a copy padded to whole chunks (a launch, 2.5 us and more, and rows a power of two apart).
@@ -432,7 +439,7 @@ namespace hipq
         const int64_t tiles = wk_tiles(M, N, 32, 32), units = device_compute_units();
         const bool few_steps = !dma && pointwise && (steps <= 3 || (steps <= 6 && tiles <= units * 40));
         const bool few_bytes = row_bytes % 4 == 0 ? pointwise || steps <= 40 : steps <= (pointwise ? 32 : 40) && tiles * steps <= (steps <= 6 || !pointwise ? 24576 : 8192);
-        return (few_steps || (few_bytes && wk_fits(M, N, steps, dma))) && wk_enabled();
+        return (few_steps || (few_bytes && wk_fits(M, N, steps, dma, 160))) && wk_enabled(); // (160: the copy is spared as well)
     }
 
     template <class XL, int MT, int NT, int KW, int TW, int U, bool X_ON_A>

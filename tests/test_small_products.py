@@ -75,3 +75,16 @@ def test_every_tile_shape(gpu_lib, pictures, N, steps, ragged):
         got = H.quantized_convolution_fused(d, f, x, w.reshape(N, K, 1, 1), bias, None, scale, None)
         assert H.last_kernel() == ("conv_mfma_wk_ragged_i8_16x16x64" if ragged else "conv_mfma_wk_i8_16x16x64")
         assert np.array_equal(got if ol == H.NXC else to_nxc(got), exp.reshape(pictures + (N,))), ol
+
+
+# (columns that are no multiple of 16; the last number of rows that the rule gives these kernels, and one more)
+@pytest.mark.parametrize("M,K,N,small", [(2976, 1088, 1001, True), (2977, 1088, 1001, False), (2080, 4160, 1001, True), (2081, 4160, 1001, False)])
+def test_long_reductions_over_many_tiles(gpu_lib, M, K, N, small):
+    print("long reduction", M, K, N, flush=True)
+    a = synth.uniform_int(81, (M, K), 0, 255, np.uint8)
+    w = synth.uniform_int(82, (N, K), -128, 127, np.int8)
+    scale = synth.uniform_f32(83, (N,), 0.5, 1.5) * np.float32(0.003 / np.sqrt(K))
+    d = H.make_dot_desc(M, K, N, out_t="i8", b_layout=H.B_NK)
+    got = H.quantized_dot_bias(d, H.make_fused_desc(has_bias=False, scale_count=N), a, w, None, scale)
+    assert H.last_kernel() == ("dot_mfma_wk_i8_16x16x64" if small else "dot_mfma_i8_32x32x32")
+    assert np.array_equal(got, dot_bias_closed_form(a, w, None, scale, "i8", False))
