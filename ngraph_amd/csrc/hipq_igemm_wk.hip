@@ -11,7 +11,8 @@
 // latency instead of one a slice, no LDS and no barrier in front of the MFMAs.  The partial tiles meet
 // in LDS once.  Fragment loads from a row-major matrix take half of every cache line they touch, so
 // a compute unit takes operands in at about half of its best rate: the launcher gives these kernels
-// only what that costs less for than the slices would.
+// only what that costs less for than the slices would (4004 of 5000 sizes of up to 24 tiles of 32 x 32 a
+// compute unit, 2.65 times as fast on average as without them).
 //
 // Measured, one launch of a replayed graph: 256 -> 256 3 x 3 on one 14 x 14 picture 17.4 -> 6.1 us,
 // 512 -> 512 3 x 3 on 7 x 7 (an unrolled copy and a skinny product before) 16.3 -> 8.3, 1024 -> 256
@@ -367,9 +368,9 @@ namespace hipq
     // Which tile: the largest that still gives every compute unit work.  From three 32 x 32 tiles for two
     // compute units on those; their reduction is worth splitting over all four wavefronts unless it is
     // short and there are many of them.  Fewer tiles: 16 x 32, and where even those leave half of the chip
-    // idle on a reduction of eight steps or more, 16 x 16 with eight wavefronts on it.  (The lines are those
-    // that cost least over 200 products and convolutions of 1 to 90 000 rows, 64 to 9 600 bytes of reduction
-    // and 16 to 4 000 outputs, each timed in five shapes: 1.7 % above the best shape of each on average.)
+    // idle on a reduction of eight steps or more, 16 x 16 with eight wavefronts on it.  (2000 products and
+    // convolutions of up to six tiles a unit, each timed in all six shapes: 1.024 times the best shape of each on
+    // average; 16 x 32 with 49 steps and more 1.10 times, 106 x 4128 x 1344 13.6 us, 8.8 with sixteen wavefronts.)
     // Reductions that eight wavefronts cannot ask for at once (more than 48 steps) and sixteen ask for in four
     // loads each take sixteen: 40 x 4096 x 512 5.6 -> 5.3 us, 100 x 4004 x 200 5.6 -> 5.1, 400 -> 400 3 x 3 on 9 x 9
     // 6.8 -> 6.2; from five loads on the larger exchange costs more (512 -> 512 3 x 3 on 7 x 7 8.0 -> 8.2).
@@ -393,7 +394,9 @@ namespace hipq
     // 1536: 8.6 us there, 9.9 us here; 985 x 512 x 512: 7.9, 5.5); up to four on reductions of at most 256
     // bytes and seven on those of one step, where their larger tiles wait for one slice as long as these do
     // and leave compute units idle (784 x 256 x 1024 6.4, 5.6; 3136 x 64 x 256 6.4, 5.2; 6272 x 64 x 256 6.8, 5.9;
-    // but 1568 x 256 x 1024, six tiles a unit: 6.8, 7.9).  Not for at most 64 outputs (12544 x 256 x 64: 6.4,
+    // but 1568 x 256 x 1024, six tiles a unit: 6.8, 7.9; looped on hot inputs 49 sizes of one step and four to
+    // seven tiles take 1.06 times as long here, inside a pass they gain: ResNet-50 of two images 390 us, with a
+    // line at four 395).  Not for at most 64 outputs (12544 x 256 x 64: 6.4,
     // 6.7).  Against the register-staged ones up to sixteen, with more than 64 outputs up to 7 + 80 / steps: those
     // take about 14 us and 0.64 a step while their 128 x 128 tiles are one round, these 4 us and 0.106 a step and
     // tile of a unit (28 x 12 x 12 pixels of 512 -> 788 3 x 3, twelve tiles: 61 us there, 108 here; 985 x 5888 x
@@ -431,7 +434,9 @@ namespace hipq
     // twice its time in the memory path, so only while there are few of them: 32 steps of 64 bytes (40 with a
     // window's taps, which hit the same lines) and 8192 step-tiles (24576 with taps or up to six steps):
     // 77 x 2001 x 1003 7.1 there, 6.2 in place; 600 x 1301 x 1003 12.0, 14.4; 16 x 4001 x 150 6.7, 8.7;
-    // 90 -> 150 channels 3 x 3 on 8 x 35 x 35 pixels 15.4, 14.8, on 64 x 35 x 35 68, 82.
+    // 90 -> 150 channels 3 x 3 on 8 x 35 x 35 pixels 15.4, 14.8, on 64 x 35 x 35 68, 82.  Of 3974 sizes 2792 stay in
+    // place, 1.52 times as fast as with the copy; 17 of them more than 5 % slower, at worst 1.34 times (20 x 10 x 10 of
+    // 261 -> 304 3 x 3: 16.0, 21.4).
     // Where no kernel that loads straight into LDS would take the call, short reductions stay here beyond
     // the sizes of wk_preferred: 90 -> 150 channels 1 x 1 on 128 x 56 x 56 179 there, 79 in place.
     bool ragged_preferred(int64_t M, int64_t N, int64_t row_bytes, int64_t steps, bool dma, bool pointwise)
