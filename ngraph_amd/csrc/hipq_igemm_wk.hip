@@ -401,7 +401,9 @@ namespace hipq
     // take about 14 us and 0.64 a step while their 128 x 128 tiles are one round, these 4 us and 0.106 a step and
     // tile of a unit (28 x 12 x 12 pixels of 512 -> 788 3 x 3, twelve tiles: 61 us there, 108 here; 985 x 5888 x
     // 2971, eleven: 72, 127; 1824 x 4160 x 1001, seven: 59, 48); at most 64 outputs leave most units idle there
-    // (42 x 32 x 32 of 288 -> 46 3 x 3, ten: 79, 45).
+    // (42 x 32 x 32 of 288 -> 46 3 x 3, ten: 79, 45).  Where the others stream the weights past up to 256 rows, or
+    // leave Gelu to a launch of its own (`tiles` unset), sixteen for any reduction (128 x 4096 x 20001, ten: 93 us
+    // there, 55 here; 256 x 1024 x 14001, fourteen: 46, 21; 250 x 9600 x 9001, nine: 224, 100).
     static bool wk_enabled()
     {
         // one walk over the environment where nothing of the library's is set, as in any program that runs in
@@ -418,6 +420,7 @@ namespace hipq
         return true;
     }
     // spare: step-tiles a compute unit that these may take longer (80: the start of the register-staged ones)
+    constexpr int64_t kWkSpare = 80, kWkAnyReduction = 1ll << 40;
     static bool wk_fits(int64_t M, int64_t N, int64_t steps, bool dma, int64_t spare)
     {
         const int64_t tiles = wk_tiles(M, N, 32, 32), units = device_compute_units();
@@ -425,7 +428,7 @@ namespace hipq
             return tiles <= units * 16 && (N <= 64 || tiles * steps <= units * (7 * steps + spare));
         return tiles <= units * (N <= 64 || steps > 4 ? 3 : steps > 1 ? 4 : 7);
     }
-    bool wk_preferred(int64_t M, int64_t N, int64_t steps, bool dma) { return wk_fits(M, N, steps, dma, 80) && wk_enabled(); }
+    bool wk_preferred(int64_t M, int64_t N, int64_t steps, bool dma, bool tiles) { return wk_fits(M, N, steps, dma, tiles ? kWkSpare : kWkAnyReduction) && wk_enabled(); }
 
     // Whether rows (pixels) of `row_bytes` that are no multiple of 16 are read where they lie, instead of
     // through a copy padded to whole chunks (a launch, 2.5 us and more, and rows a power of two apart).
@@ -444,7 +447,8 @@ namespace hipq
         const int64_t tiles = wk_tiles(M, N, 32, 32), units = device_compute_units();
         const bool few_steps = !dma && pointwise && (steps <= 3 || (steps <= 6 && tiles <= units * 40));
         const bool few_bytes = row_bytes % 4 == 0 ? pointwise || steps <= 40 : steps <= (pointwise ? 32 : 40) && tiles * steps <= (steps <= 6 || !pointwise ? 24576 : 8192);
-        return (few_steps || (few_bytes && wk_fits(M, N, steps, dma, 160))) && wk_enabled(); // (160: the copy is spared as well)
+        // (the copy is spared as well; up to 256 rows the other kernels stream the weights)
+        return (few_steps || (few_bytes && wk_fits(M, N, steps, dma, M <= 256 ? kWkAnyReduction : 2 * kWkSpare))) && wk_enabled();
     }
 
     template <class XL, int MT, int NT, int KW, int TW, int U, bool X_ON_A>

@@ -1019,12 +1019,12 @@ namespace hipq
     // Quantize(Gelu(rows x weights -> f32)) with Gelu and Quantize in the epilogue of the kernels that
     // load straight into LDS; HIPQ_ERR_UNSUPPORTED (nothing launched, no error text) when the call is
     // not of their kind.  epi carries the Quantize in its post_* fields; out is the 8-bit tensor.
-    bool dot_gelu_wk_preferred(const hipq_dot_desc_t& d) { return wk_preferred(d.M, d.N, (d.K + 63) / 64, d.N % 16 == 0); }
+    bool dot_gelu_wk_preferred(const hipq_dot_desc_t& d) { return wk_preferred(d.M, d.N, (d.K + 63) / 64, d.N % 16 == 0, false); }
 
     int launch_rows_gelu_q8(const void* a, bool a_unsigned, const int8_t* w_nk, const void* w_frag, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi,
                             void* out, hipStream_t s)
     {
-        if (wk_preferred(M, N, (K + 63) / 64, N % 16 == 0))
+        if (wk_preferred(M, N, (K + 63) / 64, N % 16 == 0, false))
         {
             // (128 x 768 x 3072: product, then Gelu and Quantize from the workspace 14.4 us, in one kernel 5.4)
             const int rc = launch_rows_wk(a, a_unsigned, w_nk, w_frag, wsum, M, N, K, zp, epi, out, s, "dot_gelu_q8_wk_i8_16x16x64");
@@ -1095,7 +1095,7 @@ namespace hipq
             const int64_t steps = (d.K + 63) / 64;
             const bool streamed = skinny && d.M <= 32 && w_frag && steps >= (d.M <= 16 ? 12 : 24);
             const bool rows64 = skinny && d.M > 64 && dot_rows64_eligible(d);
-            const bool wk = !streamed && (!rows64 || ((d.M + 31) / 32) * ((d.N + 31) / 32) * steps <= 8192) && wk_preferred(d.M, d.N, steps, dma);
+            const bool wk = !streamed && (!rows64 || ((d.M + 31) / 32) * ((d.N + 31) / 32) * steps <= 8192) && wk_preferred(d.M, d.N, steps, dma, !skinny);
             if (wk)
             {
                 const int rc = launch_rows_wk(a, d.a_t == HIPQ_U8, static_cast<const int8_t*>(w_nk), w_frag, wsum, d.M, static_cast<int32_t>(d.N), static_cast<int32_t>(d.K), zp, epi, out, s,
