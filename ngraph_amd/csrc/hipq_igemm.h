@@ -2143,9 +2143,9 @@ namespace hipq
     // small products and convolutions: the reduction split over a workgroup's wavefronts, fragments straight
     // from memory (hipq_igemm_wk.hip); HIPQ_ERR_UNSUPPORTED (nothing launched, no error text) when the call
     // is not of their kind
-    // steps: of 64 bytes of the reduction; dma, tiles: what else would take the call (kernels that load straight into
-    // LDS; tile kernels at all)
-    bool wk_preferred(int64_t M, int64_t N, int64_t steps, bool dma, bool tiles = true);
+    // steps: of 64 bytes of the reduction; dma, alone: what else would take the call (kernels that load straight into
+    // LDS; one kernel and nothing behind it)
+    bool wk_preferred(int64_t M, int64_t N, int64_t steps, bool dma, bool alone = true);
     bool ragged_preferred(int64_t M, int64_t N, int64_t row_bytes, int64_t steps, bool dma, bool pointwise);
     int launch_rows_wk(const void* a, bool a_unsigned, const int8_t* w_nk, const void* w_frag, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi,
                        void* out, hipStream_t s, const char* name);

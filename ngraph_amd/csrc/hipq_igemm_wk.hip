@@ -11,7 +11,7 @@
 // latency instead of one a slice, no LDS and no barrier in front of the MFMAs.  The partial tiles meet
 // in LDS once.  Fragment loads from a row-major matrix take half of every cache line they touch, so
 // a compute unit takes operands in at about half of its best rate: the launcher gives these kernels
-// only what that costs less for than the slices would (4004 of 5000 sizes of up to 24 tiles of 32 x 32 a
+// only what that costs less for than the slices would (4012 of 5000 sizes of up to 24 tiles of 32 x 32 a
 // compute unit, 2.65 times as fast on average as without them).
 //
 // Measured, one launch of a replayed graph: 256 -> 256 3 x 3 on one 14 x 14 picture 17.4 -> 6.1 us,
@@ -397,13 +397,14 @@ namespace hipq
     // but 1568 x 256 x 1024, six tiles a unit: 6.8, 7.9; looped on hot inputs 49 sizes of one step and four to
     // seven tiles take 1.06 times as long here, inside a pass they gain: ResNet-50 of two images 390 us, with a
     // line at four 395).  Not for at most 64 outputs (12544 x 256 x 64: 6.4,
-    // 6.7).  Against the register-staged ones up to sixteen, with more than 64 outputs up to 7 + 80 / steps: those
-    // take about 14 us and 0.64 a step while their 128 x 128 tiles are one round, these 4 us and 0.106 a step and
-    // tile of a unit (28 x 12 x 12 pixels of 512 -> 788 3 x 3, twelve tiles: 61 us there, 108 here; 985 x 5888 x
-    // 2971, eleven: 72, 127; 1824 x 4160 x 1001, seven: 59, 48); at most 64 outputs leave most units idle there
-    // (42 x 32 x 32 of 288 -> 46 3 x 3, ten: 79, 45).  Where the others stream the weights past up to 256 rows, or
-    // leave Gelu to a launch of its own (`tiles` unset), sixteen for any reduction (128 x 4096 x 20001, ten: 93 us
-    // there, 55 here; 256 x 1024 x 14001, fourteen: 46, 21; 250 x 9600 x 9001, nine: 224, 100).
+    // 6.7).  Against the register-staged ones up to sixteen; nine on reductions of more than 20 steps, where their
+    // larger tiles read each operand fewer times (of 14 500 sizes 136 lie above that line, 1.27 times as fast there on average:
+    // 28 x 12 x 12 pixels of 512 -> 788 3 x 3, twelve tiles: 61 us there, 108 here; 985 x 5888 x 2971, eleven: 72, 127;
+    // on shorter ones as many would lose: 806 x 960 x 4593, fifteen: 35, 21).  Sixteen all the same for at most 64 outputs,
+    // which leave most units idle there (42 x 32 x 32 of 288 -> 46 3 x 3, ten: 79, 45), for at most 512 rows, which
+    // wait for weights out of HBM there, on the tile kernels and on those that stream them past up to 256 rows
+    // (137 x 2192 x 23255, fourteen: 157, 66; 128 x 4096 x 20001, ten: 93, 55), and where Gelu is a launch of its
+    // own there (`alone` unset).
     static bool wk_enabled()
     {
         // one walk over the environment where nothing of the library's is set, as in any program that runs in
@@ -419,16 +420,13 @@ namespace hipq
                 return false;
         return true;
     }
-    // spare: step-tiles a compute unit that these may take longer (80: the start of the register-staged ones)
-    constexpr int64_t kWkSpare = 80, kWkAnyReduction = 1ll << 40;
-    static bool wk_fits(int64_t M, int64_t N, int64_t steps, bool dma, int64_t spare)
+    // long_limit: tiles a compute unit on long reductions
+    static bool wk_fits(int64_t M, int64_t N, int64_t steps, bool dma, int64_t long_limit)
     {
-        const int64_t tiles = wk_tiles(M, N, 32, 32), units = device_compute_units();
-        if (!dma)
-            return tiles <= units * 16 && (N <= 64 || tiles * steps <= units * (7 * steps + spare));
-        return tiles <= units * (N <= 64 || steps > 4 ? 3 : steps > 1 ? 4 : 7);
+        const int64_t limit = dma ? (N <= 64 || steps > 4 ? 3 : steps > 1 ? 4 : 7) : (N <= 64 || M <= 512 || steps <= 20 ? 16 : long_limit);
+        return wk_tiles(M, N, 32, 32) <= static_cast<int64_t>(device_compute_units()) * limit;
     }
-    bool wk_preferred(int64_t M, int64_t N, int64_t steps, bool dma, bool tiles) { return wk_fits(M, N, steps, dma, tiles ? kWkSpare : kWkAnyReduction) && wk_enabled(); }
+    bool wk_preferred(int64_t M, int64_t N, int64_t steps, bool dma, bool alone) { return wk_fits(M, N, steps, dma, alone ? 9 : 16) && wk_enabled(); }
 
     // Whether rows (pixels) of `row_bytes` that are no multiple of 16 are read where they lie, instead of
     // through a copy padded to whole chunks (a launch, 2.5 us and more, and rows a power of two apart).
@@ -447,8 +445,7 @@ namespace hipq
         const int64_t tiles = wk_tiles(M, N, 32, 32), units = device_compute_units();
         const bool few_steps = !dma && pointwise && (steps <= 3 || (steps <= 6 && tiles <= units * 40));
         const bool few_bytes = row_bytes % 4 == 0 ? pointwise || steps <= 40 : steps <= (pointwise ? 32 : 40) && tiles * steps <= (steps <= 6 || !pointwise ? 24576 : 8192);
-        // (the copy is spared as well; up to 256 rows the other kernels stream the weights)
-        return (few_steps || (few_bytes && wk_fits(M, N, steps, dma, M <= 256 ? kWkAnyReduction : 2 * kWkSpare))) && wk_enabled();
+        return (few_steps || (few_bytes && wk_fits(M, N, steps, dma, 12))) && wk_enabled(); // (12: the copy is spared as well)
     }
 
     template <class XL, int MT, int NT, int KW, int TW, int U, bool X_ON_A>

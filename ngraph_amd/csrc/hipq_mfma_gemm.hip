@@ -1095,7 +1095,7 @@ namespace hipq
             const int64_t steps = (d.K + 63) / 64;
             const bool streamed = skinny && d.M <= 32 && w_frag && steps >= (d.M <= 16 ? 12 : 24);
             const bool rows64 = skinny && d.M > 64 && dot_rows64_eligible(d);
-            const bool wk = !streamed && (!rows64 || ((d.M + 31) / 32) * ((d.N + 31) / 32) * steps <= 8192) && wk_preferred(d.M, d.N, steps, dma, !skinny);
+            const bool wk = !streamed && (!rows64 || ((d.M + 31) / 32) * ((d.N + 31) / 32) * steps <= 8192) && wk_preferred(d.M, d.N, steps, dma);
             if (wk)
             {
                 const int rc = launch_rows_wk(a, d.a_t == HIPQ_U8, static_cast<const int8_t*>(w_nk), w_frag, wsum, d.M, static_cast<int32_t>(d.N), static_cast<int32_t>(d.K), zp, epi, out, s,

@@ -77,9 +77,9 @@ def test_every_tile_shape(gpu_lib, pictures, N, steps, ragged):
         assert np.array_equal(got if ol == H.NXC else to_nxc(got), exp.reshape(pictures + (N,))), ol
 
 
-# (columns that are no multiple of 16; the last number of rows that the rule gives these kernels, and one more; as
-# many tiles of few rows, where the kernels that stream the weights are the others)
-@pytest.mark.parametrize("M,K,N,small", [(2976, 1088, 1001, True), (2977, 1088, 1001, False), (2080, 4160, 1001, True), (2081, 4160, 1001, False), (250, 4160, 8651, True)])
+# (columns that are no multiple of 16; the last number of rows that the rule gives these kernels, and one more; as many
+# tiles with a step less, of few rows, of few columns)
+@pytest.mark.parametrize("M,K,N,small", [(2304, 1344, 1001, True), (2305, 1344, 1001, False), (2305, 1280, 1001, True), (512, 1344, 4609, True), (36900, 1344, 63, True)])
 def test_long_reductions_over_many_tiles(gpu_lib, M, K, N, small):
     print("long reduction", M, K, N, flush=True)
     a = synth.uniform_int(81, (M, K), 0, 255, np.uint8)
