@@ -423,7 +423,9 @@ namespace hipq
     // long_limit: tiles a compute unit on long reductions
     static bool wk_fits(int64_t M, int64_t N, int64_t steps, bool dma, int64_t long_limit)
     {
-        const int64_t limit = dma ? (N <= 64 || steps > 4 ? 3 : steps > 1 ? 4 : 7) : (N <= 64 || M <= 512 || steps <= 20 ? 16 : long_limit);
+        // (the entry point that allocates nothing keeps sixteen: the tile kernels may want more scratch than it has)
+        const bool few = N <= 64 || M <= 512 || steps <= 20 || !workspace_holds(SIZE_MAX);
+        const int64_t limit = dma ? (N <= 64 || steps > 4 ? 3 : steps > 1 ? 4 : 7) : (few ? 16 : long_limit);
         return wk_tiles(M, N, 32, 32) <= static_cast<int64_t>(device_compute_units()) * limit;
     }
     bool wk_preferred(int64_t M, int64_t N, int64_t steps, bool dma, bool alone) { return wk_fits(M, N, steps, dma, alone ? 9 : 16) && wk_enabled(); }

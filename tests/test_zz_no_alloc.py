@@ -84,6 +84,21 @@ def test_noalloc_split_reduction_two_calls(gpu_lib, monkeypatch):
 
 
 @pytest.mark.gpu
+def test_noalloc_takes_a_long_reduction_without_partial_sums(gpu_lib):
+    """180 tiles whose partial sums would not fit the array: the kernels that need none, the regular entry point's bytes"""
+    say("noalloc long reduction")
+    d = H.make_conv_desc(6, 240, 704, (25, 25), (3, 3), pad_below=(1, 1), pad_above=(1, 1), data_layout=H.NXC, out_layout=H.NXC)
+    data = synth.uniform_int(3600, d.data_shape(), 0, 255, np.uint8)
+    filt = synth.uniform_int(3601, d.filter_shape(), -127, 127, np.int8)
+    args = (d, data, filt, 0.02, 7, 0.005, 0, 2.0, 0)
+    noalloc = H.quantized_convolution(*args, noalloc=True)
+    assert H.last_kernel() == "conv_mfma_wk_i8_16x16x64"
+    regular = H.quantized_convolution(*args)
+    assert H.last_kernel() == "conv_mfma_i8_32x32x32"
+    assert np.array_equal(noalloc, regular) and len(np.unique(regular)) > 50
+
+
+@pytest.mark.gpu
 def test_noalloc_refuses_what_does_not_fit(gpu_lib, monkeypatch):
     monkeypatch.setenv("HIPQ_NO_REGW", "1")  # the kernel that reads NCHW itself needs no scratch and would take this call
     lib = gpu_lib
