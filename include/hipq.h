@@ -662,7 +662,7 @@ HIPQ_API int hipq_batch_matmul_view_f32(const float* a,
  * on the compute unit.  Q is [queries, depth], K and V are [keys, depth] per batch element, addressed
  * like the views above (strides in elements); factor may be null (no Multiply); out may be null when
  * quant is given.  Returns HIPQ_ERR_UNSUPPORTED (nothing launched) unless depth == 64 and either queries ==
- * keys, up to 512 of them but not 64, or keys == 128 and queries is a multiple of 32: callers then run the three
+ * keys, up to 512 of them, or keys == 128 and queries is a multiple of 32: callers then run the three
  * ops.  No counterpart as a single reference op. */
 typedef struct hipq_attention_view
 {

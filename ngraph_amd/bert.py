@@ -163,10 +163,10 @@ class DevicePlan:
     the kernel launches of every layer on `stream`; `capture()` turns the pass into one HIP graph.
 
     fused=False launches the graph op by op, 19 launches a layer.  fused=True (what a backend's fusion
-    pass makes of the same graph, 9 calls a layer, 7 where a head has 17 to 512 keys (not 64) of depth 64) folds the ops that only re-read and re-write a
+    pass makes of the same graph, 9 calls a layer, 7 where a head has 17 to 512 keys of depth 64) folds the ops that only re-read and re-write a
     tensor into their producers, each through an entry point whose result equals the op-by-op one bit
     for bit: the head split and merge become views of the attention products (scores, Softmax and
-    context of a head are one kernel at 17 to 512 keys (not 64) of depth 64), Multiply goes into Softmax, the residual Add into LayerNorm, Gelu into the projection in front of it, and every
+    context of a head are one kernel at 17 to 512 keys of depth 64), Multiply goes into Softmax, the residual Add into LayerNorm, Gelu into the projection in front of it, and every
     Quantize into the kernel that produces its input (the context product, LayerNorm, that projection)."""
 
     def __init__(self, lib, stream, batch, cfg=BASE, fused=True):
@@ -232,8 +232,8 @@ class DevicePlan:
             # {0, H, 2H} + head * hd; scores [B * heads, S, S] dense; the context goes straight into [T, H]
             v_scores = self._keep(H.MatmulView(nh, S * H3, hd, H3, S * H3, hd, H3, nh * S * S, S * S, S))
             v_context = self._keep(H.MatmulView(nh, nh * S * S, S * S, S, S * H3, hd, H3, S * h, hd, h))
-            # sequences of 17 to 512 but not 64, depth 64: scores, Softmax and context of a head in one kernel
-            self.one_kernel_attention = 16 < S <= 512 and S != 64 and hd == 64
+            # sequences of 17 to 512, depth 64: scores, Softmax and context of a head in one kernel
+            self.one_kernel_attention = 16 < S <= 512 and hd == 64
             v_attention = self._keep(H.AttentionView(nh, S * H3, hd, H3, S * H3, hd, H3, S * H3, hd, H3, S * h, hd, h))
             for l in range(cfg.layers):
                 w = layer_weights(cfg, l)

@@ -680,11 +680,11 @@ int hipq_attention_f32(const float* q, const float* k, const float* v, const flo
 {
     HIPQ_REQUIRE(view, "null view");
     HIPQ_REQUIRE(batch >= 0 && queries >= 0 && keys >= 0 && depth >= 0, "negative extent");
-    // (64 keys stay refused as they were when this took 128 only, so that callers that rely on it run the three ops.
-    // Not for time: 12 heads 6.2 us here and 15.8 in three launches, 384 heads 16.5 and 28.8, 768 28.3 and 35.4)
-    const bool self = queries == keys && keys > 0 && keys <= AMAX && keys != 64;
+    // (every length up to the largest: 17 x 17 12 heads 6.0 us here and 17.6 in three launches, 64 x 64, a whole tile of
+    // the products' own kernel, 6.2 and 15.8, 768 heads 28.3 and 35.4, 65 x 65 48.7 and 96.6)
+    const bool self = queries == keys && keys > 0 && keys <= AMAX;
     if (depth != AD || !(self || (keys == AKEYS && queries % 32 == 0)))
-        return fail(HIPQ_ERR_UNSUPPORTED, "the one-kernel attention takes depth 64 and as many queries as keys, up to 512 but not 64, or 128 keys and query rows in multiples of 32 (run the three ops otherwise)");
+        return fail(HIPQ_ERR_UNSUPPORTED, "the one-kernel attention takes depth 64 and as many queries as keys, up to 512, or 128 keys and query rows in multiples of 32 (run the three ops otherwise)");
     if (batch == 0 || queries == 0)
         return HIPQ_OK;
     MatQuant mq{nullptr, nullptr, nullptr, HIPQ_I8, HIPQ_ROUND_NEAREST_TOWARD_EVEN};

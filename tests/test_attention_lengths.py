@@ -11,7 +11,7 @@ f32 = np.float32
 
 # (lengths around 16 rows, a chunk of 128 keys and the largest; few heads and, the last five, enough for items of 32
 # rows with one to four chunks)
-@pytest.mark.parametrize("B,S,nh", [(2, 1, 3), (1, 15, 2), (3, 17, 4), (2, 63, 2), (1, 65, 2), (24, 100, 12), (2, 127, 3), (9, 129, 8), (1, 197, 4), (2, 256, 1), (8, 257, 12), (1, 385, 2),
+@pytest.mark.parametrize("B,S,nh", [(2, 1, 3), (1, 15, 2), (3, 17, 4), (2, 63, 2), (1, 64, 1), (3, 64, 5), (25, 64, 12), (1, 65, 2), (24, 100, 12), (2, 127, 3), (9, 129, 8), (1, 197, 4), (2, 256, 1), (8, 257, 12), (1, 385, 2),
                                     (1, 509, 3), (25, 96, 12), (25, 128, 12), (10, 256, 12), (12, 384, 8), (16, 512, 4)])
 def test_attention_of_any_length_equals_the_three_ops(gpu_lib, B, S, nh):
     print("attention", B, S, nh, flush=True)

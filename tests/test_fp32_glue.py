@@ -291,7 +291,7 @@ def test_attention_in_one_kernel_rejects_other_shapes(gpu_lib):
     say("attention shapes")
     qkv = synth.normal_f32(49, (2 * 64, 3 * 64))
     view = H.AttentionView(1, 64 * 192, 64, 192, 64 * 192, 64, 192, 64 * 192, 64, 192, 64 * 64, 64, 64)
-    for queries, keys, depth in ((64, 64, 64), (128, 128, 32), (100, 128, 64)):
+    for queries, keys, depth in ((32, 64, 64), (64, 32, 64), (128, 128, 32), (100, 128, 64)):
         with pytest.raises(H.HipqError) as e:
             H.attention(qkv, 0, 64, 128, 2 * 64 * 64, view, 2, queries, keys, depth)
         assert e.value.code == H.ERR_UNSUPPORTED
