@@ -286,8 +286,7 @@ namespace hipq
         uint32_t bytes; // M * K
         static constexpr bool kUniform = true;
         static constexpr bool kFloatOut = true; // GEMM outputs may be floats; also: the loader is light enough on registers for three workgroups per compute unit
-        static constexpr bool kDeep = true;     // 128-byte-deep slices are possible
-        bool deep_ok() const { return true; }
+        static constexpr bool kDeep = false;    // (reductions of 256 bytes and more run on the tiles of hipq_igemm_ring.hip)
         static constexpr bool kPads = false; // no reads of padding: an out-of-range chunk is never used
         struct Row
         {
@@ -1870,7 +1869,7 @@ namespace hipq
         return check_launch(name);
     }
 
-    template <class XL, int WAVES_M, int WAVES_N, int MODE, bool HAS_SUM, int KIND = OUT_Q8, int BKT = BK, int WM = 2>
+    template <class XL, int WAVES_M, int WAVES_N, int MODE, bool HAS_SUM, int KIND = OUT_Q8, int BKT = BK>
     static int launch_pipe(const XL& xl,
                            const int8_t* w,
                            const int32_t* wsum,
@@ -1885,7 +1884,7 @@ namespace hipq
                            hipStream_t s,
                            const char* name)
     {
-        constexpr int BM = WAVES_M * WM * 32, BN = WAVES_N * 64;
+        constexpr int WM = 2, BM = WAVES_M * WM * 32, BN = WAVES_N * 64;
         constexpr bool DMA = XL::kUniform;
         // (the kernels that load into LDS and take no residual stage their outputs in an operand buffer)
         constexpr size_t lds_bytes = (DMA && BKT == BK && !HAS_SUM && WAVES_N > 1 ? 3 : 2) * static_cast<size_t>(BM + BN) * BKT + (DMA && !HAS_SUM ? 0 : 4 * WM * 32 * 64) + 3 * BN * sizeof(float) + 16;
@@ -1935,7 +1934,7 @@ namespace hipq
             // measured on ResNet-50's layers at batches 1, 32 and 128 and on GEMMs of 128 to 512 rows
             const int64_t units = dev >= 0 && dev < 16 && cus[dev] > 0 ? cus[dev] : 256;
             while (splits < 16 && slices % (splits * 2) == 0 &&
-                   ((tiles * splits * 2 * 4 <= units * 3 && slices * kDeep / (splits * 2) >= 8) || (WM == 2 && tiles * splits * 2 <= resident && slices * kDeep / (splits * 2) >= 16)))
+                   ((tiles * splits * 2 * 4 <= units * 3 && slices * kDeep / (splits * 2) >= 8) || (tiles * splits * 2 <= resident && slices * kDeep / (splits * 2) >= 16)))
                 splits *= 2;
         }
         int32_t* partials = nullptr;
@@ -1992,62 +1991,38 @@ namespace hipq
         const bool gelu_q8 = epi.post_scale != nullptr;
         if (gelu_q8 && (!f32 || N <= 64))
             return HIPQ_ERR_UNSUPPORTED;
-        // row matrices with reductions in whole 128-byte pieces, no residual, wide outputs: deep slices
-        bool deep = false;
+        // windows with reductions in whole 128-byte pieces, no residual, wide outputs: deep slices (what the tiles of
+        // hipq_igemm_ring.hip do not take: more than 32 taps)
+        if constexpr (XL::kFloatOut)
+            if (f32)
+            {
+                if (gelu_q8)
+                    return launch_pipe<XL, 2, 2, EPI_FUSED, false, OUT_GELU_Q8>(xl, w, wsum, M, N, Kred, x_unsigned, zp, epi, om, out, s, name);
+                if (N <= 64)
+                    return launch_pipe<XL, 4, 1, EPI_FUSED, false, OUT_F32>(xl, w, wsum, M, N, Kred, x_unsigned, zp, epi, om, out, s, name);
+                return launch_pipe<XL, 2, 2, EPI_FUSED, false, OUT_F32>(xl, w, wsum, M, N, Kred, x_unsigned, zp, epi, om, out, s, name);
+            }
         if constexpr (XL::kDeep)
         {
-            deep = xl.deep_ok() && Kred % (2 * BK) == 0 && Kred >= 4 * BK && N > 64 && epi.sum_in == nullptr && getenv("HIPQ_NO_DEEP_SLICES") == nullptr;
+            bool deep = xl.deep_ok() && Kred % (2 * BK) == 0 && Kred >= 4 * BK && N > 64 && epi.sum_in == nullptr && getenv("HIPQ_NO_DEEP_SLICES") == nullptr;
             // two of those workgroups fit a compute unit where three of the regular ones do: a
             // tile count that the regular kernel takes in one round and the deep one in two stays
-            // regular (4096 x 2304 outputs, 576 tiles on 256 units: 18.9 us against 22.9)
+            // regular
             const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
             const int64_t units = device_compute_units();
             if (tiles > 2 * units && tiles <= 3 * units)
                 deep = false;
             // few tiles with long reductions are split over workgroups, which then hold few slices
-            // each: three buffers of regular slices do better there (config 2 at 256 rows: 19.5 us
-            // against 20.9)
+            // each: three buffers of regular slices do better there
             if (tiles * 8 <= units * 3 && Kred >= 16 * BK)
                 deep = false;
-        }
-        // 128 x 128 tiles that leave compute units idle (and would have their reductions split over
-        // workgroups, partial sums through memory): 64 x 128 tiles, twice as many, no split.
-        // Row matrices only: a 3 x 3 filter's long reduction over gathered rows does better split
-        // (512 -> 512 channels on 128 x 7 x 7 pixels: 34 us split, 40 us in half tiles)
-        bool half_height = false;
-        if constexpr (XL::kDeep && !XL::kPads)
-        {
-            const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-            half_height = deep && M > 64 && tiles <= device_compute_units() && getenv("HIPQ_NO_HALF_TILES") == nullptr;
-        }
-        if constexpr (XL::kFloatOut)
-            if (f32)
-            {
-                if (half_height && gelu_q8)
-                    return launch_pipe<XL, 2, 2, EPI_FUSED, false, OUT_GELU_Q8, 2 * BK, 1>(xl, w, wsum, M, N, Kred, x_unsigned, zp, epi, om, out, s, name);
-                if (half_height)
-                    return launch_pipe<XL, 2, 2, EPI_FUSED, false, OUT_F32, 2 * BK, 1>(xl, w, wsum, M, N, Kred, x_unsigned, zp, epi, om, out, s, name);
-                if (gelu_q8)
-                {
-                    if (deep)
-                        return launch_pipe<XL, 2, 2, EPI_FUSED, false, OUT_GELU_Q8, 2 * BK>(xl, w, wsum, M, N, Kred, x_unsigned, zp, epi, om, out, s, name);
-                    return launch_pipe<XL, 2, 2, EPI_FUSED, false, OUT_GELU_Q8>(xl, w, wsum, M, N, Kred, x_unsigned, zp, epi, om, out, s, name);
-                }
-                if (N <= 64)
-                    return launch_pipe<XL, 4, 1, EPI_FUSED, false, OUT_F32>(xl, w, wsum, M, N, Kred, x_unsigned, zp, epi, om, out, s, name);
-                if (deep)
-                    return launch_pipe<XL, 2, 2, EPI_FUSED, false, OUT_F32, 2 * BK>(xl, w, wsum, M, N, Kred, x_unsigned, zp, epi, om, out, s, name);
-                return launch_pipe<XL, 2, 2, EPI_FUSED, false, OUT_F32>(xl, w, wsum, M, N, Kred, x_unsigned, zp, epi, om, out, s, name);
-            }
-        if constexpr (XL::kDeep)
             if (deep)
             {
-                if (half_height && epi.mode == EPI_FUSED)
-                    return launch_pipe<XL, 2, 2, EPI_FUSED, false, OUT_Q8, 2 * BK, 1>(xl, w, wsum, M, N, Kred, x_unsigned, zp, epi, om, out, s, name);
                 if (epi.mode == EPI_INTERP)
                     return launch_pipe<XL, 2, 2, EPI_INTERP, false, OUT_Q8, 2 * BK>(xl, w, wsum, M, N, Kred, x_unsigned, zp, epi, om, out, s, name);
                 return launch_pipe<XL, 2, 2, EPI_FUSED, false, OUT_Q8, 2 * BK>(xl, w, wsum, M, N, Kred, x_unsigned, zp, epi, om, out, s, name);
             }
+        }
         if (epi.mode == EPI_INTERP)
         {
             if (N <= 64)
@@ -2139,6 +2114,13 @@ namespace hipq
         }
         return fail(HIPQ_ERR_UNSUPPORTED, "no MFMA kernel for this epilogue / output type");
     }
+
+    // tiles that fit the chip (hipq_igemm_ring.hip); HIPQ_ERR_UNSUPPORTED (nothing launched, no error text) when the call is not of their kind
+    bool ring_preferred(int64_t M, int64_t N, int64_t K, bool conv);
+    int launch_rows_ring(const void* a, int a_unsigned, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi, void* out, hipStream_t s,
+                         const char* name);
+    int launch_conv_ring(const ConvX& cx, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, int x_unsigned, const ZeroPoints& zp, const Epilogue& epi, void* out, hipStream_t s,
+                         const char* name);
 
     // small products and convolutions: the reduction split over a workgroup's wavefronts, fragments straight
     // from memory (hipq_igemm_wk.hip); HIPQ_ERR_UNSUPPORTED (nothing launched, no error text) when the call

@@ -106,15 +106,22 @@ namespace hipq
             reinterpret_cast<const int32_t*>(static_cast<const uint8_t*>(packed) + align_up(static_cast<size_t>(g.K) * Kred, 256));
         OutMap om{out_ncx ? 1 : 0, N, xl.PQ};
         const int xu = g.data_t == HIPQ_U8 ? 1 : 0;
+        // a 1 x 1 filter over every pixel: the channels-last data is the [pixels][C] matrix itself
+        const bool rows = !out_ncx && g.taps() == 1 && g.st[1] == 1 && g.st[2] == 1 && g.pb[1] == 0 && g.pb[2] == 0 && g.out[1] == g.in[1] && g.out[2] == g.in[2];
+        if (!out_ncx && ring_preferred(M, N, Kred, true))
+        {
+            const char* const name = "conv_mfma_ring_i8_16x16x64";
+            const int rc = rows ? launch_rows_ring(data_nxc, xu, w, wsum, M, N, Kred, zp, epi, out, s, name) : launch_conv_ring(xl, w, wsum, M, N, Kred, xu, zp, epi, out, s, name);
+            if (rc != HIPQ_ERR_UNSUPPORTED)
+                return rc;
+        }
         if (conv_wk_preferred(g, epi.out_t, out_ncx))
         {
             const int rc = launch_conv_wk(xl, w, wsum, M, N, Kred, xu, zp, epi, om, out, s, "conv_mfma_wk_i8_16x16x64");
             if (rc != HIPQ_ERR_UNSUPPORTED)
                 return rc;
         }
-        // a 1 x 1 filter over every pixel: the channels-last data is the [pixels][C] matrix itself
-        if (!out_ncx && g.taps() == 1 && g.st[1] == 1 && g.st[2] == 1 && g.pb[1] == 0 && g.pb[2] == 0 && g.out[1] == g.in[1] && g.out[2] == g.in[2] &&
-            g.C % 16 == 0)
+        if (rows)
             return launch_rows_mfma(data_nxc, xu != 0, w, wsum, M, N, Kred, zp, epi, out, s, "conv_mfma_i8_32x32x32");
         // Channel counts in whole 64-byte slices take the kernels that load straight into LDS (on
         // ResNet-50's 3 x 3 and strided layers about 8 % faster than the register-staged ones);

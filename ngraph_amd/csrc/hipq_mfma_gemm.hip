@@ -1024,6 +1024,12 @@ namespace hipq
     int launch_rows_gelu_q8(const void* a, bool a_unsigned, const int8_t* w_nk, const void* w_frag, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi,
                             void* out, hipStream_t s)
     {
+        if (M > 256 && ring_preferred(M, N, K, false))
+        {
+            const int rc = launch_rows_ring(a, a_unsigned ? 1 : 0, w_nk, wsum, M, N, K, zp, epi, out, s, "dot_gelu_q8_mfma_ring_i8_16x16x64");
+            if (rc != HIPQ_ERR_UNSUPPORTED)
+                return rc;
+        }
         if (wk_preferred(M, N, (K + 63) / 64, N % 16 == 0, false))
         {
             // (128 x 768 x 3072: product, then Gelu and Quantize from the workspace 14.4 us, in one kernel 5.4)
@@ -1082,6 +1088,19 @@ namespace hipq
         if (a_row != 0)
             return launch_rows_wk_ragged(a, static_cast<int32_t>(a_row), d.a_t == HIPQ_U8, static_cast<const int8_t*>(w_nk), w_frag, wsum, d.M, static_cast<int32_t>(d.N), static_cast<int32_t>(d.K), zp,
                                          epi, out, s, "dot_mfma_wk_ragged_i8_16x16x64");
+        auto ring = [&]() {
+            return ring_preferred(d.M, d.N, d.K, false) ? launch_rows_ring(a, d.a_t == HIPQ_U8 ? 1 : 0, static_cast<const int8_t*>(w_nk), wsum, d.M, static_cast<int32_t>(d.N), static_cast<int32_t>(d.K),
+                                                                         zp, epi, out, s, "dot_mfma_ring_i8_16x16x64")
+                                                        : HIPQ_ERR_UNSUPPORTED;
+        };
+        // (up to 256 rows the kernels that stream the weights past, or split a reduction inside a workgroup, are ahead where
+        // they apply: 256 x 4096 x 3072 11.1 us there, 12.7 here; 200 x 1024 x 3072 5.9, 6.5)
+        if (d.M > 256)
+        {
+            const int rc = ring();
+            if (rc != HIPQ_ERR_UNSUPPORTED)
+                return rc;
+        }
         // Products too small to fill the chip: fragments straight from memory, the reduction split over a
         // workgroup's wavefronts.  Up to 32 rows with packed weights only short reductions: the kernel
         // below asks for whole lines of both operands, which counts from twelve steps on (1 x 1024 x 1003:
@@ -1135,6 +1154,12 @@ namespace hipq
                     return launch_skinny_wide<8>(d, a, w_nk, wsum, zp, epi, out, s);
                 return launch_skinny_wide<16>(d, a, w_nk, wsum, zp, epi, out, s);
             }
+        }
+        if (d.M <= 256)
+        {
+            const int rc = ring();
+            if (rc != HIPQ_ERR_UNSUPPORTED)
+                return rc;
         }
         return launch_rows_mfma(a, d.a_t == HIPQ_U8, static_cast<const int8_t*>(w_nk), wsum, d.M, static_cast<int32_t>(d.N), static_cast<int32_t>(d.K), zp, epi,
                                 out, s, "dot_mfma_i8_32x32x32");
