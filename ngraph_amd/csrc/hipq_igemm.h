@@ -30,6 +30,7 @@
 #include <type_traits>
 
 #include "hipq_common.h"
+#include "hipq_gelu_quantize.h"
 #include "hipq_quant_math.h"
 #include "hipq_row_math.h"
 
@@ -1383,9 +1384,7 @@ namespace hipq
         const float s256 = __fmul_rn(ec.scale, 256.0f);
         const int32_t c256 = 128 + 256 * ec.ozp;
         // (Gelu + Quantize of a float result: the Quantize's scale and zero point)
-        const float post_scale = KIND == OUT_GELU_Q8 ? *epi.post_scale : 1.0f;
-        const int32_t post_zp_i = KIND == OUT_GELU_Q8 ? load_zp(epi.post_zp, epi.post_t) : 0;
-        const float post_zp = static_cast<float>(post_zp_i);
+        const GeluQuantize gelu = gelu_quantize_of(KIND == OUT_GELU_Q8 ? *epi.post_scale : 1.0f, KIND == OUT_GELU_Q8 ? load_zp(epi.post_zp, epi.post_t) : 0, epi.post_t, epi.post_mode);
         // the fixed-point form needs |acc * scale| * 256 < 2^31 with room to spare
         const bool fast_interp = fabsf(ec.scale) * (static_cast<float>(Kred) * (255.0f * 128.0f)) < 4194304.0f;
         constexpr int SUM_LOADS = TM * TN / 16 / 64;
@@ -1522,27 +1521,16 @@ namespace hipq
                         uint32_t packed = 0;
                         if constexpr (KIND == OUT_GELU_Q8)
                         {
-                            // the float result exactly as the float kernel computes it, then Gelu and
-                            // Quantize with the arithmetic of their own kernels (gelu1, quantize4 /
-                            // quantize_one): the bytes equal the three launches'
+                            // the float result exactly as the float kernel computes it, then the bytes of Gelu and Quantize
                             v4f r4;
 #pragma unroll
                             for (int e = 0; e < 4; ++e)
                             {
                                 const float a = static_cast<float>(acc[mi][ni][4 * g + e]);
                                 const float y = __fmul_rn(FOLD ? a : __fadd_rn(a, bias4[e]), scale4[e]);
-                                r4[e] = gelu1(epi.relu ? ((y > 0.0f) ? y : __fmul_rn(y, -0.0f)) : y);
+                                r4[e] = epi.relu ? ((y > 0.0f) ? y : __fmul_rn(y, -0.0f)) : y;
                             }
-                            if (epi.post_mode == HIPQ_ROUND_NEAREST_TOWARD_EVEN) // uniform
-                                packed = epi.post_t == HIPQ_U8 ? quantize4<uint8_t, true>(r4, post_scale, post_zp, epi.post_mode) : quantize4<int8_t, true>(r4, post_scale, post_zp, epi.post_mode);
-                            else
-                            {
-#pragma unroll
-                                for (int e = 0; e < 4; ++e)
-                                    packed |= (epi.post_t == HIPQ_U8 ? static_cast<uint32_t>(quantize_one<float, uint8_t>(r4[e], post_scale, static_cast<uint8_t>(post_zp_i), epi.post_mode))
-                                                                     : static_cast<uint32_t>(static_cast<uint8_t>(quantize_one<float, int8_t>(r4[e], post_scale, static_cast<int8_t>(post_zp_i), epi.post_mode))))
-                                              << (8 * e);
-                            }
+                            packed = gelu_quantize4(r4, gelu);
                             *cell = packed;
                             continue;
                         }

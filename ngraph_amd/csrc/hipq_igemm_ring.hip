@@ -176,7 +176,7 @@ namespace hipq
             const int my_tiles = (total - vb + grid - 1) / grid;
             HeadWords hw = head_scalars_load(zp, epi, wsum);
             const float post_scale = KIND == OUT_GELU_Q8 ? *epi.post_scale : 1.0f;
-            const int32_t post_zp_i = KIND == OUT_GELU_Q8 ? load_zp(epi.post_zp, epi.post_t) : 0;
+            const int32_t post_zp = KIND == OUT_GELU_Q8 ? load_zp(epi.post_zp, epi.post_t) : 0;
             // tile t: column blocks in groups of 2^group_shift, along the group first, then down the rows (as igemm_pipe_kernel)
             auto tile_origin = [&](int j, int64_t& m0, int32_t& n0) {
                 const int t = vb + j * grid;
@@ -389,7 +389,7 @@ namespace hipq
             const float s256 = __fmul_rn(ec.scale, 256.0f);
             const int32_t c256 = 128 + 256 * ec.ozp;
             const bool fast_interp = fabsf(ec.scale) * (static_cast<float>(Kred) * (255.0f * 128.0f)) < 4194304.0f;
-            const float post_zp = static_cast<float>(post_zp_i);
+            const GeluQuantize gelu = gelu_quantize_of(post_scale, post_zp, epi.post_t, epi.post_mode);
             auto epilogue = [&](auto to_u8) {
                 constexpr bool PK_U8 = decltype(to_u8)::value;
                 constexpr int ESZ = Q8 ? 1 : 4;
@@ -432,22 +432,16 @@ namespace hipq
                     uint32_t packed = 0;
                     if constexpr (KIND == OUT_GELU_Q8)
                     {
-                        // the float result as the float kernels compute it, then Gelu and Quantize with the arithmetic of their own kernels
-                        v4f g;
+                        // the float result as the float kernels compute it, then the bytes of Gelu and Quantize
+                        v4f y;
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
                         {
-                            const float y = __fmul_rn(__fadd_rn(static_cast<float>(a[e]), b[e]), s[e]);
-                            g[e] = gelu1(epi.relu ? ((y > 0.0f) ? y : __fmul_rn(y, -0.0f)) : y);
+                            y[e] = __fmul_rn(__fadd_rn(static_cast<float>(a[e]), b[e]), s[e]);
+                            if (epi.relu) // uniform
+                                y[e] = (y[e] > 0.0f) ? y[e] : __fmul_rn(y[e], -0.0f);
                         }
-                        if (epi.post_mode == HIPQ_ROUND_NEAREST_TOWARD_EVEN) // uniform
-                            return PK_U8 ? quantize4<uint8_t, true>(g, post_scale, post_zp, epi.post_mode) : quantize4<int8_t, true>(g, post_scale, post_zp, epi.post_mode);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            packed |= (PK_U8 ? static_cast<uint32_t>(quantize_one<float, uint8_t>(g[e], post_scale, static_cast<uint8_t>(post_zp_i), epi.post_mode))
-                                             : static_cast<uint32_t>(static_cast<uint8_t>(quantize_one<float, int8_t>(g[e], post_scale, static_cast<int8_t>(post_zp_i), epi.post_mode))))
-                                      << (8 * e);
-                        return packed;
+                        return gelu_quantize4(y, gelu);
                     }
                     if constexpr (MODE == EPI_INTERP)
                     {
@@ -491,18 +485,10 @@ namespace hipq
                     }
                     return packed;
                 };
+                // row i of blocks, its accumulators in row `from`
+                auto row_of_blocks = [&](int i, int from, const v4f (&b)[B], const v4f (&s)[B]) {
 #pragma unroll
-                for (int q = 0; q < QUADS; ++q)
-                {
-                    v4f b[4], s[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                    {
-                        b[j] = bias4(4 * q + j);
-                        s[j] = scale4(4 * q + j);
-                    }
-#pragma unroll
-                    for (int i = 0; i < A; ++i)
+                    for (int q = 0; q < QUADS; ++q)
                     {
                         uint32_t sum[4] = {0, 0, 0, 0};
                         if constexpr (HAS_SUM)
@@ -516,22 +502,44 @@ namespace hipq
                         uint32_t d[4];
 #pragma unroll
                         for (int j = 0; j < 4; ++j)
-                            d[j] = bytes4(acc[i][4 * q + j], b[j], s[j], sum[j]);
+                            d[j] = bytes4(acc[from][4 * q + j], b[4 * q + j], s[4 * q + j], sum[j]);
                         transpose4(d);
                         __builtin_amdgcn_raw_buffer_store_b128(v4i{static_cast<int>(d[0]), static_cast<int>(d[1]), static_cast<int>(d[2]), static_cast<int>(d[3])}, ors, piece_offset(i, q), 0, 0);
                     }
-                }
 #pragma unroll
-                for (int j = 4 * QUADS; j < B; ++j)
+                    for (int j = 4 * QUADS; j < B; ++j)
+                    {
+                        const int row = (wm * A + i) * 16 + r16, n = cn0 + col0 + 16 * j;
+                        __builtin_amdgcn_raw_buffer_store_b32(static_cast<int>(bytes4(acc[from][j], b[j], s[j], 0u)), ors, cm0 + row < M && n < N ? row * N + n : kOob, 0, 0);
+                    }
+                };
+                v4f b[B], s[B];
+#pragma unroll
+                for (int j = 0; j < B; ++j)
                 {
-                    const v4f b = bias4(j), s = scale4(j);
-                    const int n = cn0 + col0 + 16 * j;
-#pragma unroll
+                    b[j] = bias4(j);
+                    s[j] = scale4(j);
+                }
+                if constexpr (KIND == OUT_GELU_Q8)
+                {
+                    // (one row of blocks at a time through the same instructions: all rows' together are 12 KB and more, met
+                    // once a tile, and wait for the instruction cache longer than moving the rows up takes)
+#pragma unroll 1
                     for (int i = 0; i < A; ++i)
                     {
-                        const int row = (wm * A + i) * 16 + r16;
-                        __builtin_amdgcn_raw_buffer_store_b32(static_cast<int>(bytes4(acc[i][j], b, s, 0u)), ors, cm0 + row < M && n < N ? row * N + n : kOob, 0, 0);
+                        row_of_blocks(i, 0, b, s);
+#pragma unroll
+                        for (int k = 0; k + 1 < A; ++k)
+#pragma unroll
+                            for (int j = 0; j < B; ++j)
+                                acc[k][j] = acc[k + 1][j];
                     }
+                }
+                else
+                {
+#pragma unroll
+                    for (int i = 0; i < A; ++i)
+                        row_of_blocks(i, i, b, s);
                 }
             };
 
@@ -601,7 +609,7 @@ namespace hipq
                     loader_next();
                 for (; kt < KT; ++kt)
                     slice(std::false_type{}, false);
-                if (Q8 && (KIND == OUT_GELU_Q8 ? epi.post_t == HIPQ_U8 : epi.out_t == HIPQ_U8) && MODE == EPI_FUSED) // uniform
+                if (KIND == OUT_Q8 && MODE == EPI_FUSED && epi.out_t == HIPQ_U8) // uniform
                     epilogue(std::true_type{});
                 else
                     epilogue(std::false_type{});
@@ -658,7 +666,7 @@ namespace hipq
         constexpr RingTile kRingInterp[] = {{128, 256, 0.77f, 2.4f}, {256, 128, 0.80f, 3.2f}, {128, 128, 0.435f, 2.2f}, {64, 128, 0.321f, 1.3f}};
         constexpr RingTile kRingF32[] = {{256, 144, 0.873f, 6.2f}, {256, 192, 0.989f, 7.6f}, {128, 192, 0.589f, 5.1f}, {128, 128, 0.408f, 3.4f},
                                          {128, 96, 0.390f, 2.9f},  {64, 128, 0.294f, 2.4f},  {64, 96, 0.293f, 2.1f},   {64, 64, 0.251f, 1.7f}};
-        constexpr RingTile kRingGelu[] = {{128, 256, 0.770f, 5.0f}, {128, 192, 0.589f, 4.0f}, {128, 128, 0.435f, 3.0f}, {64, 128, 0.321f, 2.0f}};
+        constexpr RingTile kRingGelu[] = {{128, 256, 0.770f, 8.2f}, {128, 192, 0.589f, 6.5f}, {128, 128, 0.435f, 4.9f}, {64, 128, 0.321f, 3.5f}};
 
         template <int COUNT>
         int ring_choose(const RingTile (&tiles)[COUNT], int64_t M, int64_t N, int64_t K)

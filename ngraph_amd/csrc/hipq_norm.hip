@@ -4,6 +4,7 @@
 #include <cmath>
 
 #include "hipq_common.h"
+#include "hipq_gelu_quantize.h"
 #include "hipq_quant_math.h"
 #include "hipq_row_math.h"
 
@@ -163,6 +164,12 @@ namespace hipq
                 if (t * 4 >= count)
                     return;
                 const f4 v = reinterpret_cast<const f4*>(in)[t];
+                if (GELU && !out) // uniform: the bytes alone
+                {
+                    const GeluQuantize g = gelu_quantize_of(qs, qz, q.quant_t, q.mode);
+                    static_cast<uint32_t*>(q.out)[t] = gelu_quantize4(v, g);
+                    return;
+                }
                 f4 r;
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
