@@ -2107,6 +2107,11 @@ namespace hipq
     bool ring_preferred(int64_t M, int64_t N, int64_t K, bool conv);
     int launch_rows_ring(const void* a, int a_unsigned, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi, void* out, hipStream_t s,
                          const char* name);
+    bool ring_any_preferred(int64_t M, int64_t N, int64_t K, int64_t C, const Epilogue& epi, bool window, bool ncx);
+    int launch_rows_ring_any(const void* a, int a_unsigned, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi, void* out, hipStream_t s,
+                             const char* name);
+    int launch_conv_ring_any(const ConvX& cx, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, int x_unsigned, const ZeroPoints& zp, const Epilogue& epi, bool ncx, void* out,
+                             hipStream_t s, const char* name);
     int launch_conv_ring(const ConvX& cx, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, int x_unsigned, const ZeroPoints& zp, const Epilogue& epi, void* out, hipStream_t s,
                          const char* name);
 

@@ -107,11 +107,18 @@ namespace hipq
         OutMap om{out_ncx ? 1 : 0, N, xl.PQ};
         const int xu = g.data_t == HIPQ_U8 ? 1 : 0;
         // a 1 x 1 filter over every pixel: the channels-last data is the [pixels][C] matrix itself
-        const bool rows = !out_ncx && g.taps() == 1 && g.st[1] == 1 && g.st[2] == 1 && g.pb[1] == 0 && g.pb[2] == 0 && g.out[1] == g.in[1] && g.out[2] == g.in[2];
+        const bool pointwise = g.taps() == 1 && g.st[1] == 1 && g.st[2] == 1 && g.pb[1] == 0 && g.pb[2] == 0 && g.out[1] == g.in[1] && g.out[2] == g.in[2];
+        const bool rows = !out_ncx && pointwise;
         if (!out_ncx && ring_preferred(M, N, Kred, true))
         {
             const char* const name = "conv_mfma_ring_i8_16x16x64";
             const int rc = rows ? launch_rows_ring(data_nxc, xu, w, wsum, M, N, Kred, zp, epi, out, s, name) : launch_conv_ring(xl, w, wsum, M, N, Kred, xu, zp, epi, out, s, name);
+            if (rc != HIPQ_ERR_UNSUPPORTED)
+                return rc;
+        }
+        if (ring_any_preferred(M, N, Kred, g.C, epi, !pointwise, out_ncx))
+        {
+            const int rc = launch_conv_ring_any(xl, w, wsum, M, N, Kred, xu, zp, epi, out_ncx, out, s, "conv_mfma_ring_any_i8_16x16x64");
             if (rc != HIPQ_ERR_UNSUPPORTED)
                 return rc;
         }

@@ -1097,7 +1097,10 @@ namespace hipq
         // they apply: 256 x 4096 x 3072 11.1 us there, 12.7 here; 200 x 1024 x 3072 5.9, 6.5)
         if (d.M > 256)
         {
-            const int rc = ring();
+            int rc = ring();
+            if (rc == HIPQ_ERR_UNSUPPORTED && ring_any_preferred(d.M, d.N, d.K, d.K, epi, false, false))
+                rc = launch_rows_ring_any(a, d.a_t == HIPQ_U8 ? 1 : 0, static_cast<const int8_t*>(w_nk), wsum, d.M, static_cast<int32_t>(d.N), static_cast<int32_t>(d.K), zp, epi, out, s,
+                                          "dot_mfma_ring_any_i8_16x16x64");
             if (rc != HIPQ_ERR_UNSUPPORTED)
                 return rc;
         }

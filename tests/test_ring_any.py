@@ -1,0 +1,110 @@
+"""Products and convolutions on the tiles for any number of columns, any multiple of 16 channels and both output layouts:
+every tile of every kind at sizes where one can go wrong -- columns that end inside 16, inside four and inside a
+block, windows whose slices lie across taps, pixels that end inside a row of four, one slice and many -- against the
+closed form, the oracle, or the other kernels."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from cases import dot_bias_closed_form, to_ncx, to_nxc
+from ngraph_amd import hipq as H
+from ngraph_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(257, 64, 17), (300, 400, 131), (391, 1424, 302), (260, 128, 3)]
+
+
+def operands(M, K, N, a_t):
+    lo, hi = (0, 255) if a_t == "u8" else (-128, 127)
+    a = synth.uniform_int(9001, (M, K), lo, hi, H.NP_OF[H.dtype_code(a_t)])
+    w = synth.uniform_int(9002, (N, K), -128, 127, np.int8)
+    bias = synth.uniform_int(9003, (N,), -(2**15), 2**15, np.int32)
+    bias[N // 2] = 2**26 + 12345  # (beyond what a float holds)
+    scale = synth.uniform_f32(9004, (N,), 0.5, 1.5) * np.float32(0.006 / np.sqrt(K))
+    return a, w, bias, scale
+
+
+@pytest.mark.parametrize("tile", range(4))
+@pytest.mark.parametrize("M,K,N", SHAPES)
+def test_products_of_any_width(gpu_lib, monkeypatch, tile, M, K, N):
+    print("ring any dot", tile, M, K, N, flush=True)
+    monkeypatch.setenv("HIPQ_RING_TILE", str(tile))
+    for a_t, out_t, relu in (("u8", "f32", False), ("i8", "f32", True), ("u8", "i8", False), ("i8", "u8", True)):
+        a, w, bias, scale = operands(M, K, N, a_t)
+        d = H.make_dot_desc(M, K, N, a_t=a_t, out_t=out_t, b_layout=H.B_NK)
+        exp = dot_bias_closed_form(a, w, bias, scale, out_t, relu)
+        got = H.quantized_dot_bias(d, H.make_fused_desc(has_bias=True, with_relu=relu, scale_count=N), a, w, bias, scale)
+        assert H.last_kernel() == "dot_mfma_ring_any_i8_16x16x64"
+        if out_t == "f32" and relu:  # (a ReLU leaves the sign of a zero open)
+            got, exp = got + np.float32(0), exp + np.float32(0)
+        assert np.array_equal(got.view(np.uint8), exp.view(np.uint8)), (a_t, out_t, relu)
+    # (a filter zero point: exact and slow; results beyond 2^31)
+    for out_t, os, azp, bzp, ozp in (("i8", 2.0, 0, 0, 0), ("u8", 0.7, 131, 0, 5), ("i32", 1e-4, 7, 0, 0), ("i32", 1e-9, 7, 0, 0), ("u8", 1.1, 9, -7, 1)):
+        d = H.make_dot_desc(M, K, N, out_t=out_t, b_layout=H.B_KN)
+        args = (d, a.view(np.uint8), np.ascontiguousarray(w.T), 0.02, azp, 0.005, bzp, os, ozp)
+        got = H.quantized_dot(*args)
+        assert H.last_kernel() == "dot_mfma_ring_any_i8_16x16x64"
+        assert np.array_equal(got, O.quantized_dot(*args)), (out_t, os, azp, bzp)
+
+
+# channels, outputs, image, window, stride, dilation, scheme of the output
+CONVS = [(16, 33, (9, 11), (3, 3), 1, 1, "nxc"), (80, 130, (13, 8), (3, 3), 2, 1, "nxc"), (48, 70, (12, 9), (3, 3), 1, 2, "nxc"), (64, 64, (7, 10), (5, 5), 1, 1, "ncx"),
+         (208, 35, (6, 7), (1, 1), 1, 1, "ncx"), (48, 144, (11, 9), (2, 3), 1, 1, "ncx"), (32, 3, (14, 14), (3, 1), 1, 1, "nxc")]
+
+
+@pytest.mark.parametrize("i", range(len(CONVS)))
+@pytest.mark.parametrize("tile", range(4))
+def test_convolutions_of_any_width(gpu_lib, monkeypatch, tile, i):
+    C, K, image, window, stride, dilation, scheme = CONVS[i]
+    print("ring any conv", tile, CONVS[i], flush=True)
+    pad = tuple((f - 1) * dilation // 2 for f in window)
+    kw = dict(stride=(stride,) * 2, dilation=(dilation,) * 2, pad_below=pad, pad_above=pad)
+    layout = dict(data_layout=H.NXC, out_layout=H.NXC) if scheme == "nxc" else {}
+    give, take = (to_nxc, to_ncx) if scheme == "nxc" else (lambda x: x, lambda x: x)
+    monkeypatch.setenv("HIPQ_RING_TILE", str(tile))
+    for data_t, out_t, res, relu in (("u8", "u8", None, True), ("i8", "i8", None, False), ("u8", "i8", "u8", False), ("i8", "u8", "i8", True)):
+        dn = H.make_conv_desc(3, C, K, image, window, data_t=data_t, out_t=out_t, **kw)
+        d = H.make_conv_desc(3, C, K, image, window, data_t=data_t, out_t=out_t, **layout, **kw)
+        lo, hi = (0, 255) if data_t == "u8" else (-128, 127)
+        data = synth.uniform_int(9101, dn.data_shape(), lo, hi, H.NP_OF[H.dtype_code(data_t)])
+        filt = synth.uniform_int(9102, dn.filter_shape(), -128, 127, np.int8)
+        bias = synth.uniform_int(9103, (K,), -20000, 20000, np.int32)
+        scale = synth.uniform_f32(9104, (K,), 0.5, 1.5) * np.float32(0.006 / np.sqrt(C * window[0] * window[1]))
+        f = H.make_fused_desc(has_bias=True, has_sum=res is not None, sum_t=res or "u8", with_relu=relu, scale_count=K)
+        summ, ss = None, None
+        if res:
+            summ, ss = synth.uniform_int(9105, dn.out_shape(), *((0, 255) if res == "u8" else (-128, 127)), H.NP_OF[H.dtype_code(res)]), 0.37
+        exp = O.quantized_convolution_fused(dn, f, data, filt, bias, summ, scale, ss)
+        got = H.quantized_convolution_fused(d, f, give(data), filt, bias, None if summ is None else give(summ), scale, ss)
+        assert H.last_kernel() == "conv_mfma_ring_any_i8_16x16x64"
+        assert np.array_equal(take(got), exp), (data_t, out_t, res)
+    for out_t, z in (("u8", (0, 0, 0)), ("i8", (128, 0, 5)), ("i32", (7, 0, 1)), ("i8", (9, -7, 1))):
+        dn = H.make_conv_desc(3, C, K, image, window, out_t=out_t, **kw)
+        d = H.make_conv_desc(3, C, K, image, window, out_t=out_t, **layout, **kw)
+        data = synth.uniform_int(9106, dn.data_shape(), 0, 255, np.uint8)
+        filt = synth.uniform_int(9107, dn.filter_shape(), -128, 127, np.int8)
+        s = (0.02, 0.005, 1.3)
+        exp = O.quantized_convolution(dn, data, filt, s[0], z[0], s[1], z[1], s[2], z[2])
+        got = H.quantized_convolution(d, give(data), filt, s[0], z[0], s[1], z[1], s[2], z[2])
+        assert H.last_kernel() == "conv_mfma_ring_any_i8_16x16x64"
+        assert np.array_equal(take(got), exp), (out_t, z)
+
+
+# more tiles than compute units, reductions of one, two and five slices
+@pytest.mark.parametrize("M,K,N", [(40000, 112, 405), (40000, 208, 403), (20001, 640, 270)])
+def test_any_width_more_tiles_than_compute_units(gpu_lib, monkeypatch, M, K, N):
+    print("ring any rounds", M, K, N, flush=True)
+    a, w, bias, scale = operands(M, K, N, "u8")
+    for out_t in ("i8", "f32"):
+        d = H.make_dot_desc(M, K, N, out_t=out_t, b_layout=H.B_NK)
+        f = H.make_fused_desc(has_bias=True, scale_count=N)
+        monkeypatch.setenv("HIPQ_NO_RING", "1")
+        exp = H.quantized_dot_bias(d, f, a, w, bias, scale)
+        assert "ring" not in H.last_kernel()
+        monkeypatch.delenv("HIPQ_NO_RING")
+        for tile in range(4):
+            monkeypatch.setenv("HIPQ_RING_TILE", str(tile))
+            assert np.array_equal(H.quantized_dot_bias(d, f, a, w, bias, scale).view(np.uint8), exp.view(np.uint8)), (out_t, tile)
+            assert H.last_kernel() == "dot_mfma_ring_any_i8_16x16x64"
+            monkeypatch.delenv("HIPQ_RING_TILE")
