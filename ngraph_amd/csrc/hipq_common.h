@@ -8,6 +8,8 @@
 #include <cstdio>
 #include <cstring>
 
+#include <unistd.h>
+
 #include "../../include/hipq.h"
 
 namespace hipq
@@ -33,6 +35,16 @@ namespace hipq
 
     inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
     int check_launch(const char* kernel);
+
+    // Whether any switch of the library is set: one walk over the environment, where a look-up by name costs as much and a
+    // rule may ask for many (93 variables: 65 ns; with a call of strncmp for each of them 440)
+    inline bool library_switched()
+    {
+        for (char** e = environ; e && *e; ++e)
+            if ((*e)[0] == 'H' && strncmp(*e, "HIPQ_", 5) == 0)
+                return true;
+        return false;
+    }
     int device_compute_units(); // compute units of the current device (cached per device; 256 when the query fails)
 
     // Grow-only device workspace, one per (device, stream): launches on different streams never

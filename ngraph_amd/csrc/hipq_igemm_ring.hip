@@ -93,13 +93,6 @@ namespace hipq
 #undef RING
         }
 
-        bool any_switch() // one walk over the environment, as wk_enabled()
-        {
-            bool any = false;
-            for (char** e = environ; e && *e && !any; ++e)
-                any = strncmp(*e, "HIPQ_", 5) == 0;
-            return any;
-        }
         bool ring_enabled()
         {
             // (the switches that name a kernel of another family mean that family)
@@ -118,7 +111,7 @@ namespace hipq
     bool ring_preferred(int64_t M, int64_t N, int64_t K, bool conv)
     {
         const int64_t steps = (K + 63) / 64, units = device_compute_units();
-        const bool switched = any_switch();
+        const bool switched = library_switched();
         if (switched && !ring_enabled())
             return false;
         if (switched && getenv("HIPQ_RING_TILE") != nullptr)
@@ -128,15 +121,15 @@ namespace hipq
     }
 
     // The tiles for any width (hipq_igemm_ring_any.hip).  What the kernels for whole 16-byte columns take they do faster, or
-    // have refused above.  The lines in 32 x 32 tiles x 64-byte steps are least squares over 970 drawn sizes; of 600 more they
-    // gave 95 to these tiles, 0.70 of the time before on average, six of them 3 to 12 % slower (us, before and here:
-    // 2044 x 1379 x 1017 product 33.2 and 12.7, 2836 x 727 x 3157 f32 50.8 and 26.4; 3 x 3 windows, 80 -> 412 channels on 30 x 19 x 7
-    // pixels 12.3 and 8.3, channels-last 64 -> 24 on 46 x 26 x 58 14.1 and 15.7, [image][channel][pixel] 335 -> 460 on 43 x 59
-    // 32.0 and 20.3).  Below them the kernels that split a reduction inside a workgroup wait for less: 2 x 12 x 36 of 16 -> 504 5.3 and 8.1.
+    // have refused above.  The lines in 32 x 32 tiles x 64-byte steps are fitted to 1 800 drawn sizes; of 700 more they
+    // gave 102 to these tiles, which took 0.67 of the time before on average, eight of them 3 to 11 % longer (us, before and here:
+    // 2044 x 1379 x 1017 product 33.2 and 12.7, 2836 x 727 x 3157 f32 50.8 and 26.4, 289 x 2607 x 695 11.7 and 12.9; 3 x 3 windows,
+    // 80 -> 412 channels on 30 x 19 x 7 pixels 12.3 and 8.3, [image][channel][pixel] 335 -> 460 on 43 x 59 32.0 and 20.3).  Below them
+    // the kernels that split a reduction inside a workgroup wait for less: 2 x 12 x 36 of 16 -> 504 5.3 and 8.1.
     bool ring_any_preferred(int64_t M, int64_t N, int64_t K, int64_t C, const Epilogue& epi, bool window, bool ncx)
     {
         const int64_t steps = (K + 63) / 64;
-        const bool switched = any_switch(), q8 = epi.out_t == HIPQ_U8 || epi.out_t == HIPQ_I8;
+        const bool switched = library_switched(), q8 = epi.out_t == HIPQ_U8 || epi.out_t == HIPQ_I8;
         if (switched && !ring_enabled())
             return false;
         if (switched && getenv("HIPQ_RING_TILE") != nullptr)
@@ -150,7 +143,8 @@ namespace hipq
         if (!ncx && q8 && (window ? whole && epi.mode == EPI_INTERP && steps > 32 : !whole && epi.mode == EPI_FUSED && epi.bias == nullptr && steps >= 20))
             return false;
         const int64_t small = ((M + 31) / 32) * ((N + 31) / 32) * steps;
-        return small > (ncx ? 3200 + 400 * steps : window ? 6000 + 250 * steps : 4800 + 100 * steps);
+        const bool filled = window && epi.mode == EPI_INTERP; // (taps in a padding become the zero point in LDS: a third of a slice more)
+        return small > (ncx ? (filled ? 4800 + 400 * steps : 4000 + 200 * steps) : window ? (filled ? 3200 + 800 * steps : 4800 + 200 * steps) : 4800 + 100 * steps);
     }
 
     int launch_rows_ring(const void* a, int a_unsigned, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi, void* out, hipStream_t s,

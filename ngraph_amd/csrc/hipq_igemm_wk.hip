@@ -409,12 +409,7 @@ namespace hipq
     // own there (`alone` unset).
     static bool wk_enabled()
     {
-        // one walk over the environment where nothing of the library's is set, as in any program that runs in
-        // earnest: a look-up by name costs as much, and there are seven
-        bool any = false;
-        for (char** e = environ; e && *e && !any; ++e)
-            any = strncmp(*e, "HIPQ_", 5) == 0;
-        if (!any)
+        if (!library_switched())
             return true;
         // (the switches that name a kernel of the other family mean that family)
         for (const char* name : {"HIPQ_NO_WK", "HIPQ_SPLIT_K", "HIPQ_NO_DMA", "HIPQ_NO_PIPE", "HIPQ_NO_CONV_DMA", "HIPQ_NO_HALF_TILES", "HIPQ_NO_REGW"})
