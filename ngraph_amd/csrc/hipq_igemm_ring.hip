@@ -144,7 +144,7 @@ namespace hipq
             return false;
         const int64_t small = ((M + 31) / 32) * ((N + 31) / 32) * steps;
         const bool filled = window && epi.mode == EPI_INTERP; // (taps in a padding become the zero point in LDS: a third of a slice more)
-        return small > (ncx ? (filled ? 4800 + 400 * steps : 4000 + 200 * steps) : window ? (filled ? 3200 + 800 * steps : 4800 + 200 * steps) : 4800 + 100 * steps);
+        return small > (ncx ? (filled ? 4800 + 400 * steps : 4000 + 260 * steps) : window ? (filled ? 3200 + 800 * steps : 4800 + 200 * steps) : 4800 + 100 * steps);
     }
 
     int launch_rows_ring(const void* a, int a_unsigned, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi, void* out, hipStream_t s,
