@@ -203,9 +203,10 @@ namespace hipq
             return static_cast<size_t>(nbuf) * ring_stage(bm, bn) + (sum ? static_cast<size_t>(bm) * bn : 0) + static_cast<size_t>(ring_param_loads(bn)) * 8 * 256;
         }
 
-        // ANY: any number of columns, any alignment of the output, channels-last or [image][channel][pixel] (`map`)
-        template <class XL, int WAVES_M, int WAVES_N, int A, int B, int NBUF, int MODE, bool HAS_SUM, int KIND, bool ANY = false>
-        __global__ __launch_bounds__(512, 2) void igemm_ring_kernel(XL xl, const int8_t* __restrict__ w, const int32_t* __restrict__ wsum, int64_t M, int32_t N, int32_t Kred, int32_t x_unsigned,
+        // ANY: any number of columns, any alignment of the output, channels-last or [image][channel][pixel] (`map`).  WGS: workgroups
+        // that share a compute unit
+        template <class XL, int WAVES_M, int WAVES_N, int A, int B, int NBUF, int MODE, bool HAS_SUM, int KIND, bool ANY = false, int WGS = 1>
+        __global__ __launch_bounds__(512, 2 * WGS) void igemm_ring_kernel(XL xl, const int8_t* __restrict__ w, const int32_t* __restrict__ wsum, int64_t M, int32_t N, int32_t Kred, int32_t x_unsigned,
                                                                    int32_t m_tiles, int32_t n_tiles, FastDiv by_m_tiles, FastDiv by_group, int32_t group_shift, ZeroPoints zp, Epilogue epi,
                                                                    RingMap map, void* __restrict__ out)
         {
@@ -848,14 +849,14 @@ namespace hipq
             }
             wait_vmcnt<0>(); // (the loads behind the last slice write zeros into LDS)
         }
-        template <class XL, int WAVES_M, int WAVES_N, int A, int B, int NBUF, int MODE, bool HAS_SUM, int KIND, bool ANY = false>
+        template <class XL, int WAVES_M, int WAVES_N, int A, int B, int NBUF, int MODE, bool HAS_SUM, int KIND, bool ANY = false, int WGS = 1>
         int launch_ring_tile(const XL& xl, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t Kred, int x_unsigned, const ZeroPoints& zp, const Epilogue& epi, const RingMap& map, void* out,
                              hipStream_t s, const char* name)
         {
             constexpr int BM = WAVES_M * A * 16, BN = WAVES_N * B * 16;
             constexpr size_t lds_bytes = ring_lds(BM, BN, NBUF, HAS_SUM && !ANY);
-            static_assert(lds_bytes <= 160 * 1024, "a compute unit's LDS");
-            auto kernel = igemm_ring_kernel<XL, WAVES_M, WAVES_N, A, B, NBUF, MODE, HAS_SUM, KIND, ANY>;
+            static_assert(WGS * lds_bytes <= 160 * 1024, "a compute unit's LDS");
+            auto kernel = igemm_ring_kernel<XL, WAVES_M, WAVES_N, A, B, NBUF, MODE, HAS_SUM, KIND, ANY, WGS>;
             static bool configured[16] = {};
             int dev = 0;
             HIPQ_HIP(hipGetDevice(&dev));
@@ -867,7 +868,7 @@ namespace hipq
             }
             const int64_t m_tiles = (M + BM - 1) / BM, n_tiles = (N + BN - 1) / BN;
             HIPQ_REQUIRE(fits_i32(m_tiles * n_tiles + 1024), "too many tiles");
-            const int64_t units = device_compute_units(), tiles = m_tiles * n_tiles;
+            const int64_t units = device_compute_units() * WGS, tiles = m_tiles * n_tiles;
             const unsigned grid = static_cast<unsigned>(tiles < units ? (tiles + 7) / 8 * 8 : units);
             int group_shift = 0;
             while (group_shift < 3 && (2ll << group_shift) <= n_tiles && grid % (2u << group_shift) == 0)
@@ -877,11 +878,13 @@ namespace hipq
             return check_launch(name);
         }
 
-        // a tile's size, and what a slice and a round cost (see the lists)
+        // a tile's size, and what a slice and a round cost (see the lists); where two workgroups share a compute unit, that
+        // of one alone there and of two at a time
         struct RingTile
         {
             int bm, bn;
             float slice, round;
+            float pair_slice = 0.0f, pair_round = 0.0f;
         };
         template <int COUNT>
         int ring_choose(const RingTile (&tiles)[COUNT], int64_t M, int64_t N, int64_t K)
@@ -895,8 +898,9 @@ namespace hipq
             for (int i = 0; i < COUNT; ++i)
             {
                 const RingTile& t = tiles[i];
-                const int64_t rounds = (((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) + units - 1) / units;
-                const float cost = static_cast<float>(rounds) * (static_cast<float>(slices) * t.slice + t.round);
+                const int64_t rounds = (((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) + units - 1) / units, pairs = t.pair_slice > 0.0f ? rounds / 2 : 0;
+                const float k = static_cast<float>(slices);
+                const float cost = static_cast<float>(rounds - 2 * pairs) * (k * t.slice + t.round) + static_cast<float>(pairs) * (k * t.pair_slice + t.pair_round);
                 if (best < 0 || cost < least)
                 {
                     best = i;

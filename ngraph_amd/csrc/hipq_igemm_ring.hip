@@ -18,7 +18,15 @@ namespace hipq
         constexpr RingTile kRingInterp[] = {{128, 256, 0.77f, 2.4f}, {256, 128, 0.80f, 3.2f}, {128, 128, 0.435f, 2.2f}, {64, 128, 0.321f, 1.3f}};
         constexpr RingTile kRingF32[] = {{256, 144, 0.873f, 6.2f}, {256, 192, 0.989f, 7.6f}, {128, 192, 0.589f, 5.1f}, {128, 128, 0.408f, 3.4f},
                                          {128, 96, 0.390f, 2.9f},  {64, 128, 0.294f, 2.4f},  {64, 96, 0.293f, 2.1f},   {64, 64, 0.251f, 1.7f}};
-        constexpr RingTile kRingGelu[] = {{128, 256, 0.770f, 8.2f}, {128, 192, 0.589f, 6.5f}, {128, 128, 0.435f, 4.9f}, {64, 128, 0.321f, 3.5f}};
+        // Gelu and Quantize: a third of a tile's time or more is its epilogue, vector work that two workgroups a compute unit
+        // overlap with each other's products where the tiles come in pairs (128 x 128 alone 4.6 us a tile beyond its
+        // slices, two together 6.4), and fewer, larger tiles spend on fewer rounds (4096 x 768 x 3072: 128 x 192 in two
+        // rounds 26.1 us, 256 x 192 in one 22.7; 2048 x 1024 x 4096: 128 x 256 18.5, 128 x 128 in pairs 17.6; fitted to 90 sizes,
+        // the tile picked is 0.8 % slower than the best one).  The other kinds gain in a loop and lose behind other layers,
+        // where two buffers are too few (256 x 192 for 256 -> 512 channels 3 x 3 on 128 x 56 x 56 pixels 36.8 -> 41.4 us in
+        // ResNet-50, pairs for 512 -> 256 36.5 -> 39.8).
+        constexpr RingTile kRingGelu[] = {{128, 256, 0.783f, 7.77f}, {128, 192, 0.635f, 6.10f}, {128, 128, 0.507f, 4.15f}, {64, 128, 0.380f, 2.38f},
+                                          {256, 192, 1.033f, 10.58f}, {128, 128, 0.513f, 4.63f, 1.084f, 6.39f}, {128, 96, 0.477f, 4.03f, 0.928f, 4.87f}};
 
         template <class XL>
         int launch_ring(const XL& xl, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t Kred, int x_unsigned, const ZeroPoints& zp, const Epilogue& epi, void* out, hipStream_t s,
@@ -34,6 +42,7 @@ namespace hipq
                 return HIPQ_ERR_UNSUPPORTED;
             if ((!q8 && !f32) || N % 16 != 0 || N > (1 << 20) || Kred < 2 * SL || Kred >= 65536 || !aligned(out) || !aligned(epi.sum_in))
                 return HIPQ_ERR_UNSUPPORTED;
+#define RING2(WM_, WN_, A_, B_, NB_, MODE_, SUM_, KIND_) launch_ring_tile<XL, WM_, WN_, A_, B_, NB_, MODE_, SUM_, KIND_, false, 2>(xl, w, wsum, M, N, Kred, x_unsigned, zp, epi, RingMap{}, out, s, name)
 #define RING(WM_, WN_, A_, B_, NB_, MODE_, SUM_, KIND_) launch_ring_tile<XL, WM_, WN_, A_, B_, NB_, MODE_, SUM_, KIND_>(xl, w, wsum, M, N, Kred, x_unsigned, zp, epi, RingMap{}, out, s, name)
             if constexpr (!XL::kConv)
             {
@@ -44,6 +53,9 @@ namespace hipq
                     case 1: return RING(2, 4, 4, 3, 3, EPI_FUSED, false, OUT_GELU_Q8);
                     case 2: return RING(4, 2, 2, 4, 4, EPI_FUSED, false, OUT_GELU_Q8);
                     case 3: return RING(4, 2, 1, 4, 6, EPI_FUSED, false, OUT_GELU_Q8);
+                    case 4: return RING(4, 2, 4, 6, 2, EPI_FUSED, false, OUT_GELU_Q8);
+                    case 5: return RING2(4, 2, 2, 4, 2, EPI_FUSED, false, OUT_GELU_Q8);
+                    case 6: return RING2(4, 2, 2, 3, 2, EPI_FUSED, false, OUT_GELU_Q8);
                     default: return HIPQ_ERR_UNSUPPORTED;
                     }
                 if (f32)

@@ -46,8 +46,8 @@ def test_dot_bias_on_every_tile(gpu_lib, monkeypatch, tile, M, K, N):
         assert np.array_equal(got + np.zeros(1, got.dtype), one + np.zeros(1, one.dtype)), (a_t, out_t, relu, "one scale, no bias")
 
 
-@pytest.mark.parametrize("tile", range(4))
-@pytest.mark.parametrize("M,K,N", SHAPES)
+@pytest.mark.parametrize("tile", range(7))
+@pytest.mark.parametrize("M,K,N", SHAPES + [(5000, 384, 2064)])  # (more tiles than two a compute unit)
 def test_gelu_quantize_on_every_tile(gpu_lib, monkeypatch, tile, M, K, N):
     print("ring gelu", tile, M, K, N, flush=True)
     a, w, bias, scale = operands(M, K, N, "i8")
