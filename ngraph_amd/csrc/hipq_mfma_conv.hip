@@ -124,7 +124,8 @@ namespace hipq
         }
         if (conv_wk_preferred(g, epi.out_t, out_ncx))
         {
-            const int rc = launch_conv_wk(xl, w, wsum, M, N, Kred, xu, zp, epi, om, out, s, "conv_mfma_wk_i8_16x16x64");
+            const char* const name = "conv_mfma_wk_i8_16x16x64";
+            const int rc = rows ? launch_rows_wk(data_nxc, xu != 0, w, nullptr, wsum, M, N, Kred, zp, epi, out, s, name) : launch_conv_wk(xl, w, wsum, M, N, Kred, xu, zp, epi, om, out, s, name);
             if (rc != HIPQ_ERR_UNSUPPORTED)
                 return rc;
         }
