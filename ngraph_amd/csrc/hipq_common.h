@@ -137,6 +137,22 @@ namespace hipq
     };
 
 #if defined(__HIPCC__)
+    // The kernel's arguments (the first BYTES of them), asked for line by line at once: the compiler loads a field where it is
+    // first needed, each first touch of a 64-byte line is a trip past the scalar cache, and the next field's
+    // address or branch waits for it -- six trips in turn in front of the first operand load of igemm_wk_kernel
+    template <int BYTES>
+    __device__ __forceinline__ void touch_arguments()
+    {
+        typedef const uint32_t __attribute__((address_space(4))) * Words; // (the address space is what makes them scalar loads)
+        const Words at = (Words)__builtin_amdgcn_kernarg_segment_ptr();
+        uint32_t any = 0;
+#pragma unroll
+        for (int i = 0; i < BYTES; i += 64)
+            any |= at[i / 4];
+        any = __builtin_amdgcn_readfirstlane(any);
+        asm volatile("" ::"s"(any));
+    }
+
     __device__ __forceinline__ int32_t load_q(const void* p, int t, size_t i)
     {
         switch (t)

@@ -129,6 +129,7 @@ namespace hipq
         static constexpr bool kPads = false; // (only read by the kernels that load straight into LDS)
         static constexpr bool kPadded = false; // no taps in a padding
         static constexpr bool kRagged = false; // 16-byte chunks of the data are aligned
+        static constexpr int kWalk = 1;        // the steps' cursors follow from each other (0: each from its place)
 
         struct Row
         {
@@ -166,6 +167,7 @@ namespace hipq
         static constexpr bool kPads = false; // (only read by the kernels that load straight into LDS)
         static constexpr bool kPadded = true; // taps in the padding are the data zero point
         static constexpr bool kRagged = false; // 16-byte chunks of the data are aligned
+        static constexpr int kWalk = 0;
         const uint8_t* x; // [N][H][W][C]
         int32_t H, W, C, Q, R, S, sh, sw, dh, dw, pbh, pbw;
         int64_t PQ;
@@ -252,6 +254,77 @@ namespace hipq
                     }
                 }
             return acc;
+        }
+    };
+
+    // The same windows for reductions walked in steps of 64 bytes, fewer than 2^31 output pixels: a step's cursor follows
+    // from the one before in a few additions, where ConvX divides twice a step in front of its load.  UNIFORM: a
+    // multiple of 64 channels, a step lies inside one tap and its cursor is the same for every lane (scalar registers;
+    // a lane's chunk is in Row::off); else one a lane, for its 16-byte chunk.
+    template <bool UNIFORM>
+    struct ConvStepX : ConvX
+    {
+        static constexpr int kWalk = UNIFORM ? 2 : 1;
+        // a step on: `rest` channels, `cols` columns and `rows` rows of the window (in pixels), `step` bytes; `tap_step` and `row_step`
+        // bytes more where the channel or the column wraps; width of the window with its dilation
+        int32_t rest, cols, rows, step, tap_step, row_step, width;
+        struct Row
+        {
+            int32_t off;    // of the window's first tap (may lie before the image)
+            int32_t y0, x0; // its pixel; beyond M no row of the image
+        };
+        struct Cursor
+        {
+            int32_t y, x, c, off; // tap's pixel and channel, and their distance from the window's first
+        };
+        void set_steps()
+        {
+            const int32_t taps = 64 / C;
+            rest = 64 % C;
+            cols = taps % S * dw;
+            rows = taps / S * dh;
+            step = (rows * W + cols) * C + rest;
+            tap_step = dw * C - C;
+            width = S * dw;
+            row_step = (dh * W - width) * C;
+        }
+        __device__ __forceinline__ void init_row(Row& rw, int64_t m, int64_t M) const
+        {
+            const bool valid = m < M;
+            const uint32_t mm = valid ? static_cast<uint32_t>(m) : 0u;
+            const int32_t n = static_cast<int32_t>(by_pq.div(mm));
+            const int32_t rem = static_cast<int32_t>(mm) - n * static_cast<int32_t>(PQ);
+            const int32_t p = static_cast<int32_t>(by_q.div(static_cast<uint32_t>(rem)));
+            const int32_t y0 = p * sh - pbh;
+            rw.x0 = (rem - p * Q) * sw - pbw;
+            rw.off = ((n * H + y0) * W + rw.x0) * C;
+            rw.y0 = valid ? y0 : -(1 << 30);
+        }
+        __device__ __forceinline__ void init_cursor(Cursor& cur, int kbyte) const
+        {
+            const int32_t tap = static_cast<int32_t>(by_c.div(static_cast<uint32_t>(kbyte)));
+            const int32_t r = static_cast<int32_t>(by_s.div(static_cast<uint32_t>(tap)));
+            cur.c = kbyte - tap * C;
+            cur.y = r * dh;
+            cur.x = (tap - r * S) * dw;
+            cur.off = (cur.y * W + cur.x) * C + cur.c;
+        }
+        __device__ __forceinline__ void advance(Cursor& cur, int) const
+        {
+            cur.c += rest;
+            const int32_t tap = ~((cur.c - C) >> 31); // all ones: one tap more
+            cur.c -= tap & C;
+            cur.x += cols + (tap & dw);
+            const int32_t row = ~((cur.x - width) >> 31); // all ones: the next row of taps
+            cur.x -= row & width;
+            cur.y += rows + (row & dh);
+            cur.off += step + (tap & tap_step) + (row & row_step);
+        }
+        __device__ __forceinline__ int32_t offset(const Row& rw, const Cursor& c) const
+        {
+            // (past the last tap nothing is asked for)
+            const bool ok = (static_cast<uint32_t>(rw.y0 + c.y) < static_cast<uint32_t>(H)) & (static_cast<uint32_t>(rw.x0 + c.x) < static_cast<uint32_t>(W));
+            return ok ? rw.off + c.off : kOob;
         }
     };
 
@@ -555,7 +628,8 @@ namespace hipq
         const bool interp = e.mode == EPI_INTERP;
         auto word_at = [&](const void* p, bool used) {
             const uint8_t* q = static_cast<const uint8_t*>((used && p != nullptr) ? p : safe);
-            return *reinterpret_cast<const uint32_t*>(q - (reinterpret_cast<uintptr_t>(q) & 3)); // (pointer arithmetic, not an integer cast: the load stays a global one)
+            typedef const uint32_t __attribute__((address_space(4))) * Words; // (nothing writes them while the kernel runs: scalar loads wherever they stand)
+            return *(Words)(q - (reinterpret_cast<uintptr_t>(q) & 3));
         };
         HeadWords h;
         h.x = word_at(zp.data_zp, true);
