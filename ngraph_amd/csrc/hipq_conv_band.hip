@@ -337,6 +337,7 @@ namespace hipq
                                                                     Epilogue epi,
                                                                     void* __restrict__ out)
     {
+        touch_arguments<sizeof(BandParams) + 16 + sizeof(ZeroPoints) + sizeof(Epilogue) + sizeof(void*)>();
         extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
         const int tid = threadIdx.x;
         const int lane = tid & 63;

@@ -58,6 +58,7 @@ namespace hipq
         template <int CIN, bool HAS_SUM>
         __global__ __launch_bounds__(256, 3) void conv_pw64_kernel(const PwParams p)
         {
+            touch_arguments<sizeof(PwParams)>();
             constexpr int KS = CIN / 32;
             constexpr int NB = CIN == 64 ? 2 : 1; // accumulator blocks of 32 channels live at a time (registers: the weight fragments take 8 KS)
             constexpr int kPwData = kPwRows * CIN; // bytes of a tile's data in LDS

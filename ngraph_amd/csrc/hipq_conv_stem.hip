@@ -89,6 +89,7 @@ namespace hipq
         template <bool POOL, int KS, int UNIT>
         __global__ __launch_bounds__(kStemThreads) void conv_stem_kernel(const StemParams p)
         {
+            touch_arguments<sizeof(StemParams)>();
             extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
             const int tid = static_cast<int>(threadIdx.x);
             const int lane = tid & 63;

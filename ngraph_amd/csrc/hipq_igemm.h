@@ -173,6 +173,21 @@ namespace hipq
         int64_t PQ;
         uint32_t bytes; // N * H * W * C
         FastDiv by_pq, by_q, by_c, by_s; // by_pq.sh == 0xffffffff: more than 2^31 output pixels, plain division
+        // ConvStepX: 64 bytes of the reduction on are `rest` channels, `cols` columns and `rows` rows of the window (in pixels), `step`
+        // bytes of the data; `tap_step` and `row_step` bytes more where the channel or the column wraps; width of the
+        // window with its dilation
+        int32_t rest, cols, rows, step, tap_step, row_step, width;
+        void set_steps()
+        {
+            const int32_t taps = 64 / C;
+            rest = 64 % C;
+            cols = taps % S * dw;
+            rows = taps / S * dh;
+            step = (rows * W + cols) * C + rest;
+            tap_step = dw * C - C;
+            width = S * dw;
+            row_step = (dh * W - width) * C;
+        }
 
         struct Row
         {
@@ -257,17 +272,11 @@ namespace hipq
         }
     };
 
-    // The same windows for reductions walked in steps of 64 bytes, fewer than 2^31 output pixels: a step's cursor follows
-    // from the one before in a few additions, where ConvX divides twice a step in front of its load.  UNIFORM: a
-    // multiple of 64 channels, a step lies inside one tap and its cursor is the same for every lane (scalar registers;
-    // a lane's chunk is in Row::off); else one a lane, for its 16-byte chunk.
-    template <bool UNIFORM>
+    // The same windows for reductions walked in steps of 64 bytes, fewer than 2^31 output pixels: the cursor of a lane's
+    // chunk follows from the one before in a few additions, where ConvX divides twice a step in front of its load.
     struct ConvStepX : ConvX
     {
-        static constexpr int kWalk = UNIFORM ? 2 : 1;
-        // a step on: `rest` channels, `cols` columns and `rows` rows of the window (in pixels), `step` bytes; `tap_step` and `row_step`
-        // bytes more where the channel or the column wraps; width of the window with its dilation
-        int32_t rest, cols, rows, step, tap_step, row_step, width;
+        static constexpr int kWalk = 1;
         struct Row
         {
             int32_t off;    // of the window's first tap (may lie before the image)
@@ -277,17 +286,6 @@ namespace hipq
         {
             int32_t y, x, c, off; // tap's pixel and channel, and their distance from the window's first
         };
-        void set_steps()
-        {
-            const int32_t taps = 64 / C;
-            rest = 64 % C;
-            cols = taps % S * dw;
-            rows = taps / S * dh;
-            step = (rows * W + cols) * C + rest;
-            tap_step = dw * C - C;
-            width = S * dw;
-            row_step = (dh * W - width) * C;
-        }
         __device__ __forceinline__ void init_row(Row& rw, int64_t m, int64_t M) const
         {
             const bool valid = m < M;
@@ -1128,6 +1126,7 @@ namespace hipq
                                                                 OutMap om,
                                                                 void* __restrict__ out)
     {
+        touch_arguments<sizeof(XL) + 72 + 2 * sizeof(FastDiv) + sizeof(ZeroPoints) + sizeof(Epilogue) + sizeof(OutMap)>();
         static_assert(WAVES_M * WAVES_N == 4, "four wavefronts per workgroup");
         constexpr int BM = WAVES_M * WM * 32;
         constexpr int BN = WAVES_N * WN * 32;

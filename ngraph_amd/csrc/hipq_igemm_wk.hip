@@ -21,8 +21,9 @@
 //
 // A launch of a single picture's layer is mostly the way to its first operands: the arguments' lines are touched at once
 // (touch_arguments), operands are asked for before anything that the epilogue needs, and a window's steps follow
-// from each other (ConvStepX) instead of two divisions each.  ResNet-50 on one picture 306 -> 287 us, the encoder of one
-// sequence 458 -> 443, u8 [8,90,35,29] x i8 [150,90,3,3] 13.1 -> 12.5.
+// from each other (ConvStepX) instead of two divisions each.  With that and the row loader for 1 x 1 filters ResNet-50
+// on one picture 340 -> 275 us (306 with the row loader alone), the encoder of one sequence 457 -> 442, u8 [8,90,35,29] x
+// i8 [150,90,3,3] 13.1 -> 12.5.
 //
 // Rows and pixels that are no multiple of 16 bytes are read where they lie (ragged_preferred): u8
 // [8,90,35,29] x i8 [150,90,3,3] 14.4 -> 13.1 us, 77 x 1000 x 1003 8.2 -> 4.1 with the copy's launch gone.
@@ -64,8 +65,11 @@ namespace hipq
     // X_ON_A: the activations are MFMA source A, so that a lane's four accumulators are four consecutive
     // pixels of one channel (NCHW outputs); otherwise four consecutive channels of one pixel
     template <class XL, int MT, int NT, int KW, int TW, int U, bool X_ON_A>
-    __global__ __launch_bounds__(KW * TW * 64) void igemm_wk_kernel(XL xl, WkParams p, ZeroPoints zp, Epilogue epi, OutMap om, void* __restrict__ out)
+    __global__ __launch_bounds__(KW * TW * 64) void igemm_wk_kernel(XL arg, WkParams p, ZeroPoints zp, Epilogue epi, OutMap om, void* __restrict__ out)
     {
+        using Loader = typename std::conditional<std::is_same<XL, ConvX>::value, ConvStepX, XL>::type;
+        Loader xl;
+        static_cast<XL&>(xl) = arg;
         constexpr int BM = MT * 16, BN = NT * 16;
         constexpr int BLOCKS = MT * NT;
         static_assert(BLOCKS % KW == 0 || KW % BLOCKS == 0, "the wavefronts of a tile share its blocks evenly");
@@ -98,17 +102,13 @@ namespace hipq
         const int s_end = min(steps, s_begin + per);
         const __amdgpu_buffer_rsrc_t xrs = make_rsrc(xl.x, xl.bytes);
         const __amdgpu_buffer_rsrc_t wrs = make_rsrc(p.w, p.w_bytes);
-        typename XL::Row xr[MT];
+        typename Loader::Row xr[MT];
 #pragma unroll
         for (int i = 0; i < MT; ++i)
-        {
             xl.init_row(xr[i], m0 + i * 16 + r16, p.M);
-            if constexpr (XL::kWalk == 2)
-                xr[i].off += kc * 16;
-        }
-        typename XL::Cursor cur; // kWalk: of the next step to load
-        if constexpr (XL::kWalk != 0)
-            xl.init_cursor(cur, s_begin * 64 + (XL::kWalk == 2 ? 0 : kc * 16));
+        typename Loader::Cursor cur; // kWalk: of the next step to load
+        if constexpr (Loader::kWalk != 0)
+            xl.init_cursor(cur, s_begin * 64 + kc * 16);
         int32_t woff[NT];
 #pragma unroll
         for (int j = 0; j < NT; ++j)
@@ -130,7 +130,7 @@ namespace hipq
         auto load = [&](int u, int s) {
             const int kbyte = s * 64 + kc * 16;
             const bool in_k = (s < s_end) & (kbyte < p.Kred);
-            if constexpr (XL::kWalk == 0)
+            if constexpr (Loader::kWalk == 0)
                 xl.init_cursor(cur, kbyte);
 #pragma unroll
             for (int i = 0; i < MT; ++i)
@@ -152,7 +152,7 @@ namespace hipq
 #pragma unroll
             for (int j = 0; j < NT; ++j)
                 wf[u][j] = buffer_load16(wrs, (in_k && woff[j] != kOob) ? woff[j] + s * p.w_step : kOob);
-            if constexpr (XL::kWalk != 0)
+            if constexpr (Loader::kWalk != 0)
                 xl.advance(cur, 64);
         };
 #pragma unroll
@@ -556,23 +556,14 @@ namespace hipq
         return launch_wk<ConvRaggedX, false>(xl, p, zp, epi, om, out, s, name);
     }
 
-    template <bool UNIFORM>
-    static int launch_conv_steps(const ConvX& cx, const WkParams& p, const ZeroPoints& zp, const Epilogue& epi, const OutMap& om, void* out, hipStream_t s, const char* name)
-    {
-        ConvStepX<UNIFORM> xl;
-        static_cast<ConvX&>(xl) = cx;
-        xl.set_steps();
-        if (om.ncx)
-            return launch_wk<ConvStepX<UNIFORM>, true>(xl, p, zp, epi, om, out, s, name);
-        return launch_wk<ConvStepX<UNIFORM>, false>(xl, p, zp, epi, om, out, s, name);
-    }
-
     int launch_conv_wk(const ConvX& xl, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, int x_unsigned, const ZeroPoints& zp, const Epilogue& epi, const OutMap& om, void* out,
                        hipStream_t s, const char* name)
     {
         if (M >= (1ll << 31))
             return HIPQ_ERR_UNSUPPORTED;
         const WkParams p = wk_params(w, nullptr, wsum, M, N, K, x_unsigned);
-        return xl.C % 64 == 0 ? launch_conv_steps<true>(xl, p, zp, epi, om, out, s, name) : launch_conv_steps<false>(xl, p, zp, epi, om, out, s, name);
+        if (om.ncx)
+            return launch_wk<ConvX, true>(xl, p, zp, epi, om, out, s, name);
+        return launch_wk<ConvX, false>(xl, p, zp, epi, om, out, s, name);
     }
 }

@@ -360,6 +360,7 @@ namespace hipq
                                                                               const float* __restrict__ factor, float* __restrict__ out, AttnView view, MatQuant mq, int32_t queries,
                                                                               int32_t keys_, int32_t row_blocks)
         {
+            touch_arguments<40 + sizeof(AttnView) + sizeof(MatQuant)>();
             const int keys = WHOLE ? CH * AKEYS : keys_;
             constexpr int QB = RB * 16;
             constexpr int ROWS = WAVES * 4;      // rows that one piece a thread covers

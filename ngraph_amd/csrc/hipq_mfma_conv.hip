@@ -66,6 +66,7 @@ namespace hipq
         xl.by_q = fast_div(xl.Q);
         xl.by_c = fast_div(xl.C);
         xl.by_s = fast_div(xl.S);
+        xl.set_steps();
         return xl;
     }
 

@@ -204,6 +204,7 @@ namespace hipq
                                                                        const float* __restrict__ bias, float* __restrict__ out, QuantOut qo, float* __restrict__ mean_out,
                                                                        float* __restrict__ var_out, int64_t rows, int32_t cols, float eps)
         {
+            touch_arguments<40 + sizeof(QuantOut) + 28>();
             // addend (may be null): the input is Add(in, addend), the sum rounded to f32 as the Add op rounds it;
             // qo.out (may be null): Quantize of the result beside it
             const int lane = threadIdx.x & 63;

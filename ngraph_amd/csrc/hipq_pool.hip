@@ -172,6 +172,7 @@ namespace hipq
     template <bool AVG, bool SIGNED, int VEC, int PARTS>
     __global__ __launch_bounds__(256) void pool8_nxc_kernel(Pool8Geom g, const uint32_t* __restrict__ in, uint32_t* __restrict__ out, uint32_t tasks)
     {
+        touch_arguments<sizeof(Pool8Geom) + 16>();
         typedef uint32_t vec_t __attribute__((ext_vector_type(VEC)));
         const uint32_t bias = (!AVG && SIGNED) ? 0x80808080u : 0u;
         // workgroups are dealt round-robin to the 8 XCDs, each with an L2 of its own: give every XCD a
