@@ -227,7 +227,7 @@ namespace hipq
             static_assert((NBUF - 1) * L + PL < 64 && (NBUF - 2) * L + RES + STORES < 64, "vmcnt is a 6-bit counter");
             extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [NBUF][x | w], residual tile, [3][64 WS] wsum, bias, scale
 
-            touch_arguments<sizeof(XL) + 72 + 2 * sizeof(FastDiv) + sizeof(ZeroPoints) + sizeof(Epilogue) + sizeof(RingMap)>();
+            touch_arguments<sizeof(XL) + 72 + 2 * sizeof(FastDiv) + sizeof(ZeroPoints) + sizeof(Epilogue) + sizeof(RingMap)>(); // (72: 56 of arguments, then the grid)
             const int tid = threadIdx.x;
             const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
             const int wm = wave / WAVES_N, wn = wave % WAVES_N;
