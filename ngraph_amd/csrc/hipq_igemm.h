@@ -177,6 +177,9 @@ namespace hipq
         // bytes of the data; `tap_step` and `row_step` bytes more where the channel or the column wraps; width of the
         // window with its dilation
         int32_t rest, cols, rows, step, tap_step, row_step, width;
+        // A 1 x 1 filter over every pixel in its place: the data is the [pixels][C] matrix itself.  (Rows and columns each: the
+        // padding above may be negative, and 28 x 29 pixels give 29 x 28 outputs, as many and others.)
+        bool every_pixel() const { return R * S == 1 && sh == 1 && sw == 1 && pbh == 0 && pbw == 0 && Q == W && PQ == static_cast<int64_t>(H) * W; }
         void set_steps()
         {
             const int32_t taps = 64 / C;

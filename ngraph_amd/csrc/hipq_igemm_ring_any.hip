@@ -71,8 +71,7 @@ namespace hipq
         if (cx.R * cx.S > 32 || M >= (1ll << 31) - 1024)
             return HIPQ_ERR_UNSUPPORTED;
         const RingMap map{ncx ? 1 : 0, static_cast<int32_t>(cx.PQ), cx.by_pq};
-        // a 1 x 1 filter over every pixel: the channels-last data is the [pixels][C] matrix itself
-        if (cx.R * cx.S == 1 && cx.sh == 1 && cx.sw == 1 && cx.pbh == 0 && cx.pbw == 0 && cx.PQ == static_cast<int64_t>(cx.H) * cx.W)
+        if (cx.every_pixel())
             return launch_any_of(RingRows{cx.x, cx.bytes, cx.C}, w, wsum, M, N, K, x_unsigned, zp, epi, map, out, s, name);
         RingConvAny xl;
         static_cast<RingWindow&>(xl) = ring_window(cx);

@@ -107,8 +107,7 @@ namespace hipq
             reinterpret_cast<const int32_t*>(static_cast<const uint8_t*>(packed) + align_up(static_cast<size_t>(g.K) * Kred, 256));
         OutMap om{out_ncx ? 1 : 0, N, xl.PQ};
         const int xu = g.data_t == HIPQ_U8 ? 1 : 0;
-        // a 1 x 1 filter over every pixel: the channels-last data is the [pixels][C] matrix itself
-        const bool pointwise = g.taps() == 1 && g.st[1] == 1 && g.st[2] == 1 && g.pb[1] == 0 && g.pb[2] == 0 && g.out[1] == g.in[1] && g.out[2] == g.in[2];
+        const bool pointwise = xl.every_pixel();
         const bool rows = !out_ncx && pointwise;
         if (!out_ncx && ring_preferred(M, N, Kred, true))
         {

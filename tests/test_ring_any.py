@@ -91,6 +91,32 @@ def test_convolutions_of_any_width(gpu_lib, monkeypatch, tile, i):
         assert np.array_equal(take(got), exp), (out_t, z)
 
 
+# as many output pixels as input pixels, and not the same ones: a row more and a column fewer, a column more and a row fewer
+@pytest.mark.parametrize("scheme", ["nxc", "ncx"])
+@pytest.mark.parametrize("image,above", [((9, 10), (1, -1)), ((10, 9), (-1, 1))])
+def test_one_tap_over_other_pixels(gpu_lib, monkeypatch, image, above, scheme):
+    print("ring any one tap", image, above, scheme, flush=True)
+    C, K = 48, 33
+    kw = dict(pad_below=(0, 0), pad_above=above)
+    layout = dict(data_layout=H.NXC, out_layout=H.NXC) if scheme == "nxc" else {}
+    give, take = (to_nxc, to_ncx) if scheme == "nxc" else (lambda x: x, lambda x: x)
+    monkeypatch.setenv("HIPQ_RING_TILE", "2")
+    dn, d = H.make_conv_desc(3, C, K, image, (1, 1), **kw), H.make_conv_desc(3, C, K, image, (1, 1), **layout, **kw)
+    assert np.prod(dn.out_shape()[2:]) == np.prod(image) and tuple(dn.out_shape()[2:]) != image
+    data = synth.uniform_int(9401, dn.data_shape(), 0, 255, np.uint8)
+    filt = synth.uniform_int(9402, dn.filter_shape(), -128, 127, np.int8)
+    args = (filt, 0.02, 131, 0.005, 0, 1.3, 5)
+    got = H.quantized_convolution(d, give(data), *args)
+    assert H.last_kernel() == "conv_mfma_ring_any_i8_16x16x64"
+    assert np.array_equal(take(got), O.quantized_convolution(dn, data, *args))
+    f = H.make_fused_desc(has_bias=True, scale_count=K)
+    bias = synth.uniform_int(9403, (K,), -20000, 20000, np.int32)
+    scale = synth.uniform_f32(9404, (K,), 0.5, 1.5) * np.float32(0.006 / np.sqrt(C))
+    got = H.quantized_convolution_fused(d, f, give(data), filt, bias, None, scale, None)
+    assert H.last_kernel() == "conv_mfma_ring_any_i8_16x16x64"
+    assert np.array_equal(take(got), O.quantized_convolution_fused(dn, f, data, filt, bias, None, scale, None))
+
+
 # more tiles than compute units, reductions of one, two and five slices
 @pytest.mark.parametrize("M,K,N", [(40000, 112, 405), (40000, 208, 403), (20001, 640, 270)])
 def test_any_width_more_tiles_than_compute_units(gpu_lib, monkeypatch, M, K, N):
