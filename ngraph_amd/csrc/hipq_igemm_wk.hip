@@ -64,8 +64,11 @@ namespace hipq
     // make a workgroup; U: reduction steps of 64 bytes a wavefront has in flight.
     // X_ON_A: the activations are MFMA source A, so that a lane's four accumulators are four consecutive
     // pixels of one channel (NCHW outputs); otherwise four consecutive channels of one pixel
+    // Short reductions over ragged rows are launches of many workgroups, which live on how many a compute unit holds: they
+    // are held to the registers of five wavefronts a SIMD (left to itself the compiler takes 97: four; 9320 x 71 x 1683 26.2 us,
+    // with five 22.4).
     template <class XL, int MT, int NT, int KW, int TW, int U, bool X_ON_A>
-    __global__ __launch_bounds__(KW * TW * 64) void igemm_wk_kernel(XL arg, WkParams p, ZeroPoints zp, Epilogue epi, OutMap om, void* __restrict__ out)
+    __global__ __launch_bounds__(KW * TW * 64, (std::is_same<XL, GemmRaggedX>::value && KW == 1 ? 5 : 0)) void igemm_wk_kernel(XL arg, WkParams p, ZeroPoints zp, Epilogue epi, OutMap om, void* __restrict__ out)
     {
         using Loader = typename std::conditional<std::is_same<XL, ConvX>::value, ConvStepX, XL>::type;
         Loader xl;
