@@ -433,6 +433,20 @@ def load():
     lib.hipq_pool_infer_output.argtypes = [C.POINTER(PoolDesc)]
     lib.hipq_pool.argtypes = [C.POINTER(PoolDesc), vp, vp, vp]
     lib.hipq_concat.argtypes = [i32, i32, C.POINTER(vp), C.POINTER(C.c_int64), i64, i64, vp, vp]
+    lib.hipq_slice.argtypes = [i32, vp, vp, i32] + [vp] * 5
+    lib.hipq_quantized_dot_bias_gelu_quantize.argtypes = [vp] * 9
+    lib.hipq_softmax_f32.argtypes = [vp, vp, i64, i64, i64, vp]
+    lib.hipq_softmax_scaled_f32.argtypes = [vp, vp, vp, i64, i64, i64, vp]
+    for n in ("hipq_erf_f32", "hipq_gelu_f32"):
+        getattr(lib, n).argtypes = [vp, vp, i64, vp]
+    lib.hipq_gelu_quantize_f32.argtypes = [vp, vp, vp, i64, vp]
+    for n in ("hipq_layer_norm_f32", "hipq_add_layer_norm_f32"):
+        getattr(lib, n).argtypes = [vp] * 6 + [i64, i64, C.c_double, vp]
+    lib.hipq_batch_matmul_f32.argtypes = [vp] * 3 + [i64] * 4 + [i32] * 2 + [vp]
+    lib.hipq_batch_matmul_view_f32.argtypes = [vp] * 5 + [i64] * 4 + [i32] * 2 + [vp]
+    lib.hipq_attention_f32.argtypes = [vp] * 7 + [i64] * 4 + [vp]
+    for n in ("hipq_last_error", "hipq_version", "hipq_last_kernel"):
+        getattr(lib, n).argtypes = []
     _lib = lib
     return lib
 
@@ -729,7 +743,6 @@ def slice_(x, lower, upper, strides=None):
     bx = _dev(x)
     out = DeviceBuffer(max(x.nbytes, 1))  # (a slice is never larger than its input)
     i64 = C.c_int64 * x.ndim
-    lib.hipq_slice.argtypes = [C.c_int32, C.c_void_p, C.c_void_p, C.c_int32] + [C.c_void_p] * 5
     check(lib.hipq_slice(x.dtype.itemsize, bx.ptr, out.ptr, x.ndim, i64(*x.shape), i64(*lower), i64(*upper), i64(*strides), None))
     check(lib.hipq_stream_sync(None))
     out_shape = [(u - l + s - 1) // s for l, u, s in zip(lower, upper, strides)]
@@ -778,7 +791,6 @@ def quantized_dot_bias_gelu_quantize(desc, fused, a, w, bias, scale, q_scale, q_
     bb = _dev(None if bias is None else np.asarray(bias, dtype=np.int32))
     bsc = _dev(np.asarray(scale, dtype=np.float32))
     q, keep, qt = _quant_out(int(desc.M * desc.N), q_scale, q_zp, quant_t, round_mode)
-    lib.hipq_quantized_dot_bias_gelu_quantize.argtypes = [C.c_void_p] * 9
     check(lib.hipq_quantized_dot_bias_gelu_quantize(C.byref(desc), C.byref(fused), ba.ptr, bw.ptr, _p(wsum), _p(bb), bsc.ptr, C.byref(q), None))
     check(lib.hipq_stream_sync(None))
     return keep[0].to_numpy(NP_OF[qt], (int(desc.M), int(desc.N)))
@@ -803,7 +815,6 @@ def softmax(x, axes=()):
     x = np.ascontiguousarray(x, dtype=np.float32)
     outer, axis, inner = _axes_run(x.shape, axes)
     src, dst = _dev(x), DeviceBuffer(max(x.nbytes, 4))
-    lib.hipq_softmax_f32.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_void_p]
     check(lib.hipq_softmax_f32(src.ptr, dst.ptr, outer, axis, inner, None))
     check(lib.hipq_stream_sync(None))
     return dst.to_numpy(np.float32, x.shape)
@@ -814,7 +825,6 @@ def _unary_f32(name, x):
     x = np.ascontiguousarray(x, dtype=np.float32)
     src, dst = _dev(x), DeviceBuffer(max(x.nbytes, 4))
     fn = getattr(lib, name)
-    fn.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p]
     check(fn(src.ptr, dst.ptr, x.size, None))
     check(lib.hipq_stream_sync(None))
     return dst.to_numpy(np.float32, x.shape)
@@ -840,7 +850,6 @@ def layer_norm(x, scale=None, bias=None, begin_norm_axis=1, epsilon=1e-5, keep_s
     bi = _dev(np.ascontiguousarray(bias, dtype=np.float32)) if bias is not None else None
     mean = DeviceBuffer(max(rows, 1) * 4) if keep_stats else None
     var = DeviceBuffer(max(rows, 1) * 4) if keep_stats else None
-    lib.hipq_layer_norm_f32.argtypes = [C.c_void_p] * 6 + [C.c_int64, C.c_int64, C.c_double, C.c_void_p]
     check(lib.hipq_layer_norm_f32(src.ptr, sc.ptr if sc else None, bi.ptr if bi else None, dst.ptr, mean.ptr if mean else None, var.ptr if var else None, rows, cols, float(epsilon), None))
     check(lib.hipq_stream_sync(None))
     stats_shape = x.shape[:n_axis]
@@ -860,7 +869,6 @@ def batch_matmul(a, b, transpose_a=False, transpose_b=False):
     assert (b.shape[2] if transpose_b else b.shape[1]) == K and b.shape[0] == batch
     da, db = _dev(a) if a.size else None, _dev(b) if b.size else None
     out = DeviceBuffer(max(batch * M * N * 4, 4))
-    lib.hipq_batch_matmul_f32.argtypes = [C.c_void_p] * 3 + [C.c_int64] * 4 + [C.c_int32] * 2 + [C.c_void_p]
     check(lib.hipq_batch_matmul_f32(da.ptr if da else None, db.ptr if db else None, out.ptr, batch, M, K, N, int(transpose_a), int(transpose_b), None))
     check(lib.hipq_stream_sync(None))
     r = out.to_numpy(np.float32, (batch, M, N))
@@ -882,7 +890,6 @@ def softmax_scaled(x, factor):
     lib = load()
     x = np.ascontiguousarray(x, dtype=np.float32)
     src, dst, fac = _dev(x), DeviceBuffer(max(x.nbytes, 4)), _dev(np.asarray(factor, dtype=np.float32))
-    lib.hipq_softmax_scaled_f32.argtypes = [C.c_void_p] * 3 + [C.c_int64] * 3 + [C.c_void_p]
     check(lib.hipq_softmax_scaled_f32(src.ptr, fac.ptr, dst.ptr, int(np.prod(x.shape[:-1], dtype=np.int64)), x.shape[-1], 1, None))
     check(lib.hipq_stream_sync(None))
     return dst.to_numpy(np.float32, x.shape)
@@ -899,7 +906,6 @@ def add_layer_norm(a, b, scale, bias, epsilon=1e-5, q_scale=None, q_zp=0, quant_
     q = keep = qt = None
     if q_scale is not None:
         q, keep, qt = _quant_out(a.size, q_scale, q_zp, quant_t, round_mode)
-    lib.hipq_add_layer_norm_f32.argtypes = [C.c_void_p] * 6 + [C.c_int64, C.c_int64, C.c_double, C.c_void_p]
     check(lib.hipq_add_layer_norm_f32(ba.ptr, bb.ptr if bb else None, sc.ptr, bi.ptr, dst.ptr, C.byref(q) if q else None, rows, cols, float(epsilon), None))
     check(lib.hipq_stream_sync(None))
     return dst.to_numpy(np.float32, a.shape), (keep[0].to_numpy(NP_OF[qt], a.shape) if q else None)
@@ -912,7 +918,6 @@ def gelu_quantize(x, q_scale, q_zp=0, quant_t="i8", round_mode=RNE, keep_f32=Tru
     src = _dev(x)
     dst = DeviceBuffer(max(x.nbytes, 4)) if keep_f32 else None
     q, keep, qt = _quant_out(x.size, q_scale, q_zp, quant_t, round_mode)
-    lib.hipq_gelu_quantize_f32.argtypes = [C.c_void_p] * 3 + [C.c_int64, C.c_void_p]
     check(lib.hipq_gelu_quantize_f32(src.ptr, dst.ptr if dst else None, C.byref(q), x.size, None))
     check(lib.hipq_stream_sync(None))
     return (dst.to_numpy(np.float32, x.shape) if dst else None), keep[0].to_numpy(NP_OF[qt], x.shape)
@@ -930,7 +935,6 @@ def attention(qkv, q_off, k_off, v_off, out_elems, view, batch, queries, keys, d
     if q_scale is not None:
         q, keep, qt = _quant_out(out_elems, q_scale, q_zp, quant_t, RNE)
         check(lib.hipq_fill_bytes(keep[0].ptr, 0, out_elems, None))
-    lib.hipq_attention_f32.argtypes = [C.c_void_p] * 7 + [C.c_int64] * 4 + [C.c_void_p]
     check(lib.hipq_attention_f32(buf.ptr + 4 * q_off, buf.ptr + 4 * k_off, buf.ptr + 4 * v_off, fac.ptr if fac else None, dst.ptr if dst else None, C.byref(view),
                                  C.byref(q) if q else None, batch, queries, keys, depth, None))
     check(lib.hipq_stream_sync(None))
@@ -948,7 +952,6 @@ def batch_matmul_view(a, a_off, b, b_off, out_elems, out_off, view, batch, M, K,
     if q_scale is not None:
         q, keep, qt = _quant_out(out_elems, q_scale, q_zp, quant_t, RNE)
         check(lib.hipq_fill_bytes(keep[0].ptr, 0, out_elems, None))
-    lib.hipq_batch_matmul_view_f32.argtypes = [C.c_void_p] * 5 + [C.c_int64] * 4 + [C.c_int32] * 2 + [C.c_void_p]
     check(lib.hipq_batch_matmul_view_f32(ba.ptr + 4 * a_off, bb.ptr + 4 * b_off, (dst.ptr + 4 * out_off) if dst else None, C.byref(view), C.byref(q) if q else None, batch, M, K, N,
                                          1 if transpose_a else 0, 1 if transpose_b else 0, None))
     check(lib.hipq_stream_sync(None))

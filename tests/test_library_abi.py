@@ -25,6 +25,25 @@ def test_exports_match_header():
     assert sorted(H.EXPORTS) == names
 
 
+def test_loaded_functions_know_their_arguments():
+    """ctypes passes a Python int as 32 bits where no type is declared: half a device pointer"""
+    text = re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", "hipq.h")).read(), flags=re.S)
+    kinds = {"int": C.c_int, "int32_t": C.c_int32, "uint32_t": C.c_uint32, "int64_t": C.c_int64, "size_t": C.c_size_t, "double": C.c_double}
+    lib = H.load()
+    seen = 0
+    for name, params in re.findall(r"HIPQ_API[\w\s\*]+?\b(hipq_\w+)\s*\(([^)]*)\)", text):
+        want = [p.strip() for p in params.split(",") if p.strip() != "void"]
+        got = getattr(lib, name).argtypes
+        assert got is not None and len(got) == len(want), name
+        for p, t in zip(want, got):
+            if "*" in p:
+                assert C.sizeof(t) == C.sizeof(C.c_void_p) and t not in (C.c_int64, C.c_size_t), (name, p)
+            else:
+                assert t is kinds[p.split()[0]], (name, p)
+        seen += 1
+    assert seen == len(_declared())
+
+
 def test_product_library_exports_only_the_declared_abi():
     """libhipq.so exports what include/hipq.h declares (plus hipq_last_kernel, the tests' window on the
     dispatcher) and no development or measurement symbol; those live in libhipq_probe.so"""
