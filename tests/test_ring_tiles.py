@@ -138,13 +138,46 @@ def test_more_tiles_than_compute_units(gpu_lib, monkeypatch, M, K, N):
             assert np.array_equal(H.quantized_dot_bias(d, f, a, w, bias, scale).view(np.uint8), exp.view(np.uint8)), (out_t, tile)
             assert H.last_kernel() == "dot_mfma_ring_i8_16x16x64"
             monkeypatch.delenv("HIPQ_RING_TILE")
-    dc = H.make_conv_desc(1, K, N, (M, 1), (1, 1), out_t="u8", data_layout=H.NXC, out_layout=H.NXC)
+    rows = next(r for r in range(int(M**0.5), 0, -1) if M % r == 0)  # (an image of M x 1 would be too tall for the tile kernels)
+    image = (rows, M // rows)
+    dc = H.make_conv_desc(1, K, N, image, (1, 1), out_t="u8", data_layout=H.NXC, out_layout=H.NXC)
     f = H.make_fused_desc(has_bias=True, has_sum=True, sum_t="i8", scale_count=N)
-    res = synth.uniform_int(9201, (1, M, 1, N), -128, 127, np.int8)
+    res = synth.uniform_int(9201, (1, *image, N), -128, 127, np.int8)
     monkeypatch.setenv("HIPQ_NO_RING", "1")
-    args = (dc, f, a.reshape(1, M, 1, K), w.reshape(N, K, 1, 1), bias, res, scale, 0.41)
+    args = (dc, f, a.reshape(1, *image, K), w.reshape(N, K, 1, 1), bias, res, scale, 0.41)
     exp = H.quantized_convolution_fused(*args)
+    assert "ring" not in H.last_kernel()
     monkeypatch.delenv("HIPQ_NO_RING")
     for tile in range(4):
         monkeypatch.setenv("HIPQ_RING_TILE", str(tile))
         assert np.array_equal(H.quantized_convolution_fused(*args), exp), ("residual", tile)
+        assert H.last_kernel() == "conv_mfma_ring_i8_16x16x64"
+
+
+# windows over more tiles than compute units: the loader's cursor and the queue of chunks in the padding cross from a tile to the
+# next, under the last slice of one, between and under the first (reductions of 2, 3 and 5 slices, rings of 2 to 8)
+@pytest.mark.parametrize("window", [(2, 1), (3, 1), (5, 1)])
+@pytest.mark.parametrize("kind,C,K,name", [("whole", 128, 528, "conv_mfma_ring_i8_16x16x64"), ("nxc", 112, 531, "conv_mfma_ring_any_i8_16x16x64"), ("ncx", 112, 531, "conv_mfma_ring_any_i8_16x16x64")])
+def test_windows_over_more_tiles_than_compute_units(gpu_lib, monkeypatch, kind, C, K, name, window):
+    print("ring window rounds", kind, window, flush=True)
+    layout = dict(data_layout=H.NXC, out_layout=H.NCX if kind == "ncx" else H.NXC)
+    kw = dict(pad_below=(window[0] // 2, 0), pad_above=((window[0] - 1) // 2, 0), **layout)
+    data = synth.uniform_int(9501, (17, 37, 27, C), 0, 255, np.uint8)
+    filt = synth.uniform_int(9502, (K, C) + window, -128, 127, np.int8)
+    bias = synth.uniform_int(9503, (K,), -20000, 20000, np.int32)
+    scale = synth.uniform_f32(9504, (K,), 0.5, 1.5) * np.float32(0.006 / np.sqrt(C * window[0]))
+    interp = (H.quantized_convolution, (H.make_conv_desc(17, C, K, (37, 27), window, out_t="i8", **kw), data, filt, 0.02, 131, 0.005, 0, 1.3, 5))
+    d = H.make_conv_desc(17, C, K, (37, 27), window, out_t="u8", **kw)
+    res = synth.uniform_int(9505, d.out_shape(), -128, 127, np.int8)
+    fused = [(H.quantized_convolution_fused, (d, H.make_fused_desc(has_bias=True, has_sum=r is not None, sum_t="i8", scale_count=K), data, filt, bias, r, scale, None if r is None else 0.41)) for r in (None, res)]
+    tiles = (4, 6, 4) if kind == "whole" else (4, 4, 4)
+    for (call, args), count in zip([interp] + fused, tiles):
+        monkeypatch.setenv("HIPQ_NO_RING", "1")
+        exp = call(*args)
+        assert "ring" not in H.last_kernel() and len(np.unique(exp)) > 50
+        monkeypatch.delenv("HIPQ_NO_RING")
+        for tile in range(count):
+            monkeypatch.setenv("HIPQ_RING_TILE", str(tile))
+            assert np.array_equal(call(*args), exp), tile
+            assert H.last_kernel() == name
+            monkeypatch.delenv("HIPQ_RING_TILE")
