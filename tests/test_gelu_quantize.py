@@ -40,3 +40,31 @@ def test_gelu_quantize_bytes(gpu_lib, scale, quant_t, zp):
     bad = np.nonzero(got != exp)[0]
     assert bad.size == 0, (x[bad[:5]], got[bad[:5]], exp[bad[:5]])
     assert np.array_equal(H.gelu_quantize(x, s, zp, quant_t)[1], exp)
+
+
+# no quotient is sure (scales beyond 2^30, below 2^-30 and below the error of the short form), a negative scale, what is no number
+@pytest.mark.parametrize("quant_t,zp", [("i8", -77), ("u8", 131)])
+@pytest.mark.parametrize("scale", [1e-7, 1e-10, 2e9, -0.05, np.inf, np.nan])
+def test_gelu_quantize_ends(gpu_lib, scale, quant_t, zp):
+    print("gelu quantize ends", scale, quant_t, flush=True)
+    s = np.float32(scale)
+    wide = min(abs(scale), 1e30) if scale == scale else 1.0
+    ends = np.array([np.nan, np.inf, -np.inf, 0.0, -0.0, 1e-40, -1e-40, 3e38, -3e38, 1.0, -1.0, 2e9], np.float32)
+    x = np.concatenate([np.repeat(ends, 4), np.tile(ends, 5), synth.uniform_f32(9311, (1 << 18,), -8.0, 8.0), synth.uniform_f32(9312, (1 << 18,), -300 * wide, 300 * wide)])
+    assert x.size % 4 == 0
+    exp = H.quantize(H.gelu(x), s, zp, quant_t)
+    got = H.gelu_quantize(x, s, zp, quant_t, keep_f32=False)[1]
+    bad = np.nonzero(got != exp)[0]
+    assert bad.size == 0, (x[bad[:5]], got[bad[:5]], exp[bad[:5]])
+
+
+def test_gelu_quantize_through_the_floats(gpu_lib):
+    """every 127th float, of either sign, infinities and what is no number among them"""
+    print("gelu quantize floats", flush=True)
+    for first in range(0, 1 << 32, 1 << 30):
+        x = np.arange(first, first + (1 << 30), 127, dtype=np.int64).astype(np.uint32)
+        x = x[: x.size // 4 * 4].view(np.float32)
+        for scale in (0.0175, 3e-6):
+            exp = H.quantize(H.gelu(x), np.float32(scale), 3, "i8")
+            bad = np.nonzero(H.gelu_quantize(x, np.float32(scale), 3, "i8", keep_f32=False)[1] != exp)[0]
+            assert bad.size == 0, (scale, x[bad[:5]])
