@@ -2180,7 +2180,7 @@ namespace hipq
     }
 
     // tiles that fit the chip (hipq_igemm_ring.hip); HIPQ_ERR_UNSUPPORTED (nothing launched, no error text) when the call is not of their kind
-    bool ring_preferred(int64_t M, int64_t N, int64_t K, bool conv);
+    bool ring_preferred(int64_t M, int64_t N, int64_t K, const Epilogue& epi, bool window);
     int launch_rows_ring(const void* a, int a_unsigned, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi, void* out, hipStream_t s,
                          const char* name);
     bool ring_any_preferred(int64_t M, int64_t N, int64_t K, int64_t C, const Epilogue& epi, bool window, bool ncx);
@@ -2197,6 +2197,7 @@ namespace hipq
     // steps: of 64 bytes of the reduction; dma, alone: what else would take the call (kernels that load straight into
     // LDS; one kernel and nothing behind it)
     bool wk_preferred(int64_t M, int64_t N, int64_t steps, bool dma, bool alone = true);
+    bool wk_fits(int64_t M, int64_t N, int64_t steps, bool dma, int64_t long_limit); // the same but for the switches
     bool ragged_preferred(int64_t M, int64_t N, int64_t row_bytes, int64_t steps, bool dma, bool pointwise);
     int launch_rows_wk(const void* a, bool a_unsigned, const int8_t* w_nk, const void* w_frag, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi,
                        void* out, hipStream_t s, const char* name);

@@ -115,48 +115,79 @@ namespace hipq
         }
     }
 
-    // Below a line in 32 x 32 tiles x 64-byte steps the kernels that split a reduction inside a workgroup have less
-    // to wait for (us, those first: 600 x 768 x 768 product 6.1 and 5.7, 400 x 2048 x 256 6.1 and 8.0, 2352 x 2304 -> 256
-    // window 17.2 and 9.6, 784 x 1152 -> 128 5.9 and 6.9; 985 x 4096 x 768 27.6 and 12.7).  Short reductions whose
-    // 64 x 64 tiles leave more than 0.6 of the compute units idle stay there as well (1500 x 1024 x 256, 96 tiles: 7.3, 6.2;
-    // 400 x 1024 x 768, 84: 7.1, 6.1).
-    bool ring_preferred(int64_t M, int64_t N, int64_t K, bool conv)
+    // The lines against the kernels that split a reduction inside a workgroup: from how many 64-byte steps on the tiles here are
+    // ahead, by 32 x 32 tiles a compute unit (from 5/8, 1, 2, 3, 4, 6 and 9 on).  Few tiles leave units idle here and few
+    // steps the fill of the ring exposed, where those kernels wait for less; many of both they pay for reading their operands
+    // more times.  At most 32 columns count half, since the tiles here are 64 wide and more.  Read off 34 400 drawn sizes that
+    // both families take, looped, three in four between 1 500 and 30 000 tiles x steps: the side taken is 0.6 % behind the better
+    // one on average (lines linear in tiles x steps, fitted to fewer and wider sizes, before: 1.9 %; sizes that take more than
+    // 1.1 times as long here as there 1 600, now 288; the other way round 921, now 420).  The first columns of kLineRows and
+    // kLineWindow are a little early for a loop: behind other layers these tiles, which load a ring ahead, gain (ResNet-50 of
+    // five images 388 us so, 405 with 20 for rows and 256 -> 256 channels 3 x 3 on 14 x 14 pixels on the other kernels).  us,
+    // those kernels and these, of sizes that the lines before gave to the wrong side: 1012 x 464 x 464 with Gelu 5.0 and 8.2,
+    // 1329 x 2320 x 192 8.0 and 12.7; 3 x 3 over 384 channels on 4800 pixels -> 16, INTERPRETER policy, 10.2 and 15.5;
+    // 368 x 3040 x 704 8.1 and 10.8; 1 x 1 over 32 channels on 3 x 74 x 59 pixels -> 226, [image][channel][pixel], 16.5 and
+    // 9.1.  Of the right one: 985 x 4096 x 768 27.6 and 12.7.  Gelu and Quantize are an epilogue of 4 us and more that nothing
+    // overlaps; in windows of the INTERPRETER policy taps in a padding become the zero point in LDS, a third of a slice more.
+    struct RingLine
     {
-        const int64_t steps = (K + 63) / 64, units = device_compute_units();
-        const bool switched = library_switched();
+        int16_t least[7];
+        bool reached(int64_t M, int64_t N, int64_t steps, bool halve) const
+        {
+            const int64_t tiles = ((M + 31) / 32) * ((N + 31) / 32) / (halve ? 2 : 1), units = device_compute_units(), per = tiles / units;
+            if (tiles * 8 < units * 5)
+                return false;
+            return steps >= least[per < 4 ? per : per < 6 ? 4 : per < 9 ? 5 : 6];
+        }
+    };
+    constexpr int16_t kNever = 0x7fff; // (a reduction is shorter)
+    constexpr RingLine kLineRows = {{kNever, 16, 8, 4, 4, 3, 1}}, kLineGelu = {{kNever, kNever, 28, 5, 5, 5, 5}}, kLineWindow = {{32, 16, 8, 5, 5, 3, 1}},
+                       kLineNarrowWindow = {{kNever, 32, 32, 32, 32, 32, 32}}, kLineFilled = {{kNever, 32, 12, 8, 8, 5, 5}};
+    constexpr RingLine kLineAnyRows = {{kNever, 20, 10, 5, 4, 3, 2}}, kLineAnyWindow = {{kNever, 48, 16, 12, 5, 5, 3}}, kLineAnyFilled = {{kNever, kNever, 96, 16, 12, 6, 4}};
+    constexpr RingLine kLineNcxRows = {{kNever, 5, 3, 2, 1, 1, 1}}, kLineNcxWindow = {{kNever, 20, 12, 3, 3, 1, 1}}, kLineNcxFilled = {{kNever, kNever, 20, 16, 12, 5, 3}};
+
+    // Calls that the kernels for small products do not take are better off here than on the other tile kernels (5 250 of those
+    // sizes: 0.66 of the time, 76 of them more than 1.03 times as long, the worst 1.3: 3981 x 288 x 2400 12.2 us there, 15.9 here).
+    bool ring_preferred(int64_t M, int64_t N, int64_t K, const Epilogue& epi, bool window)
+    {
+        const int64_t steps = (K + 63) / 64;
+        const bool switched = library_switched(), narrow = N <= 32;
         if (switched && !ring_enabled())
             return false;
         if (switched && getenv("HIPQ_RING_TILE") != nullptr)
             return true;
-        const int64_t small = ((M + 31) / 32) * ((N + 31) / 32) * steps, tiles = ((M + 63) / 64) * ((N + 63) / 64);
-        return small > (conv ? 1400 + 120 * steps : 1800 + 200 * steps) && (tiles * 10 >= units * 4 || steps >= 32);
+        if (!wk_fits(M, N, steps, true, 0))
+            return true;
+        if (window && epi.mode == EPI_FUSED)
+            return (narrow ? kLineNarrowWindow : kLineWindow).reached(M, N, steps, false);
+        return (epi.post_scale ? kLineGelu : window ? kLineFilled : kLineRows).reached(M, N, steps, narrow);
     }
 
-    // The tiles for any width (hipq_igemm_ring_any.hip).  What the kernels for whole 16-byte columns take they do faster, or
-    // have refused above.  The lines in 32 x 32 tiles x 64-byte steps are fitted to 1 800 drawn sizes; of 700 more they
-    // gave 102 to these tiles, which took 0.67 of the time before on average, eight of them 3 to 11 % longer (us, before and here:
-    // 2044 x 1379 x 1017 product 33.2 and 12.7, 2836 x 727 x 3157 f32 50.8 and 26.4, 289 x 2607 x 695 11.7 and 12.9; 3 x 3 windows,
-    // 80 -> 412 channels on 30 x 19 x 7 pixels 12.3 and 8.3, [image][channel][pixel] 335 -> 460 on 43 x 59 32.0 and 20.3).  Below them
-    // the kernels that split a reduction inside a workgroup wait for less: 2 x 12 x 36 of 16 -> 504 5.3 and 8.1.
+    // The tiles for any width (hipq_igemm_ring_any.hip).  Rows of whole 16-byte columns are taken, or refused, above, and so
+    // are windows over multiples of 128 channels; windows over 64, 192, 320 ... channels into whole columns stay on the kernel that
+    // loads 64-byte slices.  (Not because that is faster in a loop: 1 050 such sizes took 0.70 of its time here, the worst 1.54.
+    // Inside a pass, where the ring kernels lose some of that, it has not been measured.)
+    // us, before and here: 2044 x 1379 x 1017 product 33.2 and 12.7, 2836 x 727 x 3157 f32 50.8 and 26.4, 2304 x 1344 x 1001 without
+    // a bias 23.7 and 11.4; 3 x 3 windows, 80 -> 412 channels on 30 x 19 x 7 pixels 12.3 and 8.3, 240 -> 704 on 6 x 25 x 25 of the
+    // INTERPRETER policy 32.8 and 20.3, [image][channel][pixel] 335 -> 460 on 43 x 59 32.0 and 20.3.
     bool ring_any_preferred(int64_t M, int64_t N, int64_t K, int64_t C, const Epilogue& epi, bool window, bool ncx)
     {
         const int64_t steps = (K + 63) / 64;
-        const bool switched = library_switched(), q8 = epi.out_t == HIPQ_U8 || epi.out_t == HIPQ_I8;
+        const bool switched = library_switched(), q8 = epi.out_t == HIPQ_U8 || epi.out_t == HIPQ_I8, narrow = N <= 32;
         if (switched && !ring_enabled())
             return false;
         if (switched && getenv("HIPQ_RING_TILE") != nullptr)
             return true;
-        const bool whole = N % 16 == 0 && !ncx && (q8 || epi.mode == EPI_FUSED);
-        if (whole && (!window || C % 64 == 0))
+        if (N % 16 == 0 && !ncx && (q8 || epi.mode == EPI_FUSED) && (!window || C % 64 == 0))
             return false;
-        // Long reductions that stay where they were, though these tiles would be ahead, because their route is fixed by the tests
-        // of the kernels that have them: products without a bias (2304 x 1344 x 1001 23.7 us there, 11.4 here) and windows
-        // of the INTERPRETER policy over whole columns (240 -> 704 channels 3 x 3 on 6 x 25 x 25 32.8, 20.3).
-        if (!ncx && q8 && (window ? whole && epi.mode == EPI_INTERP && steps > 32 : !whole && epi.mode == EPI_FUSED && epi.bias == nullptr && steps >= 20))
-            return false;
-        const int64_t small = ((M + 31) / 32) * ((N + 31) / 32) * steps;
-        const bool filled = window && epi.mode == EPI_INTERP; // (taps in a padding become the zero point in LDS: a third of a slice more)
-        return small > (ncx ? (filled ? 4800 + 400 * steps : 4000 + 260 * steps) : window ? (filled ? 3200 + 800 * steps : 4800 + 200 * steps) : 4800 + 100 * steps);
+        const bool interp = epi.mode == EPI_INTERP, filled = window && interp;
+        // More tiles than the kernels for small products take: here, but for channels-last outputs of at most 32 columns and few
+        // steps, which the other tile kernels have tiles of 512 rows for (16 -> 36 channels 1 x 1 on 79 x 112 x 26 pixels,
+        // INTERPRETER policy, 12.2 us there, 17.3 here; 217 such sizes take 1.26 times as long here on average, 2 100 others 0.55).
+        if (!wk_fits(M, N, steps, false, 9))
+            return ncx || !narrow || steps > (filled ? 7 : interp ? 2 : 1);
+        const RingLine& line = ncx ? (filled ? kLineNcxFilled : window ? kLineNcxWindow : kLineNcxRows) : (filled ? kLineAnyFilled : window ? kLineAnyWindow : kLineAnyRows);
+        return line.reached(M, N, steps, narrow);
     }
 
     int launch_rows_ring(const void* a, int a_unsigned, const int8_t* w, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi, void* out, hipStream_t s,

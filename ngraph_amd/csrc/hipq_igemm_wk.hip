@@ -433,7 +433,7 @@ namespace hipq
         return true;
     }
     // long_limit: tiles a compute unit on long reductions
-    static bool wk_fits(int64_t M, int64_t N, int64_t steps, bool dma, int64_t long_limit)
+    bool wk_fits(int64_t M, int64_t N, int64_t steps, bool dma, int64_t long_limit)
     {
         // (the entry point that allocates nothing keeps sixteen: the tile kernels may want more scratch than it has)
         const bool few = N <= 64 || M <= 512 || steps <= 20 || !workspace_holds(SIZE_MAX);

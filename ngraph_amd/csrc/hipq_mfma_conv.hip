@@ -109,7 +109,7 @@ namespace hipq
         const int xu = g.data_t == HIPQ_U8 ? 1 : 0;
         const bool pointwise = xl.every_pixel();
         const bool rows = !out_ncx && pointwise;
-        if (!out_ncx && ring_preferred(M, N, Kred, true))
+        if (!out_ncx && ring_preferred(M, N, Kred, epi, !pointwise))
         {
             const char* const name = "conv_mfma_ring_i8_16x16x64";
             const int rc = rows ? launch_rows_ring(data_nxc, xu, w, wsum, M, N, Kred, zp, epi, out, s, name) : launch_conv_ring(xl, w, wsum, M, N, Kred, xu, zp, epi, out, s, name);

@@ -1024,7 +1024,7 @@ namespace hipq
     int launch_rows_gelu_q8(const void* a, bool a_unsigned, const int8_t* w_nk, const void* w_frag, const int32_t* wsum, int64_t M, int32_t N, int32_t K, const ZeroPoints& zp, const Epilogue& epi,
                             void* out, hipStream_t s)
     {
-        if (M > 256 && ring_preferred(M, N, K, false))
+        if (M > 256 && ring_preferred(M, N, K, epi, false))
         {
             const int rc = launch_rows_ring(a, a_unsigned ? 1 : 0, w_nk, wsum, M, N, K, zp, epi, out, s, "dot_gelu_q8_mfma_ring_i8_16x16x64");
             if (rc != HIPQ_ERR_UNSUPPORTED)
@@ -1089,7 +1089,7 @@ namespace hipq
             return launch_rows_wk_ragged(a, static_cast<int32_t>(a_row), d.a_t == HIPQ_U8, static_cast<const int8_t*>(w_nk), w_frag, wsum, d.M, static_cast<int32_t>(d.N), static_cast<int32_t>(d.K), zp,
                                          epi, out, s, "dot_mfma_wk_ragged_i8_16x16x64");
         auto ring = [&]() {
-            return ring_preferred(d.M, d.N, d.K, false) ? launch_rows_ring(a, d.a_t == HIPQ_U8 ? 1 : 0, static_cast<const int8_t*>(w_nk), wsum, d.M, static_cast<int32_t>(d.N), static_cast<int32_t>(d.K),
+            return ring_preferred(d.M, d.N, d.K, epi, false) ? launch_rows_ring(a, d.a_t == HIPQ_U8 ? 1 : 0, static_cast<const int8_t*>(w_nk), wsum, d.M, static_cast<int32_t>(d.N), static_cast<int32_t>(d.K),
                                                                          zp, epi, out, s, "dot_mfma_ring_i8_16x16x64")
                                                         : HIPQ_ERR_UNSUPPORTED;
         };

@@ -117,6 +117,57 @@ def test_one_tap_over_other_pixels(gpu_lib, monkeypatch, image, above, scheme):
     assert np.array_equal(take(got), O.quantized_convolution_fused(dn, f, data, filt, bias, None, scale, None))
 
 
+# either side of a line against the kernels that split a reduction in a workgroup: whole columns, any width, with a bias and
+# without (the line does not ask), at most 32 columns (which count half), more tiles than those kernels take.  On 256
+# compute units
+@pytest.mark.parametrize("M,K,N,kernel", [
+    (2304, 1344, 1001, "ring_any"), (2305, 1344, 1001, "ring_any"), (512, 1344, 4609, "ring_any"), (961, 640, 513, "ring_any"), (961, 576, 513, "wk"), (12800, 1280, 31, "wk"), (6400, 1280, 33, "ring_any"),
+    (800, 1024, 640, "ring"), (800, 960, 640, "wk"), (12800, 2048, 32, "wk"), (6400, 2048, 48, "ring"), (1056, 256, 1024, "ring"), (736, 256, 1024, "wk")])
+def test_lines_for_products(gpu_lib, M, K, N, kernel):
+    print("ring line", M, K, N, flush=True)
+    a, w, bias, scale = operands(M, K, N, "u8")
+    d = H.make_dot_desc(M, K, N, out_t="i8", b_layout=H.B_NK)
+    for b in (bias, None):
+        got = H.quantized_dot_bias(d, H.make_fused_desc(has_bias=b is not None, scale_count=N), a, w, b, scale)
+        assert H.last_kernel() == {"wk": "dot_mfma_wk_i8_16x16x64", "ring": "dot_mfma_ring_i8_16x16x64", "ring_any": "dot_mfma_ring_any_i8_16x16x64"}[kernel]
+        assert np.array_equal(got, dot_bias_closed_form(a, w, b, scale, "i8", False)), b is None
+
+
+@pytest.mark.parametrize("M,K,N,kernel", [(1012, 464, 464, "wk"), (1329, 2320, 192, "wk"), (1024, 1728, 512, "wk"), (1024, 1792, 512, "ring"), (2048, 512, 512, "ring")])
+def test_lines_for_gelu(gpu_lib, M, K, N, kernel):
+    print("ring line gelu", M, K, N, flush=True)
+    a, w, bias, scale = operands(M, K, N, "i8")
+    d = H.make_dot_desc(M, K, N, a_t="i8", out_t="f32", b_layout=H.B_NK)
+    got = H.quantized_dot_bias_gelu_quantize(d, H.make_fused_desc(has_bias=True, scale_count=N), a, w, bias, scale, 0.03, 0, "i8")
+    assert H.last_kernel() == {"wk": "dot_gelu_q8_wk_i8_16x16x64", "ring": "dot_gelu_q8_mfma_ring_i8_16x16x64"}[kernel]
+    assert np.array_equal(got, H.gelu_quantize(dot_bias_closed_form(a, w, bias, scale, "f32", False), 0.03, 0, "i8")[1])
+
+
+# the same for convolutions: pictures, channels, image, outputs, window, scheme, fused policy or the INTERPRETER's, kernel
+@pytest.mark.parametrize("case", [
+    (6, 240, (25, 25), 704, 3, "nxc", False, "ring_any"), (1, 240, (25, 25), 176, 3, "nxc", False, "wk"), (4, 384, (40, 30), 16, 3, "nxc", False, "wk"), (4, 384, (40, 30), 112, 3, "nxc", False, "ring"),
+    (3, 128, (28, 28), 128, 3, "nxc", True, "ring"), (1, 128, (28, 28), 128, 3, "nxc", True, "wk"), (5, 256, (14, 14), 256, 3, "nxc", True, "ring"),
+    (2, 256, (14, 14), 256, 3, "nxc", True, "wk"), (6, 80, (28, 28), 200, 3, "nxc", True, "ring_any"), (2, 80, (28, 28), 200, 3, "nxc", True, "wk"),
+    (10, 1728, (8, 8), 640, 1, "ncx", True, "ring_any"), (1, 256, (8, 8), 640, 1, "ncx", True, "wk"), (4, 80, (28, 28), 200, 3, "ncx", True, "ring_any"), (1, 80, (28, 28), 200, 3, "ncx", True, "wk"),
+    (40, 48, (64, 64), 30, 3, "nxc", False, "i8_32x32x32"), (40, 80, (64, 64), 30, 3, "nxc", False, "ring_any")])
+def test_lines_for_convolutions(gpu_lib, monkeypatch, case):
+    n, C, image, K, f, scheme, fused, kernel = case
+    print("ring line conv", case, flush=True)
+    layout = dict(data_layout=H.NXC, out_layout=H.NXC if scheme == "nxc" else H.NCX)
+    d = H.make_conv_desc(n, C, K, image, (f, f), pad_below=(f // 2,) * 2, pad_above=(f // 2,) * 2, out_t="i8", **layout)
+    data = synth.uniform_int(9601, d.data_shape(), 0, 255, np.uint8)
+    filt = synth.uniform_int(9602, d.filter_shape(), -128, 127, np.int8)
+    bias = synth.uniform_int(9603, (K,), -20000, 20000, np.int32)
+    scale = synth.uniform_f32(9604, (K,), 0.5, 1.5) * np.float32(0.006 / np.sqrt(C * f * f))
+    fd = H.make_fused_desc(has_bias=True, scale_count=K)
+    call = lambda: H.quantized_convolution_fused(d, fd, data, filt, bias, None, scale, None) if fused else H.quantized_convolution(d, data, filt, 0.02, 131, 0.005, 0, 2.0, 5)
+    got = call()
+    assert H.last_kernel() == "conv_mfma_%s" % (kernel if kernel.startswith("i8") else kernel + "_i8_16x16x64")
+    for switch in ("HIPQ_NO_RING", "HIPQ_NO_WK", "HIPQ_NO_BAND"):
+        monkeypatch.setenv(switch, "1")
+    assert np.array_equal(call(), got) and H.last_kernel() == "conv_mfma_i8_32x32x32" and len(np.unique(got)) > 50
+
+
 # more tiles than compute units, reductions of one, two and five slices
 @pytest.mark.parametrize("M,K,N", [(40000, 112, 405), (40000, 208, 403), (20001, 640, 270)])
 def test_any_width_more_tiles_than_compute_units(gpu_lib, monkeypatch, M, K, N):

@@ -52,8 +52,9 @@ SHAPES = (
 
 @pytest.mark.parametrize("pictures,N,steps", SHAPES)
 @pytest.mark.parametrize("ragged", [False, True])
-def test_every_tile_shape(gpu_lib, pictures, N, steps, ragged):
+def test_every_tile_shape(gpu_lib, monkeypatch, pictures, N, steps, ragged):
     """products and 1 x 1 convolutions of these sizes, rows in whole steps and rows that are not, against the closed form"""
+    monkeypatch.setenv("HIPQ_NO_RING", "1")  # (some of them lie beyond the ring tiles' lines)
     K, M = 64 * steps - (4 if ragged else 0), int(np.prod(pictures))
     print("small product", M, K, N, flush=True)
     a = synth.uniform_int(71, (M, K), 0, 255, np.uint8)
@@ -80,8 +81,9 @@ def test_every_tile_shape(gpu_lib, pictures, N, steps, ragged):
 # (columns that are no multiple of 16; the last number of rows that the rule gives these kernels, and one more; as many
 # tiles with a step less, of few rows, of few columns)
 @pytest.mark.parametrize("M,K,N,small", [(2304, 1344, 1001, True), (2305, 1344, 1001, False), (2305, 1280, 1001, True), (512, 1344, 4609, True), (36900, 1344, 63, True)])
-def test_long_reductions_over_many_tiles(gpu_lib, M, K, N, small):
+def test_long_reductions_over_many_tiles(gpu_lib, monkeypatch, M, K, N, small):
     print("long reduction", M, K, N, flush=True)
+    monkeypatch.setenv("HIPQ_NO_RING", "1")  # (the line between the two families that the ring tiles stand before)
     a = synth.uniform_int(81, (M, K), 0, 255, np.uint8)
     w = synth.uniform_int(82, (N, K), -128, 127, np.int8)
     scale = synth.uniform_f32(83, (N,), 0.5, 1.5) * np.float32(0.003 / np.sqrt(K))

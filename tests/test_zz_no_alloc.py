@@ -84,9 +84,10 @@ def test_noalloc_split_reduction_two_calls(gpu_lib, monkeypatch):
 
 
 @pytest.mark.gpu
-def test_noalloc_takes_a_long_reduction_without_partial_sums(gpu_lib):
+def test_noalloc_takes_a_long_reduction_without_partial_sums(gpu_lib, monkeypatch):
     """180 tiles whose partial sums would not fit the array: the kernels that need none, the regular entry point's bytes"""
     say("noalloc long reduction")
+    monkeypatch.setenv("HIPQ_NO_RING", "1")  # (the ring tiles take the call from both entry points: below)
     d = H.make_conv_desc(6, 240, 704, (25, 25), (3, 3), pad_below=(1, 1), pad_above=(1, 1), data_layout=H.NXC, out_layout=H.NXC)
     data = synth.uniform_int(3600, d.data_shape(), 0, 255, np.uint8)
     filt = synth.uniform_int(3601, d.filter_shape(), -127, 127, np.int8)
@@ -96,6 +97,10 @@ def test_noalloc_takes_a_long_reduction_without_partial_sums(gpu_lib):
     regular = H.quantized_convolution(*args)
     assert H.last_kernel() == "conv_mfma_i8_32x32x32"
     assert np.array_equal(noalloc, regular) and len(np.unique(regular)) > 50
+    monkeypatch.delenv("HIPQ_NO_RING")
+    for entry in (False, True):
+        assert np.array_equal(H.quantized_convolution(*args, noalloc=entry), regular), entry
+        assert H.last_kernel() == "conv_mfma_ring_any_i8_16x16x64"
 
 
 @pytest.mark.gpu
