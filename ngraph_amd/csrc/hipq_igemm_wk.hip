@@ -158,6 +158,15 @@ namespace hipq
             if constexpr (Loader::kWalk != 0)
                 xl.advance(cur, 64);
         };
+        // The byte of the padding, which a window of the INTERPRETER policy waits for before its first product: in front of the
+        // operands where a tile is 16 rows, as a trip of its own behind them it was 0.4 us of a launch of 4.4 (213 drawn
+        // sizes of one and two steps, channels-last: 1.05 times the time that they took when the operands came behind the epilogue's
+        // words, so 0.96; 1457 others 0.97 of it behind).  Tiles of 32 rows, sixteen wavefronts and 16 x 16 tiles
+        // of [image][channel][pixel] outputs lose by it, up to 1.1 times.
+        constexpr bool kByteFirst = Loader::kWalk != 0 && MT == 1 && KW <= 8 && (NT == 2 || !X_ON_A);
+        int32_t xzp_early = 0;
+        if constexpr (XL::kPadded && kByteFirst)
+            xzp_early = load_zp(zp.data_zp, zp.data_t);
 #pragma unroll
         for (int u = 0; u < U; ++u)
             load(u, s_begin + u);
@@ -200,7 +209,8 @@ namespace hipq
         }
 
         const int xor_mask = p.x_unsigned ? static_cast<int>(0x80808080u) : 0;
-        const int32_t xzp_early = XL::kPadded ? load_zp(zp.data_zp, zp.data_t) : 0;
+        if constexpr (XL::kPadded && !kByteFirst)
+            xzp_early = load_zp(zp.data_zp, zp.data_t);
         const int fill = (xzp_early & 0xFF) * 0x01010101;
         v4acc acc[MT][NT];
 #pragma unroll
