@@ -555,7 +555,7 @@ def _conv_sweep():
     """seeded channels-last layers of the kinds a ResNet holds -- 1 x 1 and 3 x 3, stride 1 and 2, 64 to
     512 channels either side, with and without a residual -- at image sizes and batches that put their
     tile counts on both sides of the dispatch edges (pointwise / tile kernels, 64- and 128-byte
-    slices, 64 x 128 tiles, split reductions)"""
+    slices, ring tiles, split reductions)"""
     rng = np.random.default_rng(777)
     out = []
     for _ in range(60):
@@ -606,9 +606,10 @@ def test_conv_register_staged(gpu_lib, i, monkeypatch):
 
 @pytest.mark.parametrize("stride", [1, 2])
 def test_conv_deep_slices_padding(gpu_lib, stride, monkeypatch):
-    """windows over 128 channels with enough tiles to take the 128-byte-deep slices (two operand
-    buffers): padded borders with a non-zero data zero point are patched in after the loads land,
-    one slice ahead instead of two; both policies, against the oracle and the regular slices"""
+    """windows over 128 channels on the ring tiles, which take them, and on the kernels that take what has more than 32
+    taps: 128-byte-deep slices (two operand buffers; padded borders with a non-zero data zero point are
+    patched in after the loads land, one slice ahead instead of two) and 64-byte ones; both
+    policies, against the oracle and each other"""
     say("conv deep slices with padding, stride", stride)
     N, Cc, K = (4, 128, 128) if stride == 1 else (16, 128, 256)
     in_sp, f_sp = (56, 56), (3, 3)
@@ -622,13 +623,15 @@ def test_conv_deep_slices_padding(gpu_lib, stride, monkeypatch):
         s = (0.02, 0.005, 2.5)
         exp = O.quantized_convolution(dn, data, filt, s[0], z[0], s[1], z[1], s[2], z[2])
         got = H.quantized_convolution(d, cases.to_nxc(data), filt, s[0], z[0], s[1], z[1], s[2], z[2])
-        assert H.last_kernel().startswith("conv_mfma"), H.last_kernel()
+        assert H.last_kernel().startswith("conv_mfma_ring"), H.last_kernel()
         assert np.array_equal(cases.to_ncx(got), exp), z
         assert len(np.unique(exp)) > 50
-        monkeypatch.setenv("HIPQ_NO_DEEP_SLICES", "1")
-        regular = H.quantized_convolution(d, cases.to_nxc(data), filt, s[0], z[0], s[1], z[1], s[2], z[2])
-        monkeypatch.delenv("HIPQ_NO_DEEP_SLICES")
-        assert np.array_equal(regular, got), z
+        for switch in ("HIPQ_NO_RING", "HIPQ_NO_DEEP_SLICES"):  # (deep slices, regular ones)
+            monkeypatch.setenv(switch, "1")
+            other = H.quantized_convolution(d, cases.to_nxc(data), filt, s[0], z[0], s[1], z[1], s[2], z[2])
+            monkeypatch.delenv(switch)
+            assert H.last_kernel() == "conv_mfma_i8_32x32x32"
+            assert np.array_equal(other, got), (z, switch)
     df = H.make_conv_desc(N, Cc, K, in_sp, f_sp, out_t="i8", data_layout=H.NXC, out_layout=H.NXC, **kw)
     dfn = H.make_conv_desc(N, Cc, K, in_sp, f_sp, out_t="i8", **kw)
     f = H.make_fused_desc(has_bias=True, with_relu=False, scale_count=K)
@@ -637,7 +640,31 @@ def test_conv_deep_slices_padding(gpu_lib, stride, monkeypatch):
     exp = O.quantized_convolution_fused(dfn, f, data, filt, bias, None, scales, None)
     got = H.quantized_convolution_fused(df, f, cases.to_nxc(data), filt, bias, None, scales, None)
     assert np.array_equal(cases.to_ncx(got), exp)
+    monkeypatch.setenv("HIPQ_NO_RING", "1")
+    got = H.quantized_convolution_fused(df, f, cases.to_nxc(data), filt, bias, None, scales, None)
+    assert H.last_kernel() == "conv_mfma_i8_32x32x32" and np.array_equal(cases.to_ncx(got), exp)
     O.port().orc_set_threads(1)
+
+
+def test_conv_deep_slices_many_taps(gpu_lib, monkeypatch):
+    """36 taps over 128 channels, where deep slices are what the library chooses: against the regular slices and the
+    register-staged kernel, both policies, padding with a non-zero data zero point"""
+    say("conv deep slices, 36 taps")
+    kw = dict(pad_below=(3, 3), pad_above=(2, 2), data_layout=H.NXC, out_layout=H.NXC)
+    d, df = (H.make_conv_desc(4, 128, 128, (56, 56), (6, 6), out_t=t, **kw) for t in ("u8", "i8"))
+    data = synth.uniform_int(3110, d.data_shape(), 0, 255, np.uint8)
+    filt = synth.uniform_int(3210, d.filter_shape(), -128, 127, np.int8)
+    f = H.make_fused_desc(has_bias=True, with_relu=False, scale_count=128)
+    bias = synth.uniform_int(3310, (128,), -20000, 20000, np.int32)
+    scales = synth.uniform_f32(3311, (128,), 3e-5, 1.5e-4)
+    for call in (lambda: H.quantized_convolution(d, data, filt, 0.02, 131, 0.005, 0, 5.0, 7), lambda: H.quantized_convolution_fused(df, f, data, filt, bias, None, scales, None)):
+        got = call()
+        assert H.last_kernel() == "conv_mfma_i8_32x32x32" and len(np.unique(got)) > 50
+        for switch in ("HIPQ_NO_DEEP_SLICES", "HIPQ_NO_CONV_DMA"):
+            monkeypatch.setenv(switch, "1")
+            assert np.array_equal(call(), got), switch
+            assert H.last_kernel() == "conv_mfma_i8_32x32x32"
+            monkeypatch.delenv(switch)
 
 
 @pytest.mark.parametrize("i", range(len(SPLIT_CONV_SHAPES)))
@@ -902,9 +929,9 @@ def test_dot_tile_order(gpu_lib, family, shape):
 
 @pytest.mark.parametrize("shape", [(1000, 768, 400), (2000, 512, 1104), (4096, 768, 768)])
 def test_dot_half_height_tiles(gpu_lib, family, shape, monkeypatch):
-    """row matrices whose 128 x 128 tiles would leave compute units idle run on 64 x 128 tiles with
-    whole reductions: ragged last tiles in both directions, 8-bit and float outputs, against the
-    oracle and against the 128 x 128 tiles (reductions split over workgroups) behind the switch"""
+    """row matrices whose 128 x 128 tiles would leave compute units idle: ragged last tiles in both directions,
+    8-bit and float outputs, on the kernels that take them and, behind the switch of the tiles they once had,
+    on the 128 x 128 tiles (reductions split over workgroups), against the oracle"""
     M, K, N = shape
     say("dot half-height tiles", shape)
     O.port().orc_set_threads(8)
@@ -963,8 +990,8 @@ def test_dot_dispatch_sweep(gpu_lib, family, shape):
 
 @pytest.mark.parametrize("split", ["2", "4"])
 def test_dot_deep_slices_split(gpu_lib, split, monkeypatch):
-    """reductions in whole 128-byte pieces run with slices twice as deep and two operand buffers;
-    here with the reduction also cut over workgroups, and against the regular slices"""
+    """reductions in whole 128-byte pieces, cut over workgroups on the 128 x 128 tiles (64-byte slices: rows no longer
+    have deep ones), and on the kernel that takes them unasked"""
     say("dot deep slices, split", split)
     M, K, N = 300, 1024, 272
     O.port().orc_set_threads(8)
@@ -978,10 +1005,10 @@ def test_dot_deep_slices_split(gpu_lib, split, monkeypatch):
         exp = O.quantized_dot_bias(d, f, a, w, bias, scales)
         monkeypatch.setenv("HIPQ_SPLIT_K", split)
         got = H.quantized_dot_bias(d, f, a, w, bias, scales)
-        monkeypatch.setenv("HIPQ_NO_DEEP_SLICES", "1")
-        regular = H.quantized_dot_bias(d, f, a, w, bias, scales)
-        monkeypatch.delenv("HIPQ_NO_DEEP_SLICES")
+        assert H.last_kernel() == "dot_mfma_i8_32x32x32"
         monkeypatch.delenv("HIPQ_SPLIT_K")
+        regular = H.quantized_dot_bias(d, f, a, w, bias, scales)
+        assert H.last_kernel() != "dot_mfma_i8_32x32x32"
         assert np.array_equal(got.view(np.uint8), exp.view(np.uint8)), out_t
         assert np.array_equal(regular.view(np.uint8), exp.view(np.uint8)), out_t
     O.port().orc_set_threads(1)
