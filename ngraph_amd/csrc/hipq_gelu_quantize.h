@@ -10,7 +10,8 @@ namespace hipq
     // distribution), and phi(-a) is 2 to a polynomial of degree 7 in a (least squares on log2 phi, weighted by what an error
     // there does to the product and reweighted to the smallest largest error: 7.3e-8, the leading coefficient held below
     // zero so that it falls for good beyond the range that counts).  The difference from gelu1, mostly gelu1's own
-    // roundings, is at most 2.4e-7 + 1.8e-7 |gelu(x)|, every float tried on the device.  Where the quotient lies
+    // roundings, is at most 2.4e-7 + 1.8e-7 |gelu(x)| (the largest seen when it was fitted; the bytes that rest on it are held
+    // next to every rounding step and for every 127th float by tests/test_gelu_quantize.py).  Where the quotient lies
     // further from every half than what that and the roundings of reciprocal, product and division amount to, both
     // round to the same integer; the other elements (about one in 15 000 at a scale of 0.0175: each holds up its
     // workgroup for 0.8 us), a NaN or an infinity are computed as the ops do.

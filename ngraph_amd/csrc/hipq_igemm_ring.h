@@ -16,8 +16,6 @@
 // channels on 15 680 pixels 25.6 -> 14.5, over 512 on 2352 26.9 -> 17.1, inside ResNet-50 of 128 images 28.9 -> 24.0 and
 // 33.7 -> 25.2 (the whole pass 1554 -> 1391).  What bounds it: see kRing*.
 #pragma once
-#include <unistd.h>
-
 #include "hipq_igemm.h"
 
 namespace hipq

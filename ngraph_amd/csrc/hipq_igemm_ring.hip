@@ -103,6 +103,7 @@ namespace hipq
             default: return HIPQ_ERR_UNSUPPORTED;
             }
 #undef RING
+#undef RING2
         }
 
         bool ring_enabled()
