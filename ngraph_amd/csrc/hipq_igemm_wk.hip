@@ -30,7 +30,6 @@
 #include <cstdlib>
 #include <cstring>
 
-#include <unistd.h>
 
 #include "hipq_igemm.h"
 

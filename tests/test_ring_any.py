@@ -133,6 +133,18 @@ def test_lines_for_products(gpu_lib, M, K, N, kernel):
         assert np.array_equal(got, dot_bias_closed_form(a, w, b, scale, "i8", False)), b is None
 
 
+# (rows of the INTERPRETER policy into at most 64 columns: one round of 256-row tiles, a row more, a column more, a long reduction)
+@pytest.mark.parametrize("M,K,N,kernel", [(65536, 256, 64, "ring"), (65537, 256, 64, "i8_32x32x32"), (65537, 256, 80, "ring"), (65537, 1024, 48, "ring")])
+def test_lines_for_narrow_rows(gpu_lib, M, K, N, kernel):
+    print("ring line narrow", M, K, N, flush=True)
+    a, w, _, _ = operands(M, K, N, "u8")
+    got = H.quantized_dot(H.make_dot_desc(M, K, N, out_t="i8", b_layout=H.B_NK), a, w, 0.02, 0, 0.005, 0, 2.0, 0)
+    assert H.last_kernel() == "dot_mfma_%s" % (kernel if kernel.startswith("i8") else kernel + "_i8_16x16x64")
+    rows = np.r_[0:300, M // 2 : M // 2 + 300, M - 300 : M]
+    few = H.make_dot_desc(rows.size, K, N, out_t="i8", b_layout=H.B_NK)
+    assert np.array_equal(got[rows], O.quantized_dot(few, a[rows], w, 0.02, 0, 0.005, 0, 2.0, 0))
+
+
 @pytest.mark.parametrize("M,K,N,kernel", [(1012, 464, 464, "wk"), (1329, 2320, 192, "wk"), (1024, 1728, 512, "wk"), (1024, 1792, 512, "ring"), (2048, 512, 512, "ring")])
 def test_lines_for_gelu(gpu_lib, M, K, N, kernel):
     print("ring line gelu", M, K, N, flush=True)
