@@ -523,6 +523,40 @@ HIPQ_API int hipq_quantized_convolution_fused_max_pool(const hipq_conv_desc_t* d
                                                        void* out,
                                                        void* stream);
 
+/*
+ * A bottleneck block's widening 1 x 1 layer and the next block's narrowing one in one launch:
+ *   wide   = hipq_quantized_convolution_fused(widen, residual)
+ *   narrow = hipq_quantized_convolution_fused(narrow, over wide)
+ * where the residual is the tensor `sum_in`, or, with `shortcut`, the result of that projection over its
+ * own data (then `sum_in` is null and the projection's result is never written).  Both results are
+ * written; the bytes equal the separate calls'
+ * (src/ngraph/runtime/cpu/builder/quantized_conv.cpp:332-766).  `sum_scale`: the widening layer's, as there.
+ * Eligible (hipq_pointwise_chain_fusable returns 1; only descriptors are looked at, data pointers may
+ * be null): 1 x 1 filters of stride 1 over channels-last pixels; 64 channels to 256 to 64 or 128, or
+ * 128 to 512 to 128, or to 256 over many pixels; the wide result after a ReLU, of the residual's type; the narrow result u8 without a
+ * residual; a shortcut with an i8 result from 64 channels, to 256 and then 64.  Filters packed
+ * (hipq_conv_pack_filter), tensors 16-byte aligned; HIPQ_ERR_UNSUPPORTED for anything else: the
+ * caller then makes the separate calls.
+ */
+typedef struct
+{
+    const hipq_conv_desc_t* conv;
+    const hipq_fused_desc_t* fused;
+    const void* data; /* not read for the narrowing layer, whose data is `wide` */
+    const void* packed_filter;
+    const int32_t* bias;
+    const float* scale;
+} hipq_pointwise_layer_t;
+HIPQ_API int hipq_pointwise_chain_fusable(const hipq_pointwise_layer_t* widen, const hipq_pointwise_layer_t* shortcut, const hipq_pointwise_layer_t* narrow);
+HIPQ_API int hipq_pointwise_chain(const hipq_pointwise_layer_t* widen,
+                                  const hipq_pointwise_layer_t* shortcut,
+                                  const hipq_pointwise_layer_t* narrow,
+                                  const void* sum_in,
+                                  const float* sum_scale,
+                                  void* wide_out,
+                                  void* narrow_out,
+                                  void* stream);
+
 /* op::v0::Concat (src/ngraph/runtime/reference/concat.hpp): piece i is [outer][extent[i]][inner]
  * elements, the result [outer][sum extent][inner]; `inputs` and `extents` are host arrays of
  * device pointers / axis extents. */

@@ -343,6 +343,11 @@ namespace hipq
     // weights in registers, tile loads one tile ahead (hipq_conv_pw.hip)
     bool conv_pw64_eligible(const ConvGeom& g, const Epilogue& epi, const ZeroPoints& zp);
     int launch_conv_pw64(const ConvGeom& g, const void* data, const void* packed, const Epilogue& epi, void* out, hipStream_t s);
+    // such a layer, with its residual or the projection that makes it, and the 1 x 1 layer that narrows its result again, in one
+    // launch (hipq_conv_chain.hip); gs / es: the projection, or null.  e1.sum_in is the residual or the projection's data
+    bool conv_chain_eligible(const ConvGeom& g1, const Epilogue& e1, const ConvGeom* gs, const Epilogue* es, const ConvGeom& g2, const Epilogue& e2);
+    int launch_conv_chain(const ConvGeom& g1, const Epilogue& e1, const void* data, const void* packed1, const ConvGeom* gs, const Epilogue* es, const void* packed_s, const ConvGeom& g2,
+                          const Epilogue& e2, const void* packed2, void* out, void* narrow, hipStream_t s);
     int launch_row_sums_i8(const void* w, int64_t rows, int64_t cols, int32_t* sums, hipStream_t s);
     // [N][K] weights in the fragment order of v_mfma_i32_16x16x64_i8 (K a multiple of 64): ceil(N / 16) * K / 64 blocks of 1 KB
     int launch_pack_dot_fragments(const void* w_nk, int64_t N, int64_t K, void* frag, hipStream_t s);

@@ -470,6 +470,73 @@ int hipq_quantized_convolution_fused_max_pool(const hipq_conv_desc_t* desc,
     return launch_conv_stem(g, data, packed_filter, zp, e, &pf, out, as_stream(stream));
 }
 
+// the layers of a chain of pointwise convolutions, pointers and all; `sum` stands for the residual or the shortcut's data
+static int chain_layers(const hipq_pointwise_layer_t* widen, const hipq_pointwise_layer_t* shortcut, const hipq_pointwise_layer_t* narrow, const void* sum, const float* sum_scale, ConvGeom (&g)[3],
+                        Epilogue (&e)[3])
+{
+    const hipq_pointwise_layer_t* const layers[3] = {widen, shortcut, narrow};
+    HIPQ_REQUIRE(widen && narrow, "layer is null");
+    for (int i = 0; i < 3; ++i)
+    {
+        if (!layers[i])
+            continue;
+        int rc = make_geom(layers[i]->conv, &g[i]);
+        if (rc)
+            return rc;
+        rc = check_conv_types(g[i], true);
+        if (rc)
+            return rc;
+        rc = fused_epilogue(layers[i]->fused, g[i].out_t, g[i].K, layers[i]->bias, i == 0 ? sum : nullptr, layers[i]->scale, i == 0 ? sum_scale : nullptr, &e[i]);
+        if (rc)
+            return rc;
+    }
+    if (!widen->fused->has_sum || !conv_chain_eligible(g[0], e[0], shortcut ? &g[1] : nullptr, shortcut ? &e[1] : nullptr, g[2], e[2]))
+        return fail(HIPQ_ERR_UNSUPPORTED, "these pointwise layers have no common kernel (hipq_pointwise_chain_fusable is 0)");
+    return HIPQ_OK;
+}
+
+int hipq_pointwise_chain_fusable(const hipq_pointwise_layer_t* widen, const hipq_pointwise_layer_t* shortcut, const hipq_pointwise_layer_t* narrow)
+{
+    if (!widen || !narrow)
+        return 0;
+    // (only what the descriptors say counts: any address stands for a tensor that will be there)
+    static const int32_t there[4] = {};
+    auto with = [](const hipq_pointwise_layer_t* l) {
+        hipq_pointwise_layer_t r = *l;
+        r.bias = there;
+        r.scale = reinterpret_cast<const float*>(there);
+        return r;
+    };
+    const hipq_pointwise_layer_t w = with(widen), s = shortcut ? with(shortcut) : w, n = with(narrow);
+    ConvGeom g[3];
+    Epilogue e[3];
+    return chain_layers(&w, shortcut ? &s : nullptr, &n, there, reinterpret_cast<const float*>(there), g, e) == HIPQ_OK ? 1 : 0;
+}
+
+int hipq_pointwise_chain(const hipq_pointwise_layer_t* widen,
+                         const hipq_pointwise_layer_t* shortcut,
+                         const hipq_pointwise_layer_t* narrow,
+                         const void* sum_in,
+                         const float* sum_scale,
+                         void* wide_out,
+                         void* narrow_out,
+                         void* stream)
+{
+    HIPQ_REQUIRE(!shortcut || !sum_in, "either a residual or a shortcut");
+    ConvGeom g[3];
+    Epilogue e[3];
+    const int rc = chain_layers(widen, shortcut, narrow, shortcut ? shortcut->data : sum_in, sum_scale, g, e);
+    if (rc)
+        return rc;
+    HIPQ_REQUIRE(widen->data && widen->packed_filter && narrow->packed_filter && (!shortcut || shortcut->packed_filter) && wide_out && narrow_out, "null tensor pointer");
+    auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    HIPQ_REQUIRE(aligned(widen->data) && aligned(widen->packed_filter) && aligned(e[0].sum_in) && aligned(narrow->packed_filter) && (!shortcut || aligned(shortcut->packed_filter)) &&
+                     aligned(wide_out) && aligned(narrow_out),
+                 "tensors must be 16-byte aligned");
+    return launch_conv_chain(g[0], e[0], widen->data, widen->packed_filter, shortcut ? &g[1] : nullptr, shortcut ? &e[1] : nullptr, shortcut ? shortcut->packed_filter : nullptr, g[2], e[2],
+                             narrow->packed_filter, wide_out, narrow_out, as_stream(stream));
+}
+
 size_t hipq_dot_packed_bytes(const hipq_dot_desc_t* d)
 {
     if (!d || !dot_mfma_eligible(dot_seen(*d)))

@@ -110,6 +110,10 @@ class FusedDesc(C.Structure):
     ]
 
 
+class PointwiseLayer(C.Structure):
+    _fields_ = [("conv", C.POINTER(ConvDesc)), ("fused", C.POINTER(FusedDesc)), ("data", C.c_void_p), ("packed_filter", C.c_void_p), ("bias", C.c_void_p), ("scale", C.c_void_p)]
+
+
 class DotDesc(C.Structure):
     _fields_ = [
         ("a_t", C.c_int32),
@@ -302,6 +306,8 @@ EXPORTS = [
     "hipq_quantized_convolution_fused",
     "hipq_conv_max_pool_fusable",
     "hipq_quantized_convolution_fused_max_pool",
+    "hipq_pointwise_chain_fusable",
+    "hipq_pointwise_chain",
     "hipq_dot_packed_bytes",
     "hipq_dot_pack",
     "hipq_quantized_dot",
@@ -412,6 +418,8 @@ def load():
     lib.hipq_quantized_convolution_fused.argtypes = [C.POINTER(ConvDesc), C.POINTER(FusedDesc)] + [vp] * 9
     lib.hipq_conv_max_pool_fusable.argtypes = [C.POINTER(ConvDesc), C.POINTER(FusedDesc), C.POINTER(PoolDesc)]
     lib.hipq_quantized_convolution_fused_max_pool.argtypes = [C.POINTER(ConvDesc), C.POINTER(FusedDesc), C.POINTER(PoolDesc)] + [vp] * 6
+    lib.hipq_pointwise_chain_fusable.argtypes = [C.POINTER(PointwiseLayer)] * 3
+    lib.hipq_pointwise_chain.argtypes = [C.POINTER(PointwiseLayer)] * 3 + [vp] * 5
     lib.hipq_dot_packed_bytes.restype = C.c_size_t
     lib.hipq_dot_packed_bytes.argtypes = [C.POINTER(DotDesc)]
     lib.hipq_dot_pack.argtypes = [C.POINTER(DotDesc), vp, vp, vp]
@@ -607,6 +615,41 @@ def quantized_convolution_fused_max_pool(desc, fused, pool_desc, data, filt, bia
     check(lib.hipq_quantized_convolution_fused_max_pool(C.byref(desc), C.byref(fused), C.byref(pool_desc), bd.ptr, _p(packed), _p(bb), bsc.ptr, out.ptr, None))
     check(lib.hipq_stream_sync(None))
     return out.to_numpy(NP_OF[desc.out_t], oshape)
+
+
+def _layer_ref(layer):
+    return None if layer is None else C.byref(layer)
+
+
+def pointwise_layer(desc, fused, data=None, packed=None, bias=None, scale=None):
+    """one layer of a pointwise chain; buffers may be left out where only the descriptors are looked at"""
+    ptr = lambda b: None if b is None else b.ptr
+    layer = PointwiseLayer(C.pointer(desc), C.pointer(fused), ptr(data), ptr(packed), ptr(bias), ptr(scale))
+    layer.keep = (desc, fused, data, packed, bias, scale)
+    return layer
+
+
+def pointwise_chain_fusable(widen, shortcut, narrow) -> bool:
+    return bool(load().hipq_pointwise_chain_fusable(_layer_ref(widen), _layer_ref(shortcut), _layer_ref(narrow)))
+
+
+def pointwise_chain(widen, shortcut, narrow, sum_in, sum_scale):
+    """(wide, narrow) of a chain in one launch.  A layer is (desc, fused desc, data, filter, bias, scale) of arrays, `shortcut` may be
+    None; raises HipqError (UNSUPPORTED) for layers without a common kernel"""
+    lib = load()
+
+    def layer(l):
+        if l is None:
+            return None
+        d, f, data, filt, bias, scale = l
+        return pointwise_layer(d, f, _dev(data), pack_filter(d, _dev(filt)), _dev(None if bias is None else np.asarray(bias, dtype=np.int32)), _dev(np.asarray(scale, dtype=np.float32)))
+
+    w, s, n = layer(widen), layer(shortcut), layer(narrow)
+    outs = [DeviceBuffer(int(np.prod(l[0].out_shape())) * np.dtype(NP_OF[l[0].out_t]).itemsize) for l in (widen, narrow)]
+    bsum, bss = _dev(sum_in), _dev(np.float32(sum_scale))
+    check(lib.hipq_pointwise_chain(_layer_ref(w), _layer_ref(s), _layer_ref(n), _p(bsum), bss.ptr, outs[0].ptr, outs[1].ptr, None))
+    check(lib.hipq_stream_sync(None))
+    return tuple(o.to_numpy(NP_OF[l[0].out_t], l[0].out_shape()) for o, l in zip(outs, (widen, narrow)))
 
 
 def pool(desc, x):

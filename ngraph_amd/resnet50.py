@@ -159,9 +159,10 @@ class DevicePlan:
     """The network with every tensor resident in HBM, weights packed once: the f32 images arrive in the
     reference's NCHW order, Quantize writes u8 NCHW, the stem reads that and writes channels-last, and
     everything up to the logits stays channels-last.  `launch()` issues the kernel launches of one
-    forward pass on `stream`; `capture()` turns them into one HIP graph for `replay()`."""
+    forward pass on `stream`; `capture()` turns them into one HIP graph for `replay()`.  With `fuse_pointwise`, a
+    block's last layer and the next block's first are one launch where the library has one for them."""
 
-    def __init__(self, lib, stream, N, hw=224, fuse_pool=True):
+    def __init__(self, lib, stream, N, hw=224, fuse_pool=True, fuse_pointwise=True):
         self.lib, self.stream, self.N = lib, stream, N
         self._replay = None
         self.calls, self.keep, self.graph = [], [], None
@@ -176,6 +177,7 @@ class DevicePlan:
             for key in ("src", "sum_src"):
                 if op.get(key) is not None:
                     readers[op[key]] = readers.get(op[key], 0) + 1
+        convs = {}      # a convolution's call by the name of its result: (its index, layer, op)
         pending = None  # a convolution whose only reader is the MaxPool behind it, held back for the fused call
         for i, op in enumerate(ops):
             Cc, h = shape[op["src"]]
@@ -216,6 +218,7 @@ class DevicePlan:
                 ss = dev(np.asarray(op["sum_scale"], np.float32)) if has_sum else None
                 sm = buf[op["sum_src"]] if has_sum else None
                 self.calls.append((lib.hipq_quantized_convolution_fused, (self._keep(d), self._keep(f), src, bf, packed, bb, sm, bs, ss, out)))
+                convs[op["name"]] = (len(self.calls) - 1, H.pointwise_layer(d, f, src, packed, bb, bs), op)
                 buf[op["name"]] = out
             elif op["op"] in ("maxpool", "avgpool"):
                 ho = out_hw(h, op["window"], op["stride"], op["pad"])
@@ -242,6 +245,35 @@ class DevicePlan:
                 self.ops_per_image += 2 * op["K"] * op["N"]
         self.logits = buf["logits"]
         self.buffers = buf
+        self.left_out = {}  # calls whose results only a common launch needs, and which it does not write: made when they are read
+        if fuse_pointwise:
+            self._join_pointwise(convs, ops, readers)
+
+    def _join_pointwise(self, convs, ops, readers):
+        """a block's widening layer, the projection that makes its residual, if only it reads that, and the next block's narrowing layer, one launch"""
+        same = {op["name"]: op["src"] for op in ops if op["op"] == "convert_u8"}  # shares its input's bytes
+        gone = set()
+        for at, narrow, op in list(convs.values()):
+            wide_name = same.get(op["src"], op["src"])
+            if op["sum_src"] is not None or wide_name not in convs:
+                continue
+            wide_at, widen, wide = convs[wide_name]
+            if wide["sum_src"] is None or wide_at != at - 1:
+                continue
+            short_at, shortcut, _ = convs.get(wide["sum_src"], (None, None, None))
+            wide_args, sm = self.calls[wide_at][1], self.calls[wide_at][1][6]
+            if shortcut is not None and (short_at != wide_at - 1 or readers[wide["sum_src"]] != 1 or not H.pointwise_chain_fusable(widen, shortcut, narrow)):
+                shortcut = None
+            if shortcut is None and not H.pointwise_chain_fusable(widen, None, narrow):
+                continue
+            if shortcut is not None:
+                self.left_out[wide["sum_src"]] = self.calls[short_at]
+                gone.add(short_at)
+                sm = None
+            gone.add(wide_at)
+            layers = [self._keep(x) if x is not None else None for x in (widen, shortcut, narrow)]
+            self.calls[at] = (self.lib.hipq_pointwise_chain, (*layers, sm, wide_args[8], wide_args[9], self.calls[at][1][9]))
+        self.calls = [c for i, c in enumerate(self.calls) if i not in gone]
 
     def _keep(self, x):
         self.keep.append(x)
@@ -253,12 +285,15 @@ class DevicePlan:
         assert x.nbytes == self.input.nbytes
         H.check(self.lib.hipq_memcpy_h2d(self.input.ptr, x.ctypes.data, x.nbytes, None))
 
+    def _call(self, fn, args):
+        a = [C.byref(x) if isinstance(x, C.Structure) else (None if x is None else x.ptr) for x in args]
+        rc = fn(*a, self.stream)
+        if rc:
+            H.check(rc)
+
     def launch(self):
         for fn, args in self.calls:
-            a = [C.byref(x) if isinstance(x, C.Structure) else (None if x is None else x.ptr) for x in args]
-            rc = fn(*a, self.stream)
-            if rc:
-                H.check(rc)
+            self._call(fn, args)
 
     def capture(self):
         """records the pass into a HIP graph (after one eager pass that sizes the library's scratch)"""
@@ -284,5 +319,7 @@ class DevicePlan:
 
     def read(self, name, channels, hw, dtype=np.uint8):
         """a named activation as an NCHW numpy tensor"""
+        if name in self.left_out:
+            self._call(*self.left_out[name])
         H.check(self.lib.hipq_stream_sync(self.stream))
         return np.ascontiguousarray(np.moveaxis(self.buffers[name].to_numpy(dtype, (self.N, hw, hw, channels)), -1, 1))

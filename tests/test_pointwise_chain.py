@@ -1,0 +1,126 @@
+"""Two or three 1 x 1 layers in one launch (hipq_pointwise_chain) against the CPU oracle and against the separate calls."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from ngraph_amd import hipq as H
+from ngraph_amd import synth
+
+
+def _conv(pixels, Cc, K, data_t, out_t):
+    n, h, w = pixels
+    return H.make_conv_desc(n, Cc, K, (h, w), (1, 1), data_t=data_t, out_t=out_t, data_layout=H.NXC, out_layout=H.NXC)
+
+
+def _layer(seed, d, f, data, bias=True, scalar=False, gain=1.0):
+    Cc, K = d.C, d.K
+    filt = synth.uniform_int(seed, (K, Cc, 1, 1), -127, 127, np.int8)
+    b = synth.uniform_int(seed + 1, (K,), -3000, 3000, np.int32) if bias is True else bias
+    s = synth.uniform_f32(seed + 2, (1 if scalar else K,), 0.8, 1.2) * np.float32(gain * 50.0 / (73.3 * 73.9 * 2 * np.sqrt(Cc)))
+    return d, f, data, filt, b, s.astype(np.float32)
+
+
+def _chain(seed, pixels, Cc, N1, N2, shortcut=False, data_t="u8", wide_t="u8", bias=True, scalar=False, gain=1.0):
+    byte = lambda t: (0, 255, np.uint8) if t == "u8" else (-127, 127, np.int8)
+    n, h, w = pixels
+    count = lambda: 1 if scalar else None
+    fused = lambda K, relu, has_sum=False, sum_t="u8": H.make_fused_desc(has_bias=bias is not None, has_sum=has_sum, sum_t=sum_t, with_relu=relu, scale_count=count() or K)
+    d1, d2 = _conv(pixels, Cc, N1, data_t, wide_t), _conv(pixels, N1, N2, "u8", "u8")
+    x = synth.uniform_int(seed, (n, h, w, Cc), *byte(data_t))
+    widen = _layer(seed + 10, d1, fused(N1, True, True, wide_t), x, bias, scalar, gain)
+    short, residual = None, None
+    if shortcut:
+        ds = _conv(pixels, 64, N1, "u8", "i8")
+        short = _layer(seed + 20, ds, fused(N1, False), synth.uniform_int(seed + 1, (n, h, w, 64), *byte("u8")), bias, scalar, gain)
+    else:
+        residual = synth.uniform_int(seed + 2, (n, h, w, N1), *byte(wide_t))
+    narrow = _layer(seed + 30, d2, fused(N2, True), None, bias, scalar, gain)
+    return widen, short, narrow, residual, 0.5
+
+
+def _apart(call, widen, short, narrow, residual, sum_scale):
+    """the separate calls through `call(desc, fused, data, filt, bias, sum_in, scale, sum_scale)`"""
+    if short is not None:
+        d, f, x, filt, b, s = short
+        residual = call(d, f, x, filt, b, None, s, None)
+    d, f, x, filt, b, s = widen
+    wide = call(d, f, x, filt, b, residual, s, sum_scale)
+    d, f, _, filt, b, s = narrow
+    return wide, call(d, f, wide.view(np.uint8), filt, b, None, s, None)
+
+
+def _oracle(d, f, x, filt, b, sum_in, s, sum_scale):
+    return O.quantized_convolution_fused(d, f, x, filt, b, sum_in, s, sum_scale)
+
+
+CHAINS = [(64, 256, 64, False, "u8"), (64, 256, 64, False, "i8"), (64, 256, 128, False, "u8"), (64, 256, 128, False, "i8"), (64, 256, 64, True, "i8"), (128, 512, 128, False, "u8"),
+          (128, 512, 128, False, "i8"), (128, 512, 256, False, "u8"), (128, 512, 256, False, "i8")]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Cc,N1,N2,shortcut,wide_t", CHAINS)
+@pytest.mark.parametrize("pixels", [(1, 1, 1), (1, 3, 5), (1, 4, 4), (1, 1, 17), (1, 1, 31), (2, 4, 4), (3, 11, 1), (2, 28, 28)])
+def test_chain_against_the_oracle(gpu_lib, Cc, N1, N2, shortcut, wide_t, pixels):
+    if N2 == 256:
+        pixels = (1, 8, 256 + pixels[0] * pixels[1] * pixels[2] % 40)  # a kernel of many pixels: 2048 and more
+    print("[case] chain", Cc, N1, N2, shortcut, wide_t, pixels, flush=True)
+    for kw in (dict(), dict(data_t="i8", scalar=True), dict(bias=None)):
+        c = _chain(7, pixels, Cc, N1, N2, shortcut, wide_t=wide_t, **kw)
+        got = H.pointwise_chain(*c)
+        assert H.last_kernel().startswith("conv_chain")
+        exp = _apart(_oracle, *c)
+        for a, b in zip(got, exp):
+            assert np.array_equal(a, b), kw
+        assert np.unique(got[0]).size > 2 and np.unique(got[1]).size > 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Cc,N1,N2,shortcut,wide_t", CHAINS)
+def test_chain_over_several_rounds_equals_the_separate_calls(gpu_lib, Cc, N1, N2, shortcut, wide_t):
+    """more tiles than the wavefronts of a launch, the last one with six pixels"""
+    pixels = (3, 2, 16385)
+    print("[case] chain", Cc, N1, N2, shortcut, wide_t, pixels, flush=True)
+    c = _chain(9, pixels, Cc, N1, N2, shortcut, wide_t=wide_t)
+    for a, b in zip(H.pointwise_chain(*c), _apart(H.quantized_convolution_fused, *c)):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Cc,N1,N2,shortcut,wide_t", CHAINS)
+def test_chain_at_the_ends_of_its_arithmetic(gpu_lib, Cc, N1, N2, shortcut, wide_t):
+    """biases beyond 2^24, which are added as floats, and results that saturate, vanish or are no numbers"""
+    print("[case] chain ends", Cc, N1, N2, shortcut, wide_t, flush=True)
+    for gain in (1.0, 1e6, 1e-6, np.float32(np.inf), np.float32(np.nan)):
+        c = list(_chain(11, (2, 9, 5) if N2 != 256 else (3, 29, 53), Cc, N1, N2, shortcut, wide_t=wide_t, gain=gain))
+        for i in range(3):
+            if c[i] is not None and gain in (1.0, 1e-6):
+                d, f, x, filt, b, s = c[i]
+                b = np.where(np.arange(b.size) % 3 == 0, (1 << 24) + 12345 + b, -(1 << 26) + 1 + b).astype(np.int32)
+                c[i] = (d, f, x, filt, b, s)
+        for a, b in zip(H.pointwise_chain(*c), _apart(H.quantized_convolution_fused, *c)):
+            assert np.array_equal(a, b), gain
+
+
+def test_only_such_layers_have_a_common_kernel():
+    px = (1, 8, 8)
+    rows = lambda c: [None if l is None else H.pointwise_layer(l[0], l[1]) for l in c[:3]]
+    assert H.pointwise_chain_fusable(*rows(_chain(1, px, 64, 256, 64)))
+    assert H.pointwise_chain_fusable(*rows(_chain(1, px, 64, 256, 64, True, wide_t="i8")))
+    assert not H.pointwise_chain_fusable(*rows(_chain(1, px, 64, 256, 64, True, wide_t="u8")))  # the projection's result is i8, the wide one must be
+    assert not H.pointwise_chain_fusable(*rows(_chain(1, px, 64, 512, 64)))
+    assert not H.pointwise_chain_fusable(*rows(_chain(1, px, 256, 1024, 256)))
+    w, s, n = _chain(1, px, 64, 256, 64)[:3]
+    for change in (dict(with_relu=0), dict(has_sum=0), dict(sum_t=H.DTYPE_OF["i8"] if hasattr(H, "DTYPE_OF") else H.I8)):
+        f = H.make_fused_desc(has_bias=True, has_sum=True, sum_t="u8", with_relu=True, scale_count=256)
+        for k, v in change.items():
+            setattr(f, k, v)
+        assert not H.pointwise_chain_fusable(H.pointwise_layer(w[0], f), None, H.pointwise_layer(n[0], n[1])), change
+    strided = H.make_conv_desc(1, 64, 256, (8, 8), (1, 1), stride=(2, 2), data_layout=H.NXC, out_layout=H.NXC, out_t="u8")
+    assert not H.pointwise_chain_fusable(H.pointwise_layer(strided, w[1]), None, H.pointwise_layer(n[0], n[1]))
+    planes = H.make_conv_desc(1, 64, 256, (8, 8), (1, 1), out_t="u8")
+    assert not H.pointwise_chain_fusable(H.pointwise_layer(planes, w[1]), None, H.pointwise_layer(n[0], n[1]))
+    assert H.load().hipq_pointwise_chain(None, None, None, None, None, None, None, None) == H.ERR_INVALID
+    wl, nl = H.pointwise_layer(w[0], w[1]), H.pointwise_layer(n[0], n[1])
+    import ctypes as C
+
+    assert H.load().hipq_pointwise_chain(C.byref(wl), None, C.byref(nl), None, None, None, None, None) == H.ERR_INVALID
