@@ -343,6 +343,9 @@ namespace hipq
     // weights in registers, tile loads one tile ahead (hipq_conv_pw.hip)
     bool conv_pw64_eligible(const ConvGeom& g, const Epilogue& epi, const ZeroPoints& zp);
     int launch_conv_pw64(const ConvGeom& g, const void* data, const void* packed, const Epilogue& epi, void* out, hipStream_t s);
+    // other 1 x 1 layers of short reductions over many pixels, any stride, fused policy, channels-last (hipq_conv_stream.hip)
+    bool conv_stream_eligible(const ConvGeom& g, const Epilogue& epi, const ZeroPoints& zp);
+    int launch_conv_stream(const ConvGeom& g, const void* data, const void* packed, const Epilogue& epi, void* out, hipStream_t s);
     // such a layer, with its residual or the projection that makes it, and the 1 x 1 layer that narrows its result again, in one
     // launch (hipq_conv_chain.hip); gs / es: the projection, or null.  e1.sum_in is the residual or the projection's data
     bool conv_chain_eligible(const ConvGeom& g1, const Epilogue& e1, const ConvGeom* gs, const Epilogue* es, const ConvGeom& g2, const Epilogue& e2);

@@ -100,6 +100,8 @@ namespace hipq
         // layers bound by HBM traffic that widen 64 channels: weights in registers, loads a tile ahead
         if (conv_pw64_eligible(g, epi, zp))
             return launch_conv_pw64(g, x, packed, epi, out, s);
+        if (conv_stream_eligible(g, epi, zp))
+            return launch_conv_stream(g, x, packed, epi, out, s);
 
         // 3x3 layers over 64 channels with an NCHW output keep their filter in registers and read the
         // input in whichever layout it has: no transposition, no scratch
