@@ -436,7 +436,7 @@ namespace hipq
         const int fill = (xzp & 0xFF) * 0x01010101;
         const int32_t mult = (x_unsigned ? 128 : 0) - xzp;
         const int32_t corr[2] = {mult * wsum_n[0], mult * wsum_n[1]};
-        // INTERPRETER requantization in fixed point needs |acc * scale| * 256 < 2^31
+        // interp_small needs |acc * scale| < 2^22
         const float acc_max = static_cast<float>(kred) * (255.0f * 128.0f);
         const bool fast_interp = fabsf(ec.scale) * acc_max < 4194304.0f;
 
@@ -592,8 +592,7 @@ namespace hipq
                     constexpr int ti0 = decltype(ti0_c)::value, ti1 = decltype(ti1_c)::value;
                     constexpr bool FAST = decltype(fast_c)::value;
                     constexpr bool SUM = decltype(sum_c)::value;
-                    const float s256 = __fmul_rn(ec.scale, 256.0f);
-                    const int32_t c256 = 128 + 256 * ec.ozp;
+                    const float away = interp_magic(ec);
                     const float lo = fmaxf(ec.lo, ec.relu_floor);
 #pragma unroll
                     for (int ni = 0; ni < 2; ++ni)
@@ -620,9 +619,7 @@ namespace hipq
                                                 s4[e] = static_cast<float>(load_q(epi.sum_in, epi.sum_t, (img_pix0 + bpix + e) * p.K + n));
                                     }
                                 }
-                                // x[e]: the output byte sits in byte BYTE of x[e]
-                                constexpr int BYTE = (MODE == EPI_INTERP && FAST && KIND == OUT_Q8) ? 1 : 0;
-                                int32_t x[4];
+                                int32_t x[4]; // (8-bit outputs: in the low byte)
 #pragma unroll
                                 for (int e = 0; e < 4; ++e)
                                 {
@@ -630,12 +627,7 @@ namespace hipq
                                     if (KIND != OUT_Q8)
                                         x[e] = epi_interp<KIND>(ec, a);
                                     else if (MODE == EPI_INTERP && FAST)
-                                    {
-                                        // t = trunc(256 v); round-half-away(v) = (t + 128 - (t < 0)) >> 8, exactly:
-                                        // for t >= 0 it is floor(v + 1/2), for t < 0 it is ceil(v - 1/2)
-                                        const int32_t t = static_cast<int32_t>(__fmul_rn(static_cast<float>(a), s256));
-                                        x[e] = t + (t >> 31) + c256;
-                                    }
+                                        x[e] = interp_small(__fmul_rn(static_cast<float>(a), ec.scale), away);
                                     else if (MODE == EPI_INTERP)
                                         x[e] = epi_interp<KIND>(ec, a);
                                     else
@@ -652,7 +644,7 @@ namespace hipq
                                 {
                                     if (OUT_NCX)
                                     {
-                                        constexpr uint32_t sel = BYTE ? 0x0c0c0501u : 0x0c0c0400u;
+                                        constexpr uint32_t sel = 0x0c0c0400u;
                                         const uint32_t lo2 = __builtin_amdgcn_perm(x[1], x[0], sel);
                                         const uint32_t hi2 = __builtin_amdgcn_perm(x[3], x[2], sel);
                                         *reinterpret_cast<uint32_t*>(stage + n * kStagePitch + lpix - (kStageHalf ? ti0 * 32 : 0)) = (hi2 << 16) | lo2;
@@ -661,7 +653,7 @@ namespace hipq
                                     {
 #pragma unroll
                                         for (int e = 0; e < 4; ++e)
-                                            stage[(lpix - (kStageHalf ? ti0 * 32 : 0) + e) * 64 + n] = static_cast<uint8_t>(BYTE ? (x[e] >> 8) : x[e]);
+                                            stage[(lpix - (kStageHalf ? ti0 * 32 : 0) + e) * 64 + n] = static_cast<uint8_t>(x[e]);
                                     }
                                 }
                                 else if (n < p.K && bpix < npix)

@@ -449,8 +449,7 @@ namespace hipq
             };
             const float clamp_lo = fmaxf(ec.lo, ec.relu_floor);
             const float magic = 12582912.0f; // 1.5 * 2^23: adding it rounds half to even into the low mantissa bits
-            const float s256 = __fmul_rn(ec.scale, 256.0f);
-            const int32_t c256 = 128 + 256 * ec.ozp;
+            const float away = interp_magic(ec);
             const bool fast_interp = fabsf(ec.scale) * (static_cast<float>(Kred) * (255.0f * 128.0f)) < 4194304.0f;
             const GeluQuantize gelu = gelu_quantize_of(post_scale, post_zp, epi.post_t, epi.post_mode);
             auto epilogue = [&](auto to_u8) {
@@ -559,14 +558,11 @@ namespace hipq
                             for (int e = 0; e < 4; ++e)
                             {
                                 if (fast_interp) // uniform
-                                {
-                                    const int32_t t = static_cast<int32_t>(__fmul_rn(static_cast<float>(a[e]), s256));
-                                    x[e] = t + (t >> 31) + c256;
-                                }
+                                    x[e] = interp_small(__fmul_rn(static_cast<float>(a[e]), ec.scale), away);
                                 else
-                                    x[e] = epi_interp<OUT_Q8>(ec, a[e]) << 8;
+                                    x[e] = epi_interp<OUT_Q8>(ec, a[e]);
                             }
-                            return (__builtin_amdgcn_perm(x[3], x[2], 0x0c0c0501u) << 16) | __builtin_amdgcn_perm(x[1], x[0], 0x0c0c0501u);
+                            return (__builtin_amdgcn_perm(x[3], x[2], 0x0c0c0400u) << 16) | __builtin_amdgcn_perm(x[1], x[0], 0x0c0c0400u);
                         }
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
