@@ -283,6 +283,297 @@ namespace hipq
             return check_launch("conv_chain_i8_16x16x64");
         }
 
+        // ---- 256 -> 1024 -> 256 channels --------------------------------------------------------------------
+        // Both layers' weights are 512 KB: no wavefronts hold them.  A workgroup takes all channels of 16 (P0 + P1) pixels, whose data
+        // stay in LDS, and streams the weights past them once, in slices of 256 rows x 128 bytes through a ring of three in LDS: for
+        // every 256 channels of the wide result two slices of the widening layer, then (requantized, through LDS) two of the narrow
+        // one, whose sums stay in registers to the end.  A wavefront has 64 channels of half of the pixels (four blocks of 16 and three
+        // for 112 pixels: the two halves share each SIMD); rows of weights are dealt to lanes as above.  The residual arrives where the
+        // wide bytes will stand, a lane's bytes in place of its own.  One barrier a slice; loads two slices ahead.
+        //
+        // Bound by the matrix cores and the LDS reads that feed them, which a barrier a slice keeps from overlapping: 25 088 pixels are
+        // 26 GOP and 64 MB (10 us each way); a workgroup of 112 pixels takes 4.0 us for 256 channels of the wide result, 1.4 for a
+        // block of 16 pixels and 5.2 before and after them.  Two launches and one, looped: 25 088 pixels 32.4 -> 25.0 us, 12 544
+        // 23.0 -> 16.6, 6 272 15.2 -> 12.9.  ResNet-50 of 128 images 1222 -> 1196 us, of 64 806 -> 788, of 32 578 -> 573.
+        // Tried and taken back: all fragments of a slice read ahead of its products, with the wavefront's priority raised or not (no
+        // faster).  Without the loads of weights the same time, without the requantization 0.8 us less.
+        constexpr int kBlockC = 256, kBlockN1 = 1024, kBlockN2 = 256;
+        constexpr int kBlockSlice = 256 * 128; // bytes of a slice of weights
+        constexpr size_t chain_block_lds(int blocks) { return 2 * static_cast<size_t>(blocks) * 4096 + 3 * static_cast<size_t>(kBlockSlice) + 4096; }
+
+        template <int P0, int P1, bool I8>
+        __global__ __launch_bounds__(512, 2) void conv_chain_block_kernel(const ChainParams p)
+        {
+            touch_arguments<sizeof(ChainParams)>();
+            constexpr int PB = P0 + P1;
+            constexpr int PIECES = PB * 4;                     // of the data: 16 pixels x 64 channels, as the lanes read them
+            extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [PB][4][1024] data, [PB][4][1024] wide, [3] slices, [3][256] wsum, bias, scale, 1 KB for loads of nothing
+            uint8_t* const xs = lds;
+            uint8_t* const ys = lds + PB * 4096;
+            uint8_t* const ring = lds + 2 * PB * 4096;
+            const uint8_t* const params = ring + 3 * kBlockSlice;
+            const int tid = static_cast<int>(threadIdx.x);
+            const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+            const int r16 = lane & 15, kc = lane >> 4;
+            const int wm = wave >> 2, wn = wave & 3;
+            const int m0 = static_cast<int>(blockIdx.x) * 16 * PB;
+            const int channel = wn * 64 + kc * 16; // the lane's first channel within 256
+
+            // ---- constants of the narrow layer, and whether biases go into the accumulators (as above) ---------
+            auto words = [](const void* from, int at) { return *reinterpret_cast<const v4i_at4*>(static_cast<const int32_t*>(from) + at); };
+            bool small = true;
+            auto look = [&](const int32_t* bias, int n) {
+                if (bias && n >= 0)
+                    small = small && bias[n] >= -(1 << 24) && bias[n] <= (1 << 24);
+            };
+            look(p.l1.bias, tid);
+            look(p.l1.bias, tid + 512);
+            look(p.l2.bias, tid & 255);
+            v4i wsum2[4], bias2[4];
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+            {
+                wsum2[b] = words(p.l2.wsum, channel + 4 * b);
+                bias2[b] = p.l2.bias ? words(p.l2.bias, channel + 4 * b) : v4i{0, 0, 0, 0};
+            }
+            const float sum_scale = *p.sum_scale, one1 = p.l1.scale[0], one2 = p.l2.scale[0];
+
+            // ---- loads ---------------------------------------------------------------------------------------
+            const v4i xw = rsrc_words(p.x, static_cast<uint32_t>(p.M) * kBlockC), sw = rsrc_words(p.sum, static_cast<uint32_t>(p.M) * kBlockN1);
+            const v4i w1 = rsrc_words(p.l1.w, kBlockN1 * kBlockC), w2 = rsrc_words(p.l2.w, kBlockN2 * kBlockN1);
+            const __amdgpu_buffer_rsrc_t ors = make_rsrc(p.out, static_cast<uint32_t>(p.M) * kBlockN1);
+            const __amdgpu_buffer_rsrc_t nrs = make_rsrc(p.narrow, static_cast<uint32_t>(p.M) * kBlockN2);
+            const uint32_t xs_at = lds_address(xs), ys_at = lds_address(ys), ring_at = lds_address(ring), params_at = lds_address(params);
+            auto dma4 = [](v4i rsrc, int32_t off, uint32_t to) {
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(to), "v"(off), "s"(rsrc));
+            };
+            // wsum, bias, scale of 256 channels from `first` (zeros for absent arrays): twelve pieces of 64
+            auto load_params = [&](const ChainLayer& l, int first) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                {
+                    const int piece = j * 8 + wave, array = piece >> 2; // uniform
+                    const void* const from = array == 0 ? static_cast<const void*>(l.wsum) : array == 1 ? static_cast<const void*>(l.bias) : static_cast<const void*>(l.scale);
+                    const bool there = array == 0 || (array == 1 && l.bias != nullptr) || (array == 2 && l.per_channel != 0);
+                    dma4(rsrc_words(from, there ? kBlockN1 * 4u : 0u), (first + (piece & 3) * 64 + lane) * 4, __builtin_amdgcn_readfirstlane(params_at + piece * 256));
+                }
+            };
+            // a load of the workgroup covers 64 rows of a slice, eight lanes a row: whole lines.  Chunk c of row r stands at position
+            // c ^ (r % 4 / 2 + r / 16 % 4 * 2) of the row: sixteen lanes of a fragment meet sixteen columns of the banks
+            const int lrow = wave * 8 + (lane >> 3);
+            const int chunk = ((lane & 7) ^ (((lrow >> 1) & 1) | (((lrow >> 4) & 3) << 1))) * 16;
+            const int at1 = lrow * kBlockC + chunk, at2 = lrow * kBlockN1 + chunk;
+            // slice j % 4 of channels 256 (j / 4) ..: two of the widening layer's rows, two of the narrow layer's columns.  (Beyond
+            // the last: rows beyond the weights, zeros)
+            auto load_widen = [&](int blk, int half, int slot) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    lds_dma16_unfenced(w1, at1 + (blk * 256 + i * 64) * kBlockC + half * 128, __builtin_amdgcn_readfirstlane(ring_at + slot * kBlockSlice + i * 8192 + wave * 1024));
+            };
+            auto load_narrow = [&](int blk, int half, int slot) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    lds_dma16_unfenced(w2, at2 + i * 64 * kBlockN1 + blk * 256 + half * 128, __builtin_amdgcn_readfirstlane(ring_at + slot * kBlockSlice + i * 8192 + wave * 1024));
+            };
+#pragma unroll
+            for (int j = 0; j < (PIECES + 7) / 8; ++j)
+            {
+                const int piece = j * 8 + wave; // uniform
+                const int m = m0 + (piece >> 2) * 16 + r16;
+                lds_dma16_unfenced(xw, piece < PIECES && m < p.M ? m * kBlockC + (piece & 3) * 64 + kc * 16 : kOob,
+                                   __builtin_amdgcn_readfirstlane(piece < PIECES ? xs_at + piece * 1024 : params_at + 3072));
+            }
+            load_params(p.l1, 0);
+            load_widen(0, 0, 0);
+            load_widen(0, 1, 1);
+            wait_vmcnt<8>(); // data and constants
+            auto flip = [](v4i v, int mask) { return v4i{v[0] ^ mask, v[1] ^ mask, v[2] ^ mask, v[3] ^ mask}; };
+            const int n_mask = p.l2.x_unsigned ? static_cast<int>(0x80808080u) : 0;
+            if (p.l1.x_unsigned) // uniform
+#pragma unroll
+                for (int j = 0; j < (PIECES + 7) / 8; ++j)
+                    if (j * 8 + wave < PIECES) // uniform; the lane's own bytes
+                    {
+                        v4i* const at = reinterpret_cast<v4i*>(xs + (j * 8 + wave) * 1024 + lane * 16);
+                        *at = flip(*at, static_cast<int>(0x80808080u));
+                    }
+            const bool fold = __syncthreads_and(small) != 0;
+
+            // fragments of a slice: rows 64 wn + 16 (r / 4) + 4 b + r % 4, 64 bytes
+            const int f_row = (wn * 64 + 16 * (r16 >> 2) + (r16 & 3)) * 128;
+            const int f_at[2] = {f_row + ((kc ^ (r16 >> 1)) << 4), f_row + (((4 + kc) ^ (r16 >> 1)) << 4)};
+
+            auto run = [&](auto folded, auto blocks) {
+                constexpr bool FOLD = decltype(folded)::value;
+                constexpr int P = decltype(blocks)::value; // the wavefront's blocks of pixels
+                const int px0 = wm * P0;
+                const uint8_t* const xl = xs + px0 * 4096 + lane * 16;
+                uint8_t* const yl = ys + px0 * 4096 + lane * 16;
+                auto pixel = [&](int i) { return m0 + (px0 + i) * 16 + r16; };
+                auto pack = [](float v, int e, uint32_t packed) { return __builtin_amdgcn_cvt_pk_u8_f32(v, e, packed); };
+                v4i acc1[P][4], acc2[P][4];
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+                {
+                    const v4i start = (p.l2.x_unsigned ? 128 * wsum2[b] : v4i{0, 0, 0, 0}) + (FOLD ? bias2[b] : v4i{0, 0, 0, 0});
+#pragma unroll
+                    for (int i = 0; i < P; ++i)
+                        acc2[i][b] = start;
+                }
+                // 128 bytes of the reduction: `from` is the lane's place in the first of their two pieces of the data
+                auto multiply = [&](v4i (&acc)[P][4], const uint8_t* from, int slot) {
+#pragma unroll
+                    for (int k = 0; k < 2; ++k)
+                    {
+                        v4i wf[4], xf[P];
+#pragma unroll
+                        for (int b = 0; b < 4; ++b)
+                            wf[b] = *reinterpret_cast<const v4i*>(ring + slot * kBlockSlice + f_at[k] + b * 512);
+#pragma unroll
+                        for (int i = 0; i < P; ++i)
+                            xf[i] = *reinterpret_cast<const v4i*>(from + i * 4096 + k * 1024);
+#pragma unroll
+                        for (int i = 0; i < P; ++i)
+#pragma unroll
+                            for (int b = 0; b < 4; ++b)
+                                acc[i][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[b], xf[i], acc[i][b], 0, 0, 0);
+                    }
+                };
+                // the slice's loads have landed (LATER loads and stores of this wavefront since may be in flight), and behind the
+                // barrier everyone's; everyone has read the slice before, whose place the loads two slices ahead take
+                auto next_slice = [](auto later) { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(decltype(later)::value) : "memory"); };
+                auto after = [](int slot, int n) { return slot + n >= 3 ? slot + n - 3 : slot + n; };
+                int slot = 0;
+                for (int blk = 0; blk < kBlockN1 / 256; ++blk)
+                {
+                    next_slice(std::integral_constant<int, 4>{});
+#pragma unroll
+                    for (int i = 0; i < P; ++i)
+                        lds_dma16_unfenced(sw, pixel(i) < p.M ? pixel(i) * kBlockN1 + blk * 256 + channel : kOob, __builtin_amdgcn_readfirstlane(ys_at + (px0 + i) * 4096 + wn * 1024));
+                    load_narrow(blk, 0, after(slot, 2));
+                    const v4i* const constants = reinterpret_cast<const v4i*>(params + channel * 4);
+#pragma unroll
+                    for (int b = 0; b < 4; ++b)
+                    {
+                        const v4i start = (p.l1.x_unsigned ? 128 * constants[b] : v4i{0, 0, 0, 0}) + (FOLD ? constants[64 + b] : v4i{0, 0, 0, 0});
+#pragma unroll
+                        for (int i = 0; i < P; ++i)
+                            acc1[i][b] = start;
+                    }
+                    multiply(acc1, xl, slot);
+                    slot = after(slot, 1);
+                    next_slice(std::integral_constant<int, 4 + P>{});
+                    load_narrow(blk, 1, after(slot, 2));
+                    multiply(acc1, xl + 2048, slot);
+                    slot = after(slot, 1);
+                    wait_vmcnt<8>(); // the residual, the lane's own bytes
+#pragma unroll
+                    for (int i = 0; i < P; ++i)
+                    {
+                        v4i* const place = reinterpret_cast<v4i*>(yl + i * 4096 + wn * 1024);
+                        const v4i res = *place;
+                        v4i y;
+#pragma unroll
+                        for (int b = 0; b < 4; ++b)
+                        {
+                            const v4f scale = p.l1.per_channel ? __builtin_bit_cast(v4f, constants[128 + b]) : v4f{one1, one1, one1, one1};
+                            const v4i bias = FOLD ? v4i{0, 0, 0, 0} : constants[64 + b];
+                            uint32_t packed = 0;
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                            {
+                                const uint32_t byte = (static_cast<uint32_t>(res[b]) >> (8 * e)) & 0xFFu;
+                                const float r = I8 ? static_cast<float>(static_cast<int8_t>(byte)) : static_cast<float>(byte);
+                                const float f = static_cast<float>(acc1[i][b][e]);
+                                packed = pack(fmaf(sum_scale, r, __fmul_rn(FOLD ? f : __fadd_rn(f, static_cast<float>(bias[e])), scale[e])), e, packed);
+                            }
+                            if constexpr (I8) // 127 at most
+                            {
+                                const uint32_t high = packed & 0x80808080u;
+                                packed = (packed | (high - (high >> 7))) & 0x7f7f7f7fu;
+                            }
+                            y[b] = static_cast<int>(packed);
+                        }
+                        __builtin_amdgcn_raw_buffer_store_b128(y, ors, pixel(i) < p.M ? pixel(i) * kBlockN1 + blk * 256 + channel : kOob, 0, 0);
+                        *place = flip(y, n_mask);
+                    }
+                    next_slice(std::integral_constant<int, 4 + P>{});
+                    load_params(blk + 1 < kBlockN1 / 256 ? p.l1 : p.l2, (blk + 1) % (kBlockN1 / 256) * 256);
+                    load_widen(blk + 1, 0, after(slot, 2));
+                    multiply(acc2, yl, slot);
+                    slot = after(slot, 1);
+                    next_slice(std::integral_constant<int, 6 + P>{});
+                    load_widen(blk + 1, 1, after(slot, 2));
+                    multiply(acc2, yl + 2048, slot);
+                    slot = after(slot, 1);
+                }
+                next_slice(std::integral_constant<int, 4>{}); // the narrow layer's constants
+#pragma unroll
+                for (int i = 0; i < P; ++i)
+                {
+                    const v4i* const constants = reinterpret_cast<const v4i*>(params + channel * 4);
+                    v4i z;
+#pragma unroll
+                    for (int b = 0; b < 4; ++b)
+                    {
+                        const v4f scale = p.l2.per_channel ? __builtin_bit_cast(v4f, constants[128 + b]) : v4f{one2, one2, one2, one2};
+                        const v4i bias = FOLD ? v4i{0, 0, 0, 0} : constants[64 + b];
+                        uint32_t packed = 0;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                        {
+                            const float f = static_cast<float>(acc2[i][b][e]);
+                            packed = pack(__fmul_rn(FOLD ? f : __fadd_rn(f, static_cast<float>(bias[e])), scale[e]), e, packed);
+                        }
+                        z[b] = static_cast<int>(packed);
+                    }
+                    __builtin_amdgcn_raw_buffer_store_b128(z, nrs, pixel(i) < p.M ? pixel(i) * kBlockN2 + channel : kOob, 0, 0);
+                }
+            };
+            auto half = [&](auto folded) {
+                if (P0 == P1 || wm == 0) // uniform over the wavefront; both sides meet the same barriers
+                    run(folded, std::integral_constant<int, P0>{});
+                else
+                    run(folded, std::integral_constant<int, P1>{});
+            };
+            if (fold) // uniform
+                half(std::true_type{});
+            else
+                half(std::false_type{});
+            wait_vmcnt<0>(); // nothing may still be on its way into LDS when the wavefront ends
+        }
+
+        template <int P0, int P1, bool I8>
+        int launch_chain_block(const ChainParams& p, hipStream_t s)
+        {
+            constexpr size_t bytes = chain_block_lds(P0 + P1);
+            static_assert(bytes + 512 <= 160 * 1024, "512 bytes are the barrier's that counts votes");
+            const auto kernel = conv_chain_block_kernel<P0, P1, I8>;
+            static bool configured[16] = {};
+            int dev = 0;
+            HIPQ_HIP(hipGetDevice(&dev));
+            if (dev >= 0 && dev < 16 && !configured[dev])
+            {
+                HIPQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)));
+                configured[dev] = true;
+            }
+            kernel<<<static_cast<unsigned>((p.M + 16 * (P0 + P1) - 1) / (16 * (P0 + P1))), 512, bytes, s>>>(p);
+            return check_launch("conv_chain_block_i8_16x16x64");
+        }
+
+        // pixels of a workgroup, 0: two launches are as fast.  us, 32 / 64 / 112 pixels a workgroup and two launches:
+        //    3 136 pixels  12.3  15.6  21.1  12.4      16 384  25.6  18.7  23.8  27.7      32 768  48.7  35.2  43.6  38.0      57 344  84  66  51.8  57.6
+        //    4 704         12.7  15.8  21.3  14.9      25 088  45.9  31.6  25.0  32.4      33 712  58.9  47.7  43.6  42.8      65 536  96  69  70.6  61.1
+        //    8 192         13.4  16.2  21.6  15.7      28 672  47.1  32.9  28.1  35.3      40 000  60.0  48.4  44.3  46.5     100 352 153 115  95.8  92.6
+        // A round takes what it takes: the fewest pixels with one round to them, then the two sizes with two
+        int block_pixels(int64_t M)
+        {
+            const int64_t units = device_compute_units();
+            if (M < 16 * units || M > 224 * units || (M > 128 * units && M < 144 * units))
+                return 0;
+            return M <= 32 * units ? 32 : M <= 64 * units || (M > 112 * units && M <= 128 * units) ? 64 : 112;
+        }
+
         bool pointwise(const ConvGeom& g)
         {
             if (g.in[0] != 1 || g.taps() != 1)
@@ -315,8 +606,10 @@ namespace hipq
             return g1.C == 64 && g1.K == 256 && g2.K == 64;
         // (256 channels of 512 for few pixels: 128 KB of weights are too many for a unit that has one tile, 784 pixels 10.2 us, apart
         // 8.7; the next stage of ResNet-50 begins with this pair, of three images 2352 pixels: 347 -> 345 us for the pass)
-        if (g2.K == 256 && M < 8 * device_compute_units())
+        if (g1.C == 128 && g2.K == 256 && M < 8 * device_compute_units())
             return false;
+        if (g1.C == kBlockC && g1.K == kBlockN1 && g2.K == kBlockN2)
+            return block_pixels(M) != 0;
         return (g1.C == 64 && g1.K == 256 && (g2.K == 64 || g2.K == 128)) || (g1.C == 128 && g1.K == 512 && (g2.K == 128 || g2.K == 256));
     }
 
@@ -345,6 +638,15 @@ namespace hipq
         const bool i8 = e1.out_t == HIPQ_I8;
         if (gs)
             return launch_chain<64, 256, 64, true, true>(p, s);
+        if (g1.C == kBlockC)
+        {
+            switch (block_pixels(p.M))
+            {
+            case 112: return i8 ? launch_chain_block<4, 3, true>(p, s) : launch_chain_block<4, 3, false>(p, s);
+            case 64: return i8 ? launch_chain_block<2, 2, true>(p, s) : launch_chain_block<2, 2, false>(p, s);
+            default: return i8 ? launch_chain_block<1, 1, true>(p, s) : launch_chain_block<1, 1, false>(p, s);
+            }
+        }
         if (g1.C == 64 && g2.K == 64)
             return i8 ? launch_chain<64, 256, 64, false, true>(p, s) : launch_chain<64, 256, 64, false, false>(p, s);
         if (g1.C == 64)

@@ -101,6 +101,58 @@ def test_chain_at_the_ends_of_its_arithmetic(gpu_lib, Cc, N1, N2, shortcut, wide
             assert np.array_equal(a, b), gain
 
 
+# a workgroup's pixels by the size: 32, 64, 112, two rounds of 64 and of 112; the last one of the first, one and all but one pixel
+BLOCKS = [(1, 64, 64), (1, 1, 4097), (3, 91, 30), (1, 127, 129), (2, 4, 1025), (1, 59, 261), (1, 4, 7168), (1, 233, 125), (1, 8, 4096), (1, 8, 4625), (2, 4, 7168)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pixels", BLOCKS)
+@pytest.mark.parametrize("wide_t", ["u8", "i8"])
+def test_chain_of_blocks_equals_the_separate_calls(gpu_lib, pixels, wide_t):
+    """256 -> 1024 -> 256 channels: weights streamed past the pixels of a workgroup"""
+    for kw in (dict(), dict(data_t="i8", scalar=True), dict(bias=None)) if pixels[1] < 128 else (dict(),):
+        print("[case] chain of blocks", pixels, wide_t, kw, flush=True)
+        c = _chain(13, pixels, 256, 1024, 256, wide_t=wide_t, **kw)
+        got = H.pointwise_chain(*c)
+        assert H.last_kernel().startswith("conv_chain_block")
+        for a, b in zip(got, _apart(H.quantized_convolution_fused, *c)):
+            assert np.array_equal(a, b), kw
+            assert np.unique(a).size > 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pixels", [(1, 5, 821), (1, 9, 961), (1, 25, 673)])
+def test_chain_of_blocks_against_the_oracle(gpu_lib, pixels):
+    print("[case] chain of blocks, oracle", pixels, flush=True)
+    O.port().orc_set_threads(8)
+    c = _chain(17, pixels, 256, 1024, 256)
+    for a, b in zip(H.pointwise_chain(*c), _apart(_oracle, *c)):
+        assert np.array_equal(a, b)
+    O.port().orc_set_threads(1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pixels", [(1, 5, 821), (1, 9, 961), (1, 25, 673)])
+@pytest.mark.parametrize("wide_t", ["u8", "i8"])
+def test_chain_of_blocks_at_the_ends_of_its_arithmetic(gpu_lib, pixels, wide_t):
+    for gain in (1.0, 1e6, 1e-6, np.float32(np.inf), np.float32(np.nan)):
+        print("[case] chain of blocks, ends", pixels, wide_t, gain, flush=True)
+        c = list(_chain(19, pixels, 256, 1024, 256, wide_t=wide_t, gain=gain))
+        for i in (0, 2):
+            if gain in (1.0, 1e-6):
+                d, f, x, filt, b, s = c[i]
+                c[i] = (d, f, x, filt, np.where(np.arange(b.size) % 3 == 0, (1 << 24) + 12345 + b, -(1 << 26) + 1 + b).astype(np.int32), s)
+        for a, b in zip(H.pointwise_chain(*c), _apart(H.quantized_convolution_fused, *c)):
+            assert np.array_equal(a, b), gain
+
+
+def test_blocks_are_for_sizes_that_fill_the_chip():
+    for pixels, fused in ((4095, False), (4096, True), (32768, True), (32769, False), (36864, True), (57344, True), (57345, False)):
+        c = [_conv((1, 1, pixels), *k, "u8", "u8") for k in ((256, 1024), (1024, 256))]
+        f = [H.make_fused_desc(has_bias=True, has_sum=s, sum_t="u8", with_relu=True, scale_count=k) for s, k in ((True, 1024), (False, 256))]
+        assert bool(H.pointwise_chain_fusable(H.pointwise_layer(c[0], f[0]), None, H.pointwise_layer(c[1], f[1]))) == fused, pixels
+
+
 def test_only_such_layers_have_a_common_kernel():
     px = (1, 8, 8)
     rows = lambda c: [None if l is None else H.pointwise_layer(l[0], l[1]) for l in c[:3]]
