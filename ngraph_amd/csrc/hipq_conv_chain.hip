@@ -294,7 +294,7 @@ namespace hipq
         // Bound by the matrix cores and the LDS reads that feed them, which a barrier a slice keeps from overlapping: 25 088 pixels are
         // 26 GOP and 64 MB (10 us each way); a workgroup of 112 pixels takes 4.0 us for 256 channels of the wide result, 1.4 for a
         // block of 16 pixels and 5.2 before and after them.  Two launches and one, looped: 25 088 pixels 32.4 -> 25.0 us, 12 544
-        // 23.0 -> 16.6, 6 272 15.2 -> 12.9.  ResNet-50 of 128 images 1222 -> 1196 us, of 64 806 -> 788, of 32 578 -> 573.
+        // 23.0 -> 16.6, 6 272 15.2 -> 12.9.  ResNet-50 of 128 images 1222 -> 1179 us, of 64 806 -> 773, of 32 578 -> 569.
         // Tried and taken back: all fragments of a slice read ahead of its products, with the wavefront's priority raised or not (no
         // faster).  Without the loads of weights the same time, without the requantization 0.8 us less.
         constexpr int kBlockC = 256, kBlockN1 = 1024, kBlockN2 = 256;
@@ -375,6 +375,18 @@ namespace hipq
                 for (int i = 0; i < 4; ++i)
                     lds_dma16_unfenced(w2, at2 + i * 64 * kBlockN1 + blk * 256 + half * 128, __builtin_amdgcn_readfirstlane(ring_at + slot * kBlockSlice + i * 8192 + wave * 1024));
             };
+            // The workgroups of a compute die (consecutive ones go to the eight of them in turn) touch a line of the weights a lane, all of
+            // them together: what the ring asks for later is then on its way into their L2, or there.  (ResNet-50, where other layers
+            // have been through it: 128 images 1190 -> 1179 us, 64 781 -> 773, 32 575 -> 569, 26, whose launch is 160 workgroups, 546 -> 541;
+            // 24, with 147, 523 either way, and 22 502 -> 504: the line is at 148)
+            if (gridDim.x >= 148) // uniform
+            {
+                constexpr int parts = 2 * kBlockN1 * kBlockC / (64 * 128); // of 64 lines
+                const int each = (parts + (static_cast<int>(gridDim.x) >> 3) - 1) / (static_cast<int>(gridDim.x) >> 3);
+                const int part = static_cast<int>(blockIdx.x >> 3) * each + wave; // uniform
+                const bool second = part >= parts / 2;
+                dma4(second ? w2 : w1, wave < each && part < parts ? (part - (second ? parts / 2 : 0)) * (64 * 128) + lane * 128 : kOob, __builtin_amdgcn_readfirstlane(params_at + 3072));
+            }
 #pragma unroll
             for (int j = 0; j < (PIECES + 7) / 8; ++j)
             {
