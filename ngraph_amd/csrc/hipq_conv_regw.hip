@@ -355,9 +355,8 @@ namespace hipq
         // ---- everyone multiplies from here on ---------------------------------------------------------
         const int32_t mult = (x_unsigned ? 128 : 0) - xzp;
         const int32_t corr[2] = {mult * wsum_n[0], mult * wsum_n[1]};
-        // interp_small needs |acc * scale| < 2^22
+        // INTERPRETER requantization in fixed point needs |acc * scale| * 256 < 2^31
         const bool fast_interp = fabsf(ec.scale) * (static_cast<float>(kRwKred) * (255.0f * 128.0f)) < 4194304.0f;
-        const float away = interp_magic(ec);
         const float s256 = __fmul_rn(ec.scale, 256.0f);
         const int32_t c256 = 128 + 256 * ec.ozp;
         const float lo = fmaxf(ec.lo, ec.relu_floor);
@@ -423,7 +422,7 @@ namespace hipq
             }
         };
         // the other half: requantize and store.  Accumulator register 4g + e is pixel 32t + 8g + 4 * (lane / 32) + e,
-        // channel ni * 32 + lane % 32.  FAST: the INTERPRETER policy by interp_small (a compile-time choice: a
+        // channel ni * 32 + lane % 32.  FAST: the INTERPRETER policy in fixed point (a compile-time choice: a
         // uniform branch per output would cost more than the arithmetic)
         auto tile_store = [&](int t, const v16i (&acc)[2], auto fast_c) {
             constexpr bool FAST = decltype(fast_c)::value;
@@ -450,10 +449,9 @@ namespace hipq
                         const int32_t a = acc[ni][4 * g + e] + corr[ni];
                         if (MODE == EPI_INTERP && FAST)
                         {
-                            // t = trunc(256 v); round-half-away(v) = (t + 128 - (t < 0)) >> 8, exactly.  (interp_small costs a wavefront
-                            // that is alone on its SIMD more: one picture of 56 x 56 5.57 us, as here 5.48)
-                            const int32_t t256 = static_cast<int32_t>(__fmul_rn(static_cast<float>(a), s256));
-                            x[e] = t256 + (t256 >> 31) + c256;
+                            // t = trunc(256 v); round-half-away(v) = (t + 128 - (t < 0)) >> 8, exactly
+                            const int32_t tt = static_cast<int32_t>(__fmul_rn(static_cast<float>(a), s256));
+                            x[e] = tt + (tt >> 31) + c256;
                         }
                         else if (MODE == EPI_INTERP)
                             x[e] = epi_interp<OUT_Q8>(ec, a);
@@ -538,12 +536,13 @@ namespace hipq
                 {
                     if (MODE == EPI_INTERP && FAST)
                     {
+                        // t = trunc(256 v); round-half-away(v) = (t + 128 - (t < 0)) >> 8, exactly
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            x[e] = __float_as_int(__fmul_rn(__int_as_float(x[e]), ec.scale));
+                            x[e] = __float_as_int(__fmul_rn(__int_as_float(x[e]), s256));
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            x[e] = x[e] + 1; // (interp_small)
+                            x[e] = static_cast<int32_t>(__int_as_float(x[e]));
                     }
                     else if (MODE == EPI_FUSED)
                     {
@@ -559,9 +558,13 @@ namespace hipq
                 {
                     if (MODE == EPI_INTERP && FAST)
                     {
+                        int32_t sg[4];
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            x[e] = __float_as_int(fmaf(__int_as_float(x[e]), kInterpTowardZero, away));
+                            sg[e] = x[e] >> 31;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            x[e] = x[e] + sg[e] + c256;
                     }
                     else if (MODE == EPI_INTERP)
                     {
@@ -588,7 +591,7 @@ namespace hipq
                 }
                 else
                 {
-                    constexpr uint32_t sel = 0x0c0c0400u;
+                    constexpr uint32_t sel = (MODE == EPI_INTERP && FAST) ? 0x0c0c0501u : 0x0c0c0400u;
                     const uint32_t lo2 = __builtin_amdgcn_perm(x[1], x[0], sel);
                     const uint32_t hi2 = __builtin_amdgcn_perm(x[3], x[2], sel);
                     d[g] = (hi2 << 16) | lo2;

@@ -669,11 +669,14 @@ namespace hipq
         return r;
     }
 
-    // INTERPRETER, 8-bit outputs, |v| < 2^22 (interp_small): roundf(v) + ozp in the low byte, two instructions.  With w the next
-    // float beyond v, w (1 - 2^-24) lies in (v, v + ulp(v) / 2): past v where that is a tie, and before the next tie where it is
-    // none (ties are floats below 2^22).  The fused sum with 1.5 * 2^23 + ozp rounds it to a whole number once.  Against trunc(256 v)
-    // with the sign added and 128, which took four, one of them a conversion at half the rate: 64 -> 64 channels 3 x 3 over 128
-    // pictures of 56 x 56 20.9 -> 20.0 us
+    // INTERPRETER, 8-bit outputs, |v| < 2^22: roundf(v) + ozp in the low byte, two instructions.  With w the next float beyond v,
+    // w (1 - 2^-24) lies in (v, v + ulp(v) / 2): past v where that is a tie, and before the next tie where it is none (ties are
+    // floats below 2^22).  The fused sum with 1.5 * 2^23 + ozp rounds it to a whole number once.  trunc(256 v) with its sign and 128
+    // added takes three, two of them at half rate.  us, with that and so: 64 -> 64 channels 3 x 3, channels-last, over 64 pictures of
+    // 56 x 56 14.5 -> 13.8, 64 -> 256 1 x 1 over 64 22.4 -> 21.4, 128 -> 128 3 x 3 over 64 of 28 x 28 15.6 -> 15.4, 2048 x 2048 x 512
+    // 7.04 -> 6.82.  conv_regw_kernel, whose requantization runs between its products, keeps trunc(256 v): 128 pictures 20.9 -> 20.0
+    // on some machines, but 22.2 -> 23.1 on those whose clock falls under this load (the same source and command; the multiplier's
+    // power is the likely reason), one picture, a wavefront alone on its SIMD, 5.48 -> 5.57.
     constexpr float kInterpTowardZero = 0x1.fffffep-1f;
     __device__ __forceinline__ float interp_magic(const EpiConst& c) { return 12582912.0f + static_cast<float>(c.ozp); }
     __device__ __forceinline__ int32_t interp_small(float v, float magic)
