@@ -436,9 +436,8 @@ namespace hipq
         const int fill = (xzp & 0xFF) * 0x01010101;
         const int32_t mult = (x_unsigned ? 128 : 0) - xzp;
         const int32_t corr[2] = {mult * wsum_n[0], mult * wsum_n[1]};
-        // interp_small needs |acc * scale| < 2^22
         const float acc_max = static_cast<float>(kred) * (255.0f * 128.0f);
-        const bool fast_interp = fabsf(ec.scale) * acc_max < 4194304.0f;
+        const bool fast_interp = fabsf(ec.scale) * acc_max < kInterpSmallEnd; // what interp_small takes
 
         // moves a band into the group's buffer; the first batch is already in xb0
         // rows of a band a lane fetches in one go: the bands of two-tile items are short

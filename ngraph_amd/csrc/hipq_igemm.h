@@ -669,15 +669,17 @@ namespace hipq
         return r;
     }
 
-    // INTERPRETER, 8-bit outputs, |v| < 2^22: roundf(v) + ozp in the low byte, two instructions.  With w the next float beyond v,
+    // INTERPRETER, 8-bit outputs, |v| < kInterpSmallEnd: roundf(v) + ozp in the low byte, two instructions.  With w the next float beyond v,
     // w (1 - 2^-24) lies in (v, v + ulp(v) / 2): past v where that is a tie, and before the next tie where it is none (ties are
-    // floats below 2^22).  The fused sum with 1.5 * 2^23 + ozp rounds it to a whole number once.  trunc(256 v) with its sign and 128
-    // added takes three, two of them at half rate.  us, with that and so: 64 -> 64 channels 3 x 3, channels-last, over 64 pictures of
+    // floats below 2^22).  The fused sum with 1.5 * 2^23 + ozp rounds it to a whole number once, as long as it stays in [2^23, 2^24),
+    // where floats are whole numbers apart: v must stay away from 2^22 by |ozp| <= 255, and by the rounding of a guard that bounds it in
+    // floats (two units).  trunc(256 v) with its sign and 128 added takes three, two of them at half rate.  us, with that and so: 64 -> 64 channels 3 x 3, channels-last, over 64 pictures of
     // 56 x 56 14.5 -> 13.8, 64 -> 256 1 x 1 over 64 22.4 -> 21.4, 128 -> 128 3 x 3 over 64 of 28 x 28 15.6 -> 15.4, 2048 x 2048 x 512
     // 7.04 -> 6.82.  conv_regw_kernel, whose requantization runs between its products, keeps trunc(256 v): 128 pictures 20.9 -> 20.0
     // on some machines, but 22.2 -> 23.1 on those whose clock falls under this load (the same source and command; the multiplier's
     // power is the likely reason), one picture, a wavefront alone on its SIMD, 5.48 -> 5.57.
     constexpr float kInterpTowardZero = 0x1.fffffep-1f;
+    constexpr float kInterpSmallEnd = 4194304.0f - 512.0f;
     __device__ __forceinline__ float interp_magic(const EpiConst& c) { return 12582912.0f + static_cast<float>(c.ozp); }
     __device__ __forceinline__ int32_t interp_small(float v, float magic)
     {
@@ -1474,8 +1476,7 @@ namespace hipq
         const float away = interp_magic(ec);
         // (Gelu + Quantize of a float result: the Quantize's scale and zero point)
         const GeluQuantize gelu = gelu_quantize_of(KIND == OUT_GELU_Q8 ? *epi.post_scale : 1.0f, KIND == OUT_GELU_Q8 ? load_zp(epi.post_zp, epi.post_t) : 0, epi.post_t, epi.post_mode);
-        // interp_small needs |acc * scale| < 2^22
-        const bool fast_interp = fabsf(ec.scale) * (static_cast<float>(Kred) * (255.0f * 128.0f)) < 4194304.0f;
+        const bool fast_interp = fabsf(ec.scale) * (static_cast<float>(Kred) * (255.0f * 128.0f)) < kInterpSmallEnd; // what interp_small takes
         constexpr int SUM_LOADS = TM * TN / 16 / 64;
         v4i sum_regs[SUM_LOADS];
         const __amdgpu_buffer_rsrc_t srs = make_rsrc(epi.sum_in, has_sum ? static_cast<uint32_t>(M * N) : 0u);

@@ -450,7 +450,7 @@ namespace hipq
             const float clamp_lo = fmaxf(ec.lo, ec.relu_floor);
             const float magic = 12582912.0f; // 1.5 * 2^23: adding it rounds half to even into the low mantissa bits
             const float away = interp_magic(ec);
-            const bool fast_interp = fabsf(ec.scale) * (static_cast<float>(Kred) * (255.0f * 128.0f)) < 4194304.0f;
+            const bool fast_interp = fabsf(ec.scale) * (static_cast<float>(Kred) * (255.0f * 128.0f)) < kInterpSmallEnd;
             const GeluQuantize gelu = gelu_quantize_of(post_scale, post_zp, epi.post_t, epi.post_mode);
             auto epilogue = [&](auto to_u8) {
                 constexpr bool PK_U8 = decltype(to_u8)::value;
