@@ -124,7 +124,9 @@ namespace hipq
 #pragma unroll
                 for (int g = 0; g < G; ++g)
                     w2[b][g] = fragment(p.l2.w, N1, o2, NB2, b, g);
-            // (a bias of up to 2^24 is carried exactly in the accumulators, which stay below 2^25 and are rounded to float once either way)
+            // (A bias of up to 2^24 is carried in the accumulators: as the sums of up to 512 products are exact as floats, float(sum + bias)
+            // rounds once, as float(sum) + float(bias) does)
+            static_assert(N1 * 255 * 128 <= (1 << 24) && C <= N1 && CS <= N1, "sums of products that are exact as floats");
             bool small = true;
             auto look = [&](const ChainLayer& l, int n) {
                 if (l.bias && tid < n) // (no more channels than threads)
@@ -319,7 +321,9 @@ namespace hipq
             const int m0 = static_cast<int>(blockIdx.x) * 16 * PB;
             const int channel = wn * 64 + kc * 16; // the lane's first channel within 256
 
-            // ---- constants of the narrow layer, and whether biases go into the accumulators (as above) ---------
+            // ---- constants of the narrow layer, and whether the widening layer's bias goes into the accumulators (as above; the narrow
+            // layer's sums reach 1024 * 255 * 128 > 2^24: float(sum) rounds before float(bias) is added, so they are never folded) ------
+            static_assert(kBlockC * 255 * 128 <= (1 << 24), "sums of products that are exact as floats");
             auto words = [](const void* from, int at) { return *reinterpret_cast<const v4i_at4*>(static_cast<const int32_t*>(from) + at); };
             bool small = true;
             auto look = [&](const int32_t* bias, int n) {
@@ -328,14 +332,10 @@ namespace hipq
             };
             look(p.l1.bias, tid);
             look(p.l1.bias, tid + 512);
-            look(p.l2.bias, tid & 255);
-            v4i wsum2[4], bias2[4];
+            v4i wsum2[4];
 #pragma unroll
             for (int b = 0; b < 4; ++b)
-            {
                 wsum2[b] = words(p.l2.wsum, channel + 4 * b);
-                bias2[b] = p.l2.bias ? words(p.l2.bias, channel + 4 * b) : v4i{0, 0, 0, 0};
-            }
             const float sum_scale = *p.sum_scale, one1 = p.l1.scale[0], one2 = p.l2.scale[0];
 
             // ---- loads ---------------------------------------------------------------------------------------
@@ -427,7 +427,7 @@ namespace hipq
 #pragma unroll
                 for (int b = 0; b < 4; ++b)
                 {
-                    const v4i start = (p.l2.x_unsigned ? 128 * wsum2[b] : v4i{0, 0, 0, 0}) + (FOLD ? bias2[b] : v4i{0, 0, 0, 0});
+                    const v4i start = p.l2.x_unsigned ? 128 * wsum2[b] : v4i{0, 0, 0, 0}; // uniform
 #pragma unroll
                     for (int i = 0; i < P; ++i)
                         acc2[i][b] = start;
@@ -529,13 +529,12 @@ namespace hipq
                     for (int b = 0; b < 4; ++b)
                     {
                         const v4f scale = p.l2.per_channel ? __builtin_bit_cast(v4f, constants[128 + b]) : v4f{one2, one2, one2, one2};
-                        const v4i bias = FOLD ? v4i{0, 0, 0, 0} : constants[64 + b];
+                        const v4i bias = constants[64 + b];
                         uint32_t packed = 0;
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
                         {
-                            const float f = static_cast<float>(acc2[i][b][e]);
-                            packed = pack(__fmul_rn(FOLD ? f : __fadd_rn(f, static_cast<float>(bias[e])), scale[e]), e, packed);
+                            packed = pack(__fmul_rn(__fadd_rn(static_cast<float>(acc2[i][b][e]), static_cast<float>(bias[e])), scale[e]), e, packed);
                         }
                         z[b] = static_cast<int>(packed);
                     }

@@ -102,6 +102,7 @@ namespace hipq
 #pragma unroll
                 for (int k = 0; k < KS; ++k)
                     wf[b4][k] = *reinterpret_cast<const v4i*>(p.w + (n_wave + 16 * (r16 >> 2) + 4 * b4 + (r16 & 3)) * C + k * 64 + kc * 16);
+            static_assert(C * 255 * 128 <= (1 << 24), "sums of products that are exact as floats: float(sum + bias) rounds once, as float(sum) + float(bias) does");
             bool small = true;
             if (p.bias)
             {

@@ -146,6 +146,40 @@ def test_chain_of_blocks_at_the_ends_of_its_arithmetic(gpu_lib, pixels, wide_t):
             assert np.array_equal(a, b), gain
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("pixels", [(1, 5, 821), (1, 9, 961), (1, 25, 673)])
+@pytest.mark.parametrize("bias", [-(1 << 24), -(1 << 24) + 255, -(1 << 24) - 2])
+def test_chain_of_blocks_where_sums_are_no_floats(gpu_lib, pixels, bias):
+    """wide bytes that are the residual's, 255 but for a few, under narrow weights of one sign: odd sums beyond 2^24, which are rounded as
+    they become floats, before a bias that leaves a byte's worth of them"""
+    print("[case] chain of blocks, sums", pixels, bias, flush=True)
+    O.port().orc_set_threads(8)
+    widen, _, narrow, residual, _ = _chain(23, pixels, 256, 1024, 256)
+    d, f, x, filt, b, s = widen
+    widen = (d, f, x, filt, b, np.full_like(s, 1e-12))
+    residual = (255 - (synth.uniform_int(3, residual.shape, 0, 1023, np.int32) == 0)).astype(np.uint8)
+    d, f, _, filt, b, s = narrow
+    weights = np.full((256, 1024), 64, np.int32)
+    weights[:, ::4] = 65
+    weights[:, : 4 * 5 : 4] -= np.arange(256)[:, None] % 6 == np.arange(5)
+    weights[:, 1] += 3 + np.arange(256) % 2  # sums of 255 * (65 794 and a little), odd and even
+    sums = 255 * weights.sum(1)
+    assert sums.min() > 2**24 and (sums % 2 == 1).any() and (sums % 2 == 0).any()
+    b = np.full(256, bias, np.int32)
+    s = (0.5 + np.arange(256) % 3 * 0.25).astype(np.float32)
+    for sign in (1, -1):
+        c = widen, None, (d, f, None, (sign * weights).astype(np.int8).reshape(256, 1024, 1, 1), sign * b, sign * s), residual, 1.0
+        got = H.pointwise_chain(*c)
+        assert H.last_kernel().startswith("conv_chain_block")
+        apart = _apart(H.quantized_convolution_fused, *c)
+        for a, e in zip(got, apart):
+            assert np.array_equal(a, e)
+        for a, e in zip(got, _apart(_oracle, *c) if pixels[1] == 5 else ()):
+            assert np.array_equal(a, e)
+        assert np.array_equal(got[0], residual) and np.unique(got[1]).size > 8
+    O.port().orc_set_threads(1)
+
+
 def test_blocks_are_for_sizes_that_fill_the_chip():
     for pixels, fused in ((4095, False), (4096, True), (32768, True), (32769, False), (36864, True), (57344, True), (57345, False)):
         c = [_conv((1, 1, pixels), *k, "u8", "u8") for k in ((256, 1024), (1024, 256))]
