@@ -253,6 +253,8 @@ namespace hipq
             return false;
         if (g.data_layout != HIPQ_LAYOUT_NXC || g.out_layout != HIPQ_LAYOUT_NXC)
             return false;
+        if ((reinterpret_cast<uintptr_t>(epi.sum_in) & 15) != 0) // (the tile kernels take a residual at any word)
+            return false;
         if ((g.C != 64 && g.C != 128 && g.C != 256 && g.C != 512) || g.K % (g.C == 512 ? 256 : g.C == 256 ? 128 : 64) != 0 || g.K > 2048)
             return false;
         // From how many outputs a compute unit on: the weights' way into the registers has to be paid for, the more so the longer the
@@ -272,8 +274,7 @@ namespace hipq
 
     int launch_conv_stream(const ConvGeom& g, const void* data, const void* packed, const Epilogue& epi, void* out, hipStream_t s)
     {
-        HIPQ_REQUIRE((reinterpret_cast<uintptr_t>(data) & 15) == 0 && (reinterpret_cast<uintptr_t>(packed) & 15) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0 &&
-                         (reinterpret_cast<uintptr_t>(epi.sum_in) & 15) == 0,
+        HIPQ_REQUIRE((reinterpret_cast<uintptr_t>(data) & 15) == 0 && (reinterpret_cast<uintptr_t>(packed) & 15) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0,
                      "MFMA convolution needs 16-byte aligned tensors");
         StreamParams p;
         memset(&p, 0, sizeof(p));

@@ -60,6 +60,23 @@ def test_stream_equals_the_tile_kernels(gpu_lib, n, hw, Cc, K, stride, monkeypat
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,hw,Cc,K,stride", [(1, (64, 64), 64, 64, (1, 1)), (2, (128, 65), 64, 256, (2, 1)), (21, (28, 28), 512, 2048, (1, 1))])
+def test_a_residual_off_16_bytes_takes_the_tile_kernels(gpu_lib, n, hw, Cc, K, stride):
+    d, f, x, filt, b, res, s, ss = _case(6, n, hw, Cc, K, stride, sum_t="u8")
+    want = H.quantized_convolution_fused(d, f, x, filt, b, res, s, ss)
+    assert H.last_kernel() == "conv_stream_i8_16x16x64"
+    bx, bf, bb, bs, bss = (H._dev(a) for a in (x, filt, b, s, np.float32(ss)))
+    packed, out = H.pack_filter(d, bf), H.DeviceBuffer(want.size)
+    for offset in (4, 8, 12, 16):
+        print("[case] stream, residual at", offset, n, hw, Cc, K, flush=True)
+        br = H._dev(np.concatenate([np.full(offset, 77, np.uint8), res.ravel(), np.full(64 - offset, 77, np.uint8)]))
+        H.check(gpu_lib.hipq_quantized_convolution_fused(H.C.byref(d), H.C.byref(f), bx.ptr, bf.ptr, packed.ptr, bb.ptr, br.ptr + offset, bs.ptr, bss.ptr, out.ptr, None))
+        assert ("stream" if offset == 16 else "mfma") in H.last_kernel()
+        H.check(gpu_lib.hipq_stream_sync(None))
+        assert np.array_equal(out.to_numpy(np.uint8, want.shape), want), offset
+
+
+@pytest.mark.gpu
 def test_stream_takes_the_layers_it_is_for(gpu_lib):
     for n, hw, Cc, K, sum_t, stream in ((1, 63, 64, 64, None, False), (1, 64, 64, 64, None, True), (2, 112, 128, 192, None, False), (21, 56, 128, 192, None, True), (8, 56, 256, 512, None, False),
                                         (11, 56, 256, 512, "u8", True), (21, 28, 512, 2048, "u8", True), (20, 56, 96, 192, None, False), (20, 56, 64, 80, None, False)):
