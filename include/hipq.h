@@ -535,8 +535,8 @@ HIPQ_API int hipq_quantized_convolution_fused_max_pool(const hipq_conv_desc_t* d
  * be null): 1 x 1 filters of stride 1 over channels-last pixels; 64 channels to 256 to 64 or 128, or
  * 128 to 512 to 128, or to 256 over many pixels, or 256 to 1024 to 256 over as many as fill the chip in one or two rounds; the wide result after a ReLU, of the residual's type; the narrow result u8 without a
  * residual; a shortcut with an i8 result from 64 channels, to 256 and then 64.  Filters packed
- * (hipq_conv_pack_filter), tensors 16-byte aligned; HIPQ_ERR_UNSUPPORTED for anything else: the
- * caller then makes the separate calls.
+ * (hipq_conv_pack_filter), tensors 16-byte aligned; HIPQ_ERR_UNSUPPORTED for anything else that the
+ * separate calls may take: the caller then makes those.
  */
 typedef struct
 {

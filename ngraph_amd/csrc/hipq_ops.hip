@@ -488,6 +488,8 @@ static int chain_layers(const hipq_pointwise_layer_t* widen, const hipq_pointwis
         rc = check_conv_types(g[i], true);
         if (rc)
             return rc;
+        if (i != 0 && layers[i]->fused && layers[i]->fused->has_sum)
+            return fail(HIPQ_ERR_UNSUPPORTED, "the narrowing layer and the shortcut of a pointwise chain have no residual");
         rc = fused_epilogue(layers[i]->fused, g[i].out_t, g[i].K, layers[i]->bias, i == 0 ? sum : nullptr, layers[i]->scale, i == 0 ? sum_scale : nullptr, &e[i]);
         if (rc)
             return rc;
@@ -532,9 +534,9 @@ int hipq_pointwise_chain(const hipq_pointwise_layer_t* widen,
         return rc;
     HIPQ_REQUIRE(widen->data && widen->packed_filter && narrow->packed_filter && (!shortcut || shortcut->packed_filter) && wide_out && narrow_out, "null tensor pointer");
     auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    HIPQ_REQUIRE(aligned(widen->data) && aligned(widen->packed_filter) && aligned(e[0].sum_in) && aligned(narrow->packed_filter) && (!shortcut || aligned(shortcut->packed_filter)) &&
-                     aligned(wide_out) && aligned(narrow_out),
-                 "tensors must be 16-byte aligned");
+    if (!aligned(widen->data) || !aligned(widen->packed_filter) || !aligned(e[0].sum_in) || !aligned(narrow->packed_filter) || (shortcut && !aligned(shortcut->packed_filter)) || !aligned(wide_out) ||
+        !aligned(narrow_out))
+        return fail(HIPQ_ERR_UNSUPPORTED, "tensors of a pointwise chain must be 16-byte aligned");
     return launch_conv_chain(g[0], e[0], widen->data, widen->packed_filter, shortcut ? &g[1] : nullptr, shortcut ? &e[1] : nullptr, shortcut ? shortcut->packed_filter : nullptr, g[2], e[2],
                              narrow->packed_filter, wide_out, narrow_out, as_stream(stream));
 }

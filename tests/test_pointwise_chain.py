@@ -1,4 +1,6 @@
 """Two or three 1 x 1 layers in one launch (hipq_pointwise_chain) against the CPU oracle and against the separate calls."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -207,6 +209,27 @@ def test_only_such_layers_have_a_common_kernel():
     assert not H.pointwise_chain_fusable(H.pointwise_layer(planes, w[1]), None, H.pointwise_layer(n[0], n[1]))
     assert H.load().hipq_pointwise_chain(None, None, None, None, None, None, None, None) == H.ERR_INVALID
     wl, nl = H.pointwise_layer(w[0], w[1]), H.pointwise_layer(n[0], n[1])
-    import ctypes as C
-
     assert H.load().hipq_pointwise_chain(C.byref(wl), None, C.byref(nl), None, None, None, None, None) == H.ERR_INVALID
+
+
+def _refused(widen, short, narrow, sum_at=None, wide_at=1 << 32, narrow_at=2 << 32, data_at=3 << 32, short_at=4 << 32):
+    """the error of a chain whose tensors stand at made-up addresses, which no call that is refused looks at"""
+    layer = lambda l, at: None if l is None else H.PointwiseLayer(C.pointer(l[0]), C.pointer(l[1]), at, 5 << 32, 6 << 32, 7 << 32)
+    w, s, n = layer(widen, data_at), layer(short, short_at), layer(narrow, None)
+    rc = H.load().hipq_pointwise_chain(H._layer_ref(w), H._layer_ref(s), H._layer_ref(n), sum_at, 8 << 32, wide_at, narrow_at, None)
+    assert rc != 0
+    return rc
+
+
+def test_what_the_separate_calls_may_take_is_unsupported_not_invalid():
+    px = (1, 8, 8)
+    for shortcut in (False, True):
+        w, s, n = _chain(1, px, 64, 256, 64, shortcut, wide_t="i8")[:3]
+        at = dict(sum_at=None if shortcut else 9 << 32)
+        more = H.make_fused_desc(has_bias=True, has_sum=True, sum_t="u8", with_relu=True, scale_count=64)
+        assert _refused(w, s, (n[0], more), **at) == H.ERR_UNSUPPORTED
+        if shortcut:
+            more = H.make_fused_desc(has_bias=True, has_sum=True, sum_t="i8", scale_count=256)
+            assert _refused(w, (s[0], more), n, **at) == H.ERR_UNSUPPORTED
+        for off in ("wide_at", "narrow_at", "data_at", "short_at" if shortcut else "sum_at"):
+            assert _refused(w, s, n, **{**at, off: (10 << 32) + 8}) == H.ERR_UNSUPPORTED, off
