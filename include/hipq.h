@@ -537,6 +537,9 @@ HIPQ_API int hipq_quantized_convolution_fused_max_pool(const hipq_conv_desc_t* d
  * residual; a shortcut with an i8 result from 64 channels, to 256 and then 64.  Filters packed
  * (hipq_conv_pack_filter), tensors 16-byte aligned; HIPQ_ERR_UNSUPPORTED for anything else that the
  * separate calls may take: the caller then makes those.
+ * All of one launch, so neither result may overlap the other or an input (HIPQ_ERR_UNSUPPORTED), even one
+ * that is dead by the time the separate calls write it; but a result may take the place of an input
+ * with as many channels, at the same address: wide_out of sum_in, narrow_out of the data.
  */
 typedef struct
 {

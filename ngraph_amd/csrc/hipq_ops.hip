@@ -537,6 +537,16 @@ int hipq_pointwise_chain(const hipq_pointwise_layer_t* widen,
     if (!aligned(widen->data) || !aligned(widen->packed_filter) || !aligned(e[0].sum_in) || !aligned(narrow->packed_filter) || (shortcut && !aligned(shortcut->packed_filter)) || !aligned(wide_out) ||
         !aligned(narrow_out))
         return fail(HIPQ_ERR_UNSUPPORTED, "tensors of a pointwise chain must be 16-byte aligned");
+    // A workgroup writes its pixels of both results while others have not read theirs: an output may stand on an input only pixel by pixel
+    const int64_t pixels = g[0].N * g[0].in[1] * g[0].in[2];
+    auto clash = [&](const void* out, int64_t out_row, const void* in, int64_t in_row) {
+        const uintptr_t o = reinterpret_cast<uintptr_t>(out), i = reinterpret_cast<uintptr_t>(in);
+        return o < i + pixels * in_row && i < o + pixels * out_row && !(o == i && out_row == in_row);
+    };
+    const int64_t sum_row = shortcut ? g[1].C : g[0].K;
+    if (clash(wide_out, g[0].K, widen->data, g[0].C) || clash(wide_out, g[0].K, e[0].sum_in, sum_row) || clash(narrow_out, g[2].K, widen->data, g[0].C) ||
+        clash(narrow_out, g[2].K, e[0].sum_in, sum_row) || clash(narrow_out, g[2].K, wide_out, g[0].K))
+        return fail(HIPQ_ERR_UNSUPPORTED, "results of a pointwise chain overlap its inputs or each other");
     return launch_conv_chain(g[0], e[0], widen->data, widen->packed_filter, shortcut ? &g[1] : nullptr, shortcut ? &e[1] : nullptr, shortcut ? shortcut->packed_filter : nullptr, g[2], e[2],
                              narrow->packed_filter, wide_out, narrow_out, as_stream(stream));
 }

@@ -233,3 +233,40 @@ def test_what_the_separate_calls_may_take_is_unsupported_not_invalid():
             assert _refused(w, (s[0], more), n, **at) == H.ERR_UNSUPPORTED
         for off in ("wide_at", "narrow_at", "data_at", "short_at" if shortcut else "sum_at"):
             assert _refused(w, s, n, **{**at, off: (10 << 32) + 8}) == H.ERR_UNSUPPORTED, off
+
+
+def test_results_that_overlap_an_input_or_each_other_are_refused():
+    n_px = 64
+    for Cc, N1, N2, shortcut in ((64, 256, 64, False), (64, 256, 128, False), (64, 256, 64, True), (128, 512, 128, False)):
+        w, s, n = _chain(1, (1, 8, 8), Cc, N1, N2, shortcut, wide_t="i8")[:3]
+        at = dict(sum_at=None if shortcut else 9 << 32)
+        for name, row, channels in (("data_at", Cc, Cc), ("short_at", 64, 64) if shortcut else ("sum_at", N1, N1)):
+            a = 10 << 32
+            bytes_in = n_px * row
+            for out, width in (("wide_at", N1), ("narrow_at", N2)):
+                bytes_out = n_px * width
+                for there in (a - bytes_out + 16, a - 16, a + 16, a + bytes_in - 16) + (() if width == channels else (a,)):
+                    assert _refused(w, s, n, **{**at, name: a, out: there}) == H.ERR_UNSUPPORTED, (name, out, there - a)
+        a = 10 << 32
+        for there in (a, a - n_px * N2 + 16, a + n_px * N1 - 16):
+            assert _refused(w, s, n, **{**at, "wide_at": a, "narrow_at": there}) == H.ERR_UNSUPPORTED
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Cc,N1,N2,shortcut,wide_t,pixels", [(64, 256, 64, False, "u8", (3, 2, 16385)), (64, 256, 64, True, "i8", (3, 2, 16385)), (128, 512, 128, False, "i8", (3, 2, 16385)),
+                                                            (64, 256, 128, False, "u8", (3, 2, 4097)), (128, 512, 256, False, "u8", (3, 2, 4097)), (256, 1024, 256, False, "u8", (1, 25, 673))])
+def test_results_in_place_of_inputs_as_wide(gpu_lib, Cc, N1, N2, shortcut, wide_t, pixels):
+    print("[case] chain in place", Cc, N1, N2, shortcut, wide_t, pixels, flush=True)
+    c = _chain(29, pixels, Cc, N1, N2, shortcut, wide_t=wide_t)
+    want = _apart(H.quantized_convolution_fused, *c)
+    for over_data in (True, False):
+        dev = [None if l is None else H.pointwise_layer(l[0], l[1], None if l[2] is None else H._dev(l[2]), H.pack_filter(l[0], H._dev(l[3])), H._dev(l[4]), H._dev(l[5])) for l in c[:3]]
+        res, ss = H._dev(c[3]), H._dev(np.float32(c[4]))
+        wide = H.DeviceBuffer(want[0].size) if shortcut else res
+        stands_on = dev[0].keep[2] if over_data or not shortcut else dev[1].keep[2]
+        narrow = stands_on if N2 == Cc else H.DeviceBuffer(want[1].size)
+        H.check(gpu_lib.hipq_pointwise_chain(*(H._layer_ref(l) for l in dev), H._p(res), ss.ptr, wide.ptr, narrow.ptr, None))
+        H.check(gpu_lib.hipq_stream_sync(None))
+        assert np.array_equal(wide.to_numpy(want[0].dtype, want[0].shape), want[0]) and np.array_equal(narrow.to_numpy(np.uint8, want[1].shape), want[1])
+        if not shortcut:
+            break
