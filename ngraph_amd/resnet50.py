@@ -155,6 +155,27 @@ class HipProvider:
         return H.quantized_dot_bias(d, f, a, w, bias, scales)
 
 
+def _call(fn, args, stream):
+    a = [C.byref(x) if isinstance(x, C.Structure) else (None if x is None else x.ptr) for x in args]
+    rc = fn(*a, stream)
+    if rc:
+        H.check(rc)
+
+
+class _Tensors(dict):
+    """a plan's activations by name; one of `left_out`, which a common launch needs and does not write, is made, on the plan's stream, when
+    it is looked up (it holds no reference to the plan, whose buffers go with it)"""
+
+    def __init__(self, written, left_out, stream):
+        super().__init__(written)
+        self.left_out, self.stream = left_out, stream
+
+    def __missing__(self, name):
+        fn, args = self.left_out[name]
+        _call(fn, args, self.stream)
+        return args[-1]
+
+
 class DevicePlan:
     """The network with every tensor resident in HBM, weights packed once: the f32 images arrive in the
     reference's NCHW order, Quantize writes u8 NCHW, the stem reads that and writes channels-last, and
@@ -244,8 +265,8 @@ class DevicePlan:
                 buf[op["name"]], shape[op["name"]] = out, (op["N"], 1)
                 self.ops_per_image += 2 * op["K"] * op["N"]
         self.logits = buf["logits"]
-        self.buffers = buf
-        self.left_out = {}  # calls whose results only a common launch needs, and which it does not write: made when they are read
+        self.left_out = {}  # calls whose results only a common launch needs, and which it does not write: made when they are looked up
+        self.buffers = _Tensors(buf, self.left_out, stream)
         if fuse_pointwise:
             self._join_pointwise(convs, ops, readers)
 
@@ -268,6 +289,7 @@ class DevicePlan:
                 continue
             if shortcut is not None:
                 self.left_out[wide["sum_src"]] = self.calls[short_at]
+                del self.buffers[wide["sum_src"]]
                 gone.add(short_at)
                 sm = None
             gone.add(wide_at)
@@ -285,15 +307,9 @@ class DevicePlan:
         assert x.nbytes == self.input.nbytes
         H.check(self.lib.hipq_memcpy_h2d(self.input.ptr, x.ctypes.data, x.nbytes, None))
 
-    def _call(self, fn, args):
-        a = [C.byref(x) if isinstance(x, C.Structure) else (None if x is None else x.ptr) for x in args]
-        rc = fn(*a, self.stream)
-        if rc:
-            H.check(rc)
-
     def launch(self):
         for fn, args in self.calls:
-            self._call(fn, args)
+            _call(fn, args, self.stream)
 
     def capture(self):
         """records the pass into a HIP graph (after one eager pass that sizes the library's scratch)"""
@@ -319,7 +335,6 @@ class DevicePlan:
 
     def read(self, name, channels, hw, dtype=np.uint8):
         """a named activation as an NCHW numpy tensor"""
-        if name in self.left_out:
-            self._call(*self.left_out[name])
+        tensor = self.buffers[name]
         H.check(self.lib.hipq_stream_sync(self.stream))
-        return np.ascontiguousarray(np.moveaxis(self.buffers[name].to_numpy(dtype, (self.N, hw, hw, channels)), -1, 1))
+        return np.ascontiguousarray(np.moveaxis(tensor.to_numpy(dtype, (self.N, hw, hw, channels)), -1, 1))

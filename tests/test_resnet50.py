@@ -145,6 +145,38 @@ def test_resnet50_device_plan_and_graph_replay(gpu_lib):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N", [1, 8])
+def test_resnet50_plan_makes_the_tensors_that_common_launches_leave_out(gpu_lib, N):
+    """a projection whose result is never written is made where it is read or looked up, from the last pass, eager or replayed"""
+    lib = gpu_lib
+    sp = C.c_void_p()
+    H.check(lib.hipq_stream_create(C.byref(sp)))
+    plan, apart = R.DevicePlan(lib, sp.value, N), R.DevicePlan(lib, sp.value, N, fuse_pointwise=False)
+    assert plan.left_out and not apart.left_out
+    shapes = {op["name"]: (op["K"], 56) for op in R.layers() if op["name"] in plan.left_out}
+    for seed, run in ((7, "launch"), (8, "launch"), (9, "replay"), (10, "replay")):
+        images = R.synthetic_images(N, seed=seed)
+        for p in (plan, apart):
+            p.set_images_nchw(images)
+            getattr(p, run)()
+        for name, (ch, hw) in shapes.items():
+            print("[case] resnet50 left out", N, seed, name, flush=True)
+            want = apart.read(name, ch, hw, np.int8)
+            assert np.unique(want).size > 16
+            if seed % 2:
+                assert np.array_equal(plan.read(name, ch, hw, np.int8), want)
+            tensor = plan.buffers[name]
+            H.check(lib.hipq_stream_sync(sp.value))
+            assert np.array_equal(np.moveaxis(tensor.to_numpy(np.int8, (N, hw, hw, ch)), -1, 1), want)
+        assert np.array_equal(plan.read_logits(), apart.read_logits())
+    with pytest.raises(KeyError):
+        plan.buffers["no such tensor"]
+    for p in (plan, apart):
+        p.close()
+    H.check(lib.hipq_stream_destroy(sp.value))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("N", [32, 128])
 def test_resnet50_benchmarked_batches_against_oracle(gpu_lib, N):
     """The batches the benchmark times.  Kernel choice depends on the batch (tile shapes, split
