@@ -22,21 +22,23 @@ def _layer(seed, d, f, data, bias=True, scalar=False, gain=1.0):
     return d, f, data, filt, b, s.astype(np.float32)
 
 
-def _chain(seed, pixels, Cc, N1, N2, shortcut=False, data_t="u8", wide_t="u8", bias=True, scalar=False, gain=1.0):
+def _chain(seed, pixels, Cc, N1, N2, shortcut=False, data_t="u8", wide_t="u8", bias=True, scalar=False, gain=1.0, narrow_t="u8", short_t="u8"):
+    """`bias`: of all layers, or of each of widen, shortcut, narrow; `narrow_t`: what the narrow layer reads the wide bytes as"""
     byte = lambda t: (0, 255, np.uint8) if t == "u8" else (-127, 127, np.int8)
     n, h, w = pixels
     count = lambda: 1 if scalar else None
-    fused = lambda K, relu, has_sum=False, sum_t="u8": H.make_fused_desc(has_bias=bias is not None, has_sum=has_sum, sum_t=sum_t, with_relu=relu, scale_count=count() or K)
-    d1, d2 = _conv(pixels, Cc, N1, data_t, wide_t), _conv(pixels, N1, N2, "u8", "u8")
+    bias = bias if isinstance(bias, tuple) else (bias,) * 3
+    fused = lambda K, relu, i, has_sum=False, sum_t="u8": H.make_fused_desc(has_bias=bias[i] is not None, has_sum=has_sum, sum_t=sum_t, with_relu=relu, scale_count=count() or K)
+    d1, d2 = _conv(pixels, Cc, N1, data_t, wide_t), _conv(pixels, N1, N2, narrow_t, "u8")
     x = synth.uniform_int(seed, (n, h, w, Cc), *byte(data_t))
-    widen = _layer(seed + 10, d1, fused(N1, True, True, wide_t), x, bias, scalar, gain)
+    widen = _layer(seed + 10, d1, fused(N1, True, 0, True, wide_t), x, bias[0], scalar, gain)
     short, residual = None, None
     if shortcut:
-        ds = _conv(pixels, 64, N1, "u8", "i8")
-        short = _layer(seed + 20, ds, fused(N1, False), synth.uniform_int(seed + 1, (n, h, w, 64), *byte("u8")), bias, scalar, gain)
+        ds = _conv(pixels, 64, N1, short_t, "i8")
+        short = _layer(seed + 20, ds, fused(N1, False, 1), synth.uniform_int(seed + 1, (n, h, w, 64), *byte(short_t)), bias[1], scalar, gain)
     else:
         residual = synth.uniform_int(seed + 2, (n, h, w, N1), *byte(wide_t))
-    narrow = _layer(seed + 30, d2, fused(N2, True), None, bias, scalar, gain)
+    narrow = _layer(seed + 30, d2, fused(N2, True, 2), None, bias[2], scalar, gain)
     return widen, short, narrow, residual, 0.5
 
 
@@ -48,7 +50,7 @@ def _apart(call, widen, short, narrow, residual, sum_scale):
     d, f, x, filt, b, s = widen
     wide = call(d, f, x, filt, b, residual, s, sum_scale)
     d, f, _, filt, b, s = narrow
-    return wide, call(d, f, wide.view(np.uint8), filt, b, None, s, None)
+    return wide, call(d, f, wide.view(H.NP_OF[d.data_t]), filt, b, None, s, None)
 
 
 def _oracle(d, f, x, filt, b, sum_in, s, sum_scale):
@@ -74,6 +76,35 @@ def test_chain_against_the_oracle(gpu_lib, Cc, N1, N2, shortcut, wide_t, pixels)
         for a, b in zip(got, exp):
             assert np.array_equal(a, b), kw
         assert np.unique(got[0]).size > 2 and np.unique(got[1]).size > 2
+
+
+# what a narrow layer reads, which layers have biases (widening, shortcut, narrow), and the shortcut's data
+MIXED = [dict(narrow_t="i8"), dict(narrow_t="i8", data_t="i8", short_t="i8", scalar=True), dict(short_t="i8"), dict(bias=(True, None, None)), dict(bias=(None, True, None)),
+         dict(bias=(None, None, True)), dict(bias=(True, None, True), narrow_t="i8")]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Cc,N1,N2,shortcut,wide_t", CHAINS + [(256, 1024, 256, False, "u8"), (256, 1024, 256, False, "i8")])
+def test_chain_of_layers_that_differ(gpu_lib, Cc, N1, N2, shortcut, wide_t):
+    """each layer's own type and bias, biases within and beyond 2^24"""
+    pixels = (1, 5, 821) if N1 == 1024 else (1, 8, 261) if N2 == 256 else (2, 9, 7)
+    O.port().orc_set_threads(8)
+    for kw in MIXED:
+        if "short_t" in kw and len(kw) == 1 and not shortcut:
+            continue
+        for large in (False, True):
+            print("[case] chain, layers differ", Cc, N1, N2, shortcut, wide_t, kw, large, flush=True)
+            c = list(_chain(31, pixels, Cc, N1, N2, shortcut, wide_t=wide_t, **kw))
+            if large:
+                for i, l in enumerate(c[:3]):
+                    if l is not None and l[4] is not None:
+                        c[i] = l[:4] + (np.where(np.arange(l[4].size) % 7 == 3, (1 << 24) + 12345, l[4]).astype(np.int32),) + l[5:]
+            got = H.pointwise_chain(*c)
+            assert H.last_kernel().startswith("conv_chain")
+            for a, b in zip(got, _apart(H.quantized_convolution_fused if N1 == 1024 and large else _oracle, *c)):
+                assert np.array_equal(a, b), kw
+                assert np.unique(a).size > 2
+    O.port().orc_set_threads(1)
 
 
 @pytest.mark.gpu
