@@ -728,7 +728,9 @@ def main():
                     row["boundary_over_c_abi"] = row["ms_per_call"] / row["c_abi_ms"]
             backend["gap"] = ("Executable::call replays one captured HIP graph and then waits for the stream (hipStreamSynchronize) before it returns, once per call; the C-ABI loop "
                               "of this process enqueues all its steps and waits once at the end.  The per-call wait and graph launch cost about the same few tens of microseconds at "
-                              "every size: a large part of a 20 us convolution, a few per cent of a ResNet-50 pass.")
+                              "every size: a large part of a 20 us convolution, a few per cent of a ResNet-50 pass.  The C-ABI plan of ResNet-50 also makes pairs of 1 x 1 layers in one "
+                              "launch (hipq_pointwise_chain), which the backend launches one by one: from a batch of 32 on that is most of the ratio (of 128 images 1.18 ms with common "
+                              "launches, 1.34 without).")
         results["backend"] = backend
 
     derived_peak = info.compute_units * info.clock_mhz * 1e6 * 8192 / 1e12

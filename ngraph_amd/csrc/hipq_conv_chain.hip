@@ -376,9 +376,11 @@ namespace hipq
                     lds_dma16_unfenced(w2, at2 + i * 64 * kBlockN1 + blk * 256 + half * 128, __builtin_amdgcn_readfirstlane(ring_at + slot * kBlockSlice + i * 8192 + wave * 1024));
             };
             // The workgroups of a compute die (consecutive ones go to the eight of them in turn) touch a line of the weights a lane, all of
-            // them together: what the ring asks for later is then on its way into their L2, or there.  (ResNet-50, where other layers
-            // have been through it: 128 images 1190 -> 1179 us, 64 781 -> 773, 32 575 -> 569, 26, whose launch is 160 workgroups, 546 -> 541;
-            // 24, with 147, 523 either way, and 22 502 -> 504: the line is at 148)
+            // them together: what the ring asks for later is then on its way into their L2, or there.  ResNet-50, where other layers have
+            // been through it, with the touch over without, both in turn, 29 numbers of images: 0.97 to 0.998 for each with one round of
+            // 148 workgroups or more (30 images 548 -> 530 us, 64 776 -> 770, 128 1190 -> 1183), 1.00 for two rounds.  Below, with 32
+            // pixels a workgroup, mixed: 129 workgroups 1.015, 135 0.988, 141 1.005, 147 0.993.  (With 64 pixels 129 to 147 workgroups gain
+            // 1 %, which the line leaves)
             if (gridDim.x >= 148) // uniform
             {
                 constexpr int parts = 2 * kBlockN1 * kBlockC / (64 * 128); // of 64 lines
@@ -615,8 +617,10 @@ namespace hipq
             return false;
         if (gs)
             return g1.C == 64 && g1.K == 256 && g2.K == 64;
-        // (256 channels of 512 for few pixels: 128 KB of weights are too many for a unit that has one tile, 784 pixels 10.2 us, apart
-        // 8.7; the next stage of ResNet-50 begins with this pair, of three images 2352 pixels: 347 -> 345 us for the pass)
+        // (256 channels of 512 for few pixels: 128 KB of weights are too many for a unit that has one tile.  One launch and two, looped, by
+        // pixels: 512 10.2 and 7.2 us, 1024 10.2 and 7.9, 1536 10.3 and 9.4, 2048 10.4 and 9.7, 2304 10.4 and 10.9, 3072 10.6 and 10.8,
+        // 6272 12.0 and 12.5, 12 544 14.0 and 13.6.  In a pass of ResNet-50, whose next stage begins with this pair: 784 pixels 1.012 times
+        // the two launches' time, 1568 0.996, 2352 and more, up to 12 544, 0.991 to 0.995)
         if (g1.C == 128 && g2.K == 256 && M < 8 * device_compute_units())
             return false;
         if (g1.C == kBlockC && g1.K == kBlockN1 && g2.K == kBlockN2)
